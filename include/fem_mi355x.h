@@ -63,6 +63,9 @@ enum {                                       /* storage form of the matrix    */
   FEM_FORM_DIFFERENCE = 1,    /* diagonal slot holds R_i = sum_j A_ij and the
                                  product is y_i = sum_{j!=i} A_ij (x_j - x_i)
                                  + R_i x_i (exact on translations)            */
+  FEM_FORM_OPERATOR = 3,      /* AMG level 0 only: no matrix; the level's
+                                 sell_vals is a host pointer to a
+                                 fem_patch_operator_t (FP64 products)          */
   FEM_FORM_SCALED_DIFF16 = 2  /* AMG level 0 only: FP16 values of D^-1 A (rows
                                  scaled by the point-Jacobi inverse diagonal)
                                  in difference form                          */
@@ -323,6 +326,57 @@ int fem_export_csr(const fem_pattern_t* pat, int32_t precision, int32_t form, co
 /* y = dR/du(u) x (FP64, matrix-free, BC rows = identity). */
 int fem_operator_apply(const fem_operator_t* op, const double* x, double* y, void* stream);
 
+/* ---- matrix-free products over patches of cells (problem.py:261-296, 426-445)
+ * A patch is a run of fem_patch_cells consecutive cells; the plan (built once
+ * per mesh) lists each patch's distinct nodes ("slots", ascending) with the
+ * (cell in patch, local node) entries that add up to them, and each node's
+ * slots.  Covered: HEX8 cells with the 2x2x2 Gauss rule. */
+typedef struct {
+  int64_t         num_patches;     /* ceil(num_cells / cells_per_patch)         */
+  int64_t         entries;         /* slot_ptr[num_patches]                     */
+  int32_t         cells_per_patch; /* fem_patch_cells(mesh)                     */
+  int32_t         pad;
+  double          val[9];          /* 1-D shape values (point, node), row-major
+                                      with the rule's points per axis squared
+                                      entries (HEX8: 4)                         */
+  double          der[9];          /* 1-D shape derivatives, likewise           */
+  const int32_t*  slot_ptr;        /* (num_patches + 1)                         */
+  const uint16_t* slot_end;        /* (entries) end of the slot's run in the
+                                      patch's part of contrib                   */
+  const uint16_t* contrib;         /* (num_cells*N) cell-in-patch * N + a       */
+  const int32_t*  inc_ptr;         /* (num_nodes + 1) node -> its slots, as
+                                      fem_incidence gives them (N = 1)          */
+  const int32_t*  inc_idx;
+} fem_patch_plan_t;
+
+/* Cells per patch of this mesh's plan; 0: the mesh is not covered. */
+int fem_patch_cells(const fem_mesh_t* mesh);
+/* Plan, pass 1: distinct nodes per patch (counts, to be scanned into slot_ptr). */
+int fem_patch_counts(const fem_mesh_t* mesh, int32_t* counts, void* stream);
+/* Plan, pass 2: slot_node (entries) is the connectivity for the node -> slot
+ * lists (fem_incidence with one node per entity). */
+int fem_patch_fill(const fem_mesh_t* mesh, const int32_t* slot_ptr, int32_t* slot_node, uint16_t* slot_end,
+                   uint16_t* contrib, void* stream);
+
+/* Tangent operator at u: Poisson, elastic, SIMP and Neo-Hookean laws. */
+typedef struct {
+  const fem_mesh_t*       mesh;
+  const fem_material_t*   mat;
+  const fem_patch_plan_t* plan;
+  const double*  u;              /* linearisation point (Neo-Hookean; else NULL) */
+  const uint8_t* bc_mask;        /* NULL, or (num_nodes*vec): 1 on identity rows */
+  const double*  modulus;        /* NULL, or E per point (fem_patch_modulus)    */
+  double*        partials;       /* scratch, (plan->entries * vec)              */
+} fem_patch_operator_t;
+
+/* modulus[c*Q+q] = E(theta) of a SIMP law. */
+int fem_patch_modulus(const fem_mesh_t* mesh, const fem_material_t* mat, double* modulus, void* stream);
+/* y = A x, with y = x on the rows of bc_mask. */
+int fem_patch_apply(const fem_patch_operator_t* op, const double* x, double* y, void* stream);
+/* res = base + internal force at u (base may be NULL); op->u and op->bc_mask are not read. */
+int fem_patch_residual(const fem_patch_operator_t* op, const double* u, const double* base, double* res,
+                       void* stream);
+
 /* ---- single-pass HEX8 assembly (problem.py:447-460 and solver.py:522-526 in
  *      one kernel, optionally with the residual scatter of problem.py:426-437)
  * The cell tangents are formed and summed straight into the SELL values: a
@@ -382,6 +436,13 @@ int fem_pcg_solve(const fem_pattern_t* pat, const void* vals, const void* dinv,
                   const fem_operator_t* op, const double* b, double* x,
                   const fem_pcg_options_t* opt, void* ws, void* host_status,
                   fem_pcg_result_t* result /* host */, void* stream);
+
+/* fem_pcg_solve with matrix-free products (FP64 arithmetic; FEM_F32 keeps FP32
+ * vectors and the FP64 residual replacement): no matrix is read.  dinv is the
+ * inverse diagonal in opt->precision; ws as for fem_pcg_solve. */
+int fem_pcg_solve_patch(const fem_pattern_t* pat, const fem_patch_operator_t* op, const void* dinv, const double* b,
+                        double* x, const fem_pcg_options_t* opt, void* ws, void* host_status,
+                        fem_pcg_result_t* result /* host */, void* stream);
 
 /* Bytes of the library-held device scratch of fem_pcg_solve_noalloc (one
  * array per GPU the library runs on, held until the process ends). */
@@ -459,7 +520,8 @@ typedef struct {
 
 typedef struct {
   const fem_pattern_t* pat;      /* level 0: SELL pattern of the matrix       */
-  const void*    sell_vals;      /* level 0: standard-form SELL values        */
+  const void*    sell_vals;      /* level 0: SELL values in level0_form, or the
+                                    operator (host) of FEM_FORM_OPERATOR      */
   fem_bcsr_t     A;              /* levels >= 1: Galerkin operator            */
   fem_bcsr_t     P;              /* prolongator from the next level           */
   fem_bcsr_t     R;              /* restriction P^T                           */
@@ -479,7 +541,8 @@ typedef struct {
   int32_t        level0_form;    /* form of the level-0 SELL values: FEM_FORM_
                                     STANDARD, FEM_FORM_DIFFERENCE (FP32), or
                                     FEM_FORM_SCALED_DIFF16 (FP16 D^-1 A, with
-                                    the level's dinv; FP32 hierarchy)        */
+                                    the level's dinv; FP32 hierarchy), or
+                                    FEM_FORM_OPERATOR                        */
   const fem_amg_level_t* levels; /* host array [num_levels]                   */
   int64_t        coarse_n;       /* unknowns of the coarsest level            */
   const double*  coarse_inv;     /* (coarse_n x coarse_n) dense inverse       */
@@ -533,7 +596,8 @@ int fem_amg_sell_to_bcsr(const fem_pattern_t* pat, const double* sell_vals, void
 /* Both FP32 copies above (block CSR and difference-form SELL) in one pass over
  * the FP64 SELL values: the level-0 inputs of an FP32 hierarchy.  dinv (n, may
  * be NULL): the inverse diagonal of the block-CSR copy, as fem_amg_dinv forms
- * it (1 / the rounded diagonal entries, 0 for a zero entry). */
+ * it (1 / the rounded diagonal entries, 0 for a zero entry).  diff_vals may be
+ * NULL: no SELL copy. */
 int fem_amg_sell_to_f32_copies(const fem_pattern_t* pat, const double* sell_vals, float* bcsr_vals,
                                float* diff_vals, double* dinv, void* stream);
 /* dinv = 1 / diag(A) (FP64 A); on levels >= 1 (fix_zero = 1) a zero
@@ -543,7 +607,9 @@ int fem_amg_dinv(const fem_bcsr_t* A, int32_t fix_zero, double* dinv, void* stre
  * start vector.  A is the SELL matrix (pat, sell_vals) if pat != NULL --
  * sell_f32 = 0: FP64 standard form, 1: FP32 difference form, 2: FP16 scaled
  * difference form (FEM_FORM_SCALED_DIFF16) -- else the FP64 block CSR matrix
- * A.  ws >= fem_amg_lmax_ws_bytes(unknowns).  Synchronises the stream. */
+ * A.  sell_f32 = 3: sell_vals is a host fem_patch_operator_t (pat is not read
+ * beyond its sizes).  ws >= fem_amg_lmax_ws_bytes(unknowns).  Synchronises the
+ * stream. */
 int64_t fem_amg_lmax_ws_bytes(int64_t n);
 int fem_amg_lmax(const fem_bcsr_t* A, const fem_pattern_t* pat, const void* sell_vals, int32_t sell_f32,
                  const double* dinv,
@@ -607,7 +673,9 @@ int fem_amg_vcycle(const fem_amg_t* amg, const double* r, double* z, void* ws, v
  * x0).  The outer operator is the FP64 standard-form SELL matrix `vals`, or,
  * if vals32 != NULL, the FP32 difference-form copy vals32 with FP64 residual
  * replacement through `vals` (opt->reliable_delta; convergence is decided on
- * the FP64 true residual; result->replacements counts them).  Uses
+ * the FP64 true residual; result->replacements counts them).  A hierarchy of
+ * FEM_FORM_OPERATOR runs the outer products on its operator (vals and vals32
+ * NULL).  Uses
  * ws >= fem_amg_solve_ws_bytes(pat, amg).  Synchronises.  Returns FEM_OK
  * when the solve ran; its outcome (FEM_OK / FEM_ERR_NOT_CONVERGED /
  * FEM_ERR_NAN) is result->status. */

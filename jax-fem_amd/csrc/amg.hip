@@ -15,7 +15,7 @@
 //   solve  CG whose scalars stay on the device; the host reads a status block
 //          every `check_every` iterations
 // No floating-point atomics: every result is bit-reproducible run to run.
-#include "fem_common.hpp"
+#include "patch.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -27,6 +27,7 @@ namespace {
 
 constexpr int kXCap = 1024;     // max blocks in one row of the left SpGEMM operand (sorted-pair kernel)
 constexpr int kDotBlocks = 1024;
+static_assert(kPatchDotBlocks <= kDotBlocks, "the partials of a matrix-free <p, A p> fit the same buffer");
 constexpr double kRankTol = 1e-10;
 
 // ------------------------------------------------------------- priorities
@@ -274,7 +275,7 @@ __global__ void k_bc_mask_set(int64_t n_bc, const int32_t* __restrict__ dofs, ui
 // One block per slice: KC slots of the slice's 64 rows are read coalesced into
 // LDS, then each row's KC*V*V entries (contiguous in the block CSR) are stored
 // as one contiguous run, so the stores fill whole cache lines.  DIFF: the same
-// pass also writes the FP32 difference-form SELL copy (dout): off-diagonal
+// pass also writes the FP32 difference-form SELL copy (dout, may be NULL): off-diagonal
 // entries rounded as they are read, and each row's FP64 row sums (summed over
 // the slots in slot order by the thread that owns the (row, entry) pair)
 // rounded once into the diagonal slot; with dinv, also 1 / the rounded diagonal
@@ -298,7 +299,7 @@ __global__ __launch_bounds__(256) void k_sell_to_bcsr(fem_pattern_t pat, const d
     s_ds[threadIdx.x] = row >= 0 ? pat.diag_slot[row] : -1;
   }
   const double* src = sv + (size_t)base * VV;
-  float* dst = DIFF ? dout + (size_t)base * VV : nullptr;
+  float* dst = DIFF && dout ? dout + (size_t)base * VV : nullptr;
   double rs[NOWN], dg[NOWN];  // row sums; diagonal entries (of the owned pairs on the block diagonal)
 #pragma unroll
   for (int o = 0; o < NOWN; ++o) rs[o] = dg[o] = 0.0;
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(256) void k_sell_to_bcsr(fem_pattern_t pat, const d
       const size_t at = ((size_t)k0 * VV + c) * kSlice + lane;
       const double x = src[at];
       tile[lane][c] = x;
-      if (DIFF && k0 + c / VV != s_ds[lane]) dst[at] = float(x);
+      if (DIFF && dst && k0 + c / VV != s_ds[lane]) dst[at] = float(x);
     }
     __syncthreads();
     for (int f = threadIdx.x; f < nc * kSlice; f += 256) {
@@ -336,7 +337,7 @@ __global__ __launch_bounds__(256) void k_sell_to_bcsr(fem_pattern_t pat, const d
       const int p = threadIdx.x + 256 * o;
       if (p < kSlice * VV) {
         const int lane = p & (kSlice - 1), v = p >> 6;
-        if (s_ds[lane] >= 0) dst[((size_t)s_ds[lane] * VV + v) * kSlice + lane] = float(rs[o]);
+        if (dst && s_ds[lane] >= 0) dst[((size_t)s_ds[lane] * VV + v) * kSlice + lane] = float(rs[o]);
         if (dinv && v % (V + 1) == 0 && s_row[lane] >= 0) {
           const double d = double(TO(dg[o]));
           dinv[(int64_t)s_row[lane] * V + v / (V + 1)] = d != 0.0 ? 1.0 / d : 0.0;
@@ -1394,66 +1395,6 @@ __global__ __launch_bounds__(256) void k_dense_gemv(int64_t n, const double* __r
   if (lane == 0) y[i] = s;
 }
 
-// ---------------------------------------------------------- operator apply
-enum { AP_STORE = 0, AP_ADD = 1, AP_RESID = 2, AP_CHEB = 3, AP_DSTORE = 4, AP_PQ = 5 };
-
-// TX: storage of the input vector and of the Chebyshev direction, TY: of the
-// output.  Arithmetic is FP64 whatever the storage; the V-cycle's vectors are
-// FP64, the level-0 power iteration on the FP32 copy keeps FP32 iterates.
-template <typename TX = double, typename TY = double>
-struct ApplyArgsT {
-  const TX* x;         // gathered input
-  TY* y;               // output (CHEB: the new iterate)
-  const double* rhs;   // RESID, CHEB
-  const double* dinv;  // CHEB, DSTORE
-  TX* d;               // CHEB: search direction (in/out)
-  double c1, c2;       // CHEB: d = c1 d + c2 D^-1 (rhs - A x), y = x + d
-  double* part;        // PQ: per-block partials of <x, A x>
-  const int32_t* done; // NULL, or a flag: the kernel returns at once when it is set
-                       // (V-cycles queued after the outer CG converged)
-};
-using ApplyArgs = ApplyArgsT<double, double>;
-
-// The epilogue's own-entry operands (loaded ahead of the product where a kernel can
-// overlap their latency with it) and the epilogue itself.
-struct EpiOperands {
-  double y, rhs, dinv, d, x;
-};
-
-template <int MODE, typename TX, typename TY>
-__device__ inline EpiOperands epilogue_load(const ApplyArgsT<TX, TY>& a, int64_t idx) {
-  EpiOperands e{0.0, 0.0, 0.0, 0.0, 0.0};
-  if (MODE == AP_ADD) e.y = double(a.y[idx]);
-  if (MODE == AP_RESID || MODE == AP_CHEB) e.rhs = a.rhs[idx];
-  if (MODE == AP_CHEB || MODE == AP_DSTORE) e.dinv = a.dinv[idx];
-  if (MODE == AP_CHEB && a.c1 != 0.0) e.d = double(a.d[idx]);
-  if (MODE == AP_CHEB) e.x = double(a.x[idx]);
-  return e;
-}
-
-template <int MODE, typename TX, typename TY>
-__device__ inline void epilogue_store(const ApplyArgsT<TX, TY>& a, int64_t idx, double ax, const EpiOperands& e) {
-  if (MODE == AP_STORE || MODE == AP_PQ) {
-    a.y[idx] = TY(ax);
-  } else if (MODE == AP_ADD) {
-    a.y[idx] = TY(e.y + ax);
-  } else if (MODE == AP_RESID) {
-    a.y[idx] = TY(e.rhs - ax);
-  } else if (MODE == AP_DSTORE) {
-    a.y[idx] = TY(e.dinv * ax);
-  } else {
-    const double r = e.dinv * (e.rhs - ax);
-    const double dn = a.c1 != 0.0 ? fma(a.c1, e.d, a.c2 * r) : a.c2 * r;
-    a.d[idx] = TX(dn);
-    a.y[idx] = TY(e.x + dn);
-  }
-}
-
-template <int MODE, typename TX, typename TY>
-__device__ inline void apply_epilogue(const ApplyArgsT<TX, TY>& a, int64_t idx, double ax) {
-  epilogue_store<MODE>(a, idx, ax, epilogue_load<MODE>(a, idx));
-}
-
 // Block CSR operator, G lanes per block row: the lanes stride over the row's
 // (block, column) pairs and accumulate every block row entry.
 template <int BR, int BC, int G, int MODE, typename T, typename TX = double, typename TY = double>
@@ -1994,10 +1935,21 @@ struct Cheb {
   }
 };
 
+// The matrix-free operator of level 0 (FEM_FORM_OPERATOR), or NULL.
+const fem_patch_operator_t* level0_operator(const fem_amg_t& amg) {
+  return amg.num_levels > 0 && amg.level0_form == FEM_FORM_OPERATOR
+             ? static_cast<const fem_patch_operator_t*>(amg.levels[0].sell_vals)
+             : nullptr;
+}
+
 template <typename T, typename TX = double, typename TY = double>
 int level_apply(const fem_amg_t& amg, int l, int mode, const ApplyArgsT<TX, TY>& a, hipStream_t s) {
   const fem_amg_level_t& L = amg.levels[l];
   if (l == 0) {
+    if (const fem_patch_operator_t* op = level0_operator(amg)) {
+      if (mode == AP_CHEB) return patch_apply<AP_CHEB, TX, TY>(*op, a, s);
+      return patch_apply<AP_RESID, TX, TY>(*op, a, s);
+    }
     if (amg.level0_form == FEM_FORM_SCALED_DIFF16) {
       ApplyArgsT<TX, TY> b = a;
       b.dinv = L.dinv;   // the residual undoes the row scaling
@@ -2154,13 +2106,16 @@ int check_amg(const fem_amg_t* amg) {
                 "AMG hierarchy descriptor incomplete");
   FEM_CHECK_ARG(amg->precision == FEM_F32 || amg->precision == FEM_F64, "AMG precision must be FEM_F32 or FEM_F64");
   FEM_CHECK_ARG(amg->degree >= 1 && amg->degree <= 8, "AMG Chebyshev degree must be in [1, 8]");
-  FEM_CHECK_ARG(amg->level0_form == FEM_FORM_STANDARD ||
+  FEM_CHECK_ARG(amg->level0_form == FEM_FORM_STANDARD || amg->level0_form == FEM_FORM_OPERATOR ||
                     ((amg->level0_form == FEM_FORM_DIFFERENCE || amg->level0_form == FEM_FORM_SCALED_DIFF16) &&
                      amg->precision == FEM_F32),
                 "AMG level 0: the difference form is an FP32 storage form");
   if (amg->num_levels == 0) return FEM_OK;   // the dense coarse inverse is the whole preconditioner
   const fem_amg_level_t& L0 = amg->levels[0];
   FEM_CHECK_ARG(L0.pat && L0.sell_vals && L0.dinv, "AMG level 0 needs the SELL pattern, values and dinv");
+  if (const fem_patch_operator_t* op = level0_operator(*amg))
+    FEM_CHECK_ARG(patch_operator_ok(op) && op->mesh->num_nodes == L0.pat->num_rows && op->mesh->vec == L0.pat->vec,
+                  "AMG level 0: the matrix-free operator is incomplete, not covered or of another size");
   for (int l = 0; l < amg->num_levels; ++l) {
     const fem_amg_level_t& L = amg->levels[l];
     FEM_CHECK_ARG(L.dinv && L.P.vals && L.R.vals && L.lmax > 0.0, "AMG level %d incomplete", l);
@@ -2382,7 +2337,7 @@ int fem_amg_sell_to_bcsr(const fem_pattern_t* pat, const double* sell_vals, void
 
 int fem_amg_sell_to_f32_copies(const fem_pattern_t* pat, const double* sell_vals, float* bcsr_vals, float* diff_vals,
                                double* dinv, void* stream) {
-  FEM_CHECK_ARG(pat && sell_vals && bcsr_vals && diff_vals, "fem_amg_sell_to_f32_copies: NULL argument");
+  FEM_CHECK_ARG(pat && sell_vals && bcsr_vals, "fem_amg_sell_to_f32_copies: NULL argument");
   hipStream_t s = as_stream(stream);
   if (pat->num_rows == 0) return FEM_OK;
   FEM_CHECK_ARG(pat->num_slices == ceil_div(pat->num_rows, kSlice), "fem_amg_sell_to_f32_copies: num_slices mismatch");
@@ -2486,6 +2441,11 @@ int fem_amg_lmax_async(const fem_bcsr_t* A, const fem_pattern_t* pat, const void
   FEM_CHECK_ARG(dinv && lmax_dev && ws && steps >= 1, "fem_amg_lmax: bad arguments");
   FEM_CHECK_ARG(pat ? (sell_vals != nullptr && pat->num_rows > 0) : (A && A->br == A->bc && A->rows > 0),
                 "fem_amg_lmax: give a SELL matrix (pat, sell_vals) or a square block CSR matrix");
+  if (pat && sell_f32 == 3) {
+    const fem_patch_operator_t* op = static_cast<const fem_patch_operator_t*>(sell_vals);
+    FEM_CHECK_ARG(patch_operator_ok(op) && op->mesh->num_nodes == pat->num_rows && op->mesh->vec == pat->vec,
+                  "fem_amg_lmax: the matrix-free operator is incomplete, not covered or of another size");
+  }
   hipStream_t s = as_stream(stream);
   const int64_t n = pat ? pat->num_rows * pat->vec : A->rows * A->br;
   char* w = static_cast<char*>(ws);
@@ -2525,7 +2485,9 @@ int fem_amg_lmax_async(const fem_bcsr_t* A, const fem_pattern_t* pat, const void
       if constexpr (sizeof(TV) == 4) {
         rc = sell_apply<AP_DSTORE, float, true>(*pat, static_cast<const float*>(sell_vals), a, nullptr, s);
       } else {
-        rc = !pat ? (A->f32 ? bcsr_apply<AP_DSTORE, float>(*A, a, s) : bcsr_apply<AP_DSTORE, double>(*A, a, s))
+        rc = sell_f32 == 3 ? patch_apply<AP_DSTORE, double, double>(
+                                 *static_cast<const fem_patch_operator_t*>(sell_vals), a, s)
+             : !pat ? (A->f32 ? bcsr_apply<AP_DSTORE, float>(*A, a, s) : bcsr_apply<AP_DSTORE, double>(*A, a, s))
              : sell_f32 == 2 ? sell_apply<AP_DSTORE, _Float16, true>(*pat, sell_vals, a, nullptr, s)
                              : sell_apply<AP_DSTORE, double>(*pat, static_cast<const double*>(sell_vals), a, nullptr, s);
       }
@@ -2849,8 +2811,11 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
                       const double* b, double* x, const fem_amg_options_t* opt, void* ws, void* host_status,
                       fem_pcg_result_t* result, void* stream) {
   if (int rc = check_amg(amg)) return rc;
-  FEM_CHECK_ARG(pat && vals && b && x && opt && ws && host_status && result, "fem_amg_pcg_solve: NULL argument");
+  const fem_patch_operator_t* pop = level0_operator(*amg);
+  FEM_CHECK_ARG(pat && (vals || pop) && b && x && opt && ws && host_status && result,
+                "fem_amg_pcg_solve: NULL argument");
   const bool outer32 = vals32 != nullptr;
+  FEM_CHECK_ARG(!outer32 || !pop, "fem_amg_pcg_solve: an FP32 outer operator needs a matrix hierarchy");
   FEM_CHECK_ARG(!outer32 || (opt->reliable_delta > 0.0 && opt->reliable_delta < 1.0),
                 "fem_amg_pcg_solve: reliable_delta must be in (0, 1) with an FP32 outer operator");
   FEM_CHECK_ARG(amg->num_levels == 0 ? amg->coarse_n == pat->num_rows * pat->vec
@@ -2879,7 +2844,9 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
   // r = b - A x with the FP64 matrix, sc->rr = |r|^2
   auto true_residual = [&]() -> int {
     ApplyArgs ar{x, r, b, nullptr, nullptr, 0.0, 0.0, nullptr};
-    if (int rc = sell_apply<AP_RESID, double>(*pat, vals, ar, nullptr, s)) return rc;
+    if (int rc = pop ? patch_apply<AP_RESID, double, double>(*pop, ar, s)
+                     : sell_apply<AP_RESID, double>(*pat, vals, ar, nullptr, s))
+      return rc;
     hipLaunchKernelGGL(k_dot_part, dim3(kDotBlocks), dim3(256), 0, s, n, r, r, part, (const int32_t*)nullptr);
     hipLaunchKernelGGL(k_finish, dim3(1), dim3(256), 0, s, part, kDotBlocks, &sc->rr);
     FEM_LAUNCHED();
@@ -2924,11 +2891,13 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
     hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(256), 0, s, part, kDotBlocks, sc);
     hipLaunchKernelGGL(k_cg_p, dim3(g), dim3(256), 0, s, n, z, p, sc);
     FEM_LAUNCHED();
-    ApplyArgs apq{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, part};
-    if (int rc = outer32 ? sell_apply<AP_PQ, float, true>(*pat, vals32, apq, done, s)
-                         : sell_apply<AP_PQ, double>(*pat, vals, apq, done, s))
+    ApplyArgs apq{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, part, done};
+    int np = (int)pat->num_slices;
+    if (int rc = pop       ? patch_apply<AP_PQ, double, double>(*pop, apq, s, &np)
+                 : outer32 ? sell_apply<AP_PQ, float, true>(*pat, vals32, apq, done, s)
+                           : sell_apply<AP_PQ, double>(*pat, vals, apq, done, s))
       return rc;
-    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, s, part, (int)pat->num_slices, sc);
+    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, s, part, np, sc);
     hipLaunchKernelGGL(k_cg_xr, dim3(kDotBlocks), dim3(256), 0, s, n, p, q, x, r, part, sc);
     hipLaunchKernelGGL(k_cg_rr, dim3(1), dim3(256), 0, s, part, kDotBlocks, sc);
     FEM_LAUNCHED();
@@ -2968,7 +2937,9 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
   }
   // true residual
   ApplyArgs af{x, q, b, nullptr, nullptr, 0.0, 0.0, nullptr};
-  if (int rc = sell_apply<AP_RESID, double>(*pat, vals, af, nullptr, s)) return rc;
+  if (int rc = pop ? patch_apply<AP_RESID, double, double>(*pop, af, s)
+                   : sell_apply<AP_RESID, double>(*pat, vals, af, nullptr, s))
+    return rc;
   hipLaunchKernelGGL(k_dot_part, dim3(kDotBlocks), dim3(256), 0, s, n, q, q, part, (const int32_t*)nullptr);
   hipLaunchKernelGGL(k_finish, dim3(1), dim3(256), 0, s, part, kDotBlocks, &sc->rz);
   FEM_LAUNCHED();

@@ -1,0 +1,19 @@
+// Matrix-free element products over patches of consecutive cells (patch.hip):
+// the entry points the solvers call.
+#pragma once
+#include "apply.hpp"
+
+namespace fem {
+
+constexpr int kPatchDotBlocks = 1024;  // most <x, A x> partials of an AP_PQ product
+
+// True when `op` describes an element, rule and law the patch kernels run.
+bool patch_operator_ok(const fem_patch_operator_t* op);
+
+// y = epilogue(A x), A the tangent at op->u with identity rows on op->bc_mask; *parts
+// receives the number of partials an AP_PQ product writes to a.part.  TX / TY: FP64, or
+// FP32 vectors (the arithmetic is FP64).
+template <int MODE, typename TX, typename TY>
+int patch_apply(const fem_patch_operator_t& op, const ApplyArgsT<TX, TY>& a, hipStream_t s, int* parts = nullptr);
+
+}  // namespace fem

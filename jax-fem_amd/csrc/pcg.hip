@@ -27,7 +27,7 @@
 // (A applied matrix-free in FP64) each time it has dropped by reliable_delta
 // and at convergence; beta keeps the value of the recursion across a
 // replacement.
-#include "fem_common.hpp"
+#include "patch.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -332,7 +332,7 @@ static int64_t ws_layout(const fem_pattern_t* pat, int precision, void* base, Ws
   o->q = take(n * es);
   o->ones = take(n * es);
   o->y = reinterpret_cast<double*>(take(n * 8));
-  o->partA = reinterpret_cast<double*>(take(grid_a(pat) * 8));
+  o->partA = reinterpret_cast<double*>(take(std::max<int64_t>(grid_a(pat), kPatchDotBlocks) * 8));
   o->partB = reinterpret_cast<double*>(take(2 * kVecGrid * 8));
   o->partR = reinterpret_cast<double*>(take(2 * kVecGrid * 8));
   o->partT = reinterpret_cast<double*>(take(kVecGrid * 8));
@@ -340,9 +340,10 @@ static int64_t ws_layout(const fem_pattern_t* pat, int precision, void* base, Ws
   return off;
 }
 
+// pop != NULL: the products run matrix-free on it (vals and op are not read).
 template <int V, typename T>
 static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, const fem_operator_t* op,
-                   const double* b, double* x, const fem_pcg_options_t* opt, void* ws_base,
+                   const fem_patch_operator_t* pop, const double* b, double* x, const fem_pcg_options_t* opt, void* ws_base,
                    PcgScalars* host_sc, fem_pcg_result_t* res, hipStream_t s) {
   constexpr bool kMixed = std::is_same<T, float>::value;
   constexpr bool kDiff = kMixed;  // the FP32 matrix is stored in difference form
@@ -359,7 +360,7 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
     FEM_LAUNCHED();
     dinv = (T*)w.ones;
   }
-  const int gA = (int)grid_a(pat);
+  int gA = (int)grid_a(pat);  // partials of <p, q>
   const int gV = (int)std::min<int64_t>(ceil_div(n, 256), kVecGrid);
   FEM_HIP(hipMemsetAsync(w.sc, 0, sizeof(PcgScalars), s));
   hipLaunchKernelGGL(k_fill<T>, dim3(256), dim3(256), 0, s, n, p, T(0));
@@ -378,7 +379,10 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
     return read_status();
   };
   auto true_residual = [&]() -> int {
-    if (kMixed) {
+    if (pop) {
+      ApplyArgs a{x, w.y, nullptr, nullptr, nullptr, 0.0, 0.0, nullptr, nullptr};
+      if (int rc = patch_apply<AP_STORE, double, double>(*pop, a, s)) return rc;
+    } else if (kMixed) {
       if (int rc = fem_operator_apply_impl(op, x, w.y, s)) return rc;
     } else {
       hipLaunchKernelGGL((k_spmv_x<V, T>), dim3((unsigned)ceil_div(pat->num_rows, 256)), dim3(256), 0, s, *pat, vals,
@@ -430,8 +434,13 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m], s));
       hipLaunchKernelGGL(k_pcg_p<T>, dim3(gV), dim3(256), 0, s, n, (const T*)z, p, (const PcgScalars*)w.sc);
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 1], s));
-      hipLaunchKernelGGL((k_pcg_a<V, kDiff, T>), dim3(gA), dim3(SliceCfg<T>::NT), 0, s, *pat, vals, (const T*)p, q,
-                         (const PcgScalars*)w.sc, w.partA, opt->xcd_remap);
+      if (pop) {
+        ApplyArgsT<T, T> a{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, w.partA, &w.sc->done};
+        if (int rc = patch_apply<AP_PQ, T, T>(*pop, a, s, &gA)) return rc;
+      } else {
+        hipLaunchKernelGGL((k_pcg_a<V, kDiff, T>), dim3(gA), dim3(SliceCfg<T>::NT), 0, s, *pat, vals, (const T*)p, q,
+                           (const PcgScalars*)w.sc, w.partA, opt->xcd_remap);
+      }
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 2], s));
       hipLaunchKernelGGL(k_pcg_ra, dim3(1), dim3(1024), 0, s, (const double*)w.partA, gA, w.sc);
       hipLaunchKernelGGL((k_pcg_b<T, double>), dim3(gV), dim3(256), 0, s, n, x, r, z, (const T*)p, (const T*)q, dinv,
@@ -536,6 +545,28 @@ int64_t fem_pcg_ws_bytes(const fem_pattern_t* pat, int32_t precision) {
   return ws_layout(pat, precision, nullptr, nullptr) + 256;
 }
 
+static int pcg_dispatch(const fem_pattern_t* pat, const void* vals, const void* dinv, const fem_operator_t* op,
+                        const fem_patch_operator_t* pop, const double* b, double* x, const fem_pcg_options_t* opt,
+                        void* ws, void* host_status, fem_pcg_result_t* result, void* stream) {
+  hipStream_t s = as_stream(stream);
+  PcgScalars* hsc = reinterpret_cast<PcgScalars*>(host_status);
+  auto run = [&](auto vc) -> int {
+    constexpr int V = decltype(vc)::value;
+    if (opt->precision == FEM_F32)
+      return pcg_run<V, float>(pat, (const float*)vals, (const float*)dinv, op, pop, b, x, opt, ws, hsc, result, s);
+    return pcg_run<V, double>(pat, (const double*)vals, (const double*)dinv, op, pop, b, x, opt, ws, hsc, result, s);
+  };
+  switch (pat->vec) {
+    case 1: return run(std::integral_constant<int, 1>{});
+    case 2: return run(std::integral_constant<int, 2>{});
+    case 3: return run(std::integral_constant<int, 3>{});
+    case 4: return run(std::integral_constant<int, 4>{});
+    default: break;
+  }
+  set_error("fem_pcg_solve: unsupported vec %d", pat->vec);
+  return FEM_ERR_BAD_ARG;
+}
+
 int fem_pcg_solve(const fem_pattern_t* pat, const void* vals, const void* dinv, const fem_operator_t* op,
                   const double* b, double* x, const fem_pcg_options_t* opt, void* ws, void* host_status,
                   fem_pcg_result_t* result, void* stream) {
@@ -546,27 +577,21 @@ int fem_pcg_solve(const fem_pattern_t* pat, const void* vals, const void* dinv, 
   FEM_CHECK_ARG(opt->precision == FEM_F64 || op, "fem_pcg_solve: FP32 mode needs the FP64 operator");
   FEM_CHECK_ARG(opt->maxiter > 0 && opt->rtol >= 0 && opt->atol >= 0, "fem_pcg_solve: bad tolerances");
   FEM_CHECK_ARG(!opt->precond || dinv, "fem_pcg_solve: Jacobi requested without dinv");
-  hipStream_t s = as_stream(stream);
-  PcgScalars* hsc = reinterpret_cast<PcgScalars*>(host_status);
-  const int V = pat->vec;
-  if (V == 1 && opt->precision == FEM_F32)
-    return pcg_run<1, float>(pat, (const float*)vals, (const float*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 1 && opt->precision == FEM_F64)
-    return pcg_run<1, double>(pat, (const double*)vals, (const double*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 3 && opt->precision == FEM_F32)
-    return pcg_run<3, float>(pat, (const float*)vals, (const float*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 3 && opt->precision == FEM_F64)
-    return pcg_run<3, double>(pat, (const double*)vals, (const double*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 2 && opt->precision == FEM_F32)
-    return pcg_run<2, float>(pat, (const float*)vals, (const float*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 2 && opt->precision == FEM_F64)
-    return pcg_run<2, double>(pat, (const double*)vals, (const double*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 4 && opt->precision == FEM_F32)
-    return pcg_run<4, float>(pat, (const float*)vals, (const float*)dinv, op, b, x, opt, ws, hsc, result, s);
-  if (V == 4 && opt->precision == FEM_F64)
-    return pcg_run<4, double>(pat, (const double*)vals, (const double*)dinv, op, b, x, opt, ws, hsc, result, s);
-  set_error("fem_pcg_solve: unsupported vec %d", V);
-  return FEM_ERR_BAD_ARG;
+  return pcg_dispatch(pat, vals, dinv, op, nullptr, b, x, opt, ws, host_status, result, stream);
+}
+
+int fem_pcg_solve_patch(const fem_pattern_t* pat, const fem_patch_operator_t* op, const void* dinv, const double* b,
+                        double* x, const fem_pcg_options_t* opt, void* ws, void* host_status,
+                        fem_pcg_result_t* result, void* stream) {
+  FEM_CHECK_ARG(pat && pat->num_rows > 0 && b && x && opt && ws && host_status && result,
+                "fem_pcg_solve_patch: NULL argument");
+  FEM_CHECK_ARG(patch_operator_ok(op), "fem_pcg_solve_patch: the operator is incomplete or not covered");
+  FEM_CHECK_ARG(op->mesh->num_nodes == pat->num_rows && op->mesh->vec == pat->vec,
+                "fem_pcg_solve_patch: operator and pattern disagree");
+  FEM_CHECK_ARG(opt->precision == FEM_F32 || opt->precision == FEM_F64, "fem_pcg_solve_patch: bad precision");
+  FEM_CHECK_ARG(opt->maxiter > 0 && opt->rtol >= 0 && opt->atol >= 0, "fem_pcg_solve_patch: bad tolerances");
+  FEM_CHECK_ARG(!opt->precond || dinv, "fem_pcg_solve_patch: Jacobi requested without dinv");
+  return pcg_dispatch(pat, nullptr, dinv, nullptr, op, b, x, opt, ws, host_status, result, stream);
 }
 
 int fem_pcg_solve_noalloc(const fem_pattern_t* pat, const void* vals, const void* dinv, const fem_operator_t* op,

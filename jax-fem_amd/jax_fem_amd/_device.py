@@ -5,6 +5,7 @@ allocates device memory, supplies the stream and evaluates the user's own
 mass/surface callbacks at quadrature points.
 """
 import ctypes as C
+import functools
 import time
 import logging
 
@@ -14,6 +15,7 @@ from torch.func import vmap
 
 from . import _lib
 from ._lib import check, ptr, stream_ptr
+from .basis import _lagrange_1d, gauss_legendre_01, get_elements, get_shape_vals_and_grads
 from .materials import identify
 
 logger = logging.getLogger('jax_fem_amd')
@@ -25,6 +27,24 @@ def _i32(x, device):
 
 def _f64(x, device):
     return torch.as_tensor(onp.ascontiguousarray(onp.asarray(x, dtype=onp.float64)), device=device)
+
+
+@functools.lru_cache(maxsize=None)
+def _gauss_tables(ele_type, npts):
+    """The element's tables at the npts^3 Gauss rule and the 1-D (values, derivatives) they are products of."""
+    val, der = _lagrange_1d(get_elements(ele_type)[0], gauss_legendre_01(npts)[0])
+    return get_shape_vals_and_grads(ele_type, None, 2 * npts - 2), (val, der)
+
+
+def tensor_rule(fe):
+    """(values, derivatives) of the 1-D shape functions at the 1-D points when the element's tables
+    are the tensor product of them over its Gauss rule; None otherwise."""
+    npts = round(fe.num_quads ** (1. / 3.))
+    if npts ** 3 != fe.num_quads:
+        return None
+    ref, rule = _gauss_tables(fe.ele_type, npts)
+    same = all(onp.array_equal(a, b) for a, b in zip(ref, (fe.shape_vals, fe.shape_grads_ref, fe.quad_weights)))
+    return rule if same else None
 
 
 class DeviceMesh:
@@ -57,6 +77,8 @@ class DeviceMesh:
             setattr(m, name, getattr(self, name).data_ptr())
         self.desc = m
         self.ref = C.byref(m)
+        self.tensor_rule = tensor_rule(fe)
+        self._patch = None
 
     def empty(self, *shape, dtype=torch.float64):
         return torch.empty(shape, dtype=dtype, device=self.device)
@@ -92,6 +114,34 @@ class DeviceMesh:
         check(self.L.fem_incidence(E, N, ptr(conn), self.Nn, ptr(inc_ptr), ptr(inc_idx), ptr(ws), stream_ptr()),
               'fem_incidence')
         return inc_ptr, inc_idx
+
+    def patch_plan(self):
+        """Plan of the matrix-free patch products (csrc/patch.hip), built once per mesh; None where
+        they do not apply (HEX8 cells with the 2x2x2 Gauss rule only)."""
+        if self._patch is None:
+            self._patch = False
+            cpp = int(self.L.fem_patch_cells(self.ref)) if self.C > 0 else 0
+            if cpp > 0 and self.tensor_rule:
+                np_ = (self.C + cpp - 1) // cpp
+                counts = self.empty(np_, dtype=torch.int32)
+                check(self.L.fem_patch_counts(self.ref, ptr(counts), stream_ptr()), 'fem_patch_counts')
+                slot_ptr = self.scan(counts)
+                entries = int(slot_ptr[-1].item())
+                slot_node = self.empty(entries, dtype=torch.int32)
+                slot_end = self.empty(entries, dtype=torch.int16)
+                contrib = self.empty(self.C * self.N, dtype=torch.int16)
+                check(self.L.fem_patch_fill(self.ref, ptr(slot_ptr), ptr(slot_node), ptr(slot_end), ptr(contrib),
+                                            stream_ptr()), 'fem_patch_fill')
+                inc_ptr, inc_idx = self.incidence(slot_node.reshape(-1, 1))
+                p = _lib.FemPatchPlan()
+                p.num_patches, p.entries, p.cells_per_patch = np_, entries, cpp
+                for i, (v, d) in enumerate(zip(*(t.reshape(-1) for t in self.tensor_rule))):
+                    p.val[i], p.der[i] = v, d
+                keep = dict(slot_ptr=slot_ptr, slot_end=slot_end, contrib=contrib, inc_ptr=inc_ptr, inc_idx=inc_idx)
+                for k, t in keep.items():
+                    setattr(p, k, t.data_ptr())
+                self._patch = (p, keep)
+        return self._patch[0] if self._patch else None
 
     def scan(self, x):
         n = x.numel()
@@ -198,6 +248,7 @@ class DeviceProblem:
         self.cperm_inv = onp.argsort(self.cperm)
         self.inc_ptr, self.inc_idx = dm.incidence(dm.cells)
         self._build_pattern()
+        self.patch_plan = dm.patch_plan()
         self.surfaces = []
         for bi in problem.boundary_inds_list:
             faces = dm.faces_tensor(bi)
@@ -221,6 +272,7 @@ class DeviceProblem:
         self._amg_uses = 0
         self._asm_plan = None
         self.last_residual = None
+        self.fine = None
 
     # ------------------------------------------------------------ pattern
     def _build_pattern(self):
@@ -302,6 +354,8 @@ class DeviceProblem:
         self.bc_vals = _f64(v, self.dm.device)
         self.bc_dofs_long = self.bc_dofs.long()
         self.n_bc = int(d.shape[0])
+        self.bc_mask = torch.zeros(self.n, dtype=torch.uint8, device=self.dm.device)
+        self.bc_mask[self.bc_dofs_long] = 1
         self._bc_sources = sources
 
     def prepare(self):
@@ -746,10 +800,36 @@ class DeviceProblem:
         self._mat_cache[lc['key']] = Tabulated(lc['fn'], self.V)
         self.prepare()
 
+    _PATCH_KINDS = (_lib.FEM_MAT_POISSON, _lib.FEM_MAT_LINEAR_ELASTIC, _lib.FEM_MAT_SIMP, _lib.FEM_MAT_NEO_HOOKEAN)
+
+    @property
+    def patch_law(self):
+        """True when the cells' integrals are a closed-form law the patch kernels run."""
+        return self.patch_plan is not None and not self.cell_terms and self.material.kind in self._PATCH_KINDS
+
+    def patch_operator(self, mat_desc, u=None, modulus=None):
+        """Descriptor of the matrix-free tangent at u (fem_patch_operator_t); u is needed by the
+        hyperelastic law only."""
+        dm = self.dm
+        if 'patch_part' not in self.buffers:
+            self.buffers['patch_part'] = dm.empty(self.patch_plan.entries * self.V)
+        op = _lib.FemPatchOperator()
+        op.mesh, op.mat, op.plan = C.pointer(dm.desc), C.pointer(mat_desc), C.pointer(self.patch_plan)
+        op.u = u.data_ptr() if u is not None else None
+        op.bc_mask = self.bc_mask.data_ptr() if self.n_bc else None
+        op.modulus = modulus.data_ptr() if modulus is not None else None
+        op.partials = self.buffers['patch_part'].data_ptr()
+        return op
+
     def residual_unconstrained(self, u):
         """R(u) without Dirichlet rows, FP64 (problem.py:439-445)."""
         dm = self.dm
         self._check_law(u)
+        if self.patch_law:
+            base, res = self._base_load(u), dm.empty(self.n)
+            check(self.L.fem_patch_residual(C.byref(self.patch_operator(self.mat_desc)), ptr(u), ptr(base), ptr(res),
+                                            stream_ptr()), 'fem_patch_residual')
+            return res
         self._tabulate(u, False)
         cell = self.cell_buffer()
         check(self.L.fem_cell_residual(dm.ref, self.mref, ptr(u), ptr(cell), stream_ptr()), 'fem_cell_residual')
@@ -824,7 +904,41 @@ class DeviceProblem:
         self.current = (precision, Ke, vals, dinv)
         self.form = form
         self.last_residual = res
+        self.fine = self._fine_operator(u) if ke_precision == _lib.FEM_F64 else None
         return self.current
+
+    # Cells from which a solve's products run matrix-free, by the storage of the matrix they replace.
+    # One product at 28^3, 32^3, 40^3, 64^3 cells in us: elastic law, patches 9.9, 9.8, 12.5, 31;
+    # FP64 matrix 10.9, 13.8, 24, 97; FP32 matrix 6.6, 7.8, 12.9, 49.  Neo-Hookean patches 12.0, 12.2,
+    # 19, 65: faster than the FP64 matrix, slower than the FP32 one at every size.  The scalar Poisson
+    # matrix is read as fast as its cells are integrated (64^3: 19.2 against 19.6).
+    PATCH_MIN_CELLS = {_lib.FEM_F64: 24000, _lib.FEM_F32: 48000}
+
+    def fine_for(self, storage):
+        """The matrix-free tangent where it is faster than a matrix stored in `storage`, else None."""
+        if self.fine is None or self.dm.C < self.PATCH_MIN_CELLS[storage]:
+            return None
+        if storage == _lib.FEM_F32 and self.fine[0].mat.contents.kind == _lib.FEM_MAT_NEO_HOOKEAN:
+            return None
+        return self.fine
+
+    def _fine_operator(self, u):
+        """The matrix-free form of the tangent just assembled at u, with its own copies of the law's
+        constants and of what varies with u; None where no solve uses it."""
+        if (not self.patch_law or self.mass_dyn is not None or self.material.kind == _lib.FEM_MAT_POISSON
+                or self.dm.C < min(self.PATCH_MIN_CELLS.values())):
+            return None
+        if self.material.kind == _lib.FEM_MAT_SIMP:
+            # E at every point: the power is taken once per tangent
+            if 'modulus' not in self.buffers:
+                self.buffers['modulus'] = self.dm.empty(self.dm.C * self.dm.Q)
+            mod = self.buffers['modulus']
+            check(self.L.fem_patch_modulus(self.dm.ref, self.mref, ptr(mod), stream_ptr()), 'fem_patch_modulus')
+        else:
+            mod = None
+        lin = u.clone() if self.material.kind == _lib.FEM_MAT_NEO_HOOKEAN else None
+        op = self.patch_operator(self.mat_desc, lin, mod)
+        return op, (self.mat_desc, self.param, lin, mod, self.bc_mask)
 
     def operator(self, u):
         op = _lib.FemOperator()
@@ -869,9 +983,15 @@ class DeviceProblem:
             nb = int(self.L.fem_pcg_ws_bytes(self.pref, precision))
             self.buffers[key] = self.dm.empty(nb, dtype=torch.uint8)
         ws = self.buffers[key]
-        op = self.operator(u) if precision == _lib.FEM_F32 else None
         x = x0.clone()
         res = _lib.FemPcgResult()
+        fine = self.fine_for(precision)
+        if fine is not None:
+            check(self.L.fem_pcg_solve_patch(self.pref, C.byref(fine[0]), ptr(dinv), ptr(b), ptr(x), C.byref(o),
+                                             ptr(ws), C.c_void_p(self.host_status.data_ptr()), C.byref(res),
+                                             stream_ptr()), 'fem_pcg_solve_patch')
+            return x, res
+        op = self.operator(u) if precision == _lib.FEM_F32 else None
         check(self.L.fem_pcg_solve(self.pref, ptr(vals), ptr(dinv), C.byref(op) if op is not None else None,
                                    ptr(b), ptr(x), C.byref(o), ptr(ws), C.c_void_p(self.host_status.data_ptr()),
                                    C.byref(res), stream_ptr()), 'fem_pcg_solve')
@@ -958,7 +1078,14 @@ class DeviceProblem:
         from .amg import DeviceAMG
         if self._amg is None:
             self._amg = DeviceAMG(self)
-        return self._amg.setup(vals, cfg['amg_precision'], cfg['degree'], cfg.get('level0', 'fp32'))
+        return self._amg.setup(vals, cfg['amg_precision'], cfg['degree'], cfg.get('level0', 'fp32'),
+                               self._amg_operator(cfg))
+
+    def _amg_operator(self, cfg):
+        """The matrix-free operator of level 0 and the outer CG, unless the options ask for a stored matrix."""
+        if cfg.get('outer', 'fp64') != 'fp64' or cfg.get('level0', 'fp32') != 'fp32':
+            return None
+        return self.fine_for(cfg['amg_precision'])
 
     def amg_solve(self, b, x0, cfg):
         """AMG-CG on the current FP64 matrix.  With cfg['setup_reuse'] = k > 0 the
@@ -970,6 +1097,7 @@ class DeviceProblem:
         reuse = (cfg.get('setup_reuse', 0) > 0 and amg is not None and amg.amg is not None
                  and amg.precision == cfg['amg_precision'] and self._amg_uses < cfg['setup_reuse']
                  and amg.level0_f16 == (cfg.get('level0', 'fp32') == 'fp16')
+                 and (amg.fine is None) == (self._amg_operator(cfg) is None)
                  and amg.structure_current())
         if reuse:
             self._amg_uses += 1
@@ -978,6 +1106,7 @@ class DeviceProblem:
             self._amg_uses = 0
         torch.cuda.synchronize()
         t1 = time.perf_counter()
+        amg.use_operator(self._amg_operator(cfg))
         out = amg.solve(self.current[2], b, x0, cfg)
         self.amg_timing = dict(setup_s=t1 - t0, solve_s=time.perf_counter() - t1)
         return out

@@ -13,7 +13,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME)
 
 FEM_OK, FEM_ERR_BAD_ARG, FEM_ERR_NOT_CONVERGED, FEM_ERR_NAN, FEM_ERR_HIP, FEM_ERR_CAPACITY = 0, -1, -2, -3, -4, -5
 FEM_F32, FEM_F64, FEM_BF16X3 = 0, 1, 2
-FEM_FORM_STANDARD, FEM_FORM_DIFFERENCE, FEM_FORM_SCALED_DIFF16 = 0, 1, 2
+FEM_FORM_STANDARD, FEM_FORM_DIFFERENCE, FEM_FORM_SCALED_DIFF16, FEM_FORM_OPERATOR = 0, 1, 2, 3
 FEM_MAT_POISSON, FEM_MAT_LINEAR_ELASTIC, FEM_MAT_SIMP, FEM_MAT_NEO_HOOKEAN, FEM_MAT_J2_PLASTIC = 1, 2, 3, 4, 5
 FEM_MAT_TABULATED = 6
 FEM_MAT_NONE = 0
@@ -60,6 +60,17 @@ class FemConstraint(C.Structure):
 class FemAssemblyPlan(C.Structure):
     _fields_ = [('slice_cell_ptr', _vp), ('slice_cells', _vp), ('slice_pair_ptr', _vp), ('slice_pairs', _vp),
                 ('contrib_loc', _vp), ('max_slots', _i32), ('max_pairs', _i32)]
+
+
+class FemPatchPlan(C.Structure):
+    _fields_ = [('num_patches', _i64), ('entries', _i64), ('cells_per_patch', _i32), ('pad', _i32),
+                ('val', _f64 * 9), ('der', _f64 * 9), ('slot_ptr', _vp), ('slot_end', _vp), ('contrib', _vp),
+                ('inc_ptr', _vp), ('inc_idx', _vp)]
+
+
+class FemPatchOperator(C.Structure):
+    _fields_ = [('mesh', C.POINTER(FemMesh)), ('mat', C.POINTER(FemMaterial)), ('plan', C.POINTER(FemPatchPlan)),
+                ('u', _vp), ('bc_mask', _vp), ('modulus', _vp), ('partials', _vp)]
 
 
 class FemPcgOptions(C.Structure):
@@ -132,6 +143,12 @@ _SIGNATURES = {
     'fem_assembly_plan_fill': (C.c_int, [_P(FemPattern), _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     'fem_assemble': (C.c_int, [_P(FemMesh), _P(FemMaterial), _P(FemPattern), _P(FemAssemblyPlan), _vp, _i32,
                                _i32, _vp, _vp, _vp, _vp, _vp]),
+    'fem_patch_cells': (_i32, [_P(FemMesh)]),
+    'fem_patch_counts': (C.c_int, [_P(FemMesh), _vp, _vp]),
+    'fem_patch_fill': (C.c_int, [_P(FemMesh), _vp, _vp, _vp, _vp, _vp]),
+    'fem_patch_modulus': (C.c_int, [_P(FemMesh), _P(FemMaterial), _vp, _vp]),
+    'fem_patch_apply': (C.c_int, [_P(FemPatchOperator), _vp, _vp, _vp]),
+    'fem_patch_residual': (C.c_int, [_P(FemPatchOperator), _vp, _vp, _vp, _vp]),
     'fem_csr_spmv': (C.c_int, [_i64, _vp, _vp, _vp, _vp, _vp, _vp]),
     'fem_bicgstab_ws_bytes': (_i64, [_P(FemPattern), _P(FemConstraint)]),
     'fem_bicgstab_solve': (C.c_int, [_P(FemPattern), _vp, _vp, _P(FemConstraint), _vp, _vp, _P(FemPcgOptions),
@@ -139,6 +156,8 @@ _SIGNATURES = {
     'fem_pcg_ws_bytes': (_i64, [_P(FemPattern), _i32]),
     'fem_pcg_solve': (C.c_int, [_P(FemPattern), _vp, _vp, _P(FemOperator), _vp, _vp, _P(FemPcgOptions),
                                 _vp, _vp, _P(FemPcgResult), _vp]),
+    'fem_pcg_solve_patch': (C.c_int, [_P(FemPattern), _P(FemPatchOperator), _vp, _vp, _vp, _P(FemPcgOptions),
+                                      _vp, _vp, _P(FemPcgResult), _vp]),
     'fem_pcg_solve_noalloc': (C.c_int, [_P(FemPattern), _vp, _vp, _P(FemOperator), _vp, _vp, _P(FemPcgOptions),
                                         _vp, _P(FemPcgResult), _vp]),
     'fem_dot': (C.c_int, [_i64, _vp, _vp, _vp, _vp, _vp]),

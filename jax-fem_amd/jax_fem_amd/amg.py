@@ -89,6 +89,7 @@ class DeviceAMG:
         self.levels = []
         self.amg = None
         self.level0_f16 = False
+        self.fine = None
 
     # -------------------------------------------------------------- helpers
     def _empty(self, n, dtype=torch.float64):
@@ -178,14 +179,18 @@ class DeviceAMG:
                                   ptr(ws), stream_ptr()), 'fem_amg_lmax')
         return float(lam.value)
 
-    def _lmax_async(self, A, dinv, out, sell_vals=None):
+    def _lmax_async(self, A, dinv, out, sell_vals=None, op=None):
         """_lmax's estimate written to the device scalar `out` (a 1-element FP64 tensor) without
-        a host synchronisation."""
+        a host synchronisation; with `op`, on the matrix-free operator."""
         s = A.struct()
         ws = self._empty(self.L.fem_amg_lmax_ws_bytes(A.rows * A.br), torch.uint8)
-        pat = self.dev.pref if sell_vals is not None else None
-        f32 = 0 if sell_vals is None else {torch.float32: 1, torch.float16: 2}.get(sell_vals.dtype, 0)
-        check(self.L.fem_amg_lmax_async(C.byref(s), pat, ptr(sell_vals), f32, ptr(dinv), POWER_STEPS, ptr(out),
+        pat = self.dev.pref if sell_vals is not None or op is not None else None
+        if op is not None:
+            vals, f32 = C.c_void_p(C.addressof(op[0])), 3
+        else:
+            vals = ptr(sell_vals)
+            f32 = 0 if sell_vals is None else {torch.float32: 1, torch.float16: 2}.get(sell_vals.dtype, 0)
+        check(self.L.fem_amg_lmax_async(C.byref(s), pat, vals, f32, ptr(dinv), POWER_STEPS, ptr(out),
                                         ptr(ws), stream_ptr()), 'fem_amg_lmax_async')
 
     def _sell_diff32_buffer(self, vals64):
@@ -289,10 +294,11 @@ class DeviceAMG:
         self._struct_src = (dev.pat_tensors['row_ptr'], dev.bc_dofs)
         return self._struct
 
-    def setup(self, vals64, precision=_lib.FEM_F64, degree=DEGREE, level0='fp32'):
+    def setup(self, vals64, precision=_lib.FEM_F64, degree=DEGREE, level0='fp32', op=None):
         """Hierarchy of the current FP64 matrix (standard-form SELL values `vals64`).
         level0 ('fp32' or 'fp16', FP32 hierarchies only): storage of the level-0
-        smoother matrix, FP32 difference form or FP16 D^-1 A in difference form."""
+        smoother matrix, FP32 difference form or FP16 D^-1 A in difference form.
+        op: the matrix-free form of the same matrix; level 0 then has no stored copy."""
         dev, L = self.dev, self.L
         levels, coarse = self._structure()
         # an FP32 hierarchy forms its Galerkin products from FP32 values (FP64 arithmetic):
@@ -310,9 +316,9 @@ class DeviceAMG:
         sv32 = dinv0 = None
         if precision == _lib.FEM_F32 and levels and not f16:
             # level 0's FP32 block-CSR copy (the Galerkin products' input), its FP32
-            # difference-form SELL copy (the V-cycle's level-0 matrix) and its inverse
-            # diagonal in one pass
-            sv32 = self._sell_diff32_buffer(vals64)
+            # difference-form SELL copy (the V-cycle's level-0 matrix, unless that is
+            # matrix-free) and its inverse diagonal in one pass
+            sv32 = self._sell_diff32_buffer(vals64) if op is None else None
             dinv0 = self._empty(A0.rows * A0.br)
             check(L.fem_amg_sell_to_f32_copies(dev.pref, ptr(vals64), ptr(A0.vals), ptr(sv32), ptr(dinv0),
                                                stream_ptr()), 'fem_amg_sell_to_f32_copies')
@@ -328,7 +334,10 @@ class DeviceAMG:
             if l == 0 and f16:
                 sv32 = self._sell_f16(vals64, lv['dinv'])
             lam_l = lam_dev[l:l + 1]
-            self._lmax_async(A, lv['dinv'], lam_l, (vals64 if sv32 is None else sv32) if l == 0 else None)
+            if l == 0 and op is not None:
+                self._lmax_async(A, lv['dinv'], lam_l, op=op)
+            else:
+                self._lmax_async(A, lv['dinv'], lam_l, (vals64 if sv32 is None else sv32) if l == 0 else None)
             plan_w0, plan_w, plan_c = lv['plans']
             P = lv['P']
             as_, p0s, ps = A.struct(), lv['P0m'].struct(), P.struct()
@@ -352,10 +361,16 @@ class DeviceAMG:
         check(L.fem_amg_coarse_inverse(C.byref(cs), ptr(self.coarse_inv), ptr(self._gj_ws), stream_ptr()),
               'fem_amg_coarse_inverse')
         self.levels, self.coarse = levels, coarse
-        self._descriptor(vals64, precision, degree, sv32)
+        self._descriptor(vals64, precision, degree, sv32, op if levels else None)
         return self
 
-    def _descriptor(self, vals64, precision, degree, sv32=None):
+    def use_operator(self, op):
+        """Point a matrix-free level 0 at the current tangent (a reused hierarchy follows the matrix)."""
+        if self.fine is not None:
+            self.fine = op
+            self._keep[1][0].sell_vals = C.addressof(op[0])
+
+    def _descriptor(self, vals64, precision, degree, sv32=None, op=None):
         dev = self.dev
         f32 = precision == _lib.FEM_F32
         keep = []
@@ -363,7 +378,10 @@ class DeviceAMG:
         self.vals32, self._diff_fresh = None, False
         for l, lv in enumerate(self.levels):
             e = arr[l]
-            if l == 0:
+            if l == 0 and op is not None:
+                e.pat = C.pointer(dev.pat)
+                e.sell_vals = C.addressof(op[0])
+            elif l == 0:
                 e.pat = C.pointer(dev.pat)
                 sv = (sv32 if sv32 is not None else self._sell_diff32(vals64)) if f32 else vals64
                 keep.append(sv)
@@ -384,6 +402,9 @@ class DeviceAMG:
         self.level0_f16 = sv32 is not None and sv32.dtype == torch.float16
         amg.level0_form = (_lib.FEM_FORM_SCALED_DIFF16 if self.level0_f16 else _lib.FEM_FORM_DIFFERENCE) \
             if (f32 and self.levels) else _lib.FEM_FORM_STANDARD
+        if op is not None:
+            amg.level0_form = _lib.FEM_FORM_OPERATOR
+        self.fine = op
         amg.levels = arr if self.levels else None
         amg.coarse_n = self.coarse.rows * self.coarse.br
         amg.coarse_inv = self.coarse_inv.data_ptr()
