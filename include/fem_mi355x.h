@@ -330,7 +330,8 @@ int fem_operator_apply(const fem_operator_t* op, const double* x, double* y, voi
  * A patch is a run of fem_patch_cells consecutive cells; the plan (built once
  * per mesh) lists each patch's distinct nodes ("slots", ascending) with the
  * (cell in patch, local node) entries that add up to them, and each node's
- * slots.  Covered: HEX8 cells with the 2x2x2 Gauss rule. */
+ * slots.  Covered: HEX8 cells with the 2x2x2 and HEX27 cells with the 3x3x3
+ * Gauss rule. */
 typedef struct {
   int64_t         num_patches;     /* ceil(num_cells / cells_per_patch)         */
   int64_t         entries;         /* slot_ptr[num_patches]                     */
@@ -338,7 +339,7 @@ typedef struct {
   int32_t         pad;
   double          val[9];          /* 1-D shape values (point, node), row-major
                                       with the rule's points per axis squared
-                                      entries (HEX8: 4)                         */
+                                      entries (HEX8: 4, HEX27: 9)               */
   double          der[9];          /* 1-D shape derivatives, likewise           */
   const int32_t*  slot_ptr;        /* (num_patches + 1)                         */
   const uint16_t* slot_end;        /* (entries) end of the slot's run in the
@@ -358,7 +359,8 @@ int fem_patch_counts(const fem_mesh_t* mesh, int32_t* counts, void* stream);
 int fem_patch_fill(const fem_mesh_t* mesh, const int32_t* slot_ptr, int32_t* slot_node, uint16_t* slot_end,
                    uint16_t* contrib, void* stream);
 
-/* Tangent operator at u: Poisson, elastic, SIMP and Neo-Hookean laws. */
+/* Tangent operator at u: Poisson, elastic, SIMP and (HEX8 cells; HEX27 for the
+ * residual only) Neo-Hookean laws. */
 typedef struct {
   const fem_mesh_t*       mesh;
   const fem_material_t*   mat;

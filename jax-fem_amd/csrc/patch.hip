@@ -6,7 +6,8 @@
 // are recomputed from the nodal coordinates instead of read from HBM.
 //
 // Two kernels per product.
-//   k_patch_hex8    one workgroup per patch of kPatchCells consecutive cells.
+//   k_patch_hex8, k_patch_hex27
+//                   one workgroup per patch of consecutive cells (128 or 28).
 //                   Every cell's nodal vector is formed in registers, staged in
 //                   LDS and summed per distinct node of the patch (a fixed
 //                   order): one partial per (patch, node) goes to memory
@@ -35,6 +36,7 @@
 namespace fem {
 
 constexpr int kPatchCells = 128;  // HEX8 cells per patch
+constexpr int kPatchCells27 = 28;  // HEX27 cells per patch: 7 per wave, 9 lanes each
 constexpr int kPatchCap = 2048;   // most (cell, node) entries of a patch
 
 // ------------------------------------------------------------------ plan
@@ -477,6 +479,211 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
   sums.store(s_plan, s_r, part);
 }
 
+// ------------------------------------------------------------ HEX27 cells
+// LDS written by a wave and read by the same wave: its DS instructions execute in order, the
+// fence keeps the compiler from reordering them.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// VTK number of lattice node (i, j, k) of the triquadratic cell, at 9 i + 3 j + k
+__device__ const int8_t kVtk27[27] = {0, 16, 4, 11, 20, 15, 3,  19, 7,  8, 22, 12, 24, 26,
+                                      25, 10, 23, 14, 1, 17, 5, 9, 21, 13, 2, 18, 6};
+
+// Triquadratic cells with the 3x3x3 Gauss rule, sum-factorised: nine lanes per cell, each
+// holding a line of three values, contract one axis at a time with the 1-D tables and hand
+// the results on through LDS (seven cells per wave, so no barrier is needed).  MODE as in
+// k_patch_hex8; the tangent covers the laws that are linear in grad u.
+template <class MAT, int MODE, typename TX>
+__global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_material_t mat, fem_patch_plan_t plan,
+                                                     const TX* __restrict__ x, double* __restrict__ part,
+                                                     const int32_t* __restrict__ done) {
+  constexpr int N = 27, V = MAT::V, NT = 256, STRIDE = 243;  // doubles of LDS per cell: 3 fields, 3 kinds, 27 points
+  constexpr bool kLinear = !MAT::kNeedsU;
+  static_assert(MODE == 0 || kLinear, "the hyperelastic tangent runs on HEX8 patches only");
+  using Sums = PatchSums<N, V, STRIDE, kPatchCells27, NT>;
+  __shared__ double s_r[kPatchCells27 * STRIDE];
+  __shared__ typename Sums::Lds s_plan;
+  if (done && *done) return;
+  const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
+  const int lane = min((int)(threadIdx.x & 63), 62);  // lane 63 repeats lane 62
+  const int cl = (threadIdx.x >> 6) * 7 + lane / 9, t = lane % 9, ta = t / 3, tb = t % 3;
+  const int64_t c = min(patch * kPatchCells27 + cl, mesh.num_cells - 1);
+  double* L = s_r + cl * STRIDE;
+  Sums sums;
+  auto val = [&](int q, int n) { return plan.val[3 * q + n]; };
+  auto der = [&](int q, int n) { return plan.der[3 * q + n]; };
+  // nodal lines n[i][field] of lane (j, k) -> h[field][kind][k] of lane (qx, qy): kind 0 the value
+  // along both axes, 1 the y derivative, 2 the x derivative
+  auto contract = [&](auto& n, auto& h) {
+    constexpr int NC = sizeof(n[0]) / sizeof(double);
+#pragma unroll
+    for (int f = 0; f < NC; ++f)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        L[(2 * f) * 27 + q * 9 + t] = val(q, 0) * n[0][f] + val(q, 1) * n[1][f] + val(q, 2) * n[2][f];
+        L[(2 * f + 1) * 27 + q * 9 + t] = der(q, 0) * n[0][f] + der(q, 1) * n[1][f] + der(q, 2) * n[2][f];
+      }
+    wave_lds_fence();
+    double a[NC][3], b[NC][3];
+#pragma unroll
+    for (int f = 0; f < NC; ++f)
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        a[f][j] = L[(2 * f) * 27 + ta * 9 + j * 3 + tb];
+        b[f][j] = L[(2 * f + 1) * 27 + ta * 9 + j * 3 + tb];
+      }
+    wave_lds_fence();
+#pragma unroll
+    for (int f = 0; f < NC; ++f)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        double* o = L + (3 * f) * 27 + ta * 9 + q * 3 + tb;
+        o[0] = val(q, 0) * a[f][0] + val(q, 1) * a[f][1] + val(q, 2) * a[f][2];
+        o[27] = der(q, 0) * a[f][0] + der(q, 1) * a[f][1] + der(q, 2) * a[f][2];
+        o[54] = val(q, 0) * b[f][0] + val(q, 1) * b[f][1] + val(q, 2) * b[f][2];
+      }
+    wave_lds_fence();
+#pragma unroll
+    for (int f = 0; f < NC; ++f)
+#pragma unroll
+      for (int kind = 0; kind < 3; ++kind)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) h[f][kind][k] = L[(3 * f + kind) * 27 + t * 3 + k];
+    wave_lds_fence();
+  };
+  double hx[3][3][3], hf[V][3][3];
+  int vtk[3];
+  {
+    double nx[3][3], nf[3][V];
+    const int32_t* cn = mesh.cells + c * N;
+    const double* p0 = mesh.points + (int64_t)cn[0] * 3;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      vtk[i] = kVtk27[9 * i + t];
+      const int64_t id = cn[vtk[i]];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) nx[i][j] = mesh.points[id * 3 + j] - p0[j];
+#pragma unroll
+      for (int v = 0; v < V; ++v) nf[i][v] = double(x[id * V + v]);
+    }
+    sums.load(plan, patch, mesh.num_cells);
+    contract(nx, hx);
+    contract(nf, hf);
+  }
+  double s[V][3][3];
+#pragma unroll
+  for (int v = 0; v < V; ++v)
+#pragma unroll
+    for (int kind = 0; kind < 3; ++kind)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) s[v][kind][k] = 0.0;
+  // reference gradients at point q of the lane's line: M[f][dir]
+  auto columns = [&](auto& h, int q, auto& M) {
+    constexpr int NC = sizeof(M) / sizeof(M[0]);
+#pragma unroll
+    for (int f = 0; f < NC; ++f) {
+      M[f][0] = val(q, 0) * h[f][2][0] + val(q, 1) * h[f][2][1] + val(q, 2) * h[f][2][2];
+      M[f][1] = val(q, 0) * h[f][1][0] + val(q, 1) * h[f][1][1] + val(q, 2) * h[f][1][2];
+      M[f][2] = der(q, 0) * h[f][0][0] + der(q, 1) * h[f][0][1] + der(q, 2) * h[f][0][2];
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double J3[3][3], R[V][3], J[9], A[9], G[V][3], P[V][3];
+    columns(hx, q, J3);
+    columns(hf, q, R);
+#pragma unroll
+    for (int k = 0; k < 9; ++k) J[k] = J3[k / 3][k % 3];
+    adj3(J, A);
+    const double det = J[0] * A[0] + J[1] * A[3] + J[2] * A[6], id = rcp_newton(det);
+    const double w = mesh.quad_weights[t * 3 + q];
+    if constexpr (!kLinear)
+#pragma unroll
+      for (int k = 0; k < 9; ++k) A[k] *= id;
+#pragma unroll
+    for (int v = 0; v < V; ++v)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) G[v][k] = R[v][0] * A[k] + R[v][1] * A[3 + k] + R[v][2] * A[6 + k];
+    auto st = MAT::template prep<double>(mat, c * 27 + t * 3 + q, G);
+    if constexpr (kLinear) scale_state(st, w * id);
+    MAT::stress(st, G, P);
+    if constexpr (!kLinear) {
+      const double jxw = w * det;
+#pragma unroll
+      for (int v = 0; v < V; ++v)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) P[v][k] *= jxw;
+    }
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      double T[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) T[d] = P[v][0] * A[3 * d] + P[v][1] * A[3 * d + 1] + P[v][2] * A[3 * d + 2];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        s[v][2][k] = fma(val(q, k), T[0], s[v][2][k]);
+        s[v][1][k] = fma(val(q, k), T[1], s[v][1][k]);
+        s[v][0][k] = fma(der(q, k), T[2], s[v][0][k]);
+      }
+    }
+  }
+  // the transposed contractions, back to the lane's nodes
+#pragma unroll
+  for (int v = 0; v < V; ++v)
+#pragma unroll
+    for (int kind = 0; kind < 3; ++kind)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) L[(3 * v + kind) * 27 + t * 3 + k] = s[v][kind][k];
+  wave_lds_fence();
+  double a[V][3], b[V][3];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+#pragma unroll
+    for (int j = 0; j < 3; ++j) a[v][j] = b[v][j] = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const double* o = L + (3 * v) * 27 + ta * 9 + q * 3 + tb;
+      const double vv = o[0], vd = o[27], dv = o[54];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) {
+        a[v][j] = fma(val(q, j), vv, fma(der(q, j), vd, a[v][j]));
+        b[v][j] = fma(val(q, j), dv, b[v][j]);
+      }
+    }
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int v = 0; v < V; ++v)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      L[(2 * v) * 27 + ta * 9 + j * 3 + tb] = a[v][j];
+      L[(2 * v + 1) * 27 + ta * 9 + j * 3 + tb] = b[v][j];
+    }
+  wave_lds_fence();
+  double r[3][V];
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) r[i][v] = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const double va = L[(2 * v) * 27 + q * 9 + t], de = L[(2 * v + 1) * 27 + q * 9 + t];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) r[i][v] = fma(val(q, i), va, fma(der(q, i), de, r[i][v]));
+    }
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+#pragma unroll
+    for (int v = 0; v < V; ++v) L[vtk[i] * V + v] = r[i][v];
+  sums.stage(s_plan);
+  __syncthreads();
+  sums.store(s_plan, s_r, part);
+}
+
 // ------------------------------------------------------------------ gather
 // AP_STORE adds a.rhs where it is given (the residual's constant loads).
 template <int V, int MODE, typename TX, typename TY>
@@ -514,7 +721,7 @@ __global__ __launch_bounds__(256) void k_patch_gather(int64_t n, const int32_t* 
 
 // ---------------------------------------------------------------- dispatch
 template <class F>
-static int with_patch_law(const fem_patch_operator_t& op, fem_material_t* mat, bool tangent, F&& f) {
+static int with_patch_law(const fem_patch_operator_t& op, fem_material_t* mat, F&& f) {
   *mat = *op.mat;
   const int vec = op.mesh->vec;
   switch (mat->kind) {
@@ -541,12 +748,13 @@ static int with_patch_law(const fem_patch_operator_t& op, fem_material_t* mat, b
   return FEM_ERR_BAD_ARG;
 }
 
-bool patch_operator_ok(const fem_patch_operator_t* op) {
+bool patch_operator_ok(const fem_patch_operator_t* op, bool residual) {
   if (!op || !op->mesh || !op->mat || !op->plan || !op->partials) return false;
   const fem_mesh_t& m = *op->mesh;
   const fem_patch_plan_t& p = *op->plan;
-  if (m.nodes_per_cell != 8 || m.num_quads != 8 || m.num_cells <= 0 || m.num_nodes <= 0) return false;
-  if (p.cells_per_patch != kPatchCells || p.num_patches != ceil_div(m.num_cells, kPatchCells)) return false;
+  const int cpp = fem_patch_cells(&m);
+  if (cpp <= 0 || m.num_cells <= 0 || m.num_nodes <= 0) return false;
+  if (p.cells_per_patch != cpp || p.num_patches != ceil_div(m.num_cells, cpp)) return false;
   if (!m.cells || ((uintptr_t)m.cells & 15) || !m.points || !m.quad_weights) return false;  // 16-byte node id loads
   if (!p.slot_ptr || !p.slot_end || !p.contrib || !p.inc_ptr || !p.inc_idx) return false;
   const fem_material_t& t = *op->mat;
@@ -555,7 +763,7 @@ bool patch_operator_ok(const fem_patch_operator_t* op) {
     case FEM_MAT_POISSON: return m.vec == 1;
     case FEM_MAT_LINEAR_ELASTIC: return m.vec == 3;
     case FEM_MAT_SIMP: return m.vec == 3 && t.has_param;
-    case FEM_MAT_NEO_HOOKEAN: return m.vec == 3 && op->u;
+    case FEM_MAT_NEO_HOOKEAN: return m.vec == 3 && op->u && (residual || m.nodes_per_cell == 8);
     default: return false;
   }
 }
@@ -565,8 +773,16 @@ template <int MODE, typename TX>
 static int patch_cells(const fem_patch_operator_t& op, const TX* x, const int32_t* done, hipStream_t s) {
   fem_material_t mat;
   const fem_mesh_t& m = *op.mesh;
-  return with_patch_law(op, &mat, MODE == 1, [&](auto tag) -> int {
+  return with_patch_law(op, &mat, [&](auto tag) -> int {
     using MAT = decltype(tag);
+    if (m.nodes_per_cell == 27) {
+      if constexpr (MODE == 0 || !MAT::kNeedsU) {
+        hipLaunchKernelGGL((k_patch_hex27<MAT, MODE, TX>), dim3((unsigned)op.plan->num_patches), dim3(256), 0, s, m,
+                           mat, *op.plan, x, op.partials, done);
+        FEM_LAUNCHED();
+      }
+      return FEM_OK;
+    }
     hipLaunchKernelGGL((k_patch_hex8<MAT, MODE, TX>), dim3((unsigned)op.plan->num_patches), dim3(2 * kPatchCells), 0,
                        s, m, mat, *op.plan, op.u, x, op.partials, done);
     FEM_LAUNCHED();
@@ -618,9 +834,9 @@ __global__ __launch_bounds__(256) void k_modulus(int64_t n, fem_material_t mat, 
 
 static int check_patch_mesh(const fem_mesh_t* m) {
   FEM_CHECK_ARG(m && m->cells && m->num_cells > 0 && m->num_nodes > 0, "patch plan: mesh descriptor incomplete");
-  FEM_CHECK_ARG(m->nodes_per_cell == 8 && m->num_quads == 8,
-                "patch plan: covers HEX8 cells with the 2x2x2 Gauss rule (got %d nodes, %d points)", m->nodes_per_cell,
-                m->num_quads);
+  FEM_CHECK_ARG(fem_patch_cells(m) > 0,
+                "patch plan: covers HEX8 cells with the 2x2x2 and HEX27 cells with the 3x3x3 Gauss rule (got %d nodes, "
+                "%d points)", m->nodes_per_cell, m->num_quads);
   return FEM_OK;
 }
 
@@ -631,7 +847,9 @@ using namespace fem;
 extern "C" {
 
 int fem_patch_cells(const fem_mesh_t* mesh) {
-  return mesh && mesh->nodes_per_cell == 8 && mesh->num_quads == 8 ? kPatchCells : 0;
+  if (!mesh) return 0;
+  if (mesh->nodes_per_cell == 8 && mesh->num_quads == 8) return kPatchCells;
+  return mesh->nodes_per_cell == 27 && mesh->num_quads == 27 ? kPatchCells27 : 0;
 }
 
 int fem_patch_counts(const fem_mesh_t* mesh, int32_t* counts, void* stream) {
@@ -678,7 +896,7 @@ int fem_patch_residual(const fem_patch_operator_t* op, const double* u, const do
   FEM_CHECK_ARG(op && u && res, "fem_patch_residual: NULL argument");
   fem_patch_operator_t o = *op;
   o.u = u;
-  FEM_CHECK_ARG(patch_operator_ok(&o), "fem_patch_residual: the operator is incomplete or not covered");
+  FEM_CHECK_ARG(patch_operator_ok(&o, true), "fem_patch_residual: the operator is incomplete or not covered");
   hipStream_t s = as_stream(stream);
   if (int rc = patch_cells<0, double>(o, u, nullptr, s)) return rc;
   ApplyArgs a{u, res, base, nullptr, nullptr, 0.0, 0.0, nullptr, nullptr};

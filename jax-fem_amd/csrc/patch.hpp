@@ -7,8 +7,8 @@ namespace fem {
 
 constexpr int kPatchDotBlocks = 1024;  // most <x, A x> partials of an AP_PQ product
 
-// True when `op` describes an element, rule and law the patch kernels run.
-bool patch_operator_ok(const fem_patch_operator_t* op);
+// True when `op` describes an element, rule and law whose tangent (or residual) the patch kernels run.
+bool patch_operator_ok(const fem_patch_operator_t* op, bool residual = false);
 
 // y = epilogue(A x), A the tangent at op->u with identity rows on op->bc_mask; *parts
 // receives the number of partials an AP_PQ product writes to a.part.  TX / TY: FP64, or

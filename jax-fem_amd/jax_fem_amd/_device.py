@@ -912,11 +912,17 @@ class DeviceProblem:
     # FP64 matrix 10.9, 13.8, 24, 97; FP32 matrix 6.6, 7.8, 12.9, 49.  Neo-Hookean patches 12.0, 12.2,
     # 19, 65: faster than the FP64 matrix, slower than the FP32 one at every size.  The scalar Poisson
     # matrix is read as fast as its cells are integrated (64^3: 19.2 against 19.6).
-    PATCH_MIN_CELLS = {_lib.FEM_F64: 24000, _lib.FEM_F32: 48000}
+    # HEX27, elastic law, 6^3, 8^3, 10^3, 24^3 cells: patches 13, 13, 13, 21; FP64 matrix 15, 23, 30,
+    # 150; FP32 matrix 8.7, 12, 15, 72.
+    PATCH_MIN_CELLS = {(8, _lib.FEM_F64): 24000, (8, _lib.FEM_F32): 48000,
+                       (27, _lib.FEM_F64): 250, (27, _lib.FEM_F32): 1000}
+
+    def patch_min_cells(self, storage):
+        return self.PATCH_MIN_CELLS[self.dm.N, storage]
 
     def fine_for(self, storage):
         """The matrix-free tangent where it is faster than a matrix stored in `storage`, else None."""
-        if self.fine is None or self.dm.C < self.PATCH_MIN_CELLS[storage]:
+        if self.fine is None or self.dm.C < self.patch_min_cells(storage):
             return None
         if storage == _lib.FEM_F32 and self.fine[0].mat.contents.kind == _lib.FEM_MAT_NEO_HOOKEAN:
             return None
@@ -926,7 +932,8 @@ class DeviceProblem:
         """The matrix-free form of the tangent just assembled at u, with its own copies of the law's
         constants and of what varies with u; None where no solve uses it."""
         if (not self.patch_law or self.mass_dyn is not None or self.material.kind == _lib.FEM_MAT_POISSON
-                or self.dm.C < min(self.PATCH_MIN_CELLS.values())):
+                or (self.material.kind == _lib.FEM_MAT_NEO_HOOKEAN and self.dm.N != 8)
+                or self.dm.C < min(self.patch_min_cells(f) for f in (_lib.FEM_F64, _lib.FEM_F32))):
             return None
         if self.material.kind == _lib.FEM_MAT_SIMP:
             # E at every point: the power is taken once per tangent
