@@ -41,10 +41,36 @@ constexpr int kSlice = 64;  // rows per SELL slice
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------- reductions
+// v of another lane of the 16-lane row, by a DPP control (a move of the vector ALU; a shuffle
+// goes through LDS and takes some ten times as long)
+template <int CTRL>
+__device__ inline double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
+}
+constexpr int kDppXor1 = 0xB1;        // quad_perm [1, 0, 3, 2]
+constexpr int kDppXor2 = 0x4E;        // quad_perm [2, 3, 0, 1]
+constexpr int kDppHalfMirror = 0x141; // lane i of 8 <- 7 - i
+constexpr int kDppMirror = 0x140;     // lane i of 16 <- 15 - i
+
 template <typename T>
 __device__ inline T wave_sum(T v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// Sum over the wave, in every lane: within a 16-lane row each step adds a group that already
+// holds equal values, so the mirrors act as exchanges of 4 and of 8 lanes.
+template <>
+__device__ inline double wave_sum<double>(double v) {
+  v += dpp_move<kDppXor1>(v);
+  v += dpp_move<kDppXor2>(v);
+  v += dpp_move<kDppHalfMirror>(v);
+  v += dpp_move<kDppMirror>(v);
+  v += __shfl_xor(v, 16, 64);
+  v += __shfl_xor(v, 32, 64);
   return v;
 }
 
@@ -74,6 +100,27 @@ __device__ inline T block_sum(T v, T* smem) {
   for (int i = 0; i < NW; ++i) t += smem[i];
   __syncthreads();
   return t;
+}
+
+// Two block-wide sums behind one pair of barriers; smem holds >= 2 * NT / 64 values.
+template <int NT>
+__device__ inline void block_sum2(double& a, double& b, double* smem) {
+  constexpr int NW = NT / 64;
+  a = wave_sum(a);
+  b = wave_sum(b);
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    smem[2 * w] = a;
+    smem[2 * w + 1] = b;
+  }
+  __syncthreads();
+  a = b = 0.0;
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    a += smem[2 * i];
+    b += smem[2 * i + 1];
+  }
+  __syncthreads();
 }
 
 // Slice-parallel SELL-64 row product.  A slice (64 rows) is processed by W

@@ -103,11 +103,7 @@ __global__ __launch_bounds__(256) void k_patch_nodes(int64_t num_cells, int N, i
 
 // ------------------------------------------------------------ element layer
 // value of the neighbouring lane (lane ^ 1)
-__device__ inline double swap_lane1(double x) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xF, 0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xF, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
+__device__ inline double swap_lane1(double x) { return dpp_move<kDppXor1>(x); }
 
 // Reference gradients of NC nodal fields on one layer of quadrature points of a
 // trilinear cell, sum-factorised.  Two neighbouring lanes share a cell: lane h = 0
@@ -337,12 +333,31 @@ __device__ inline void neo_hookean_tangent(const fem_material_t& m, int64_t cq, 
     for (int d = 0; d < 3; ++d) T[i][d] = D[i][0] * A[3 * d] + D[i][1] * A[3 * d + 1] + D[i][2] * A[3 * d + 2];
 }
 
+// The field a cells' pass gathers: x, or z + beta x (the direction of a CG iteration that the
+// pass begins, in the vectors' precision as the gather kernel stores it).
+template <typename TX>
+struct PatchField {
+  const TX* x;
+  const TX* z;
+  PcgHead head;
+  const int32_t* done;
+};
+
+template <bool CG, typename TX, int NT>
+__device__ inline TX patch_begin(const PatchField<TX>& f, bool* done) {
+  if constexpr (CG) {
+    __shared__ double smem[2 * (NT / 64)];
+    return TX(pcg_head<NT>(f.head, smem, done));
+  }
+  *done = f.done && *f.done;
+  return TX(0);
+}
+
 // MODE 0: internal force at x (u unused); MODE 1: tangent at u times x.
-template <class MAT, int MODE, typename TX>
+template <class MAT, int MODE, typename TX, bool CG>
 __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh, fem_material_t mat,
                                                                 fem_patch_plan_t plan, const double* __restrict__ u,
-                                                                const TX* __restrict__ x, double* __restrict__ part,
-                                                                const int32_t* __restrict__ done) {
+                                                                PatchField<TX> field, double* __restrict__ part) {
   constexpr int N = 8, V = MAT::V, NT = 2 * kPatchCells, STRIDE = N * V + 1;  // odd: no bank conflicts between cells
   constexpr bool kNeo = MODE == 1 && MAT::kNeedsU;     // the tangent of the hyperelastic law
   constexpr bool kLinear = !MAT::kNeedsU;
@@ -350,7 +365,9 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
   using Sums = PatchSums<N, V, STRIDE, kPatchCells, NT>;
   __shared__ double s_r[kPatchCells * STRIDE];
   __shared__ typename Sums::Lds s_plan;
-  if (done && *done) return;
+  bool done;
+  const TX beta = patch_begin<CG, TX, NT>(field, &done);
+  if (done) return;
   const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
   Sums sums;
   const int h = threadIdx.x & 1, cl = threadIdx.x >> 1;
@@ -369,7 +386,10 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
 #pragma unroll
       for (int j = 0; j < 3; ++j) nx[k][j] = mesh.points[(int64_t)id[k] * 3 + j];
 #pragma unroll
-      for (int v = 0; v < V; ++v) nf[k][v] = double(x[(int64_t)id[k] * V + v]);
+      for (int v = 0; v < V; ++v) {
+        const int64_t at = (int64_t)id[k] * V + v;
+        nf[k][v] = double(CG ? fma(beta, field.x[at], field.z[at]) : field.x[at]);
+      }
     }
     sums.load(plan, patch, mesh.num_cells);
     // coordinates from the cell's first node, so that their differences round like the cell's size
@@ -495,17 +515,18 @@ __device__ const int8_t kVtk27[27] = {0, 16, 4, 11, 20, 15, 3,  19, 7,  8, 22, 1
 // holding a line of three values, contract one axis at a time with the 1-D tables and hand
 // the results on through LDS (seven cells per wave, so no barrier is needed).  MODE as in
 // k_patch_hex8; the tangent covers the laws that are linear in grad u.
-template <class MAT, int MODE, typename TX>
+template <class MAT, int MODE, typename TX, bool CG>
 __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_material_t mat, fem_patch_plan_t plan,
-                                                     const TX* __restrict__ x, double* __restrict__ part,
-                                                     const int32_t* __restrict__ done) {
+                                                     PatchField<TX> field, double* __restrict__ part) {
   constexpr int N = 27, V = MAT::V, NT = 256, STRIDE = 243;  // doubles of LDS per cell: 3 fields, 3 kinds, 27 points
   constexpr bool kLinear = !MAT::kNeedsU;
   static_assert(MODE == 0 || kLinear, "the hyperelastic tangent runs on HEX8 patches only");
   using Sums = PatchSums<N, V, STRIDE, kPatchCells27, NT>;
   __shared__ double s_r[kPatchCells27 * STRIDE];
   __shared__ typename Sums::Lds s_plan;
-  if (done && *done) return;
+  bool done;
+  const TX beta = patch_begin<CG, TX, NT>(field, &done);
+  if (done) return;
   const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
   const int lane = min((int)(threadIdx.x & 63), 62);  // lane 63 repeats lane 62
   const int cl = (threadIdx.x >> 6) * 7 + lane / 9, t = lane % 9, ta = t / 3, tb = t % 3;
@@ -566,7 +587,10 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
 #pragma unroll
       for (int j = 0; j < 3; ++j) nx[i][j] = mesh.points[id * 3 + j] - p0[j];
 #pragma unroll
-      for (int v = 0; v < V; ++v) nf[i][v] = double(x[id * V + v]);
+      for (int v = 0; v < V; ++v) {
+        const int64_t at = id * V + v;
+        nf[i][v] = double(CG ? fma(beta, field.x[at], field.z[at]) : field.x[at]);
+      }
     }
     sums.load(plan, patch, mesh.num_cells);
     contract(nx, hx);
@@ -686,37 +710,82 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
 
 // ------------------------------------------------------------------ gather
 // AP_STORE adds a.rhs where it is given (the residual's constant loads).
+// AP_PQ runs at most kPatchDotBlocks blocks (one partial each) of kDotThreads threads, which
+// still fill the chip; the others one thread per dof.
+constexpr int kDotThreads = 512;
+
+// sum of the partials of dof idx
+template <int V>
+__device__ inline double patch_sum(int64_t idx, const int32_t* __restrict__ inc_ptr,
+                                   const int32_t* __restrict__ inc_idx, const double* __restrict__ part) {
+  const int64_t node = idx / V;
+  const int v = (int)(idx - node * V);
+  const int k1 = inc_ptr[node + 1];
+  double t = 0.0;
+  for (int k = inc_ptr[node]; k < k1; ++k) t += part[(int64_t)inc_idx[k] * V + v];
+  return t;
+}
+
+// the dofs of a block: one contiguous range, in the order of the patches
+__device__ inline void patch_range(int64_t n, int64_t* begin, int64_t* end) {
+  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
+  const int64_t per = ((n + gridDim.x - 1) / gridDim.x + blockDim.x - 1) / blockDim.x * blockDim.x;
+  *begin = (int64_t)lb * per;
+  *end = min(n, *begin + per);
+}
+
 template <int V, int MODE, typename TX, typename TY>
-__global__ __launch_bounds__(256) void k_patch_gather(int64_t n, const int32_t* __restrict__ inc_ptr,
+__global__ __launch_bounds__(MODE == AP_PQ ? kDotThreads : 256) void k_patch_gather(int64_t n, const int32_t* __restrict__ inc_ptr,
                                                       const int32_t* __restrict__ inc_idx,
                                                       const double* __restrict__ part,
                                                       const uint8_t* __restrict__ mask, ApplyArgsT<TX, TY> a) {
-  __shared__ double red[4];
+  constexpr int NT = MODE == AP_PQ ? kDotThreads : 256;
+  __shared__ double red[NT / 64];
   if (a.done && *a.done) return;
   double pq = 0.0;
-  const int lb = xcd_logical_block(blockIdx.x, gridDim.x);
-  // one contiguous range of dofs per block, in the order of the patches
-  const int64_t per = ((n + gridDim.x - 1) / gridDim.x + 255) & ~(int64_t)255;
-  const int64_t end = min(n, (int64_t)(lb + 1) * per);
-  for (int64_t idx = (int64_t)lb * per + threadIdx.x; idx < end; idx += 256) {
-    const int64_t node = idx / V;
-    const int v = (int)(idx - node * V);
+  int64_t begin, end;
+  patch_range(n, &begin, &end);
+  for (int64_t idx = begin + threadIdx.x; idx < end; idx += NT) {
     EpiOperands e = epilogue_load<MODE>(a, idx);
     if (MODE == AP_PQ) e.x = double(a.x[idx]);
     if (MODE == AP_STORE && a.rhs) e.rhs = a.rhs[idx];
     const bool fixed = mask && mask[idx];
-    const int k1 = inc_ptr[node + 1];
-    double t = 0.0;
-    for (int k = inc_ptr[node]; k < k1; ++k) t += part[(int64_t)inc_idx[k] * V + v];
+    double t = patch_sum<V>(idx, inc_ptr, inc_idx, part);
     if (fixed) t = double(a.x[idx]);
     if (MODE == AP_STORE) t += e.rhs;
     epilogue_store<MODE>(a, idx, t, e);
     if (MODE == AP_PQ) pq = fma(e.x, double(TY(t)), pq);
   }
   if (MODE == AP_PQ) {
-    pq = block_sum_256(pq, red);
-    if (threadIdx.x == 0) a.part[lb] = pq;
+    pq = block_sum<NT>(pq, red);
+    if (threadIdx.x == 0) a.part[blockIdx.x] = pq;
   }
+}
+
+// The gather of a CG product: p_new = z + beta p_old (as the cells' pass formed it), q, <p, q>.
+template <int V, typename T>
+__global__ __launch_bounds__(kDotThreads) void k_patch_gather_cg(
+    int64_t n, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_idx,
+    const double* __restrict__ part, const uint8_t* __restrict__ mask, const PcgScalars* __restrict__ sc,
+    const T* __restrict__ z, const T* __restrict__ p_old, T* __restrict__ p_new, T* __restrict__ q,
+    double* __restrict__ pq_part) {
+  __shared__ double red[kDotThreads / 64];
+  if (sc->done) return;
+  const T beta = T(sc->beta);
+  double pq = 0.0;
+  int64_t begin, end;
+  patch_range(n, &begin, &end);
+  for (int64_t idx = begin + threadIdx.x; idx < end; idx += kDotThreads) {
+    const T p = fma(beta, p_old[idx], z[idx]);
+    const bool fixed = mask && mask[idx];
+    const double t = patch_sum<V>(idx, inc_ptr, inc_idx, part);
+    const T qi = fixed ? p : T(t);
+    p_new[idx] = p;
+    q[idx] = qi;
+    pq = fma(double(p), double(qi), pq);
+  }
+  pq = block_sum<kDotThreads>(pq, red);
+  if (threadIdx.x == 0) pq_part[blockIdx.x] = pq;
 }
 
 // ---------------------------------------------------------------- dispatch
@@ -768,23 +837,23 @@ bool patch_operator_ok(const fem_patch_operator_t* op, bool residual) {
   }
 }
 
-// the cells' pass: partials of the internal force at x (MODE 0) or of A x (MODE 1)
-template <int MODE, typename TX>
-static int patch_cells(const fem_patch_operator_t& op, const TX* x, const int32_t* done, hipStream_t s) {
+// the cells' pass: partials of the internal force (MODE 0) or of the tangent product (MODE 1)
+template <int MODE, bool CG, typename TX>
+static int patch_cells(const fem_patch_operator_t& op, const PatchField<TX>& field, hipStream_t s) {
   fem_material_t mat;
   const fem_mesh_t& m = *op.mesh;
   return with_patch_law(op, &mat, [&](auto tag) -> int {
     using MAT = decltype(tag);
     if (m.nodes_per_cell == 27) {
       if constexpr (MODE == 0 || !MAT::kNeedsU) {
-        hipLaunchKernelGGL((k_patch_hex27<MAT, MODE, TX>), dim3((unsigned)op.plan->num_patches), dim3(256), 0, s, m,
-                           mat, *op.plan, x, op.partials, done);
+        hipLaunchKernelGGL((k_patch_hex27<MAT, MODE, TX, CG>), dim3((unsigned)op.plan->num_patches), dim3(256), 0, s,
+                           m, mat, *op.plan, field, op.partials);
         FEM_LAUNCHED();
       }
       return FEM_OK;
     }
-    hipLaunchKernelGGL((k_patch_hex8<MAT, MODE, TX>), dim3((unsigned)op.plan->num_patches), dim3(2 * kPatchCells), 0,
-                       s, m, mat, *op.plan, op.u, x, op.partials, done);
+    hipLaunchKernelGGL((k_patch_hex8<MAT, MODE, TX, CG>), dim3((unsigned)op.plan->num_patches), dim3(2 * kPatchCells),
+                       0, s, m, mat, *op.plan, op.u, field, op.partials);
     FEM_LAUNCHED();
     return FEM_OK;
   });
@@ -794,14 +863,15 @@ template <int MODE, typename TX, typename TY>
 static int patch_gather(const fem_patch_operator_t& op, const uint8_t* mask, const ApplyArgsT<TX, TY>& a, hipStream_t s,
                         int* parts) {
   const int64_t n = op.mesh->num_nodes * op.mesh->vec;
-  const int64_t want = ceil_div(n, 256);
+  constexpr int NT = MODE == AP_PQ ? kDotThreads : 256;
+  const int64_t want = ceil_div(n, NT);
   const unsigned grid = (unsigned)(MODE == AP_PQ ? std::min<int64_t>(want, kPatchDotBlocks) : want);
   if (parts) *parts = (int)grid;
   if (op.mesh->vec == 3)
-    hipLaunchKernelGGL((k_patch_gather<3, MODE, TX, TY>), dim3(grid), dim3(256), 0, s, n, op.plan->inc_ptr,
+    hipLaunchKernelGGL((k_patch_gather<3, MODE, TX, TY>), dim3(grid), dim3(NT), 0, s, n, op.plan->inc_ptr,
                        op.plan->inc_idx, op.partials, mask, a);
   else
-    hipLaunchKernelGGL((k_patch_gather<1, MODE, TX, TY>), dim3(grid), dim3(256), 0, s, n, op.plan->inc_ptr,
+    hipLaunchKernelGGL((k_patch_gather<1, MODE, TX, TY>), dim3(grid), dim3(NT), 0, s, n, op.plan->inc_ptr,
                        op.plan->inc_idx, op.partials, mask, a);
   FEM_LAUNCHED();
   return FEM_OK;
@@ -809,9 +879,34 @@ static int patch_gather(const fem_patch_operator_t& op, const uint8_t* mask, con
 
 template <int MODE, typename TX, typename TY>
 int patch_apply(const fem_patch_operator_t& op, const ApplyArgsT<TX, TY>& a, hipStream_t s, int* parts) {
-  if (int rc = patch_cells<1, TX>(op, a.x, a.done, s)) return rc;
+  if (int rc = patch_cells<1, false, TX>(op, PatchField<TX>{a.x, nullptr, PcgHead{}, a.done}, s)) return rc;
   return patch_gather<MODE, TX, TY>(op, op.bc_mask, a, s, parts);
 }
+
+template <typename T>
+int patch_pcg_product(const fem_patch_operator_t& op, const PcgHead& head, const T* z, const T* p_old, T* p_new, T* q,
+                      double* part, hipStream_t s, int* parts) {
+  if (int rc = patch_cells<1, true, T>(op, PatchField<T>{p_old, z, head, nullptr}, s)) return rc;
+  const int64_t n = op.mesh->num_nodes * op.mesh->vec;
+  *parts = (int)std::min<int64_t>(ceil_div(n, kDotThreads), kPatchDotBlocks);
+  auto go = [&](auto vc) {
+    constexpr int V = decltype(vc)::value;
+    hipLaunchKernelGGL((k_patch_gather_cg<V, T>), dim3((unsigned)*parts), dim3(kDotThreads), 0, s, n,
+                       op.plan->inc_ptr, op.plan->inc_idx, op.partials, op.bc_mask, (const PcgScalars*)head.next, z,
+                       p_old, p_new, q, part);
+  };
+  if (op.mesh->vec == 3)
+    go(std::integral_constant<int, 3>{});
+  else
+    go(std::integral_constant<int, 1>{});
+  FEM_LAUNCHED();
+  return FEM_OK;
+}
+
+template int patch_pcg_product<double>(const fem_patch_operator_t&, const PcgHead&, const double*, const double*,
+                                       double*, double*, double*, hipStream_t, int*);
+template int patch_pcg_product<float>(const fem_patch_operator_t&, const PcgHead&, const float*, const float*, float*,
+                                      float*, double*, hipStream_t, int*);
 
 template int patch_apply<AP_STORE, double, double>(const fem_patch_operator_t&, const ApplyArgsT<double, double>&,
                                                    hipStream_t, int*);
@@ -898,7 +993,7 @@ int fem_patch_residual(const fem_patch_operator_t* op, const double* u, const do
   o.u = u;
   FEM_CHECK_ARG(patch_operator_ok(&o, true), "fem_patch_residual: the operator is incomplete or not covered");
   hipStream_t s = as_stream(stream);
-  if (int rc = patch_cells<0, double>(o, u, nullptr, s)) return rc;
+  if (int rc = patch_cells<0, false, double>(o, PatchField<double>{u, nullptr, PcgHead{}, nullptr}, s)) return rc;
   ApplyArgs a{u, res, base, nullptr, nullptr, 0.0, 0.0, nullptr, nullptr};
   return patch_gather<AP_STORE, double, double>(o, nullptr, a, s, nullptr);
 }

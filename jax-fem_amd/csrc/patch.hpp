@@ -2,6 +2,7 @@
 // the entry points the solvers call.
 #pragma once
 #include "apply.hpp"
+#include "pcg_scalars.hpp"
 
 namespace fem {
 
@@ -15,5 +16,11 @@ bool patch_operator_ok(const fem_patch_operator_t* op, bool residual = false);
 // FP32 vectors (the arithmetic is FP64).
 template <int MODE, typename TX, typename TY>
 int patch_apply(const fem_patch_operator_t& op, const ApplyArgsT<TX, TY>& a, hipStream_t s, int* parts = nullptr);
+
+// One CG product: begins the iteration (pcg_head), p_new = z + beta p_old, q = A p_new and the
+// *parts partials of <p_new, q> in part.
+template <typename T>
+int patch_pcg_product(const fem_patch_operator_t& op, const PcgHead& head, const T* z, const T* p_old, T* p_new, T* q,
+                      double* part, hipStream_t s, int* parts);
 
 }  // namespace fem

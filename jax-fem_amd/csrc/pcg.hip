@@ -7,15 +7,20 @@
 // exact boundary increment (solver.py:402-409), so the residual and search
 // direction vanish on those rows and CG runs on the SPD free block.
 //
-// Five launches per iteration k:
-//   P_k : p = z + beta p (row-local, in place)
+// Launches per iteration k:
+//   P_k : ends iteration k-1 (rz, rr, stop test, beta from B's partials, summed by
+//         every block); p = z + beta p (row-local, in place)
 //   A_k : q = A p, per-block <p, q> (one 64-row slice per block, W waves
-//         splitting its slots; the product gathers p only)
-//   RA_k: one block: pq = sum of A's partials, alpha = rz / pq
-//   B_k : x += alpha p, r -= alpha q, z = D^-1 r, per-block <r,z>, <r,r>
-//   RB_k: one block: rz, rr; convergence / NaN / maxiter test; beta = rz / rz_old
-// Forming p inside the product (gathering z and p_old per column) cost ~20% of
-// the product's bandwidth; the separate P pass streams 3 vectors once.
+//         splitting its slots; the product gathers p only), or the two kernels
+//         of a matrix-free product (patch.hip)
+//   B_k : alpha = rz / pq from A's partials, summed by every block;
+//         x += alpha p, r -= alpha q, z = D^-1 r, per-block <r,z>, <r,r>
+// Where the matrix stays in the caches, and in the matrix-free products, P's
+// work is done by the product's kernel, which gathers z and the old direction.
+// (On matrices read from HBM that gather costs ~20% of the product's bandwidth;
+// there P streams 3 vectors once, and a one-block kernel RA sums more than 2048
+// partials.)  The five kernels of separate reductions took 26 us per iteration
+// on small systems, of which 6 in the reductions and 8 in gaps; two take 13.
 // The reductions sum per-block partials in a fixed order (bit-reproducible);
 // no grid-wide fence or atomic is used.  Scalars live in device memory and
 // are written by one kernel and read by the next.
@@ -28,6 +33,7 @@
 // and at convergence; beta keeps the value of the recursion across a
 // replacement.
 #include "patch.hpp"
+#include "pcg_scalars.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -38,55 +44,46 @@ int fem_operator_apply_impl(const fem_operator_t* op, const double* x, double* y
 
 namespace fem {
 
-struct PcgScalars {
-  double rz;             // <r, z> of the current iteration
-  double alpha, beta;
-  double rr;             // <r, r> of the current iteration
-  double rr_true;        // |b - A x|^2 of the last true-residual evaluation
-  double pad0[3];
-  int32_t done, iter, nan, pad1;
-  int32_t pad2[4];
-};
-static_assert(sizeof(PcgScalars) <= 128, "host status buffer");
-
-// Sum of `n` partials starting at p, identical in every block (blockDim == 256).
-__device__ inline double block_reduce_partials(const double* __restrict__ p, int n, double* smem) {
-  double acc = 0.0;
-  for (int i = threadIdx.x; i < n; i += 256) acc += p[i];
-  return block_sum_256(acc, smem);
-}
-
-
-
-// Kernel P: p = z + beta p in place (beta = 0 at a start).
+// Kernel P: begins the iteration; p = z + beta p in place (beta = 0 at a start).
 template <typename T>
-__global__ __launch_bounds__(256) void k_pcg_p(int64_t n, const T* __restrict__ z, T* __restrict__ p,
-                                               const PcgScalars* sc) {
-  if (sc->done) return;
-  const T beta = T(sc->beta);
+__global__ __launch_bounds__(256) void k_pcg_p(int64_t n, const T* __restrict__ z, T* __restrict__ p, PcgHead head) {
+  __shared__ double smem[8];
+  bool done;
+  const T beta = T(pcg_head<256>(head, smem, &done));
+  if (done) return;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = z[i] + beta * p[i];
+    p[i] = fma(beta, p[i], z[i]);
 }
 
 // Kernel A: one 64-row slice per block; the W waves split the slots
 // (sell_slice_partial) and wave 0 combines them through LDS, stores
 // q = A p and the block's <p, q>.
-template <int V, bool DIFF, typename T>
-__global__ __launch_bounds__(SliceCfg<T>::NT) void k_pcg_a(fem_pattern_t pat, const T* __restrict__ vals,
-                                                           const T* __restrict__ p, T* __restrict__ q,
-                                                           const PcgScalars* sc, double* __restrict__ partA,
-                                                           int remap) {
-  constexpr int W = SliceCfg<T>::W, U = SliceCfg<T>::U, NT = SliceCfg<T>::NT;
-  __shared__ double smem[NT / 64];
+// FUSED: the kernel begins the iteration (pcg_head) and multiplies p = z + beta p_old, formed
+// where it is gathered; each row's own entries go to pn.
+template <int V, bool DIFF, typename T, bool FUSED, int W = SliceCfg<T>::W>
+__global__ __launch_bounds__(64 * W) void k_pcg_a(fem_pattern_t pat, const T* __restrict__ vals,
+                                                           const T* __restrict__ p, const T* __restrict__ z,
+                                                           T* __restrict__ pn, T* __restrict__ q,
+                                                           const PcgScalars* sc, PcgHead head,
+                                                           double* __restrict__ partA, int remap) {
+  constexpr int U = SliceCfg<T>::U, NT = 64 * W;
+  __shared__ double smem[2 * (NT / 64)];
   __shared__ double red[W][kSlice][V];
-  if (sc->done) return;
+  T beta = T(0);
+  if (FUSED) {
+    bool done;
+    beta = T(pcg_head<NT>(head, smem, &done));
+    if (done) return;
+  } else if (sc->done) {
+    return;
+  }
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t s = remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
   const int64_t row = pat.sell_row[s * kSlice + lane];
   const bool real = row >= 0;
   auto xat = [&](int64_t c, T (&xc)[V]) {
 #pragma unroll
-    for (int j = 0; j < V; ++j) xc[j] = p[c * V + j];
+    for (int j = 0; j < V; ++j) xc[j] = FUSED ? fma(beta, p[c * V + j], z[c * V + j]) : p[c * V + j];
   };
   T pr[V];
   xat(real ? row : 0, pr);
@@ -94,6 +91,10 @@ __global__ __launch_bounds__(SliceCfg<T>::NT) void k_pcg_a(fem_pattern_t pat, co
 #pragma unroll
   for (int j = 0; j < V; ++j) xr[j] = double(pr[j]);
   sell_slice_partial<V, DIFF, W, U, T>(pat, vals, s, w, lane, row, xat, xr, acc);
+  if (FUSED && w == 0 && real) {
+#pragma unroll
+    for (int j = 0; j < V; ++j) pn[row * V + j] = pr[j];
+  }
   if (w > 0) {
 #pragma unroll
     for (int i = 0; i < V; ++i) red[w][lane][i] = acc[i];
@@ -135,35 +136,24 @@ __global__ __launch_bounds__(1024) void k_pcg_ra(const double* __restrict__ part
   if (threadIdx.x == 0) sc->alpha = sc->rz / pq;
 }
 
-// RB: rz, rr of iteration k+1; stop test; beta.  nB <= 1024.
-__global__ __launch_bounds__(1024) void k_pcg_rb(const double* __restrict__ partB, int nB, PcgScalars* sc, int k,
-                                                 double tol2, int maxiter) {
-  __shared__ double smem[16];
-  const int i = threadIdx.x;
-  const double a0 = i < nB ? partB[i] : 0.0;
-  const double a1 = i < nB ? partB[nB + i] : 0.0;
-  const double rz = block_sum<1024>(a0, smem);
-  const double rr = block_sum<1024>(a1, smem);
-  if (sc->done) return;
-  if (threadIdx.x == 0) {
-    const bool bad = !isfinite(rr) || !isfinite(rz);
-    sc->beta = rz / sc->rz;
-    sc->rz = rz;
-    sc->rr = rr;
-    sc->iter = k + 1;
-    if (bad) sc->nan = 1;
-    if (bad || rr <= tol2 || k + 1 >= maxiter) sc->done = 1;
-  }
+// RB: rz, rr and beta of the iteration that ended, its stop test (head.next may be head.cur).
+__global__ __launch_bounds__(1024) void k_pcg_rb(PcgHead head) {
+  __shared__ double smem[32];
+  const PcgState s = pcg_state<1024>(head, smem);
+  __syncthreads();
+  if (threadIdx.x == 0) pcg_store(head.next, s, 1);
 }
 
 template <typename T, typename TX>
 __global__ __launch_bounds__(256) void k_pcg_b(int64_t n, TX* __restrict__ x, T* __restrict__ r,
                                                T* __restrict__ z, const T* __restrict__ p,
                                                const T* __restrict__ q, const T* __restrict__ dinv,
-                                               const PcgScalars* sc, double* __restrict__ partB) {
+                                               const PcgScalars* sc, const double* __restrict__ partA, int nA,
+                                               double* __restrict__ partB) {
   __shared__ double smem[8];
   if (sc->done) return;
-  const double alpha_d = sc->alpha;
+  // nA > 0: every block sums the <p, q> partials itself
+  const double alpha_d = nA > 0 ? sc->rz / block_reduce_partials(partA, nA, smem) : sc->alpha;
   const T alpha = T(alpha_d);
   T rz = T(0), rr = T(0);
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
@@ -241,6 +231,7 @@ __global__ __launch_bounds__(1024) void k_pcg_rr(const double* __restrict__ part
     sc->rr = rr;
     sc->done = 0;
     sc->iter = k;
+    sc->ready = 1;
     if (init) {
       sc->beta = 0.0;
       sc->nan = 0;
@@ -252,6 +243,12 @@ template <typename T>
 __global__ void k_fill(int64_t n, T* __restrict__ v, T val) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     v[i] = val;
+}
+
+template <typename T>
+__global__ void k_pcg_copy(int64_t n, const T* __restrict__ a, T* __restrict__ b) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+    b[i] = a[i];
 }
 
 // y = A x for FP64 x, y (standard form values of precision T).
@@ -283,6 +280,10 @@ __global__ __launch_bounds__(256) void k_spmv_x(fem_pattern_t pat, const T* __re
 }
 
 constexpr int kVecGrid = 1024;  // blocks of the vector kernels (partials per reduction)
+constexpr int kSumParts = 2048;  // most <p, q> partials that every block of the update kernel sums itself
+// Largest matrix whose product forms its direction itself (us per iteration, with and without):
+// FP64 3 MB 13 / 18, 28 MB 15.9 / 19.5, 38 MB 21.9 / 22.1; FP32 39 MB 17.3 / 18.9, 59 MB 35 / 32.5.
+constexpr double kFuseBytes = 48e6;
 
 struct EventPool {
   std::vector<hipEvent_t> e;
@@ -336,7 +337,7 @@ static int64_t ws_layout(const fem_pattern_t* pat, int precision, void* base, Ws
   o->partB = reinterpret_cast<double*>(take(2 * kVecGrid * 8));
   o->partR = reinterpret_cast<double*>(take(2 * kVecGrid * 8));
   o->partT = reinterpret_cast<double*>(take(kVecGrid * 8));
-  o->sc = reinterpret_cast<PcgScalars*>(take(sizeof(PcgScalars)));
+  o->sc = reinterpret_cast<PcgScalars*>(take(2 * sizeof(PcgScalars)));
   return off;
 }
 
@@ -362,7 +363,7 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
   }
   int gA = (int)grid_a(pat);  // partials of <p, q>
   const int gV = (int)std::min<int64_t>(ceil_div(n, 256), kVecGrid);
-  FEM_HIP(hipMemsetAsync(w.sc, 0, sizeof(PcgScalars), s));
+  FEM_HIP(hipMemsetAsync(w.sc, 0, 2 * sizeof(PcgScalars), s));
   hipLaunchKernelGGL(k_fill<T>, dim3(256), dim3(256), 0, s, n, p, T(0));
   FEM_LAUNCHED();
 
@@ -418,6 +419,15 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
   FEM_LAUNCHED();
   double rr_ref = rr_true;
   const int check = std::max(1, opt->check_every);
+  // Small matrices leave most of the chip idle at one workgroup of W waves per slice: up to 256
+  // slices (one per CU) 16 waves share a slice's slots, up to 768 eight (FP64 Poisson of 13,824
+  // cells 15.3 -> 12.0 us per iteration, of 32,768 cells 16.0 -> 14.9).
+  // The direction update runs inside the product (which then gathers z and the old direction) where
+  // the matrix stays in the caches or is not read; the new direction goes to a second buffer.  That is
+  // y's, free between the true residuals: so a batch of status-free iterations has to be even.
+  T* p2 = (T*)w.y;
+  const double sell_bytes = double(pat->sell_blocks) * (V * V * sizeof(T) + 4);
+  const bool fused = check % 2 == 0 && (pop ? true : sell_bytes <= kFuseBytes);
   const double delta2 = kMixed ? opt->reliable_delta * opt->reliable_delta : 0.0;
   EventPool ev(opt->timing ? 4 * check : 0);
   if (!ev.ok) {
@@ -429,29 +439,53 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
   int iter = 0;
   for (;;) {
     const int iter0 = iter;
+    T* pc = p;  // the current direction
     for (int m = 0; m < check; ++m) {
-      const int k = iter0 + m;
+      PcgScalars* sc = w.sc + 1 - (m & 1);  // the state of this iteration
+      const PcgHead head{w.sc + (m & 1), sc, w.partB, gV, tol2, opt->maxiter};
+      T* pn = fused ? (pc == p ? p2 : p) : p;
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m], s));
-      hipLaunchKernelGGL(k_pcg_p<T>, dim3(gV), dim3(256), 0, s, n, (const T*)z, p, (const PcgScalars*)w.sc);
+      if (!fused) hipLaunchKernelGGL(k_pcg_p<T>, dim3(gV), dim3(256), 0, s, n, (const T*)z, p, head);
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 1], s));
-      if (pop) {
-        ApplyArgsT<T, T> a{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, w.partA, &w.sc->done};
+      if (pop && fused) {
+        if (int rc = patch_pcg_product<T>(*pop, head, z, pc, pn, q, w.partA, s, &gA)) return rc;
+      } else if (pop) {
+        ApplyArgsT<T, T> a{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, w.partA, &sc->done};
         if (int rc = patch_apply<AP_PQ, T, T>(*pop, a, s, &gA)) return rc;
+      } else if (fused) {
+        auto product = [&](auto waves) {
+          constexpr int W = decltype(waves)::value;
+          hipLaunchKernelGGL((k_pcg_a<V, kDiff, T, true, W>), dim3(gA), dim3(64 * W), 0, s, *pat, vals, (const T*)pc,
+                             (const T*)z, pn, q, (const PcgScalars*)sc, head, w.partA, opt->xcd_remap);
+        };
+        if (gA <= 256)
+          product(std::integral_constant<int, 16>{});
+        else if (gA <= 768)
+          product(std::integral_constant<int, 8>{});
+        else
+          product(std::integral_constant<int, SliceCfg<T>::W>{});
       } else {
-        hipLaunchKernelGGL((k_pcg_a<V, kDiff, T>), dim3(gA), dim3(SliceCfg<T>::NT), 0, s, *pat, vals, (const T*)p, q,
-                           (const PcgScalars*)w.sc, w.partA, opt->xcd_remap);
+        hipLaunchKernelGGL((k_pcg_a<V, kDiff, T, false>), dim3(gA), dim3(SliceCfg<T>::NT), 0, s, *pat, vals,
+                           (const T*)p, (const T*)z, p, q, (const PcgScalars*)sc, head, w.partA, opt->xcd_remap);
       }
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 2], s));
-      hipLaunchKernelGGL(k_pcg_ra, dim3(1), dim3(1024), 0, s, (const double*)w.partA, gA, w.sc);
-      hipLaunchKernelGGL((k_pcg_b<T, double>), dim3(gV), dim3(256), 0, s, n, x, r, z, (const T*)p, (const T*)q, dinv,
-                         (const PcgScalars*)w.sc, w.partB);
-      hipLaunchKernelGGL(k_pcg_rb, dim3(1), dim3(1024), 0, s, (const double*)w.partB, gV, w.sc, k, tol2,
-                         opt->maxiter);
+      const int sumA = gA <= kSumParts ? gA : 0;
+      if (!sumA) hipLaunchKernelGGL(k_pcg_ra, dim3(1), dim3(1024), 0, s, (const double*)w.partA, gA, sc);
+      hipLaunchKernelGGL((k_pcg_b<T, double>), dim3(gV), dim3(256), 0, s, n, x, r, z, (const T*)pn, (const T*)q, dinv,
+                         (const PcgScalars*)sc, (const double*)w.partA, sumA, w.partB);
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 3], s));
+      pc = pn;
     }
+    hipLaunchKernelGGL(k_pcg_rb, dim3(1), dim3(1024), 0, s,
+                       PcgHead{w.sc + (check & 1), w.sc, w.partB, gV, tol2, opt->maxiter});
     FEM_LAUNCHED();
     if (int rc = read_status()) return rc;
     iter = host_sc->iter;
+    // the last direction of a batch that ended inside: back from the shared buffer
+    if (fused && ((iter - iter0) & 1)) {
+      hipLaunchKernelGGL(k_pcg_copy<T>, dim3(gV), dim3(256), 0, s, n, (const T*)p2, p);
+      FEM_LAUNCHED();
+    }
     if (opt->timing) {
       // only the launches that ran an iteration (the rest returned on `done`)
       for (int m = 0; m < std::min(check, iter - iter0); ++m) {

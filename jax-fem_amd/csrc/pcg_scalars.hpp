@@ -1,0 +1,87 @@
+// Scalars of the Jacobi-PCG iteration and the reductions that a consuming kernel does
+// itself (pcg.hip, patch.hip).
+#pragma once
+#include "fem_common.hpp"
+
+namespace fem {
+
+struct PcgScalars {
+  double rz;             // <r, z> of the current iteration
+  double alpha, beta;
+  double rr;             // <r, r> of the current iteration
+  double rr_true;        // |b - A x|^2 of the last true-residual evaluation
+  double pad0[3];
+  int32_t done, iter, nan;
+  int32_t ready;         // 1: rz, rr and beta are those of the partials last written; 0: to be summed
+  int32_t pad2[4];
+};
+static_assert(sizeof(PcgScalars) <= 128, "host status buffer");
+
+// Sum of `n` partials starting at p, identical in every block (blockDim == 256).
+__device__ inline double block_reduce_partials(const double* __restrict__ p, int n, double* smem) {
+  double acc = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) acc += p[i];
+  return block_sum_256(acc, smem);
+}
+
+// End of an iteration, done by every block of the kernel that begins the next one: <r, z> and
+// <r, r> from the update kernel's partials, the stop test and beta.  The state is read from
+// `cur` and block 0 writes it to `next` (two slots, so no block reads what another writes).
+// A reduction of at most 1024 partials by every block costs about 1 us of latency where a
+// kernel of its own cost 3 us and its launch 1.6 us.
+struct PcgHead {
+  const PcgScalars* cur;
+  PcgScalars* next;
+  const double* part;    // (2 * parts): <r, z>, then <r, r>
+  int parts;
+  double tol2;
+  int maxiter;
+};
+
+// The state after the partials; smem holds 2 * NT / 64 doubles.  The partials are loaded with
+// the state, not after it.
+struct PcgState {
+  double rz, rr, beta;
+  int32_t done, iter, nan;
+};
+
+template <int NT>
+__device__ inline PcgState pcg_state(const PcgHead& h, double* smem) {
+  double a0 = 0.0, a1 = 0.0;
+  for (int i = threadIdx.x; i < h.parts; i += NT) {
+    a0 += h.part[i];
+    a1 += h.part[h.parts + i];
+  }
+  PcgState s{h.cur->rz, h.cur->rr, h.cur->beta, h.cur->done, h.cur->iter, h.cur->nan};
+  if (s.done || h.cur->ready) return s;
+  block_sum2<NT>(a0, a1, smem);
+  const bool bad = !isfinite(a1) || !isfinite(a0);
+  s.beta = a0 / s.rz;
+  s.rz = a0;
+  s.rr = a1;
+  s.iter += 1;
+  if (bad) s.nan = 1;
+  if (bad || a1 <= h.tol2 || s.iter >= h.maxiter) s.done = 1;
+  return s;
+}
+
+__device__ inline void pcg_store(PcgScalars* out, const PcgState& s, int ready) {
+  out->rz = s.rz;
+  out->rr = s.rr;
+  out->beta = s.beta;
+  out->done = s.done;
+  out->iter = s.iter;
+  out->nan = s.nan;
+  out->ready = ready;
+}
+
+// beta of the iteration that begins, or done = true.
+template <int NT>
+__device__ inline double pcg_head(const PcgHead& h, double* smem, bool* done) {
+  const PcgState s = pcg_state<NT>(h, smem);
+  if (blockIdx.x == 0 && threadIdx.x == 0) pcg_store(h.next, s, 0);
+  *done = s.done != 0;
+  return s.beta;
+}
+
+}  // namespace fem

@@ -260,6 +260,8 @@ class DeviceProblem:
         self._bc_sources = None
         self._mat_cache = {}
         self.buffers = {}
+        if self.patch_plan is not None:
+            self.buffers['patch_part'] = dm.empty(self.patch_plan.entries * self.V)
         self.material = None
         self.param = None
         self.load = None
@@ -811,8 +813,6 @@ class DeviceProblem:
         """Descriptor of the matrix-free tangent at u (fem_patch_operator_t); u is needed by the
         hyperelastic law only."""
         dm = self.dm
-        if 'patch_part' not in self.buffers:
-            self.buffers['patch_part'] = dm.empty(self.patch_plan.entries * self.V)
         op = _lib.FemPatchOperator()
         op.mesh, op.mat, op.plan = C.pointer(dm.desc), C.pointer(mat_desc), C.pointer(self.patch_plan)
         op.u = u.data_ptr() if u is not None else None
