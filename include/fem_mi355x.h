@@ -249,6 +249,13 @@ int fem_cell_tangent(const fem_mesh_t* mesh, const fem_material_t* mat, int32_t 
  * U[c][q][i] = sum_a u[cells[c][a]][i] * N_a(q) (FP64, (C, Q, vec)).  Either
  * output may be NULL. */
 int fem_quad_grad(const fem_mesh_t* mesh, const double* u, double* G, double* U, void* stream);
+/* The `top` quadrature points of largest |grad u| (greatest component; points with
+ * a non-finite gradient last) and `spread` points evenly over the mesh: idx
+ * (top + spread) point numbers c*Q+q, G (top + spread, vec, 3) their grad u.
+ * top, spread <= 48; ws >= fem_grad_samples_ws_bytes(mesh). */
+int64_t fem_grad_samples_ws_bytes(const fem_mesh_t* mesh);
+int fem_grad_samples(const fem_mesh_t* mesh, const double* u, int32_t top, int32_t spread, int64_t* idx, double* G,
+                     void* ws, void* stream);
 /* Tangent of a mass term whose map depends on u (the jacfwd of the mass
  * kernel, problem.py:216-236, 262-266): adds to the per-cell tangents
  * Ke[c][a][b][i][k] += sum_q N_a(q) N_b(q) M[c][q][i][k] JxW(c, q), where

@@ -120,6 +120,8 @@ _SIGNATURES = {
     'fem_geometry': (C.c_int, [_P(FemMesh), _vp, _vp, _vp, _vp]),
     'fem_cell_tangent': (C.c_int, [_P(FemMesh), _P(FemMaterial), _i32, _vp, _vp, _vp]),
     'fem_quad_grad': (C.c_int, [_P(FemMesh), _vp, _vp, _vp, _vp]),
+    'fem_grad_samples_ws_bytes': (_i64, [_P(FemMesh)]),
+    'fem_grad_samples': (C.c_int, [_P(FemMesh), _vp, _i32, _i32, _vp, _vp, _vp, _vp]),
     'fem_cell_mass_tangent': (C.c_int, [_P(FemMesh), _vp, _i32, _vp, _vp]),
     'fem_cell_mass_jvp': (C.c_int, [_P(FemMesh), _vp, _vp, _vp, _vp]),
     'fem_cell_matvec': (C.c_int, [_P(FemMesh), _vp, _vp, _vp, _vp]),
