@@ -389,42 +389,45 @@ int fem_patch_residual(const fem_patch_operator_t* op, const double* u, const do
 /* ---- single-pass HEX8 assembly (problem.py:447-460 and solver.py:522-526 in
  *      one kernel, optionally with the residual scatter of problem.py:426-437)
  * The cell tangents are formed and summed straight into the SELL values: a
- * workgroup owns one 64-row slice and walks the cells incident to its rows in
- * chunks; no per-cell tangent buffer exists.  The plan (built once per pattern)
- * lists each slice's incident cells and re-expresses every contribution as a
- * position in that list. */
+ * wave owns eight block rows (a group of eight consecutive lanes of a slice)
+ * and walks the cells incident to them; no per-cell tangent buffer exists.  The
+ * plan (built once per pattern) lists each group's incident cells and, for each
+ * (cell, local node) pair of a row, the slots its eight blocks go to. */
 typedef struct {
   const int32_t* slice_cell_ptr; /* (num_slices + 1)                           */
-  const int32_t* slice_cells;    /* unique incident cells of each slice, in chunk
-                                    order: cells whose lowest slice lane is even
-                                    first, each group by ascending id         */
-  const int32_t* slice_pair_ptr; /* (num_slices + 1)                           */
-  const int32_t* slice_pairs;    /* the slice's (cell, local node a, row lane)
-                                    pairs, sorted keys (rank * 8 + a) * 64 +
-                                    lane, rank = position in slice_cells      */
-  const int32_t* contrib_loc;    /* (num_cells*N*N), aligned with contrib_idx:
-                                    pair * N + b (pair = index in the slice's
-                                    pair list), ascending within each slot    */
+  const int32_t* slice_cells;    /* per slice: the end offsets of its 8 groups'
+                                    lists, then the lists: the group's unique
+                                    incident cells, ascending                 */
+  const int32_t* slice_pair_ptr; /* not read (may be NULL)                     */
+  const int32_t* slice_pairs;    /* not read (may be NULL)                     */
+  const int32_t* contrib_loc;    /* (num_cells*N*N), rows where contrib_idx has
+                                    them: 8 words per (cell, local node a) pair,
+                                    by ascending cell.  Word j, of the slots
+                                    j + 8 m: bits 4m..4m+3 the column node whose
+                                    block goes there (8: none), 16-18 a, 19 the
+                                    cell names a node twice, 20-31 position of
+                                    the cell in the group's list              */
   int32_t        max_slots;      /* largest slot count of a slice (<= 32)     */
   int32_t        max_pairs;      /* largest pair count of a slice (<= 1024)   */
 } fem_assembly_plan_t;
 
-/* Plan, pass 1: unique incident cells and (cell, row node) pairs per slice
- * (counts, to be scanned into slice_cell_ptr and slice_pair_ptr).  err_flag > 0
- * after the call: a slice's rows have more than 4096 incidences (use the
- * two-pass path). */
+/* Plan, pass 1: entries of slice_cells and (cell, row node) pairs per slice
+ * (the former to be scanned into slice_cell_ptr, the latter for max_pairs).
+ * err_flag > 0 after the call: a slice's rows have more than 4096 incidences
+ * (use the two-pass path). */
 int fem_assembly_plan_counts(const fem_pattern_t* pat, const int32_t* inc_ptr, const int32_t* inc_idx,
                              int32_t* slice_cell_counts, int32_t* slice_pair_counts, int32_t* err_flag,
                              void* stream);
-/* Plan, pass 2: slice_cells, slice_pairs and contrib_loc (err_flag as above, or
- * 1 when a contribution's cell is missing from its slice list). */
+/* Plan, pass 2: slice_cells and contrib_loc (err_flag as above, or 1 when the
+ * pattern and the incidences do not belong together).  slice_pair_ptr and
+ * slice_pairs are not used (may be NULL). */
 int fem_assembly_plan_fill(const fem_pattern_t* pat, const int32_t* inc_ptr, const int32_t* inc_idx,
                            const int32_t* slice_cell_ptr, const int32_t* slice_pair_ptr, int32_t* slice_cells,
                            int32_t* slice_pairs, int32_t* contrib_loc, int32_t* err_flag, void* stream);
 /* Assemble the tangent of HEX8 cells with 8 quadrature points at u into the
  * SELL values: FP64 standard form (precision FEM_F64, form FEM_FORM_STANDARD)
  * or FP32 difference form (FEM_F32, FEM_FORM_DIFFERENCE); the cell tangents
- * are FP64 and each matrix value is their FP64 sum in the plan's chunk
+ * are FP64 and each matrix value is their FP64 sum in the plan's cell
  * order, rounded once.  dinv (may be NULL): Jacobi inverse diagonal in `precision`.  res (may
  * be NULL): R(u) without Dirichlet rows, = base (may be NULL) + the scattered
  * internal force, FP64.  Dirichlet rows are applied afterwards by

@@ -7,23 +7,24 @@
 //   solver.py:522-526   PETSc setValuesCOO: sum the COO duplicates into AIJ
 //   problem.py:426-437  scatter of the cell residuals (optional, same pass)
 //
-// Work split.  A workgroup owns one SELL slice (64 block rows, lane l = row
-// sell_row[64 s + l]), so every matrix block it writes is its own and no
-// atomics are needed.  The plan lists the slice's (cell, local node a, row
-// lane) pairs in a fixed order (cells in chunk order, see k_slice_reorder) and
-// re-expresses each slot's contributions as (pair, column node b) entries.
-// The pairs are walked in chunks of at most 16 cells / 32 pairs; per chunk the
-// cells' geometry is staged in LDS, one thread per (pair, b) forms the 3x3
-// block K_ab (and the pair's residual contribution), and the thread owning a
-// slot (wave w owns the slots w, w + 8, ... of its lane's row) adds its
-// blocks in pair order.  The sums do not depend on scheduling
-// (bit-reproducible).  After the last chunk every lane stores its slots: one
-// coalesced 64-lane store per matrix value.  The difference form's row sum and
-// the Jacobi inverse diagonal are formed from the accumulators in a fixed order.
+// Work split.  A wave owns eight block rows (a group: eight consecutive lanes
+// of one SELL slice) and shares nothing with other waves but the table of
+// reference gradients: no barrier after the start, no atomics.  The plan lists
+// the group's incident cells by ascending id and, for each row, its pairs
+// (cell, local node a) in the same order, with the slots of the row that the
+// pair's eight blocks go to.
 //
-// A cell's Jacobian is recomputed once per slice that touches it (about 4.5
-// times for a structured HEX8 box with 64-row slices); each tangent block is
-// computed exactly once.
+// A cell's geometry and point records are recomputed once per group that
+// touches it (about 4.5 times per 8 rows for a structured HEX8 box, against 4.1
+// with 64-row groups); each tangent block is computed exactly once.
+//
+// What bounds it: LDS (60 to 70 % of its cycles: gradients read per block, blocks
+// handed over) and the latencies that two waves per SIMD leave open; the matrix
+// itself is written at 6 TB/s, past the caches.  64^3 Neo-Hookean cells with FP64
+// values 2630 -> 930 us, 128 x 64 x 64 elastic cells 2000 -> 870 us (the stores alone
+// take 220 us of these, a wave's first loads 130 us), 80 x 31 x 31 SIMP cells 342 ->
+// 170 us, against one workgroup per slice that met at four barriers per chunk (80 to
+// 110 KB of LDS, one or two workgroups per CU, most threads idle in most phases).
 #include "element.hpp"
 
 #include <algorithm>
@@ -31,29 +32,57 @@
 
 namespace fem {
 
-constexpr int kAsmThreads = 512;   // 8 waves per slice
-constexpr int kAsmWaves = kAsmThreads / 64;
-constexpr int kSliceIncCap = 4096;  // incident (cell, node) entries of one slice's rows
+constexpr int kGroupRows = 8;                // rows (and cells per chunk) of a wave
+constexpr int kGroups = kSlice / kGroupRows; // groups per slice: the header of its cell list
+constexpr int kSliceIncCap = 4096;           // incident (cell, node) entries of one slice's rows
+constexpr int kSlicePairCap = 1024;          // pairs of a slice the assembly takes (the rank has 12 bits)
+constexpr int kAsmMaxK = 4;                  // slots per lane: rows of at most 8 * 4 = 32 blocks
+
+// A pair's word for slot class j (slots j, j + 8, j + 16, j + 24 of its row):
+//   bits 0-15   four nibbles: the column node b whose block goes to slot j + 8 m, 8 = none
+//   bits 16-18  a     bit 19  the cell names a node twice     bits 20-31  rank of the cell
+constexpr uint32_t kNoSlots = 0x8888u, kTwice = 1u << 19;
+constexpr int kRankShift = 20;
+
+// An LDS pointer whose value the compiler does not know: constant offsets from it go into the
+// instructions (from a known address it adds each of them up anew).
+using LdsD = __attribute__((address_space(3))) double;
+__device__ inline LdsD* lds_base(double* p) {
+  LdsD* q = (LdsD*)p;
+  asm volatile("" : "+v"(q));
+  return q;
+}
+
+// Orders LDS accesses of one wave: the hardware executes them in order, so only the compiler
+// has to keep the order.
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // ------------------------------------------------------------------ plan
-// Unique incident cells of each slice's rows, ascending.  FILL = false writes
-// the count per slice; FILL = true writes the cells at out_ptr[s].
+// Cell lists of each slice: kGroups end offsets, then the groups' unique incident
+// cells, ascending.  FILL = false writes the slice's entry and pair counts;
+// FILL = true writes the entries at out_ptr[s].  One wave per group.
 template <bool FILL>
-__global__ __launch_bounds__(256) void k_slice_cells(int64_t num_slices, int32_t N,
-                                                     const int32_t* __restrict__ sell_row,
-                                                     const int32_t* __restrict__ inc_ptr,
-                                                     const int32_t* __restrict__ inc_idx,
-                                                     const int32_t* __restrict__ out_ptr, int32_t* __restrict__ out,
-                                                     int32_t* __restrict__ pair_out, int32_t* __restrict__ err) {
-  __shared__ int32_t buf[kSliceIncCap];
-  __shared__ int32_t s_off[65];
-  __shared__ int32_t s_scan[256];
+__global__ __launch_bounds__(64 * kGroups) void k_slice_cells(int64_t num_slices,
+                                                              const int32_t* __restrict__ sell_row,
+                                                              const int32_t* __restrict__ inc_ptr,
+                                                              const int32_t* __restrict__ inc_idx,
+                                                              const int32_t* __restrict__ out_ptr,
+                                                              int32_t* __restrict__ out,
+                                                              int32_t* __restrict__ pair_out,
+                                                              int32_t* __restrict__ err) {
+  __shared__ int32_t s_buf[2 * kSliceIncCap];  // the groups' entries, each padded to a power of two
+  __shared__ int32_t s_off[kSlice + 1];        // first entry of each row
+  __shared__ int32_t s_n[kGroups];             // unique cells of each group
   const int64_t s = blockIdx.x;
-  const int t = threadIdx.x;
+  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
   if (s >= num_slices) return;
   int row = -1, b = 0, e = 0;
-  if (t < 64) {
-    row = sell_row[s * 64 + t];
+  if (t < kSlice) {
+    row = sell_row[s * kSlice + t];
     if (row >= 0) {
       b = inc_ptr[row];
       e = inc_ptr[row + 1];
@@ -63,10 +92,10 @@ __global__ __launch_bounds__(256) void k_slice_cells(int64_t num_slices, int32_t
   if (t == 0) s_off[0] = 0;
   __syncthreads();
   if (t == 0)
-    for (int i = 1; i <= 64; ++i) s_off[i] += s_off[i - 1];
+    for (int i = 1; i <= kSlice; ++i) s_off[i] += s_off[i - 1];
   __syncthreads();
-  const int total = s_off[64];
-  if (!FILL && t == 0) pair_out[s] = total <= kSliceIncCap ? total : 0;  // the slice's (cell, row node) pairs
+  const int total = s_off[kSlice];
+  if (!FILL && t == 0) pair_out[s] = total <= kSliceIncCap ? total : 0;
   if (total > kSliceIncCap) {
     if (t == 0) {
       atomicMax(err, total);
@@ -74,568 +103,625 @@ __global__ __launch_bounds__(256) void k_slice_cells(int64_t num_slices, int32_t
     }
     return;
   }
-  if (t < 64)
-    for (int j = b; j < e; ++j) buf[s_off[t] + (j - b)] = inc_idx[j] / N;
-  int P = 1;
-  while (P < total) P <<= 1;
-  for (int i = total + t; i < P; i += 256) buf[i] = INT32_MAX;
+  // the group's entries at s_buf[beg, beg + n), padded to P <= max(1, 2 n): the segments of the
+  // groups start at twice their entry offset and do not overlap (P <= 2 n for n >= 1)
+  const int g0 = s_off[w * kGroupRows], n = s_off[(w + 1) * kGroupRows] - g0;
+  int32_t* buf = s_buf + 2 * g0;
+  if (t < kSlice) {
+    const int q0 = s_off[(t / kGroupRows) * kGroupRows];
+    for (int j = b; j < e; ++j) s_buf[2 * q0 + (s_off[t] - q0) + (j - b)] = inc_idx[j] >> 3;
+  }
+  int P = n > 0 ? 1 : 0;
+  while (P < n) P <<= 1;
+  for (int i = n + lane; i < P; i += 64) buf[i] = INT32_MAX;
   __syncthreads();
-  // bitonic sort of buf[0, P)
-  for (int k = 2; k <= P; k <<= 1) {
+  for (int k = 2; k <= P; k <<= 1)
     for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = t; i < P; i += 256) {
+      for (int i = lane; i < P; i += 64) {
         const int l = i ^ j;
         if (l > i) {
           const int32_t x = buf[i], y = buf[l];
-          const bool up = (i & k) == 0;
-          if ((x > y) == up) {
+          if ((x > y) == ((i & k) == 0)) {
             buf[i] = y;
             buf[l] = x;
           }
         }
       }
-      __syncthreads();
+      wave_fence();
     }
-  }
-  // unique entries: each thread takes a contiguous run of the sorted list
-  const int per = (total + 255) / 256;
-  const int i0 = min(total, t * per), i1 = min(total, i0 + per);
+  // unique entries: each lane takes a contiguous run of the sorted list
+  const int per = (n + 63) / 64, i0 = min(n, lane * per), i1 = min(n, i0 + per);
   int cnt = 0;
   for (int i = i0; i < i1; ++i) cnt += (i == 0 || buf[i] != buf[i - 1]) ? 1 : 0;
-  s_scan[t] = cnt;
+  int scan = cnt;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int v = __shfl_up(scan, off, 64);
+    if (lane >= off) scan += v;
+  }
+  if (lane == 63) s_n[w] = scan;
   __syncthreads();
-  for (int off = 1; off < 256; off <<= 1) {
-    const int a = t >= off ? s_scan[t - off] : 0;
-    __syncthreads();
-    s_scan[t] += a;
-    __syncthreads();
+  int before = 0, all = 0;
+  for (int i = 0; i < kGroups; ++i) {
+    if (i < w) before += s_n[i];
+    all += s_n[i];
   }
   if (!FILL) {
-    if (t == 255) out[s] = s_scan[255];
+    if (t == 0) out[s] = kGroups + all;
     return;
   }
-  int pos = out_ptr[s] + s_scan[t] - cnt;
+  int32_t* o = out + out_ptr[s];
+  if (lane == 63) o[w] = before + scan;
+  o += kGroups + before + scan - cnt;
   for (int i = i0; i < i1; ++i)
-    if (i == 0 || buf[i] != buf[i - 1]) out[pos++] = buf[i];
+    if (i == 0 || buf[i] != buf[i - 1]) *o++ = buf[i];
 }
 
-// contrib_loc[t] = (position of the cell in its slice's cell list) * N*N + a*N + b
-// for every contribution t of every row (one thread per slice lane).
-__global__ __launch_bounds__(256) void k_contrib_local(fem_pattern_t pat, const int32_t* __restrict__ sc_ptr,
-                                                       const int32_t* __restrict__ sc, int32_t* __restrict__ loc,
-                                                       int32_t* __restrict__ err) {
-  const int64_t g = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (g >= pat.num_slices * kSlice) return;
-  const int row = pat.sell_row[g];
+// The words of every pair: loc[8 p + j] for slot class j of the row's pair p, rows' pairs by
+// ascending cell (a row with n pairs has 8 n contributions, so its words start where its
+// contributions do).  One thread per (row, j).
+__global__ __launch_bounds__(kSlice* kGroupRows) void k_pair_words(fem_pattern_t pat,
+                                                                   const int32_t* __restrict__ inc_ptr,
+                                                                   const int32_t* __restrict__ inc_idx,
+                                                                   const int32_t* __restrict__ sc_ptr,
+                                                                   const int32_t* __restrict__ sc,
+                                                                   uint32_t* __restrict__ loc,
+                                                                   int32_t* __restrict__ err) {
+  if (*err) return;  // the plan is refused
+  const int64_t s = blockIdx.x;
+  const int l = threadIdx.x >> 3, j = threadIdx.x & 7, g = l / kGroupRows;
+  const int row = pat.sell_row[s * kSlice + l];
   if (row < 0) return;
-  const int64_t s = g >> 6;
-  const int NN = pat.nodes_per_cell * pat.nodes_per_cell;
-  const int32_t* list = sc + sc_ptr[s];
-  const int n = sc_ptr[s + 1] - sc_ptr[s];
-  const int t0 = pat.contrib_ptr[pat.row_ptr[row]], t1 = pat.contrib_ptr[pat.row_ptr[row + 1]];
-  for (int t = t0; t < t1; ++t) {
-    const int32_t e = pat.contrib_idx[t];
-    const int32_t c = e / NN;
-    int lo = 0, hi = n;
+  const int32_t* hd = sc + sc_ptr[s];
+  const int first = g ? hd[g - 1] : 0, nc = hd[g] - first;
+  const int32_t* list = hd + kGroups + first;
+  const int32_t* inc = inc_idx + inc_ptr[row];
+  const int np = inc_ptr[row + 1] - inc_ptr[row];
+  const int rb = pat.row_ptr[row], len = pat.row_ptr[row + 1] - rb, t0 = pat.contrib_ptr[rb];
+  if (pat.contrib_ptr[rb + len] - t0 != 8 * np) {
+    atomicMax(err, 1);
+    return;
+  }
+  auto order = [&](int32_t e) {  // position of incidence e among the row's
+    int p = 0;
+    for (int i = 0; i < np; ++i) p += inc[i] < e ? 1 : 0;
+    return p;
+  };
+  for (int i = 0; i < np; ++i) {
+    const int32_t e = inc[i], c = e >> 3;
+    int lo = 0, hi = nc;
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
       if (list[mid] < c) lo = mid + 1; else hi = mid;
     }
-    if (lo >= n || list[lo] != c) {
+    if (lo >= nc || list[lo] != c || lo >= kSlicePairCap) {
       atomicMax(err, 1);
       return;
     }
-    loc[t] = lo * NN + (e - c * NN);
+    loc[t0 + 8 * order(e) + j] = ((uint32_t)lo << kRankShift) | ((uint32_t)(e & 7) << 16) | kNoSlots;
+  }
+  // every slot of the row: its own class' nibbles, and whether a pair has two blocks for it
+  for (int k = 0; k < len; ++k) {
+    const int c0 = pat.contrib_ptr[rb + k], c1 = pat.contrib_ptr[rb + k + 1];
+    int32_t prev = -1;
+    for (int t = c0; t < c1; ++t) {
+      const int32_t v = pat.contrib_idx[t], e = v >> 3;
+      if ((k & 7) != j && e != prev) {
+        prev = e;
+        continue;
+      }
+      uint32_t& word = loc[t0 + 8 * order(e) + j];
+      if (e == prev) word |= kTwice;
+      if ((k & 7) == j && k < 8 * kAsmMaxK) {
+        const int sh = 4 * (k >> 3);
+        const uint32_t b = v & 7, old = (word >> sh) & 15u;
+        word = (word & ~(15u << sh)) | (min(b, old) << sh);  // 8 = none yet; the lowest of two
+      }
+      prev = e;
+    }
   }
 }
 
-// Chunk order of each slice's cell list.  A cell is ranked by the parity of the
-// lowest slice lane among its nodes, then by id: on a structured HEX8 box in
-// natural row order, the cells of one parity touch every row of a z-line slice
-// once, so the assembly's fixed-size cell chunks keep every row lane busy
-// (in id order a chunk covers half the rows).  Rewrites the slice's cell list
-// in that order and re-expresses contrib_loc in it, each slot's contributions
-// sorted by position (the order the assembly sums them in).  One 64-thread
-// workgroup per slice; integer LDS minima only, so the result is deterministic.
-__global__ __launch_bounds__(64) void k_slice_reorder(fem_pattern_t pat, const int32_t* __restrict__ inc_ptr,
-                                                      const int32_t* __restrict__ inc_idx,
-                                                      const int32_t* __restrict__ sc_ptr, int32_t* __restrict__ sc,
-                                                      const int32_t* __restrict__ sp_ptr, int32_t* __restrict__ sp,
-                                                      int32_t* __restrict__ loc, const int32_t* __restrict__ err) {
-  __shared__ int32_t s_cell[kSliceIncCap];
-  __shared__ int32_t s_rank[kSliceIncCap];
-  __shared__ int32_t s_key[kSliceIncCap];
-  __shared__ int32_t s_cnt[64];
-  if (*err) return;  // the plan is refused (a slice over capacity or a cell missing from its list)
-  const int64_t s = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int c0 = sc_ptr[s], n = sc_ptr[s + 1] - c0;
-  const int N = pat.nodes_per_cell, NN = N * N;
-  for (int i = lane; i < n; i += 64) {
-    s_cell[i] = sc[c0 + i];
-    s_rank[i] = 64;  // lowest lane among the cell's nodes, 64 = none yet
+// ------------------------------------------------------- point records
+// What a block K_ab needs of a quadrature point besides the gradients h_a, h_b of its
+// shape functions: NR doubles, weighted with JxW (point()), and the block itself (add(),
+// summed over the points, then finish()).  kSpatial: the gradients are taken in the
+// current configuration.  kRow: the law has a vector per (a, q) that all b share.
+template <class MAT>
+struct TanPoint;
+
+// K = w k g_a . g_b
+template <>
+struct TanPoint<MatPoisson> {
+  static constexpr int NR = 1;
+  static constexpr bool kSpatial = false, kRow = false, kIso = false;
+  __device__ static void point(const MatPoisson::St<double>& s, double w, double (&r)[NR]) { r[0] = w * s.k; }
+  __device__ static void add(const LdsD* r, const double (&)[3], const double (&a)[3], const double (&b)[3], double&,
+                             double (&K)[1][1]) {
+    K[0][0] += r[0] * (a[0] * b[0] + a[1] * b[1] + a[2] * b[2]);
   }
-  __syncthreads();
-  const int row = pat.sell_row[s * kSlice + lane];
-  auto find = [&](int32_t c) {
-    int lo = 0, hi = n;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (s_cell[mid] < c) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-  };
-  if (row >= 0)
-    for (int j = inc_ptr[row]; j < inc_ptr[row + 1]; ++j) {
-      const int p = find(inc_idx[j] / N);
-      if (p < n) atomicMin(&s_rank[p], lane);
-    }
-  __syncthreads();
-  // parity-0 cells first, each group in id order: rank = group offset + count of the
-  // group's cells before it (per-lane runs, then a scan over the 64 lanes)
-  const int per = (n + 63) / 64;
-  const int i0 = min(n, lane * per), i1 = min(n, i0 + per);
-  int odd = 0;
-  for (int i = i0; i < i1; ++i) odd += s_rank[i] & 1;
-  s_cnt[lane] = odd;
-  __syncthreads();
-  if (lane == 0)
-    for (int l = 1; l < 64; ++l) s_cnt[l] += s_cnt[l - 1];
-  __syncthreads();
-  const int n_odd = s_cnt[63], n_even = n - n_odd;
-  int o = lane ? s_cnt[lane - 1] : 0;  // odd cells before i0
-  int e = i0 - o;                      // even cells before i0
-  for (int i = i0; i < i1; ++i) {
-    const bool is_odd = s_rank[i] & 1;
-    s_rank[i] = is_odd ? n_even + o++ : e++;
-  }
-  __syncthreads();
-  for (int i = lane; i < n; i += 64) sc[c0 + s_rank[i]] = s_cell[i];
-  // the slice's (cell, local node a, row lane) pairs, keyed (rank * 8 + a) * 64 + lane and
-  // sorted: the order the assembly forms and sums the blocks in
-  const int p0 = sp_ptr[s], np = sp_ptr[s + 1] - p0;
-  const int ib = row >= 0 ? inc_ptr[row] : 0, ie = row >= 0 ? inc_ptr[row + 1] : 0;
-  __syncthreads();
-  s_cnt[lane] = ie - ib;
-  __syncthreads();
-  if (lane == 0)
-    for (int l = 1; l < 64; ++l) s_cnt[l] += s_cnt[l - 1];
-  __syncthreads();
-  {
-    int pos = lane ? s_cnt[lane - 1] : 0;
-    for (int j = ib; j < ie; ++j) {
-      const int32_t e = inc_idx[j];
-      const int q = find(e / N);
-      s_key[pos++] = ((q < n ? s_rank[q] : 0) * 8 + e % N) * 64 + lane;
+};
+
+// Isotropic linear laws: lambda = c0 E and mu = c1 E at every point, so with
+// M = sum_q JxW E g_a (x) g_b,  K_ab = c0 M + c1 M^T + c1 tr(M) I.  The slots sum M.
+template <bool S>
+struct TanPoint<MatElastic<S>> {
+  static constexpr int NR = 1;
+  static constexpr bool kSpatial = false, kRow = false, kIso = true;
+  __device__ static void add(const LdsD* r, const double (&)[3], const double (&a)[3], const double (&b)[3], double&,
+                             double (&K)[3][3]) {
+    const double w = r[0];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double wa = w * a[i];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) K[i][k] += wa * b[k];
     }
   }
-  int P2 = 1;
-  while (P2 < np) P2 <<= 1;
-  for (int i = np + lane; i < P2; i += 64) s_key[i] = INT32_MAX;
-  __syncthreads();
-  for (int k = 2; k <= P2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = lane; i < P2; i += 64) {
-        const int l = i ^ j;
-        if (l > i) {
-          const int32_t x = s_key[i], y = s_key[l];
-          if ((x > y) == ((i & k) == 0)) {
-            s_key[i] = y;
-            s_key[l] = x;
-          }
-        }
-      }
-      __syncthreads();
+};
+
+// Neo-Hookean in the current configuration: with h = F^-T grad N, b = F F^T,
+//   K_ab = c_fh (b h_a (x) h_b + h_a (x) b h_b) + c_hh h_a (x) h_b + c_tr h_b (x) h_a
+//          + ma (h_a . b h_b) I,   c_fh = -2/3 ma
+// (MatNeoHookean::tangent with F g = b h).  Record: c_fh b (6), c_hh, c_tr.  The
+// row vector is t_a = c_fh b h_a + c_hh h_a: 42 operations per point instead of 106.
+template <>
+struct TanPoint<MatNeoHookean> {
+  static constexpr int NR = 8;
+  static constexpr bool kSpatial = true, kRow = true, kIso = false;
+  __device__ static void bh(const LdsD* r, const double (&h)[3], double (&f)[3]) {
+    f[0] = r[0] * h[0] + r[3 * 64] * h[1] + r[4 * 64] * h[2];
+    f[1] = r[3 * 64] * h[0] + r[1 * 64] * h[1] + r[5 * 64] * h[2];
+    f[2] = r[4 * 64] * h[0] + r[5 * 64] * h[1] + r[2 * 64] * h[2];
+  }
+  __device__ static void row(const LdsD* r, const double (&a)[3], double (&t)[3]) {
+    bh(r, a, t);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) t[i] += r[6 * 64] * a[i];
+  }
+  __device__ static void add(const LdsD* r, const double (&t)[3], const double (&a)[3], const double (&b)[3],
+                             double& d, double (&K)[3][3]) {
+    double f[3];
+    bh(r, b, f);
+    d += a[0] * f[0] + a[1] * f[1] + a[2] * f[2];
+    const double ct = r[7 * 64];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double cb = ct * b[i];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) K[i][k] += t[i] * b[k] + a[i] * f[k] + cb * a[k];
     }
   }
-  for (int i = lane; i < np; i += 64) sp[p0 + i] = s_key[i];
-  if (row < 0) return;
-  auto pair_of = [&](int32_t key) {
-    int lo = 0, hi = np;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (s_key[mid] < key) lo = mid + 1; else hi = mid;
-    }
-    return lo;
-  };
-  const int rb = pat.row_ptr[row], len = pat.row_ptr[row + 1] - rb;
-  for (int k = 0; k < len; ++k) {
-    const int t0 = pat.contrib_ptr[rb + k], t1 = pat.contrib_ptr[rb + k + 1];
-    for (int t = t0; t < t1; ++t) {
-      const int v = loc[t];  // in [0, n * NN): k_contrib_local found every contribution's cell
-      const int a = (v % NN) / N, b = v % N;
-      loc[t] = pair_of((s_rank[v / NN] * 8 + a) * 64 + lane) * N + b;
-    }
-    for (int t = t0 + 1; t < t1; ++t) {  // insertion sort of the slot's few entries
-      const int v = loc[t];
-      int u = t - 1;
-      while (u >= t0 && loc[u] > v) {
-        loc[u + 1] = loc[u];
-        --u;
-      }
-      loc[u + 1] = v;
+};
+
+// J2: MatJ2::tangent with the symmetric deviator.  Record: s (6), w lam_t, w mu_t, w gam.
+template <>
+struct TanPoint<MatJ2> {
+  static constexpr int NR = 9;
+  static constexpr bool kSpatial = false, kRow = true, kIso = false;
+  __device__ static void point(const MatJ2::St<double>& s, double w, double (&r)[NR]) {
+    r[0] = s.s[0], r[1] = s.s[4], r[2] = s.s[8], r[3] = s.s[1], r[4] = s.s[2], r[5] = s.s[5];
+    r[6] = w * s.lam_t, r[7] = w * s.mu_t, r[8] = w * s.gam;
+  }
+  __device__ static void row(const LdsD* r, const double (&a)[3], double (&t)[3]) {
+    TanPoint<MatNeoHookean>::bh(r, a, t);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) t[i] *= r[8 * 64];
+  }
+  __device__ static void add(const LdsD* r, const double (&t)[3], const double (&a)[3], const double (&b)[3],
+                             double& d, double (&K)[3][3]) {
+    double sb[3];
+    TanPoint<MatNeoHookean>::bh(r, b, sb);
+    const double l = r[6 * 64], m = r[7 * 64];
+    d += m * (a[0] * b[0] + a[1] * b[1] + a[2] * b[2]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const double la = l * a[i], mb = m * b[i];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) K[i][k] += la * b[k] + mb * a[k] - t[i] * sb[k];
     }
   }
-}
+};
 
 // ------------------------------------------------------------- assembly
-template <class MAT>
-struct alignas(8) StRow {
-  typename MAT::template St<double> s[8];
-  double pad;  // odd stride between cells
+constexpr int kAsmThreads = 128;             // 2 waves: 16 rows, whole 128-byte lines of FP64 values
+constexpr int kGQ = 25, kGC = 8 * kGQ;       // strides of the staged gradients: [cell][q][node][3]
+constexpr int kXC = 49;                      // stride of a cell's staged coordinates and u
+
+// LDS of one wave: the chunk's gradients (its coordinates and u before them), point
+// records, weighted stresses and the blocks in exchange.
+template <class MAT, bool RES>
+struct AsmWave {
+  static constexpr int NP = RES ? (MAT::V == 1 ? 3 : 6) : 0, NR = TanPoint<MAT>::NR;
+  // values of a block exchanged at a time: as many as leave eight waves' LDS on a CU (20,480 bytes
+  // each with the table), at least a row vector's three
+  static constexpr int NX = MAT::V == 1 ? 1 : NR == 1 ? 9 : NR <= 8 ? 5 : 3;
+  double g[8 * kGC];
+  double rec[NR + NP][64];
+  double ex[65 * NX];  // the last entry stays zero: the block of a slot that receives none
 };
 
-// Isotropic linear laws (elasticity, SIMP): lambda = c0 E and mu = c1 E at every
-// point, so K_ab = c0 M + c1 M^T + c1 tr(M) I with the single weighted sum
-// M = sum_q JxW E g_a (x) g_b (the closed form of MatElastic::tangent).
-template <class MAT>
-struct IsoLinear : std::false_type {
-  __device__ static double E(const fem_material_t&, int64_t) { return 1.0; }
-};
-template <bool S>
-struct IsoLinear<MatElastic<S>> : std::true_type {
-  // the modulus factor E of lambda = c0 E, mu = c1 E at point cq
-  __device__ static double E(const fem_material_t& m, int64_t cq) {
-    return S ? MatElastic<S>::modulus(m, m.param[cq]) : 1.0;
-  }
-};
-
-constexpr int kAsmMaxK = 4;               // slots per thread: rows of at most 8 * 4 = 32 blocks
-constexpr int kResWave0 = kAsmWaves - 3;  // waves summing the residual's components
-constexpr int kAsmGS = 8 * 8 * 3 + 1;     // odd stride (in doubles) between cells' gradients
-
-// Chunk sizes: at most CH cells and PM (cell, row node) pairs per chunk (on a
-// z-line slice every cell holds two of the slice's nodes, so PM = 2 CH).
-template <class MAT>
-struct AsmCfg {
-  using St = typename MAT::template St<double>;
-  static constexpr bool kBig = sizeof(St) > 4 * sizeof(double);  // Neo-Hookean, J2: large point states
-  static constexpr int CH = kBig ? 16 : 32;
-  static constexpr int PM = 2 * CH;
-};
-constexpr int kSlicePairCap = 1024;  // pairs (and cells) of one slice, staged in LDS
-
-// The slice's (cell, local node a, row lane) pairs are walked in chunks; per
-// chunk:
-//   A1  one thread per (cell, node): node coordinates (and u) to LDS;
-//   A2  one thread per (cell, quadrature point): Jacobian, inverse, JxW, the 8
-//       physical gradients, the material state (and the weighted stress);
-//   B1  one thread per (pair, column node b): the 3x3 block K_ab of the pair's
-//       cell (the pair's 8 threads share g_a and read the 8 g_b side by side)
-//       and, for b < V, component b of the pair's residual contribution, all
-//       staged in LDS;
-//   B2  every owner thread (row lane, slot) adds the staged blocks of its
-//       slots, in pair order (which is the plan's fixed cell order).
+// One wave per group.  The group's cells are walked in chunks of eight; per chunk
+//   1  lane (cell, node): coordinates (and u) to LDS, loaded one chunk ahead;
+//   2  lane (cell, q): Jacobian, inverse, the eight gradients, the point record (and the
+//      weighted stress);
+//   3  while a row has pairs in the chunk: lane (row, b) forms block K_ab of the row's next
+//      pair (the eight lanes share h_a and the records) and hands it to the lane that owns
+//      its slot (lane j of a row owns the slots j, j + 8, ...), which adds it in registers.
+// Every sum runs in the plan's order, so the result does not depend on scheduling.
+// With the residual, lane (row, q) sums its point's part over the row's pairs and the
+// eight lanes are added at the end.
 template <class MAT, typename TO, bool DIFF, bool RES>
-__global__ __launch_bounds__(kAsmThreads) void k_assemble_hex8(
+__global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
     fem_mesh_t mesh, fem_material_t mat, fem_pattern_t pat, const int32_t* __restrict__ sc_ptr,
-    const int32_t* __restrict__ sc, const int32_t* __restrict__ sp_ptr, const int32_t* __restrict__ sp,
-    const int32_t* __restrict__ cloc, const double* __restrict__ u, TO* __restrict__ vals, TO* __restrict__ dinv,
-    const double* __restrict__ base, double* __restrict__ res) {
-  constexpr int N = 8, Q = 8, V = MAT::V, VV = V * V, MAXK = kAsmMaxK, GS = kAsmGS;
-  constexpr int CH = AsmCfg<MAT>::CH, PM = AsmCfg<MAT>::PM;
-  constexpr bool kIso = IsoLinear<MAT>::value;
-  __shared__ double s_dN[Q][N][3];
-  __shared__ double s_w[Q];
-  __shared__ double s_g[CH][GS];
-  __shared__ double s_wq[CH][Q + 1];                        // JxW (elastic laws: JxW E)
-  __shared__ StRow<MAT> s_st[kIso ? 1 : CH];
-  __shared__ double s_K[PM][N][VV];                         // staged blocks of the chunk's pairs
-  __shared__ double s_R[RES ? PM : 1][V];                   // staged residual contributions
-  __shared__ int64_t s_c[CH];
-  __shared__ int32_t s_key[kSlicePairCap];   // the slice's pair keys
-  __shared__ int32_t s_cid[kSlicePairCap];   // the slice's cells, in rank order
-  // A1 stages coordinates and u in s_buf; with the residual, A2's weighted stresses reuse it
-  constexpr int kXU = CH * N * (3 + V);
-  constexpr int kP = RES ? CH * (Q * V * 3 + 1) : 0;
-  __shared__ double s_buf[kXU > kP ? kXU : kP];
-  double(*s_x)[N][3] = reinterpret_cast<double(*)[N][3]>(s_buf);
-  double(*s_u)[N][V] = reinterpret_cast<double(*)[N][V]>(s_buf + CH * N * 3);
-  double(*s_P)[Q * V * 3 + 1] = reinterpret_cast<double(*)[Q * V * 3 + 1]>(s_buf);
-  // the difference form's row sums are staged in s_K after the last chunk, half the waves at a time
-  constexpr int kHalf = kAsmWaves / 2;
-  static_assert(kHalf * kSlice * VV <= PM * N * VV, "row-sum staging does not fit in s_K");
-  double(*s_red)[kSlice][VV] = reinterpret_cast<double(*)[kSlice][VV]>(&s_K[0][0][0]);
+    const int32_t* __restrict__ sc, const uint32_t* __restrict__ loc, const double* __restrict__ u,
+    TO* __restrict__ vals, TO* __restrict__ dinv, const double* __restrict__ base, double* __restrict__ res) {
+  using TP = TanPoint<MAT>;
+  constexpr int V = MAT::V, VV = V * V, M = kAsmMaxK, NR = TP::NR;
+  constexpr bool kU = MAT::kNeedsU || RES;
+  constexpr bool kParam = !std::is_same<MAT, MatJ2>::value;
+  __shared__ double s_dN[8 * kGQ], s_w[8];
+  __shared__ AsmWave<MAT, RES> s_wave[kAsmThreads / 64];
+  for (int i = threadIdx.x; i < 8 * 24; i += kAsmThreads) s_dN[(i / 24) * kGQ + i % 24] = mesh.shape_grads_ref[i];
+  if (threadIdx.x < 8) s_w[threadIdx.x] = mesh.quad_weights[threadIdx.x];
+  __syncthreads();
+  AsmWave<MAT, RES>& L = s_wave[threadIdx.x >> 6];
+  const int lane = threadIdx.x & 63, hi8 = lane >> 3, j = lane & 7;
+  const int64_t gid = blockIdx.x * (int64_t)(kAsmThreads / 64) + (threadIdx.x >> 6);
+  const int64_t s = gid / kGroups;
+  const int gr = (int)(gid % kGroups), rl = gr * kGroupRows + hi8;  // the lane's row in the slice
 
-  const int64_t s = blockIdx.x;
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const double iso_c1 = kIso ? mat.c[1] : 0.0;  // elastic laws: the slots sum M; K is formed at the end
-  load_tables(mesh, s_dN, s_w);
-  const int sbase = pat.slice_ptr[s];
-  const int L = (pat.slice_ptr[s + 1] - sbase) >> 6;
-  const int row = pat.sell_row[s * kSlice + lane];
-  const bool real = row >= 0;
-  const int rb = real ? pat.row_ptr[row] : 0;
-  const int len = real ? pat.row_ptr[row + 1] - rb : 0;
-  const int ds = real ? pat.diag_slot[row] : -1;
-  const int c0 = sc_ptr[s], ncs = sc_ptr[s + 1] - c0;
-  const int p_base = sp_ptr[s], np = sp_ptr[s + 1] - p_base;
-  // np, ncs <= kSlicePairCap: fem_assemble refuses plans with larger slices
-  for (int i = t; i < np; i += kAsmThreads) s_key[i] = sp[p_base + i];
-  for (int i = t; i < ncs; i += kAsmThreads) s_cid[i] = sc[c0 + i];
+  const int sbase = pat.slice_ptr[s], nslots = (pat.slice_ptr[s + 1] - sbase) >> 6;
+  const int row = pat.sell_row[s * kSlice + rl];
+  int ds = -1, np = 0;  // pairs of the row
+  const uint32_t* pw = loc + j;
+  if (row >= 0) {
+    const int rb = pat.row_ptr[row], t0 = pat.contrib_ptr[rb];
+    np = (pat.contrib_ptr[pat.row_ptr[row + 1]] - t0) >> 3;
+    pw += np > 0 ? t0 : 0;
+    ds = pat.diag_slot[row];
+  }
+  // word: the row's next pair; ahead: what was loaded for pair ip, the one after it (beyond the
+  // row's last pair the load repeats that one and is not used)
+  int ip = 1;
+  uint32_t word = pw[0], ahead = pw[8 * min(1, max(np - 1, 0))];
+  if (np == 0) word = ~0u;
+  constexpr int NX = AsmWave<MAT, RES>::NX;
+  LdsD *const lg = lds_base(L.g), *const lr = lds_base(&L.rec[0][0]), *const lx = lds_base(L.ex);
+  if (lane < NX) lx[64 * NX + lane] = 0.0;
 
-  double acc[MAXK][VV];
-  // cur: next contribution of each owned slot; nxt: its entry (pair * 8 + b), loaded one
-  // contribution ahead
-  int cur[MAXK], cend[MAXK], nxt[MAXK];
+  const int32_t* cl = sc + sc_ptr[s];
+  const int first = gr ? cl[gr - 1] : 0, nc = cl[gr] - first;
+  cl += kGroups + first;
+  auto cell_at = [&](int k) { return cl[min(k * 8 + hi8, nc - 1)]; };
+
+  // the point's reference gradients: kept where the registers suffice, else read from LDS each time
+  constexpr bool kKeep = TP::kIso && !RES;
+  double kept[kKeep ? 24 : 1];
+  if constexpr (kKeep)
 #pragma unroll
-  for (int m = 0; m < MAXK; ++m) {
-    const int k = w + kAsmWaves * m;
-    cur[m] = cend[m] = 0;
-    if (k < len) {
-      cur[m] = pat.contrib_ptr[rb + k];
-      cend[m] = pat.contrib_ptr[rb + k + 1];
-    }
-    nxt[m] = cur[m] < cend[m] ? cloc[cur[m]] : INT32_MAX;
+    for (int i = 0; i < 24; ++i) kept[i] = s_dN[j * kGQ + i];
+  double acc[M][VV];
+#pragma unroll
+  for (int m = 0; m < M; ++m)
 #pragma unroll
     for (int v = 0; v < VV; ++v) acc[m][v] = 0.0;
-  }
-  // residual: component ri of the row is summed by wave kResWave0 + ri from the diagonal
-  // slot's list, whose entries are exactly the row's pairs
-  const int ri = w - kResWave0;
-  const bool resw = RES && real && ri >= 0 && ri < V;
-  int rcur = 0, rend = 0, rnxt = INT32_MAX;
-  if (resw) {
-    rcur = pat.contrib_ptr[rb + ds];
-    rend = pat.contrib_ptr[rb + ds + 1];
-    rnxt = rcur < rend ? cloc[rcur] : INT32_MAX;
-  }
-  double r = 0.0;
-  __syncthreads();
+  double rs[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) rs[i] = 0.0;
 
-  for (int p0 = 0; p0 < np;) {
-    // ---- the chunk: pairs [p0, p1), cells of ranks [r0, r0 + ncell)
-    const int r0 = s_key[p0] >> 9;
-    int lo = p0 + 1, hi = min(np, p0 + PM);  // first pair of rank >= r0 + CH, at most p0 + PM
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if ((s_key[mid] >> 9) < r0 + CH) lo = mid + 1; else hi = mid;
+  // loaded ahead: cell, node, coordinates and parameter of the coming chunk (1), cell and node of
+  // the one after it (2), cells of the third
+  double xr[3] = {0, 0, 0}, ur[V], par = 1.0;
+#pragma unroll
+  for (int i = 0; i < V; ++i) ur[i] = 0.0;
+  int32_t c1 = 0, n1 = 0, c2 = 0, n2 = 0, c3 = 0;
+  // without parameters the load reads a weight and is not used (a branch would split the geometry)
+  const bool has_par = kParam && mat.has_param;
+  const double* par_base = has_par ? mat.param : mesh.quad_weights;
+  auto load_chunk = [&]() {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) xr[i] = mesh.points[(int64_t)n1 * 3 + i];
+    if constexpr (kU)
+#pragma unroll
+      for (int i = 0; i < V; ++i) ur[i] = u[(int64_t)n1 * V + i];
+    if constexpr (kParam) par = par_base[has_par ? (int64_t)c1 * 8 + j : 0];
+  };
+  if (nc > 0) {
+    c1 = cell_at(0);
+    n1 = mesh.cells[(int64_t)c1 * 8 + j];
+    c2 = cell_at(1);
+    n2 = mesh.cells[(int64_t)c2 * 8 + j];
+    c3 = cell_at(2);
+    load_chunk();
+  }
+
+  for (int k = 0; k * 8 < nc; ++k) {
+    // ---- 1: the chunk's coordinates to LDS; fetch the next chunk's
+    wave_fence();
+    const int32_t c0 = c1;
+    const double p0 = has_par ? par : 1.0;
+    {
+      LdsD* x = lg + hi8 * kXC + j * 6;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) x[i] = xr[i];
+      if constexpr (kU)
+#pragma unroll
+        for (int i = 0; i < V; ++i) x[3 + i] = ur[i];
     }
-    const int p1 = lo;
-    const int ncell = (s_key[p1 - 1] >> 9) - r0 + 1;
-    // ---- A1: node coordinates (and u)
-    if (t < ncell * N) {
-      const int cc = t / N, a = t % N;
-      const int64_t c = s_cid[r0 + cc];
-      if (a == 0) s_c[cc] = c;
-      const int64_t na = mesh.cells[c * N + a];
-#pragma unroll
-      for (int j = 0; j < 3; ++j) s_x[cc][a][j] = mesh.points[na * 3 + j];
-      if (MAT::kNeedsU || RES)
-#pragma unroll
-        for (int i = 0; i < V; ++i) s_u[cc][a][i] = u[na * V + i];
+    c1 = c2, n1 = n2;
+    c2 = c3;
+    load_chunk();
+    n2 = mesh.cells[(int64_t)c2 * 8 + j];
+    c3 = cell_at(k + 3);
+    wave_fence();
+    __builtin_amdgcn_sched_barrier(0);
+    double E = 1.0;
+    if constexpr (std::is_same<MAT, MatElastic<true>>::value) {
+      E = MAT::modulus(mat, p0);
+      __builtin_amdgcn_sched_barrier(0);  // the power's temporaries end before the Jacobian's begin
     }
-    __syncthreads();
-    // ---- A2: per (cell, quadrature point) geometry and material state
-    double Pw[RES ? V : 1][3];
-    const int acc_cc = t / Q, acc_q = t % Q;
-    const bool a2 = t < ncell * Q;
-    if (a2) {
-      const int cc = acc_cc, q = acc_q;
-      const int64_t c = s_c[cc];
-      const double x00 = s_x[cc][0][0], x01 = s_x[cc][0][1], x02 = s_x[cc][0][2];
-      double J[9];
+    // ---- 2: geometry, gradients and records of (cell hi8, point j)
+    {
+      double J[9], U[V][3];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) J[k] = 0.0;
+      for (int i = 0; i < 9; ++i) J[i] = 0.0;
 #pragma unroll
-      for (int a = 1; a < N; ++a) {
-        const double d0 = s_x[cc][a][0] - x00, d1 = s_x[cc][a][1] - x01, d2 = s_x[cc][a][2] - x02;
+      for (int i = 0; i < V; ++i) U[i][0] = U[i][1] = U[i][2] = 0.0;
+      const LdsD* x = lg + hi8 * kXC;
+      const LdsD* tab = lds_base(&s_dN[j * kGQ]);
+      auto dn = [&](int i) { return kKeep ? kept[kKeep ? i : 0] : tab[i]; };
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const double dn = s_dN[q][a][j];
-          J[0 * 3 + j] += d0 * dn;
-          J[1 * 3 + j] += d1 * dn;
-          J[2 * 3 + j] += d2 * dn;
+      for (int a = 1; a < 8; ++a) {
+        const double e0 = dn(a * 3), e1 = dn(a * 3 + 1), e2 = dn(a * 3 + 2);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          const double d = x[a * 6 + i] - x[i];
+          J[i * 3 + 0] += d * e0;
+          J[i * 3 + 1] += d * e1;
+          J[i * 3 + 2] += d * e2;
         }
-      }
-      const double det = det3(J);
-      double iJ[9];
-      inv3(J, det, iJ);
-      const double jxw = det * s_w[q];
-      double G[V][3];
-#pragma unroll
-      for (int i = 0; i < V; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) G[i][j] = 0.0;
-#pragma unroll
-      for (int a = 0; a < N; ++a) {
-        const double e0 = s_dN[q][a][0], e1 = s_dN[q][a][1], e2 = s_dN[q][a][2];
-        double g[3];
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          g[j] = e0 * iJ[0 * 3 + j] + e1 * iJ[1 * 3 + j] + e2 * iJ[2 * 3 + j];
-          s_g[cc][(q * N + a) * 3 + j] = g[j];
-        }
-        if (MAT::kNeedsU || RES) {
+        if constexpr (kU)
 #pragma unroll
           for (int i = 0; i < V; ++i) {
-            const double ua = s_u[cc][a][i];
-#pragma unroll
-            for (int j = 0; j < 3; ++j) G[i][j] += ua * g[j];
+            const double d = x[a * 6 + 3 + i] - x[3 + i];
+            U[i][0] += d * e0;
+            U[i][1] += d * e1;
+            U[i][2] += d * e2;
           }
-        }
+        if (a == 3 || a == 5) __builtin_amdgcn_sched_barrier(0);
       }
-      const auto st = MAT::template prep<double>(mat, c * Q + q, G);
-      if constexpr (!kIso) s_st[cc].s[q] = st;
-      s_wq[cc][q] = kIso ? jxw * IsoLinear<MAT>::E(mat, c * Q + q) : jxw;  // elastic laws: JxW E
-      if (RES) {
-        double P[V][3];
-        MAT::stress(st, G, P);
+      const double det = det3(J), w = det * s_w[j];
+      double iJ[9], r[NR];
+      inv3(J, det, iJ);
+      [[maybe_unused]] double P[6];
+      if constexpr (TP::kSpatial) {
+        // F = j J^-1 with j = J + grad_ref u; h = j^-T dN
+        double jc[9], F[9];
 #pragma unroll
-        for (int i = 0; i < V; ++i)
+        for (int i = 0; i < 9; ++i) jc[i] = J[i] + U[i / 3][i % 3];
 #pragma unroll
-          for (int j = 0; j < 3; ++j) Pw[i][j] = P[i][j] * jxw;
-      }
-    }
-    if (RES) {
-      // the weighted stresses overwrite the coordinates' storage once every thread has read it
-      __syncthreads();
-      if (a2)
+        for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int i = 0; i < V; ++i)
+          for (int l = 0; l < 3; ++l)
+            F[i * 3 + l] = jc[i * 3] * iJ[l] + jc[i * 3 + 1] * iJ[3 + l] + jc[i * 3 + 2] * iJ[6 + l];
+        const double b[6] = {F[0] * F[0] + F[1] * F[1] + F[2] * F[2], F[3] * F[3] + F[4] * F[4] + F[5] * F[5],
+                             F[6] * F[6] + F[7] * F[7] + F[8] * F[8], F[0] * F[3] + F[1] * F[4] + F[2] * F[5],
+                             F[0] * F[6] + F[1] * F[7] + F[2] * F[8], F[3] * F[6] + F[4] * F[7] + F[5] * F[8]};
+        const double detc = det3(jc), Jd = detc / det;
+        inv3(jc, detc, iJ);
+        // Jd^-2/3; NaN for an inverted point, like pow(Jd, -2/3)
+        const double rc = rcbrt(Jd), wp = w * p0, I1 = b[0] + b[1] + b[2];
+        const double ma = mat.c[0] * wp * (Jd < 0.0 ? __builtin_nan("") : rc * rc), kp = mat.c[1] * wp;
 #pragma unroll
-          for (int j = 0; j < 3; ++j) s_P[acc_cc][(acc_q * V + i) * 3 + j] = Pw[i][j];
-    }
-    __syncthreads();
-    // ---- B1: one block per (pair, column node)
-    if (t < (p1 - p0) * N) {
-      const int pp = t / N, b = t % N;
-      const int key = s_key[p0 + pp];
-      const int cc = (key >> 9) - r0, a = (key >> 6) & 7;
-      double K[V][V];
+        for (int i = 0; i < 6; ++i) r[i] = (-2.0 / 3.0) * ma * b[i];
+        const double kj = kp * (Jd * Jd - Jd), mi = ma * I1 * (1.0 / 3.0);
+        r[6] = (2.0 / 3.0) * mi + kj + kp * (Jd * Jd);
+        r[7] = mi - kj;
+        if constexpr (RES)
 #pragma unroll
-      for (int i = 0; i < V; ++i)
-#pragma unroll
-        for (int k = 0; k < V; ++k) K[i][k] = 0.0;
-      if constexpr (kIso) {
-        // M = sum_q JxW E g_a (x) g_b
-#pragma unroll
-        for (int q = 0; q < Q; ++q) {
-          const double* ga = &s_g[cc][(q * N + a) * 3];
-          const double* gb = &s_g[cc][(q * N + b) * 3];
-          const double wq = s_wq[cc][q];
-          const double gb0 = gb[0], gb1 = gb[1], gb2 = gb[2];
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            const double wa = wq * ga[i];
-            K[i][0] += wa * gb0;
-            K[i][1] += wa * gb1;
-            K[i][2] += wa * gb2;
-          }
-        }
+          for (int i = 0; i < 6; ++i) P[i] = ma * b[i] + (i < 3 ? kj - mi : 0.0);  // Kirchhoff stress
       } else {
-#pragma unroll 2
-        for (int q = 0; q < Q; ++q)
-          MAT::tangent(s_st[cc].s[q], &s_g[cc][(q * N + a) * 3], &s_g[cc][(q * N + b) * 3], s_wq[cc][q], K);
+        double G[V][3];
+        if constexpr (kU)
+#pragma unroll
+          for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int l = 0; l < 3; ++l) G[i][l] = U[i][0] * iJ[l] + U[i][1] * iJ[3 + l] + U[i][2] * iJ[6 + l];
+        typename MAT::template St<double> st;
+        if constexpr (TP::kIso) {
+          r[0] = w * E;
+          st.lam = mat.c[0] * E;
+          st.mu = mat.c[1] * E;
+        } else {
+          if constexpr (std::is_same<MAT, MatPoisson>::value)
+            st.k = mat.c[0] * p0;
+          else
+            st = MAT::template prep<double>(mat, (int64_t)c0 * 8 + j, G);
+          TP::point(st, w, r);
+        }
+        if constexpr (RES) {
+          double S[V][3];
+          MAT::stress(st, G, S);
+          if constexpr (V == 1) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) P[i] = w * S[0][i];
+          } else {  // symmetric
+            P[0] = w * S[0][0], P[1] = w * S[1][1], P[2] = w * S[2][2];
+            P[3] = w * S[0][1], P[4] = w * S[0][2], P[5] = w * S[1][2];
+          }
+        }
       }
+      wave_fence();  // the gradients overwrite the coordinates
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < NR; ++i) lr[i * 64 + lane] = r[i];
+      if constexpr (RES)
+#pragma unroll
+        for (int i = 0; i < AsmWave<MAT, RES>::NP; ++i) lr[(NR + i) * 64 + lane] = P[i];
+      tab = lds_base(&s_dN[j * kGQ]);
+      LdsD* g = lg + hi8 * kGC + j * kGQ;
+#pragma unroll
+      for (int a = 0; a < 8; ++a) {
+        const double e0 = dn(a * 3), e1 = dn(a * 3 + 1), e2 = dn(a * 3 + 2);
+#pragma unroll
+        for (int l = 0; l < 3; ++l) g[a * 3 + l] = e0 * iJ[l] + e1 * iJ[3 + l] + e2 * iJ[6 + l];
+      }
+    }
+    // ---- 3: the rows' pairs of this chunk
+    const uint32_t lim = (uint32_t)(k + 1) * 8u;
+    do {  // every chunk has a pair
+      const bool active = (word >> kRankShift) < lim;
+      const uint32_t cur = active ? word : kNoSlots | ((uint32_t)k * 8u << kRankShift);
+      // no branch around the fetch: one would make the compiler copy every accumulator
+      word = active ? (ip < np ? ahead : ~0u) : word;
+      ip += active ? 1 : 0;
+      ahead = pw[8 * max(min(ip, np - 1), 0)];
+      const int cc = (int)(cur >> kRankShift) - k * 8, a = (cur >> 16) & 7;
+      const LdsD* ga = lg + cc * kGC + a * 3;
+      const LdsD* gb = lg + cc * kGC + j * 3;
+      const LdsD* rec = lr + cc * 8;
+      wave_fence();
+      if constexpr (TP::kRow || RES) {  // lane (row, q = j)
+        const double ha[3] = {ga[j * kGQ], ga[j * kGQ + 1], ga[j * kGQ + 2]};
+        if constexpr (TP::kRow) {
+          double t[3];
+          TP::row(rec + j, ha, t);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) lx[lane * 3 + i] = t[i];
+        }
+        if constexpr (RES) {
+          const LdsD* p = rec + j + NR * 64;
+          double f[3];
+          if constexpr (V == 1)
+            f[0] = p[0] * ha[0] + p[64] * ha[1] + p[128] * ha[2];
+          else
+            TanPoint<MatNeoHookean>::bh(p, ha, f);
+#pragma unroll
+          for (int i = 0; i < V; ++i) rs[i] += active ? f[i] : 0.0;
+        }
+        wave_fence();
+      }
+      double K[V][V], d = 0.0;
 #pragma unroll
       for (int i = 0; i < V; ++i)
 #pragma unroll
-        for (int k = 0; k < V; ++k) s_K[pp][b][i * V + k] = K[i][k];
-      if (RES && b < V) {
-        double rr = 0.0;
+        for (int l = 0; l < V; ++l) K[i][l] = 0.0;
 #pragma unroll
-        for (int q = 0; q < Q; ++q)
+      for (int q = 0; q < 8; ++q) {
+        const double ha[3] = {ga[q * kGQ], ga[q * kGQ + 1], ga[q * kGQ + 2]};
+        const double hb[3] = {gb[q * kGQ], gb[q * kGQ + 1], gb[q * kGQ + 2]};
+        double t[3] = {0, 0, 0};
+        if constexpr (TP::kRow)
 #pragma unroll
-          for (int j = 0; j < 3; ++j) rr += s_P[cc][(q * V + b) * 3 + j] * s_g[cc][(q * N + a) * 3 + j];
-        s_R[RES ? pp : 0][b] = rr;
+          for (int i = 0; i < 3; ++i) t[i] = lx[(hi8 * 8 + q) * 3 + i];
+        TP::add(rec + q, t, ha, hb, d, K);
       }
-    }
-    __syncthreads();
-    // ---- B2: owners add their slots' blocks of this chunk, in pair order
-    const int lim = p1 * N;
+      if constexpr (TP::kRow) {
+        const double dd = TP::kSpatial ? -1.5 * d : d;  // Neo-Hookean: the records hold c_fh = -2/3 ma
 #pragma unroll
-    for (int m = 0; m < MAXK; ++m) {
-      int e = nxt[m];
-      while (e < lim) {
-        ++cur[m];
-        const int en = cur[m] < cend[m] ? cloc[cur[m]] : INT32_MAX;
-        const double* kb = &s_K[e / N - p0][e % N][0];
+        for (int i = 0; i < V; ++i) K[i][i] += dd;
+      }
+      if (__any((cur & kTwice) != 0)) {
+        // a cell naming a node twice: the lowest lane of equal columns takes their sum
+        const int32_t node = mesh.cells[(int64_t)cl[min((int)(cur >> kRankShift), nc - 1)] * 8 + j];
+        double S[V][V];
 #pragma unroll
-        for (int v = 0; v < VV; ++v) acc[m][v] += kb[v];
-        e = en;
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+          for (int l = 0; l < V; ++l) S[i][l] = 0.0;
+        for (int b = 0; b < 8; ++b) {
+          const bool same = __shfl(node, (lane & 56) + b, 64) == node;
+#pragma unroll
+          for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int l = 0; l < V; ++l) {
+              const double v = __shfl(K[i][l], (lane & 56) + b, 64);
+              if (same) S[i][l] += v;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+          for (int l = 0; l < V; ++l) K[i][l] = S[i][l];
       }
-      nxt[m] = e;
-    }
-    if (RES && resw) {
-      while (rnxt < lim) {
-        ++rcur;
-        const int en = rcur < rend ? cloc[rcur] : INT32_MAX;
-        r += s_R[RES ? rnxt / N - p0 : 0][ri];
-        rnxt = en;
+      // hand the blocks to their slots, NX values at a time
+#pragma unroll
+      for (int r0 = 0; r0 < (VV + NX - 1) / NX; ++r0) {
+        wave_fence();
+#pragma unroll
+        for (int v = 0; v < NX; ++v)
+          if (r0 * NX + v < VV) lx[lane * NX + v] = K[(r0 * NX + v) / V][(r0 * NX + v) % V];
+        wave_fence();
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          const int b = (cur >> (4 * m)) & 15;
+          if (!__any(b < 8)) continue;  // a HEX8 box: two or three of the four
+          const LdsD* e = lx + (b < 8 ? (lane & 56) + b : 64) * NX;
+#pragma unroll
+          for (int v = 0; v < NX; ++v)
+            if (r0 * NX + v < VV) acc[m][r0 * NX + v] += e[v];
+        }
       }
-    }
-    __syncthreads();
-    p0 = p1;
+    } while (__any((word >> kRankShift) < lim));
   }
-  if constexpr (kIso) {
-    // the slots summed M: K = c0 M + c1 M^T + c1 tr(M) I
-    const double c0m = mat.c[0];
+
+  if constexpr (TP::kIso) {
+    const double l = mat.c[0], mu = mat.c[1];
 #pragma unroll
-    for (int m = 0; m < MAXK; ++m) {
-      double M[9];
+    for (int m = 0; m < M; ++m) {
+      double A[9];
 #pragma unroll
-      for (int v = 0; v < 9; ++v) M[v] = acc[m][v];
-      const double tr = iso_c1 * (M[0] + M[4] + M[8]);
+      for (int v = 0; v < 9; ++v) A[v] = acc[m][v];
+      const double tr = mu * (A[0] + A[4] + A[8]);
 #pragma unroll
       for (int i = 0; i < 3; ++i)
 #pragma unroll
-        for (int k = 0; k < 3; ++k) acc[m][i * 3 + k] = c0m * M[i * 3 + k] + iso_c1 * M[k * 3 + i] + (i == k ? tr : 0.0);
+        for (int k = 0; k < 3; ++k) acc[m][i * 3 + k] = l * A[i * 3 + k] + mu * A[k * 3 + i] + (i == k ? tr : 0.0);
     }
   }
-
-  // ---- difference form: row sums of all slots, combined in a fixed order
-  double rsum[DIFF ? VV : 1];
-  if (DIFF) {
+  // sums over the eight lanes of a row, the same in every lane
+  auto row_sum = [](double v) {
+    v += dpp_move<kDppXor1>(v);
+    v += dpp_move<kDppXor2>(v);
+    return v + dpp_move<kDppHalfMirror>(v);
+  };
+  double rsum[DIFF ? VV : 1];  // difference form: the diagonal block holds the row sum
+  if constexpr (DIFF)
 #pragma unroll
     for (int v = 0; v < VV; ++v) {
       double p = 0.0;
 #pragma unroll
-      for (int m = 0; m < MAXK; ++m) p += acc[m][v];
-      rsum[v] = p;
+      for (int m = 0; m < M; ++m) p += acc[m][v];
+      rsum[v] = row_sum(p);
     }
-    // round 1: waves kHalf.. stage, waves 0..kHalf-1 add (pairs w, w + kHalf)
-    if (w >= kHalf)
+  if (dinv && row >= 0 && ds < 0 && j < V) dinv[(int64_t)row * V + j] = TO(0);  // a node of no cell
+  // the diagonal block: its inverse diagonal, then the difference form's row sum in its place
 #pragma unroll
-      for (int v = 0; v < VV; ++v) s_red[w - kHalf][lane][v] = rsum[v];
-    __syncthreads();
-    if (w < kHalf)
+  for (int c = 0; c < V; ++c) {
+    double d = 0.0;
 #pragma unroll
-      for (int v = 0; v < VV; ++v) rsum[v] += s_red[w][lane][v];
-    __syncthreads();
-    // round 2: the pair sums, read by every thread
-    if (w < kHalf)
-#pragma unroll
-      for (int v = 0; v < VV; ++v) s_red[w][lane][v] = rsum[v];
-    __syncthreads();
-#pragma unroll
-    for (int v = 0; v < VV; ++v) {
-      double sum = s_red[0][lane][v];
-#pragma unroll
-      for (int o = 1; o < kHalf; ++o) sum += s_red[o][lane][v];
-      rsum[v] = sum;
-    }
+    for (int m = 0; m < M; ++m) d = ds == j + 8 * m ? acc[m][c * V + c] : d;
+    if (dinv && ds >= 0 && (ds & 7) == j) dinv[(int64_t)row * V + c] = d != 0.0 ? TO(1.0 / d) : TO(0);
   }
-
-  // ---- stores: one coalesced 64-lane store per value of each owned slot
-  TO* vp = vals + (size_t)sbase * VV + lane;
+  TO* vp = vals + (size_t)sbase * VV + rl;
 #pragma unroll
-  for (int m = 0; m < MAXK; ++m) {
-    const int k = w + kAsmWaves * m;
-    if (k >= L) continue;
-    if (k == ds && dinv) {
+  for (int m = 0; m < M; ++m) {
+    const int k = j + 8 * m;
+    if (k < nslots)
 #pragma unroll
-      for (int c = 0; c < V; ++c) {
-        const double d = acc[m][c * V + c];
-        dinv[(int64_t)row * V + c] = d != 0.0 ? TO(1.0 / d) : TO(0);
+      for (int v = 0; v < VV; ++v)
+        __builtin_nontemporal_store(TO((DIFF && k == ds) ? rsum[v] : acc[m][v]), &vp[((size_t)k * VV + v) * kSlice]);
+  }
+  if constexpr (RES) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const double r = row_sum(rs[i]);
+      if (j == i && row >= 0) {
+        const int64_t idx = (int64_t)row * V + i;
+        res[idx] = (base ? base[idx] : 0.0) + r;
       }
     }
-#pragma unroll
-    for (int v = 0; v < VV; ++v) vp[((size_t)k * VV + v) * kSlice] = TO((DIFF && k == ds) ? rsum[v] : acc[m][v]);
-  }
-  if (RES && resw) {
-    const int64_t idx = (int64_t)row * V + ri;
-    res[idx] = (base ? base[idx] : 0.0) + r;
   }
 }
 
@@ -677,11 +763,12 @@ int fem_assembly_plan_counts(const fem_pattern_t* pat, const int32_t* inc_ptr, c
                              void* stream) {
   FEM_CHECK_ARG(pat && inc_ptr && inc_idx && slice_cell_counts && slice_pair_counts && err_flag,
                 "fem_assembly_plan_counts: NULL argument");
+  FEM_CHECK_ARG(pat->nodes_per_cell == 8, "fem_assembly_plan_counts: HEX8 patterns only");
   if (pat->num_slices == 0) return FEM_OK;
   hipStream_t st = as_stream(stream);
   FEM_HIP(hipMemsetAsync(err_flag, 0, sizeof(int32_t), st));
-  hipLaunchKernelGGL(k_slice_cells<false>, dim3((unsigned)pat->num_slices), dim3(256), 0, st, pat->num_slices,
-                     pat->nodes_per_cell, pat->sell_row, inc_ptr, inc_idx, (const int32_t*)nullptr,
+  hipLaunchKernelGGL(k_slice_cells<false>, dim3((unsigned)pat->num_slices), dim3(64 * kGroups), 0, st,
+                     pat->num_slices, pat->sell_row, inc_ptr, inc_idx, (const int32_t*)nullptr,
                      slice_cell_counts, slice_pair_counts, err_flag);
   FEM_LAUNCHED();
   return FEM_OK;
@@ -690,21 +777,19 @@ int fem_assembly_plan_counts(const fem_pattern_t* pat, const int32_t* inc_ptr, c
 int fem_assembly_plan_fill(const fem_pattern_t* pat, const int32_t* inc_ptr, const int32_t* inc_idx,
                            const int32_t* slice_cell_ptr, const int32_t* slice_pair_ptr, int32_t* slice_cells,
                            int32_t* slice_pairs, int32_t* contrib_loc, int32_t* err_flag, void* stream) {
-  FEM_CHECK_ARG(pat && inc_ptr && inc_idx && slice_cell_ptr && slice_pair_ptr && slice_cells && slice_pairs &&
-                    contrib_loc && err_flag,
+  (void)slice_pair_ptr;
+  (void)slice_pairs;
+  FEM_CHECK_ARG(pat && inc_ptr && inc_idx && slice_cell_ptr && slice_cells && contrib_loc && err_flag,
                 "fem_assembly_plan_fill: NULL argument");
+  FEM_CHECK_ARG(pat->nodes_per_cell == 8, "fem_assembly_plan_fill: HEX8 patterns only");
   if (pat->num_slices == 0) return FEM_OK;
   hipStream_t st = as_stream(stream);
-  hipLaunchKernelGGL(k_slice_cells<true>, dim3((unsigned)pat->num_slices), dim3(256), 0, st, pat->num_slices,
-                     pat->nodes_per_cell, pat->sell_row, inc_ptr, inc_idx, slice_cell_ptr, slice_cells,
+  hipLaunchKernelGGL(k_slice_cells<true>, dim3((unsigned)pat->num_slices), dim3(64 * kGroups), 0, st,
+                     pat->num_slices, pat->sell_row, inc_ptr, inc_idx, slice_cell_ptr, slice_cells,
                      (int32_t*)nullptr, err_flag);
   FEM_LAUNCHED();
-  const int64_t lanes = pat->num_slices * kSlice;
-  hipLaunchKernelGGL(k_contrib_local, dim3((unsigned)ceil_div(lanes, 256)), dim3(256), 0, st, *pat, slice_cell_ptr,
-                     slice_cells, contrib_loc, err_flag);
-  FEM_LAUNCHED();
-  hipLaunchKernelGGL(k_slice_reorder, dim3((unsigned)pat->num_slices), dim3(64), 0, st, *pat, inc_ptr, inc_idx,
-                     slice_cell_ptr, slice_cells, slice_pair_ptr, slice_pairs, contrib_loc, err_flag);
+  hipLaunchKernelGGL(k_pair_words, dim3((unsigned)pat->num_slices), dim3(kSlice * kGroupRows), 0, st, *pat, inc_ptr,
+                     inc_idx, slice_cell_ptr, slice_cells, (uint32_t*)contrib_loc, err_flag);
   FEM_LAUNCHED();
   return FEM_OK;
 }
@@ -717,11 +802,9 @@ int fem_assemble(const fem_mesh_t* mesh, const fem_material_t* mat, const fem_pa
                 "fem_assemble: single-pass assembly covers HEX8 cells with 8 quadrature points");
   FEM_CHECK_ARG(pat->nodes_per_cell == 8 && pat->vec == mesh->vec && pat->num_cells == mesh->num_cells,
                 "fem_assemble: pattern and mesh disagree");
-  FEM_CHECK_ARG(plan->slice_cell_ptr && plan->slice_cells && plan->slice_pair_ptr && plan->slice_pairs &&
-                    plan->contrib_loc,
-                "fem_assemble: plan not built");
-  FEM_CHECK_ARG(plan->max_slots >= 0 && plan->max_slots <= kAsmWaves * kAsmMaxK,
-                "fem_assemble: a slice has %d blocks per row (at most %d)", plan->max_slots, kAsmWaves * kAsmMaxK);
+  FEM_CHECK_ARG(plan->slice_cell_ptr && plan->slice_cells && plan->contrib_loc, "fem_assemble: plan not built");
+  FEM_CHECK_ARG(plan->max_slots >= 0 && plan->max_slots <= 8 * kAsmMaxK,
+                "fem_assemble: a slice has %d blocks per row (at most %d)", plan->max_slots, 8 * kAsmMaxK);
   FEM_CHECK_ARG(plan->max_pairs >= 0 && plan->max_pairs <= kSlicePairCap,
                 "fem_assemble: a slice has %d (cell, row node) pairs (at most %d)", plan->max_pairs, kSlicePairCap);
   FEM_CHECK_ARG((precision == FEM_F64 && form == FEM_FORM_STANDARD) ||
@@ -730,19 +813,17 @@ int fem_assemble(const fem_mesh_t* mesh, const fem_material_t* mat, const fem_pa
   FEM_CHECK_ARG(!mat->has_param || mat->param, "fem_assemble: material param missing");
   if (pat->num_slices == 0) return FEM_OK;
   hipStream_t st = as_stream(stream);
-  const dim3 grid((unsigned)pat->num_slices), block(kAsmThreads);
+  const dim3 grid((unsigned)(pat->num_slices * kGroups * 64 / kAsmThreads)), block(kAsmThreads);
   return with_mat8(*mat, mesh->vec, [&](auto m) -> int {
     using MAT = decltype(m);
     auto go = [&](auto res_c) {
       constexpr bool R = decltype(res_c)::value;
       if (precision == FEM_F64)
         hipLaunchKernelGGL((k_assemble_hex8<MAT, double, false, R>), grid, block, 0, st, *mesh, *mat, *pat,
-                           plan->slice_cell_ptr, plan->slice_cells, plan->slice_pair_ptr, plan->slice_pairs,
-                           plan->contrib_loc, u, (double*)vals, (double*)dinv, base, res);
+                           plan->slice_cell_ptr, plan->slice_cells, (const uint32_t*)plan->contrib_loc, u, (double*)vals, (double*)dinv, base, res);
       else
         hipLaunchKernelGGL((k_assemble_hex8<MAT, float, true, R>), grid, block, 0, st, *mesh, *mat, *pat,
-                           plan->slice_cell_ptr, plan->slice_cells, plan->slice_pair_ptr, plan->slice_pairs,
-                           plan->contrib_loc, u, (float*)vals, (float*)dinv, base, res);
+                           plan->slice_cell_ptr, plan->slice_cells, (const uint32_t*)plan->contrib_loc, u, (float*)vals, (float*)dinv, base, res);
     };
     if (res)
       go(std::true_type{});

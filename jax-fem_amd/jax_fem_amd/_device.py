@@ -558,7 +558,7 @@ class DeviceProblem:
                     _lib.FEM_MAT_J2_PLASTIC)
 
     def assembly_plan(self):
-        """The single-pass assembly's plan (slice cell lists, slice-local contribution ids), built
+        """The single-pass assembly's plan (cell lists of eight-row groups, slots of each pair), built
         once per pattern; None where it does not apply (not HEX8 with 8 quadrature points, rows of
         more than 32 blocks, slices with more than 4096 incidences)."""
         if self._asm_plan is None:
@@ -577,20 +577,17 @@ class DeviceProblem:
                     max_pairs = int(pcounts.max().item()) if ns else 0
                     if int(err.item()) == 0 and max_pairs <= 1024:
                         sc_ptr = dm.scan(counts)
-                        sp_ptr = dm.scan(pcounts)
                         sc = dm.empty(max(int(sc_ptr[-1].item()), 1), dtype=torch.int32)
-                        sp = dm.empty(max(int(sp_ptr[-1].item()), 1), dtype=torch.int32)
                         loc = dm.empty(max(dm.C * dm.N * dm.N, 1), dtype=torch.int32)
                         check(L.fem_assembly_plan_fill(self.pref, ptr(self.inc_ptr), ptr(self.inc_idx), ptr(sc_ptr),
-                                                       ptr(sp_ptr), ptr(sc), ptr(sp), ptr(loc), ptr(err), s),
+                                                       None, ptr(sc), None, ptr(loc), ptr(err), s),
                               'fem_assembly_plan_fill')
                         if int(err.item()) == 0:
                             plan = _lib.FemAssemblyPlan()
                             plan.slice_cell_ptr, plan.slice_cells, plan.contrib_loc = (
                                 sc_ptr.data_ptr(), sc.data_ptr(), loc.data_ptr())
-                            plan.slice_pair_ptr, plan.slice_pairs = sp_ptr.data_ptr(), sp.data_ptr()
                             plan.max_slots, plan.max_pairs = max_slots, max_pairs
-                            self._asm_plan = (plan, (sc_ptr, sc, sp_ptr, sp, loc))
+                            self._asm_plan = (plan, (sc_ptr, sc, loc))
                         else:
                             logger.info("single-pass assembly plan refused (code %d): two-pass assembly",
                                         int(err.item()))
