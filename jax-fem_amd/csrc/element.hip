@@ -23,6 +23,26 @@
 
 namespace fem {
 
+// f(cell, active, first) for the cells of a workgroup that walks the mesh (CPW cells at a time,
+// every thread in every trip): the tables, 23 KB for a HEX27 cell, are read once per workgroup,
+// not once per cell.  Workgroups: as many as the chip holds at a time.  24^3 HEX27 cells, with
+// ref_grads and no gradients staged where only JxW is needed: body loads 515 -> 82 us, their
+// transpose 460 -> 82, parameter gradient 860 -> 162.
+constexpr int kCellBlocks = 1536;
+template <int CPW, class F>
+__device__ inline void for_cells(const fem_mesh_t& mesh, F&& f) {
+  for (int64_t b = blockIdx.x; b * CPW < mesh.num_cells; b += gridDim.x) {
+    const int64_t c = b * CPW + threadIdx.x / (256 / CPW);
+    f(c, c < mesh.num_cells, b == blockIdx.x);
+  }
+}
+
+// Shape values of quadrature points q0 .. q0 + qn - 1.
+template <int N, int Q>
+__device__ inline void load_shape_chunk(const fem_mesh_t& mesh, int q0, int qn, double (&s)[Q][N]) {
+  for (int i = threadIdx.x; i < qn * N; i += 256) (&s[0][0])[i] = mesh.shape_vals[(size_t)q0 * N + i];
+}
+
 // ------------------------------------------------------------------ tangent
 // Quadrature points are staged Cfg::Q at a time; each thread keeps the blocks
 // of its PPT (a, b) pairs in registers across the chunks.
@@ -640,47 +660,57 @@ __global__ __launch_bounds__(256) void k_cell_adjoint(fem_mesh_t mesh, fem_mater
   constexpr int N = Cfg::N, Q = Cfg::Q, TPC = Cfg::TPC, CPW = Cfg::CPW, V = MAT::V;
   __shared__ T s_dN[Q][N][3];
   __shared__ double s_w[Q];
-  __shared__ CellLds<N, Q, T> s_cell[CPW];
-  __shared__ T s_u[CPW][N][V];
-  __shared__ T s_l[CPW][N][V];
+  __shared__ JacLds<N, Q, T> s_cell[CPW];
+  __shared__ T s_u[CPW][N][V], s_l[CPW][N][V];
+  __shared__ T s_gu[CPW][Q][V * 3], s_gl[CPW][Q][V * 3];
   __shared__ int32_t s_node[CPW][N];
   const int w = threadIdx.x / TPC, t = threadIdx.x % TPC;
-  const int64_t c = (int64_t)blockIdx.x * CPW + w;
-  const bool active = c < mesh.num_cells;
   const int Qt = mesh.num_quads;
-  CellLds<N, Q, T>& L = s_cell[w];
-  for (int q0 = 0; q0 < Qt; q0 += Q) {
-    const int qn = min(Q, Qt - q0);
-    __syncthreads();
-    load_tables_chunk(mesh, q0, qn, s_dN, s_w);
-    __syncthreads();
-    stage_geometry<N, Q, TPC, T>(mesh, c, active, t, s_dN, s_w, L, s_node[w], qn);
-    if (active && t < N) {
-      const int64_t n = s_node[w][t];
+  JacLds<N, Q, T>& L = s_cell[w];
+  for_cells<CPW>(mesh, [&](int64_t c, bool active, bool first) {
+    for (int q0 = 0; q0 < Qt; q0 += Q) {
+      const int qn = min(Q, Qt - q0);
+      __syncthreads();
+      if (first || Qt > Q) load_tables_chunk(mesh, q0, qn, s_dN, s_w);
+      __syncthreads();
+      stage_jacobian<N, Q, TPC, T>(mesh, c, active, t, s_dN, s_w, L, s_node[w], qn);
+      if (active)
+        for (int it = t; it < N * V; it += TPC) {
+          const int64_t at = (int64_t)s_node[w][it / V] * V + it % V;
+          s_u[w][it / V][it % V] = u[at];
+          s_l[w][it / V][it % V] = lam[at];
+        }
+      __syncthreads();
+      if (active) {
+        ref_grads<N, Q, TPC, V>(s_dN, s_u[w], qn, t, &s_gu[w][0][0]);
+        ref_grads<N, Q, TPC, V>(s_dN, s_l[w], qn, t, &s_gl[w][0][0]);
+      }
+      __syncthreads();
+      if (active) {
+        for (int q = t; q < qn; q += TPC) {
+          T G[V][3], GL[V][3], dP[V][3];
+          const T* iJ = L.invJ[q];
 #pragma unroll
-      for (int i = 0; i < V; ++i) {
-        s_u[w][t][i] = u[n * V + i];
-        s_l[w][t][i] = lam[n * V + i];
+          for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+              const T *ru = &s_gu[w][q][i * 3], *rl = &s_gl[w][q][i * 3];
+              G[i][j] = ru[0] * iJ[j] + ru[1] * iJ[3 + j] + ru[2] * iJ[6 + j];
+              GL[i][j] = rl[0] * iJ[j] + rl[1] * iJ[3 + j] + rl[2] * iJ[6 + j];
+            }
+          const int64_t cq = c * Qt + q0 + q;
+          const auto st = MAT::template prep<T>(mat, cq, G);
+          MAT::dparam(mat, cq, st, G, dP);
+          T s = 0;
+#pragma unroll
+          for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) s += dP[i][j] * GL[i][j];
+          gout[cq] = -s * L.jxw[q];
+        }
       }
     }
-    __syncthreads();
-    if (active) {
-      for (int q = t; q < qn; q += TPC) {
-        T G[V][3], GL[V][3], dP[V][3];
-        quad_grad<N, Q, V, T>(L, s_u[w], q, G);
-        quad_grad<N, Q, V, T>(L, s_l[w], q, GL);
-        const int64_t cq = c * Qt + q0 + q;
-        const auto st = MAT::template prep<T>(mat, cq, G);
-        MAT::dparam(mat, cq, st, G, dP);
-        T s = 0;
-#pragma unroll
-        for (int i = 0; i < V; ++i)
-#pragma unroll
-          for (int j = 0; j < 3; ++j) s += dP[i][j] * GL[i][j];
-        gout[cq] = -s * L.jxw[q];
-      }
-    }
-  }
+  });
 }
 
 // HEX8 with 8 quadrature points: one thread per (cell, quadrature point),
@@ -787,48 +817,54 @@ __global__ __launch_bounds__(256) void k_geometry(fem_mesh_t mesh, double* __res
   }
 }
 
-// re[c][a][i] = sum_q m[c][q][i] N_a(q) JxW(c, q); the vec count is runtime (1..3).
+// re[c][a][i] = sum_q m[c][q][i] N_a(q) JxW(c, q); the vec count is runtime (1..4).
 template <class Cfg>
 __global__ __launch_bounds__(256) void k_cell_load(fem_mesh_t mesh, int V, const double* __restrict__ m,
                                                    double* __restrict__ re) {
   using T = double;
   constexpr int N = Cfg::N, Q = Cfg::Q, TPC = Cfg::TPC, CPW = Cfg::CPW;
-  constexpr int RPT = (N * 3 + TPC - 1) / TPC;  // (a, i) rows per thread for vec <= 3
-  __shared__ T s_dN[Q][N][3];
+  constexpr int RPT = (N * 4 + TPC - 1) / TPC;  // (a, i) rows per thread for vec <= 4
+  __shared__ T s_dN[Q][N][3], s_N[Q][N];
   __shared__ double s_w[Q];
-  __shared__ CellLds<N, Q, T> s_cell[CPW];
+  __shared__ JacLds<N, Q, T> s_cell[CPW];
+  __shared__ T s_m[CPW][Q * 4];  // m JxW
   __shared__ int32_t s_node[CPW][N];
   const int w = threadIdx.x / TPC, t = threadIdx.x % TPC;
-  const int64_t c = (int64_t)blockIdx.x * CPW + w;
-  const bool active = c < mesh.num_cells;
   const int Qt = mesh.num_quads;
-  CellLds<N, Q, T>& L = s_cell[w];
-  double r[RPT];
+  JacLds<N, Q, T>& L = s_cell[w];
+  for_cells<CPW>(mesh, [&](int64_t c, bool active, bool first) {
+    double r[RPT];
 #pragma unroll
-  for (int p = 0; p < RPT; ++p) r[p] = 0.0;
-  for (int q0 = 0; q0 < Qt; q0 += Q) {
-    const int qn = min(Q, Qt - q0);
-    __syncthreads();
-    load_tables_chunk(mesh, q0, qn, s_dN, s_w);
-    __syncthreads();
-    stage_geometry<N, Q, TPC, T>(mesh, c, active, t, s_dN, s_w, L, s_node[w], qn);
-    if (!active) continue;
-#pragma unroll
-    for (int p = 0; p < RPT; ++p) {
-      const int it = t + p * TPC;
-      if (it < N * V) {
-        const int a = it / V, i = it % V;
-        for (int q = 0; q < qn; ++q)
-          r[p] += m[((size_t)c * Qt + q0 + q) * V + i] * mesh.shape_vals[(size_t)(q0 + q) * N + a] * L.jxw[q];
+    for (int p = 0; p < RPT; ++p) r[p] = 0.0;
+    for (int q0 = 0; q0 < Qt; q0 += Q) {
+      const int qn = min(Q, Qt - q0);
+      __syncthreads();
+      if (first || Qt > Q) {
+        load_tables_chunk(mesh, q0, qn, s_dN, s_w);
+        load_shape_chunk(mesh, q0, qn, s_N);
       }
-    }
-  }
-  if (!active) return;
+      __syncthreads();
+      stage_jacobian<N, Q, TPC, T>(mesh, c, active, t, s_dN, s_w, L, s_node[w], qn);
+      if (active)
+        for (int it = t; it < qn * V; it += TPC) s_m[w][it] = m[((size_t)c * Qt + q0) * V + it] * L.jxw[it / V];
+      __syncthreads();
+      if (active)
 #pragma unroll
-  for (int p = 0; p < RPT; ++p) {
-    const int it = t + p * TPC;
-    if (it < N * V) re[(size_t)c * N * V + it] = r[p];
-  }
+        for (int p = 0; p < RPT; ++p) {
+          const int it = t + p * TPC;
+          if (it < N * V) {
+            const int a = it / V, i = it % V;
+            for (int q = 0; q < qn; ++q) r[p] += s_m[w][q * V + i] * s_N[q][a];
+          }
+        }
+    }
+    if (active)
+#pragma unroll
+      for (int p = 0; p < RPT; ++p) {
+        const int it = t + p * TPC;
+        if (it < N * V) re[(size_t)c * N * V + it] = r[p];
+      }
+  });
 }
 
 // Transpose of k_cell_load: lq[c][q][i] = sum_a lam[node_a][i] N_a(q) JxW(c, q).
@@ -837,29 +873,37 @@ __global__ __launch_bounds__(256) void k_cell_load_adjoint(fem_mesh_t mesh, int 
                                                            double* __restrict__ lq) {
   using T = double;
   constexpr int N = Cfg::N, Q = Cfg::Q, TPC = Cfg::TPC, CPW = Cfg::CPW;
-  __shared__ T s_dN[Q][N][3];
+  __shared__ T s_dN[Q][N][3], s_N[Q][N];
   __shared__ double s_w[Q];
-  __shared__ CellLds<N, Q, T> s_cell[CPW];
+  __shared__ JacLds<N, Q, T> s_cell[CPW];
+  __shared__ T s_l[CPW][N * 4];
   __shared__ int32_t s_node[CPW][N];
   const int w = threadIdx.x / TPC, t = threadIdx.x % TPC;
-  const int64_t c = (int64_t)blockIdx.x * CPW + w;
-  const bool active = c < mesh.num_cells;
   const int Qt = mesh.num_quads;
-  CellLds<N, Q, T>& L = s_cell[w];
-  for (int q0 = 0; q0 < Qt; q0 += Q) {
-    const int qn = min(Q, Qt - q0);
-    __syncthreads();
-    load_tables_chunk(mesh, q0, qn, s_dN, s_w);
-    __syncthreads();
-    stage_geometry<N, Q, TPC, T>(mesh, c, active, t, s_dN, s_w, L, s_node[w], qn);
-    if (!active) continue;
-    for (int it = t; it < qn * V; it += TPC) {
-      const int q = it / V, i = it % V;
-      double r = 0;
-      for (int a = 0; a < N; ++a) r += lam[(int64_t)s_node[w][a] * V + i] * mesh.shape_vals[(size_t)(q0 + q) * N + a];
-      lq[((size_t)c * Qt + q0 + q) * V + i] = r * L.jxw[q];
+  JacLds<N, Q, T>& L = s_cell[w];
+  for_cells<CPW>(mesh, [&](int64_t c, bool active, bool first) {
+    for (int q0 = 0; q0 < Qt; q0 += Q) {
+      const int qn = min(Q, Qt - q0);
+      __syncthreads();
+      if (first || Qt > Q) {
+        load_tables_chunk(mesh, q0, qn, s_dN, s_w);
+        load_shape_chunk(mesh, q0, qn, s_N);
+      }
+      __syncthreads();
+      stage_jacobian<N, Q, TPC, T>(mesh, c, active, t, s_dN, s_w, L, s_node[w], qn);
+      if (active)
+        for (int it = t; it < N * V; it += TPC) s_l[w][it] = lam[(int64_t)s_node[w][it / V] * V + it % V];
+      __syncthreads();
+      if (active)
+        for (int it = t; it < qn * V; it += TPC) {
+          const int q = it / V, i = it % V;
+          double r = 0;
+#pragma unroll
+          for (int a = 0; a < N; ++a) r += s_l[w][a * V + i] * s_N[q][a];
+          lq[((size_t)c * Qt + q0) * V + it] = r * L.jxw[q];
+        }
     }
-  }
+  });
 }
 
 // --------------------------------------------------------------- faces
@@ -925,6 +969,11 @@ __global__ void k_face(fem_mesh_t mesh, int64_t S, const int32_t* __restrict__ f
 template <class Cfg>
 static int grid_cells(const fem_mesh_t& m) {
   return (int)ceil_div(m.num_cells, Cfg::CPW);
+}
+
+template <class Cfg>
+static int cell_blocks(const fem_mesh_t& m) {
+  return std::min(grid_cells<Cfg>(m), kCellBlocks);
 }
 
 // Calls f(Cfg{}) for the supported (nodes per cell, quads) pairs.
@@ -1222,7 +1271,7 @@ int fem_cell_adjoint(const fem_mesh_t* mesh, const fem_material_t* mat, const do
     using Cfg = decltype(cfg);
     return with_mat(*mat, mesh->vec, [&](auto m) -> int {
       using MAT = decltype(m);
-      hipLaunchKernelGGL((k_cell_adjoint<Cfg, MAT>), dim3(grid_cells<Cfg>(*mesh)), dim3(256), 0, as_stream(stream),
+      hipLaunchKernelGGL((k_cell_adjoint<Cfg, MAT>), dim3(cell_blocks<Cfg>(*mesh)), dim3(256), 0, as_stream(stream),
                          *mesh, *mat, u, lam, g);
       FEM_LAUNCHED();
       return FEM_OK;
@@ -1236,7 +1285,7 @@ int fem_cell_load(const fem_mesh_t* mesh, const double* m, double* re, void* str
   if (mesh->num_cells == 0) return FEM_OK;
   return with_cfg(*mesh, [&](auto cfg) -> int {
     using Cfg = decltype(cfg);
-    hipLaunchKernelGGL(k_cell_load<Cfg>, dim3(grid_cells<Cfg>(*mesh)), dim3(256), 0, as_stream(stream), *mesh,
+    hipLaunchKernelGGL(k_cell_load<Cfg>, dim3(cell_blocks<Cfg>(*mesh)), dim3(256), 0, as_stream(stream), *mesh,
                        mesh->vec, m, re);
     FEM_LAUNCHED();
     return FEM_OK;
@@ -1287,7 +1336,7 @@ int fem_cell_load_adjoint(const fem_mesh_t* mesh, const double* lam, double* lq,
   if (mesh->num_cells == 0) return FEM_OK;
   return with_cfg(*mesh, [&](auto cfg) -> int {
     using Cfg = decltype(cfg);
-    hipLaunchKernelGGL(k_cell_load_adjoint<Cfg>, dim3(grid_cells<Cfg>(*mesh)), dim3(256), 0, as_stream(stream),
+    hipLaunchKernelGGL(k_cell_load_adjoint<Cfg>, dim3(cell_blocks<Cfg>(*mesh)), dim3(256), 0, as_stream(stream),
                        *mesh, mesh->vec, lam, lq);
     FEM_LAUNCHED();
     return FEM_OK;

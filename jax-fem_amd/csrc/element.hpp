@@ -17,21 +17,38 @@ struct ElemCfg {
   static constexpr int CPW = 256 / TPC;                   // cells per workgroup
 };
 
-// LDS state of one cell.
+// LDS state of one cell: coordinates, (inverse) Jacobians and JxW; with the physical gradients.
 template <int N, int Q, typename T>
-struct CellLds {
+struct JacLds {
   double xd[N][3];
   T invJ[Q][9];
   T jxw[Q];
+};
+template <int N, int Q, typename T>
+struct CellLds : JacLds<N, Q, T> {
   T g[Q][N][3];
 };
 
-// Stage node coordinates, Jacobians and physical gradients of cell c for the
+// Reference gradients r[q][i][j] = sum_a f[a][i] dN_a/dxi_j of a nodal field in LDS, one lane per
+// entry (q, i, j): a serial sum of N products, where a lane per point had 3 V of them one after
+// the other and left nine lanes of ten idle.
+template <int N, int Q, int TPC, int V, typename T, typename TF>
+__device__ inline void ref_grads(const T (&dN)[Q][N][3], const TF (*f)[V], int qn, int t, T* r) {
+  for (int it = t; it < qn * V * 3; it += TPC) {
+    const int q = it / (V * 3), i = (it / 3) % V, j = it % 3;
+    T s = T(0);
+#pragma unroll
+    for (int a = 0; a < N; ++a) s += f[a][i] * dN[q][a][j];
+    r[it] = s;
+  }
+}
+
+// Stage the node numbers and coordinates of cell c and the inverse Jacobians and JxW of the
 // first qn (default Q) staged quadrature points.
 // Must be called by all threads of the workgroup (contains barriers).
 template <int N, int Q, int TPC, typename T>
-__device__ inline void stage_geometry(const fem_mesh_t& mesh, int64_t c, bool active, int t,
-                                      const T (&dN)[Q][N][3], const double (&w)[Q], CellLds<N, Q, T>& L,
+__device__ inline void stage_jacobian(const fem_mesh_t& mesh, int64_t c, bool active, int t,
+                                      const T (&dN)[Q][N][3], const double (&w)[Q], JacLds<N, Q, T>& L,
                                       int32_t (&node)[N], int qn = Q) {
   if (active && t < N) {
     const int32_t n = mesh.cells[c * N + t];
@@ -41,29 +58,36 @@ __device__ inline void stage_geometry(const fem_mesh_t& mesh, int64_t c, bool ac
     L.xd[t][2] = mesh.points[(int64_t)n * 3 + 2];
   }
   __syncthreads();
-  if (active) {
+  if (active)
+    for (int it = t; it < qn * 9; it += TPC) {
+      const int q = it / 9, i = (it / 3) % 3, j = it % 3;
+      const double x0 = L.xd[0][i];
+      T s = T(0);
+#pragma unroll
+      for (int a = 1; a < N; ++a) s += T(L.xd[a][i] - x0) * dN[q][a][j];
+      L.invJ[q][i * 3 + j] = s;
+    }
+  __syncthreads();
+  if (active)
     for (int q = t; q < qn; q += TPC) {
-      T J[9];
+      T J[9], iJ[9];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) J[k] = T(0);
-      for (int a = 0; a < N; ++a) {
-        const T x0 = T(L.xd[a][0] - L.xd[0][0]);
-        const T x1 = T(L.xd[a][1] - L.xd[0][1]);
-        const T x2 = T(L.xd[a][2] - L.xd[0][2]);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          const T d = dN[q][a][j];
-          J[0 * 3 + j] += x0 * d;
-          J[1 * 3 + j] += x1 * d;
-          J[2 * 3 + j] += x2 * d;
-        }
-      }
+      for (int k = 0; k < 9; ++k) J[k] = L.invJ[q][k];
       const T det = det3(J);
-      inv3(J, det, L.invJ[q]);
+      inv3(J, det, iJ);
+#pragma unroll
+      for (int k = 0; k < 9; ++k) L.invJ[q][k] = iJ[k];
       L.jxw[q] = det * T(w[q]);
     }
-  }
   __syncthreads();
+}
+
+// stage_jacobian and the physical gradients.
+template <int N, int Q, int TPC, typename T>
+__device__ inline void stage_geometry(const fem_mesh_t& mesh, int64_t c, bool active, int t,
+                                      const T (&dN)[Q][N][3], const double (&w)[Q], CellLds<N, Q, T>& L,
+                                      int32_t (&node)[N], int qn = Q) {
+  stage_jacobian<N, Q, TPC, T>(mesh, c, active, t, dN, w, L, node, qn);
   if (active) {
     for (int it = t; it < qn * N; it += TPC) {
       const int q = it / N, a = it % N;

@@ -48,68 +48,91 @@ __global__ __launch_bounds__(256) void k_gather_nodal(int64_t num_nodes, const i
 }
 
 // ------------------------------------------------------- matrix values
-// One thread per slice lane: for every SELL slot k, sum the cell blocks that land in
-// block (row, col_k) and store them (zeros in padding slots).  DIFF stores
-// the row-sum block R_row = sum_k A(row, k) (accumulated in TS) in the
-// diagonal slot instead of the diagonal block (difference form of the SpMV).
-// dinv (may be NULL) receives 1 / A(row*V+c, row*V+c).  The slot bounds and
-// the cell-block ids are read through windows (a lane's lists are contiguous).
+// One workgroup per slice, lane = row: for every SELL slot k, sum the cell blocks that land in
+// block (row, col_k) and store them (zeros in padding slots).  Wave w takes the slots
+// [w K, (w + 1) K), K = slots / waves rounded up, so the lists a lane reads stay contiguous (they
+// are read through windows).  DIFF stores the row-sum block R_row = sum_k A(row, k) (accumulated
+// in TS, the waves' sums added in their order) in the diagonal slot instead of the diagonal block
+// (difference form of the SpMV).  dinv (may be NULL) receives 1 / A(row*V+c, row*V+c).
+// Bound by the blocks' addresses (every lane reads 72 bytes of its own: five wide loads where
+// element loads are nine); one thread per row walked a dependent chain of up to 125 slots on 1840
+// waves in all: 24^3 HEX27 cells 800 -> 630 us (4 and 16 waves per slice: 650 and 690).
+constexpr int kGatherWaves = 8;
+
+template <int VV, typename TS>
+__device__ inline void add_block(const TS* __restrict__ src, TS (&acc)[VV]) {
+  // two values a load; a block is aligned to one value
+  typedef TS Pair __attribute__((ext_vector_type(2), aligned(alignof(TS))));
+#pragma unroll
+  for (int v = 0; v + 1 < VV; v += 2) {
+    const Pair p = *reinterpret_cast<const Pair*>(src + v);
+    acc[v] += p.x;
+    acc[v + 1] += p.y;
+  }
+  if (VV & 1) acc[VV - 1] += src[VV - 1];
+}
+
 template <int V, bool DIFF, typename TS, typename T>
-__global__ __launch_bounds__(256) void k_gather_matrix(fem_pattern_t pat, const TS* __restrict__ Ke,
-                                                       T* __restrict__ vals, T* __restrict__ dinv) {
+__global__ __launch_bounds__(64 * kGatherWaves) void k_gather_matrix(fem_pattern_t pat, const TS* __restrict__ Ke,
+                                                                     T* __restrict__ vals, T* __restrict__ dinv) {
   constexpr int VV = V * V;
-  const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (t >= pat.num_slices * kSlice) return;
-  const int64_t s = t >> 6;
-  const int lane = (int)(t & 63);
+  __shared__ TS s_sum[DIFF ? kGatherWaves : 1][DIFF ? VV : 1][DIFF ? kSlice : 1];
+  const int64_t s = blockIdx.x;
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int base = pat.slice_ptr[s];
   const int L = (pat.slice_ptr[s + 1] - base) >> 6;
-  const int row = pat.sell_row[t];
+  const int row = pat.sell_row[s * kSlice + lane];
   const bool real = row >= 0;
   const int rb = real ? pat.row_ptr[row] : 0;
   const int len = real ? pat.row_ptr[row + 1] - rb : 0;
   const int ds = real ? pat.diag_slot[row] : -1;
   T* vp = vals + (size_t)base * VV + lane;
   TS rsum[VV];
-  TS diag[V];
 #pragma unroll
   for (int v = 0; v < VV; ++v) rsum[v] = TS(0);
-#pragma unroll
-  for (int c = 0; c < V; ++c) diag[c] = TS(0);
   ListWindow<4> cptr(pat.contrib_ptr, pat.nnzb + 1);
   ListWindow<8> cidx(pat.contrib_idx, (int64_t)pat.num_cells * pat.nodes_per_cell * pat.nodes_per_cell);
-  int c1 = len > 0 ? cptr[rb] : 0;
-  for (int k = 0; k < L; ++k) {
+  const int K = (L + kGatherWaves - 1) / kGatherWaves, k0 = w * K, k1 = min(L, k0 + K);
+  int c1 = k0 < len ? cptr[rb + k0] : 0;
+  for (int k = k0; k < k1; ++k) {
     TS acc[VV];
 #pragma unroll
     for (int v = 0; v < VV; ++v) acc[v] = TS(0);
     if (k < len) {
       const int c0 = c1;
       c1 = cptr[rb + k + 1];
-      for (int ci = c0; ci < c1; ++ci) {
-        const TS* src = Ke + (size_t)cidx[ci] * VV;
-#pragma unroll
-        for (int v = 0; v < VV; ++v) acc[v] += src[v];
-      }
+      for (int ci = c0; ci < c1; ++ci) add_block<VV>(Ke + (size_t)cidx[ci] * VV, acc);
     }
+    if (DIFF)
 #pragma unroll
-    for (int v = 0; v < VV; ++v) rsum[v] += acc[v];
-    if (k == ds) {
+      for (int v = 0; v < VV; ++v) rsum[v] += acc[v];
+    if (k == ds && dinv) {
 #pragma unroll
-      for (int c = 0; c < V; ++c) diag[c] = acc[c * V + c];
+      for (int c = 0; c < V; ++c) {
+        const TS d = acc[c * V + c];
+        dinv[(int64_t)row * V + c] = d != TS(0) ? T(TS(1) / d) : T(0);
+      }
     }
     if (!(DIFF && k == ds)) {
 #pragma unroll
-      for (int v = 0; v < VV; ++v) vp[((size_t)k * VV + v) * kSlice] = T(acc[v]);
+      for (int v = 0; v < VV; ++v) __builtin_nontemporal_store(T(acc[v]), &vp[((size_t)k * VV + v) * kSlice]);
     }
   }
-  if (DIFF && ds >= 0) {
+  if (w == 0 && real && ds < 0 && dinv) {  // a node of no cell
 #pragma unroll
-    for (int v = 0; v < VV; ++v) vp[((size_t)ds * VV + v) * kSlice] = T(rsum[v]);
+    for (int c = 0; c < V; ++c) dinv[(int64_t)row * V + c] = T(0);
   }
-  if (dinv && real) {
+  if (DIFF) {
 #pragma unroll
-    for (int c = 0; c < V; ++c) dinv[(int64_t)row * V + c] = diag[c] != TS(0) ? T(TS(1) / diag[c]) : T(0);
+    for (int v = 0; v < VV; ++v) s_sum[w][v][lane] = rsum[v];
+    __syncthreads();
+    if (ds >= 0)
+      for (int v = w; v < VV; v += kGatherWaves) {
+        TS t = s_sum[0][v][lane];
+#pragma unroll
+        for (int o = 1; o < kGatherWaves; ++o) t += s_sum[o][v][lane];
+        vp[((size_t)ds * VV + v) * kSlice] = T(t);
+      }
   }
 }
 
@@ -348,25 +371,25 @@ int fem_gather_matrix(const fem_pattern_t* pat, int32_t ke_precision, const void
   FEM_CHECK_ARG(ke_precision == precision || (ke_precision == FEM_F64 && precision == FEM_F32),
                 "fem_gather_matrix: Ke precision must equal the matrix precision or be FP64");
   FEM_CHECK_ARG(form == FEM_FORM_STANDARD || form == FEM_FORM_DIFFERENCE, "fem_gather_matrix: bad form");
-  const int64_t threads = pat->num_slices * kSlice;
-  const dim3 grid((unsigned)ceil_div(threads, 256));
+  if (pat->num_slices == 0) return FEM_OK;
+  const dim3 grid((unsigned)pat->num_slices), block(64 * kGatherWaves);
   return with_vt(pat->vec, precision, [&](auto vc, auto tv) -> int {
     constexpr int V = decltype(vc)::value;
     using T = decltype(tv);
     hipStream_t s = as_stream(stream);
     if (ke_precision == FEM_F64) {
       if (form == FEM_FORM_DIFFERENCE)
-        hipLaunchKernelGGL((k_gather_matrix<V, true, double, T>), grid, dim3(256), 0, s, *pat, (const double*)Ke,
+        hipLaunchKernelGGL((k_gather_matrix<V, true, double, T>), grid, block, 0, s, *pat, (const double*)Ke,
                            (T*)vals, (T*)dinv);
       else
-        hipLaunchKernelGGL((k_gather_matrix<V, false, double, T>), grid, dim3(256), 0, s, *pat, (const double*)Ke,
+        hipLaunchKernelGGL((k_gather_matrix<V, false, double, T>), grid, block, 0, s, *pat, (const double*)Ke,
                            (T*)vals, (T*)dinv);
     } else {
       if (form == FEM_FORM_DIFFERENCE)
-        hipLaunchKernelGGL((k_gather_matrix<V, true, T, T>), grid, dim3(256), 0, s, *pat, (const T*)Ke, (T*)vals,
+        hipLaunchKernelGGL((k_gather_matrix<V, true, T, T>), grid, block, 0, s, *pat, (const T*)Ke, (T*)vals,
                            (T*)dinv);
       else
-        hipLaunchKernelGGL((k_gather_matrix<V, false, T, T>), grid, dim3(256), 0, s, *pat, (const T*)Ke, (T*)vals,
+        hipLaunchKernelGGL((k_gather_matrix<V, false, T, T>), grid, block, 0, s, *pat, (const T*)Ke, (T*)vals,
                            (T*)dinv);
     }
     FEM_LAUNCHED();

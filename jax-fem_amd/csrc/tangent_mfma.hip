@@ -8,16 +8,20 @@
 // because lambda = c0 E and mu = c1 E share the modulus E:
 //   K[(a,i),(b,k)] = c0 Z[(a,i),(b,k)] + c1 Z[(a,k),(b,i)]
 //                  + delta_ik c1 (Z[(a,0),(b,0)] + Z[(a,1),(b,1)] + Z[(a,2),(b,2)]).
-// Z is formed on MFMA in 16 x 16 tiles (81 padded to 96, 36 tiles, 9 per
-// wave), staged in LDS and expanded into Ke[c][a][b][i][k] with coalesced
-// stores.  Operand layouts: A[i][k] in lane i + 16 k (f64; for bf16 the four
+// Z is formed on MFMA in tiles of 15 x 15 (five nodes by five: whole 3 x 3 blocks in a 16 x 16
+// result) and is symmetric, so the 21 tile pairs of the upper triangle are shared out over the
+// four waves; a wave stages its tile in LDS of its own and writes the blocks of Ke[c][a][b][i][k]
+// and, off the diagonal, their transposes, 45 consecutive values at a time.  Operand layouts:
+// A[i][k] in lane i + 16 k (f64; for bf16 the four
 // k of one lane are k = 4 (lane / 16) + e), B[k][j] in lane j + 16 k; the two
 // instructions place the 16 x 16 result differently (see the stores).  Two arithmetic modes:
 //   FP64 : v_mfma_f64_16x16x4f64, exact FP64 products and sums.
 //   BF16x3: each operand split x = hi + lo (hi = bf16(x), lo = bf16(x - hi));
 //          hi*hi + hi*lo + lo*hi on v_mfma_f32_16x16x16bf16_1k with FP32
 //          accumulation (about 16 significant bits per product); Ke in FP32.
-// One workgroup of 4 waves per cell, persistent over cells (LDS ~ 91 KB).
+// One workgroup of 4 waves per cell, persistent over cells.  46 KB of LDS, so three of them share
+// a CU and one's Jacobians run beside another's products and stores; with all of Z in LDS (91 KB)
+// there was one, which waited for each phase in turn: 24^3 cells 940 -> 420 us (726 MB written).
 #include "element.hpp"
 #include "tangent_mfma.hpp"
 
@@ -28,8 +32,9 @@ namespace fem {
 
 namespace {
 
-constexpr int kN = 27, kQ = 27, kM = 81, kTiles = 6;  // 81 padded to 6 tiles of 16
-constexpr int kGrid = 1024;                            // persistent workgroups
+constexpr int kN = 27, kQ = 27, kM = 81;
+constexpr int kTN = 5, kTiles = 6;  // nodes per tile; 27 nodes padded to 6 tiles
+constexpr int kGrid = 768;          // persistent workgroups: three per CU
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
@@ -58,13 +63,15 @@ __global__ __launch_bounds__(256) void k_tangent_hex27_mfma(fem_mesh_t mesh, fem
                                                             TO* __restrict__ Ke) {
   using TZ = typename std::conditional<kBf16, float, double>::type;
   __shared__ Hex27Lds S;
-  __shared__ TZ Z[kM][kM + 1];
+  __shared__ TZ s_z[4][3 * kTN][3 * kTN + 2];
   const int t = threadIdx.x;
   const int wave = t >> 6, lane = t & 63;
   load_tables(mesh, S.dN, S.w);
-  __syncthreads();
   const double c0 = mat.c[0], c1 = mat.c[1];
+  TZ(*z)[3 * kTN + 2] = s_z[wave];
+  const int l = lane & 15;  // row of A, column of B and of the result; 15 is padding
   for (int64_t c = blockIdx.x; c < mesh.num_cells; c += gridDim.x) {
+    __syncthreads();  // the previous cell's gradients are no longer read
     stage_geometry<kN, kQ, 256, double>(mesh, c, true, t, S.dN, S.w, S.cell, S.node);
     if (t < kQ) {
       const double E = kSimp ? MatElastic<true>::modulus(mat, mat.param[c * kQ + t]) : 1.0;
@@ -72,24 +79,28 @@ __global__ __launch_bounds__(256) void k_tangent_hex27_mfma(fem_mesh_t mesh, fem
     }
     __syncthreads();
     const double(*g)[kN][3] = S.cell.g;
-    for (int tile = wave; tile < kTiles * kTiles; tile += 4) {
-      const int tm = tile / kTiles, tn = tile % kTiles;
-      const int m = tm * 16 + (lane & 15);      // A row (operand lane layout)
-      const int n = tn * 16 + (lane & 15);      // B column
+    TO* out = Ke + (size_t)c * kM * kM;
+    // pair p of the upper triangle (row by row): (tm, tn), tm <= tn
+    for (int p = wave; p < kTiles * (kTiles + 1) / 2; p += 4) {
+      int tm = 0, first = 0;
+      while (p >= first + kTiles - tm) first += kTiles - tm++;
+      const int tn = tm + (p - first);
+      const int m = tm * 3 * kTN + l, n = tn * 3 * kTN + l;
+      const bool om = l < 3 * kTN && m < kM, on = l < 3 * kTN && n < kM;
       if (!kBf16) {
         double4_t acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
         for (int kk = 0; kk < 7; ++kk) {          // inner dim 27 padded to 28
           const int q = kk * 4 + (lane >> 4);
-          const double a = (q < kQ && m < kM) ? S.W[q] * g[q][m / 3][m % 3] : 0.0;
-          const double b = (q < kQ && n < kM) ? g[q][n / 3][n % 3] : 0.0;
+          const double a = (q < kQ && om) ? S.W[q] * g[q][m / 3][m % 3] : 0.0;
+          const double b = (q < kQ && on) ? g[q][n / 3][n % 3] : 0.0;
           acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
         }
         // f64 16x16x4 result: D[i][j] in lane j + 16 (i % 4), register i / 4
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int row = tm * 16 + (lane >> 4) + 4 * r, col = tn * 16 + (lane & 15);
-          if (row < kM && col < kM) Z[row][col] = TZ(acc[r]);
+          const int row = (lane >> 4) + 4 * r;
+          if (row < 3 * kTN && l < 3 * kTN) z[row][l] = TZ(acc[r]);
         }
       } else {
         float4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -99,8 +110,8 @@ __global__ __launch_bounds__(256) void k_tangent_hex27_mfma(fem_mesh_t mesh, fem
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int q = kk * 16 + 4 * (lane >> 4) + e;
-            const float a = (q < kQ && m < kM) ? float(S.W[q] * g[q][m / 3][m % 3]) : 0.f;
-            const float b = (q < kQ && n < kM) ? float(g[q][n / 3][n % 3]) : 0.f;
+            const float a = (q < kQ && om) ? float(S.W[q] * g[q][m / 3][m % 3]) : 0.f;
+            const float b = (q < kQ && on) ? float(g[q][n / 3][n % 3]) : 0.f;
             const unsigned short ah = bf16_bits(a), bh = bf16_bits(b);
             ahi[e] = (short)ah;
             alo[e] = (short)bf16_bits(a - bf16_value(ah));
@@ -114,22 +125,34 @@ __global__ __launch_bounds__(256) void k_tangent_hex27_mfma(fem_mesh_t mesh, fem
         // bf16 16x16x16 result: D[i][j] in lane j + 16 (i / 4), register i % 4
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          const int row = tm * 16 + 4 * (lane >> 4) + r, col = tn * 16 + (lane & 15);
-          if (row < kM && col < kM) Z[row][col] = TZ(acc[r]);
+          const int row = 4 * (lane >> 4) + r;
+          if (row < 3 * kTN && l < 3 * kTN) z[row][l] = TZ(acc[r]);
         }
       }
+      // (the hardware executes a wave's LDS accesses in order; the fences keep the compiler's)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const int a0 = tm * kTN, b0 = tn * kTN;
+      const int na = min(kTN, kN - a0), nb = min(kTN, kN - b0);
+      // value (i, k) of block (a, b) of the tile
+      auto value = [&](int a, int b, int i, int k) {
+        double v = c0 * double(z[3 * a + i][3 * b + k]) + c1 * double(z[3 * a + k][3 * b + i]);
+        if (i == k)
+          v += c1 * (double(z[3 * a][3 * b]) + double(z[3 * a + 1][3 * b + 1]) + double(z[3 * a + 2][3 * b + 2]));
+        return TO(v);
+      };
+      for (int e = lane; e < kTN * kTN * 9; e += 64) {
+        const int a = e / (9 * kTN), b = (e / 9) % kTN, ik = e % 9;
+        if (a < na && b < nb) out[((a0 + a) * kN + b0 + b) * 9 + ik] = value(a, b, ik / 3, ik % 3);
+      }
+      if (tm != tn)
+        for (int e = lane; e < kTN * kTN * 9; e += 64) {
+          const int b = e / (9 * kTN), a = (e / 9) % kTN, ki = e % 9;
+          if (a < na && b < nb) out[((b0 + b) * kN + a0 + a) * 9 + ki] = value(a, b, ki % 3, ki / 3);
+        }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
-    __syncthreads();
-    TO* out = Ke + (size_t)c * kM * kM;
-    for (int e = t; e < kM * kM; e += 256) {
-      const int k = e % 3, i = (e / 3) % 3, ab = e / 9;
-      const int a = ab / kN, b = ab % kN;
-      double v = c0 * double(Z[3 * a + i][3 * b + k]) + c1 * double(Z[3 * a + k][3 * b + i]);
-      if (i == k)
-        v += c1 * (double(Z[3 * a][3 * b]) + double(Z[3 * a + 1][3 * b + 1]) + double(Z[3 * a + 2][3 * b + 2]));
-      out[e] = TO(v);
-    }
-    __syncthreads();
   }
 }
 
