@@ -315,19 +315,19 @@ __global__ __launch_bounds__(256) void k_cell_vector_q8(fem_mesh_t mesh, fem_mat
 }
 
 // ------------------------------------------------------- quadrature gradients
-// grad u (and u) at quadrature point q of cell c (problem.py:200-203); dN: the point's reference
-// gradients; Jacobian from coordinates relative to the first node.
+// grad u (and u) at a quadrature point (problem.py:200-203).  x, f: the cell's node coordinates
+// and u in LDS; dN, Nq: the point's reference gradients and shape values; Jacobian from
+// coordinates relative to the first node.
 template <int N, int V>
-__device__ inline void point_grad(const fem_mesh_t& mesh, const double (*dN)[3], int64_t c, int q,
-                                  const double* __restrict__ u, double (&Gl)[V][3], double (&Ul)[V]) {
-  const int32_t* cn = mesh.cells + c * N;
-  const double* p0 = mesh.points + (int64_t)cn[0] * 3;
+__device__ inline void point_grad(const double (*x)[3], const double (*f)[V], const double (*dN)[3],
+                                  const double* __restrict__ Nq, double (&Gl)[V][3], double (&Ul)[V]) {
+  constexpr int kUnroll = N <= 8 ? N : 3;
   double J[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) J[k] = 0.0;
+#pragma unroll kUnroll
   for (int a = 1; a < N; ++a) {
-    const double* pa = mesh.points + (int64_t)cn[a] * 3;
-    const double d0 = pa[0] - p0[0], d1 = pa[1] - p0[1], d2 = pa[2] - p0[2];
+    const double d0 = x[a][0] - x[0][0], d1 = x[a][1] - x[0][1], d2 = x[a][2] - x[0][2];
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       const double dn = dN[a][j];
@@ -344,20 +344,76 @@ __device__ inline void point_grad(const fem_mesh_t& mesh, const double (*dN)[3],
 #pragma unroll
     for (int j = 0; j < 3; ++j) Gl[i][j] = 0.0;
   }
+#pragma unroll kUnroll
   for (int a = 0; a < N; ++a) {
     const double e0 = dN[a][0], e1 = dN[a][1], e2 = dN[a][2];
-    const double na = mesh.shape_vals[q * N + a];
     double g[3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) g[j] = e0 * iJ[0 * 3 + j] + e1 * iJ[1 * 3 + j] + e2 * iJ[2 * 3 + j];
-    const int64_t node = cn[a];
 #pragma unroll
     for (int i = 0; i < V; ++i) {
-      const double ua = u[node * V + i];
-      Ul[i] += ua * na;
+      const double ua = f[a][i];
+      if (Nq) Ul[i] += ua * Nq[a];
 #pragma unroll
       for (int j = 0; j < 3; ++j) Gl[i][j] += ua * g[j];
     }
+  }
+}
+
+// The coordinates and u of the cells of a workgroup's round of points, in LDS.  One lane per (cell,
+// node); a lane per point loading all its cell's nodes issues Qt times the loads.
+template <class Cfg, int V>
+struct PointCells {
+  static constexpr int N = Cfg::N, kCells = 256 / Cfg::Q + 2;  // 256 points, not aligned to cells
+  double x[kCells][N][3], f[kCells][N][V];
+  int64_t c0;
+
+  // points of a round: 256, or whole cells where they have fewer points than Cfg::Q
+  __host__ __device__ static int round(const fem_mesh_t& mesh) {
+    return mesh.num_quads * (kCells - 2) < 256 ? mesh.num_quads * (kCells - 2) : 256;
+  }
+
+  __device__ void load(const fem_mesh_t& mesh, const double* __restrict__ u, int64_t e0, int64_t e1) {
+    const int Qt = mesh.num_quads;
+    const int64_t first = e0 / Qt;
+    const int cells = (int)((e1 - 1) / Qt - first) + 1;
+    if (threadIdx.x == 0) c0 = first;
+    for (int it = threadIdx.x; it < cells * N; it += blockDim.x) {
+      const int64_t node = mesh.cells[first * N + it];
+#pragma unroll
+      for (int j = 0; j < 3; ++j) x[it / N][it % N][j] = mesh.points[node * 3 + j];
+#pragma unroll
+      for (int i = 0; i < V; ++i) f[it / N][it % N][i] = u[node * V + i];
+    }
+  }
+};
+
+// f(round, point, inside, grad u, u) for the points of a workgroup, P rounds of them; every thread
+// calls f in every round.  The tables are in LDS when all the points fit, else read where they are (cached).
+template <class Cfg, int V, int P, bool VALUES, class F>
+__device__ inline void for_points(const fem_mesh_t& mesh, const double* __restrict__ u, F&& f) {
+  constexpr int N = Cfg::N, Q = Cfg::Q;
+  __shared__ double s_dN[Q][N][3];
+  __shared__ double s_w[Q];
+  __shared__ PointCells<Cfg, V> S;
+  const int Qt = mesh.num_quads;
+  if (Qt <= Q) load_tables_chunk(mesh, 0, Qt, s_dN, s_w);
+  const double(*dN)[N][3] = Qt <= Q ? s_dN : reinterpret_cast<const double(*)[N][3]>(mesh.shape_grads_ref);
+  const int64_t n = mesh.num_cells * Qt;
+  const int per = PointCells<Cfg, V>::round(mesh);
+#pragma unroll
+  for (int r = 0; r < P; ++r) {
+    const int64_t e0 = ((int64_t)blockIdx.x * P + r) * per, e1 = min(e0 + per, n), e = e0 + threadIdx.x;
+    __syncthreads();
+    if (e0 < n) S.load(mesh, u, e0, e1);
+    __syncthreads();
+    double Gl[V][3], Ul[V];
+    if (e < e1) {
+      const int64_t c = e / Qt;
+      const int q = (int)(e - c * Qt), k = (int)(c - S.c0);
+      point_grad<N, V>(S.x[k], S.f[k], dN[q], VALUES ? mesh.shape_vals + (size_t)q * N : nullptr, Gl, Ul);
+    }
+    f(r, e, e < e1, Gl, Ul);
   }
 }
 
@@ -365,162 +421,244 @@ __device__ inline void point_grad(const fem_mesh_t& mesh, const double (*dN)[3],
 template <class Cfg, int V>
 __global__ __launch_bounds__(256) void k_quad_grad(fem_mesh_t mesh, const double* __restrict__ u,
                                                    double* __restrict__ G, double* __restrict__ U) {
-  constexpr int N = Cfg::N, Q = Cfg::Q;
-  const int Qt = mesh.num_quads;
-  // reference gradients from LDS when all points fit, else straight from the (cached) table
-  __shared__ double s_dN[Q][N][3];
-  __shared__ double s_w[Q];
-  if (Qt <= Q) load_tables_chunk(mesh, 0, Qt, s_dN, s_w);
-  __syncthreads();
-  const double(*dN)[N][3] = Qt <= Q ? s_dN : reinterpret_cast<const double(*)[N][3]>(mesh.shape_grads_ref);
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= mesh.num_cells * Qt) return;
-  const int64_t c = e / Qt;
-  const int q = (int)(e - c * Qt);
-  double Gl[V][3], Ul[V];
-  point_grad<N, V>(mesh, dN[q], c, q, u, Gl, Ul);
+  for_points<Cfg, V, 1, true>(mesh, u, [&](int, int64_t e, bool in, const double(&Gl)[V][3], const double(&Ul)[V]) {
+    if (!in) return;
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
-    if (U) U[e * V + i] = Ul[i];
-    if (G) {
+    for (int i = 0; i < V; ++i) {
+      if (U) U[e * V + i] = Ul[i];
+      if (G) {
 #pragma unroll
-      for (int j = 0; j < 3; ++j) G[(e * V + i) * 3 + j] = Gl[i][j];
+        for (int j = 0; j < 3; ++j) G[(e * V + i) * 3 + j] = Gl[i][j];
+      }
     }
-  }
+  });
 }
 
-// The quadrature points of largest |grad u| (the greatest component), in two passes: every wave
-// extracts the kTop largest of its kPerWave points from registers (pass 1: a sorted list per
-// wave), one workgroup merges the lists (pass 2).  Points whose gradient is not finite come last.
-// Replaces a sort of all the magnitudes (0.4 ms at 2 M points; this takes about 0.1).
+// ------------------------------------------------ points of largest gradient
+// The kTop quadrature points of largest |grad u| (the greatest component), points whose gradient
+// is not finite last: every workgroup forms the keys of four rounds of points and keeps the kTop largest,
+// workgroups of kMergeKeys reduce the lists while there are more, and one orders the last list and
+// adds points spread evenly over the mesh.  A selection is a radix search for the kTop-th key, a
+// byte at a time from the top (about four rounds of an LDS histogram for keys that differ early,
+// eight at most): extracting one maximum after the other took 48 rounds of wave reductions, about
+// 60 us in either pass whatever the mesh.  All of it: 64^3 HEX8 cells 165 -> 100 us, 24^3
+// HEX27 cells 370 -> 125, 9^3 cells 150 -> 40.
 constexpr int kTop = 48;
-constexpr int kPerLane = 16;
-constexpr int kPerWave = 64 * kPerLane;
+constexpr int kListRounds = 4;
+constexpr int kMergeKeys = 8192;  // keys of a merging workgroup: eight per thread
+constexpr int kMergeThreads = 1024;
 
-// the lane of the wave with the greatest key (the lowest among equals)
-__device__ inline int wave_argmax(double key) {
-  double best = key;
+using TopKey = unsigned long long;  // 0: not finite; else the bits of the magnitude, plus 1
+
+// Selects the kTop largest of the workgroup's NT * PER keys, `m` of them real (the others 0 and
+// not counted), ties by position (thread t holds positions t PER + s).  f(slot, s) for each
+// selected key, slot in [0, min(m, kTop)).  Every thread calls.
+template <int NT, int PER, class F>
+__device__ inline void select_top(const TopKey (&key)[PER], const bool (&real)[PER], int m, F&& f) {
+  __shared__ int s_hist[256];
+  __shared__ int s_pick[3];  // digit, keys wanted of it, keys of it
+  __shared__ int s_scan[NT / 64][2];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int want = min(m, kTop);
+  TopKey prefix = 0, mask = 0;
+  bool all = m <= kTop;
+  for (int shift = 56; shift >= 0 && !all; shift -= 8) {
+    for (int i = t; i < 256; i += NT) s_hist[i] = 0;
+    __syncthreads();
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) best = fmax(best, __shfl_xor(best, off, 64));
-  return __ffsll((unsigned long long)__ballot(key == best)) - 1;
+    for (int s = 0; s < PER; ++s)
+      if (real[s] && (key[s] & mask) == prefix) atomicAdd(&s_hist[(int)((key[s] >> shift) & 255u)], 1);
+    __syncthreads();
+    if (w == 0) {
+      // lane l holds the digits 255 - 4 l .. 252 - 4 l; the digit where the count from the top
+      // reaches `want`
+      int c[4], sum = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum += c[i] = s_hist[255 - 4 * lane - i];
+      int above = sum;
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) {
+        const int v = __shfl_up(above, off, 64);
+        if (lane >= off) above += v;
+      }
+      above -= sum;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (above < want && above + c[i] >= want) {
+          s_pick[0] = 255 - 4 * lane - i;
+          s_pick[1] = want - above;
+          s_pick[2] = c[i];
+        }
+        above += c[i];
+      }
+    }
+    __syncthreads();
+    prefix |= (TopKey)s_pick[0] << shift;
+    mask |= (TopKey)255u << shift;
+    want = s_pick[1];
+    if (s_pick[2] == want) break;  // the whole digit is wanted
+    __syncthreads();
+  }
+  // above the prefix: all; equal to it under the mask: the first `want` by position
+  int up = 0, eq = 0;
+#pragma unroll
+  for (int s = 0; s < PER; ++s) {
+    up += real[s] && (all || (key[s] & mask) > prefix) ? 1 : 0;
+    eq += real[s] && !all && (key[s] & mask) == prefix ? 1 : 0;
+  }
+  int su = up, se = eq;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int a = __shfl_up(su, off, 64), b = __shfl_up(se, off, 64);
+    if (lane >= off) su += a, se += b;
+  }
+  if (lane == 63) s_scan[w][0] = su, s_scan[w][1] = se;
+  __syncthreads();
+  int pu = su - up, pe = se - eq, total = 0;
+  for (int k = 0; k < NT / 64; ++k) {
+    if (k < w) pu += s_scan[k][0], pe += s_scan[k][1];
+    total += s_scan[k][0];
+  }
+#pragma unroll
+  for (int s = 0; s < PER; ++s) {
+    if (!real[s]) continue;
+    if (all || (key[s] & mask) > prefix)
+      f(pu++, s);
+    else if ((key[s] & mask) == prefix && pe++ < want)
+      f(total + pe - 1, s);
+  }
 }
 
 template <class Cfg, int V>
 __global__ __launch_bounds__(256) void k_grad_top(fem_mesh_t mesh, const double* __restrict__ u,
-                                                  double* __restrict__ key, int32_t* __restrict__ idx) {
-  constexpr int N = Cfg::N, Q = Cfg::Q;
-  const int Qt = mesh.num_quads;
-  __shared__ double s_dN[Q][N][3];
-  __shared__ double s_w[Q];
-  if (Qt <= Q) load_tables_chunk(mesh, 0, Qt, s_dN, s_w);
-  __syncthreads();
-  const double(*dN)[N][3] = Qt <= Q ? s_dN : reinterpret_cast<const double(*)[N][3]>(mesh.shape_grads_ref);
-  const int lane = threadIdx.x & 63;
-  const int64_t n = mesh.num_cells * Qt;
-  const int64_t wave = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), first = wave * kPerWave;
-  if (first >= n) return;
-  double m[kPerLane];
-  // (a rolled loop over the points, the magnitudes in statically indexed registers)
-#pragma unroll 1
-  for (int k = 0; k < kPerLane; ++k) {
-    const int64_t e = first + (int64_t)k * 64 + lane;
-    double v = -2.0;  // past the end
-    if (e < n) {
-      const int64_t c = e / Qt;
-      const int q = (int)(e - c * Qt);
-      double Gl[V][3], Ul[V];
-      point_grad<N, V>(mesh, dN[q], c, q, u, Gl, Ul);
-      v = 0.0;
-      bool finite = true;
+                                                  TopKey* __restrict__ key, int32_t* __restrict__ idx) {
+  const int per = PointCells<Cfg, V>::round(mesh);
+  const int64_t n = mesh.num_cells * mesh.num_quads, first = (int64_t)blockIdx.x * kListRounds * per;
+  TopKey k[kListRounds];
+  bool real[kListRounds];
+  for_points<Cfg, V, kListRounds, false>(
+      mesh, u, [&](int r, int64_t, bool in, const double(&Gl)[V][3], const double(&)[V]) {
+        real[r] = in;
+        k[r] = 0;
+        if (!in) return;
+        double v = 0.0;
+        bool finite = true;
 #pragma unroll
-      for (int i = 0; i < V; ++i)
+        for (int i = 0; i < V; ++i)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) {
-          v = fmax(v, fabs(Gl[i][j]));
-          finite = finite && isfinite(Gl[i][j]);
-        }
-      if (!finite) v = -1.0;
-    }
-#pragma unroll
-    for (int s = 0; s < kPerLane; ++s) m[s] = s == k ? v : m[s];
-  }
-  for (int t = 0; t < kTop; ++t) {
-    double best = m[0];
-    int at = 0;
-#pragma unroll
-    for (int s = 1; s < kPerLane; ++s) {
-      at = m[s] > best ? s : at;
-      best = fmax(best, m[s]);
-    }
-    const int w = wave_argmax(best);
-    if (lane == w) {
-      key[wave * kTop + t] = best;
-      idx[wave * kTop + t] = (int32_t)(first + (int64_t)at * 64 + lane);
-#pragma unroll
-      for (int s = 0; s < kPerLane; ++s) m[s] = s == at ? -3.0 : m[s];
-    }
-  }
+          for (int j = 0; j < 3; ++j) {
+            v = fmax(v, fabs(Gl[i][j]));
+            finite = finite && isfinite(Gl[i][j]);
+          }
+        if (finite) k[r] = (TopKey)__double_as_longlong(v) + 1u;
+      });
+  // (position here is thread by thread, not the point's number: ties fall to the lower threads)
+  const int m = (int)min((int64_t)kListRounds * per, n - first);
+  TopKey* ko = key + (int64_t)blockIdx.x * kTop;
+  int32_t* io = idx + (int64_t)blockIdx.x * kTop;
+  select_top<256, kListRounds>(k, real, m, [&](int slot, int r) {
+    ko[slot] = k[r];
+    io[slot] = (int32_t)(first + r * per + threadIdx.x);
+  });
+  if ((int)threadIdx.x >= m && threadIdx.x < kTop) io[threadIdx.x] = -1;  // a last list of fewer points
 }
 
-// Pass 2: out[0, kTop) = the largest of the lists' points, out[kTop, kTop + spread) = points spread
-// evenly over the mesh; G receives their gradients.  pos (lists): scratch.
-template <class Cfg, int V>
-__global__ __launch_bounds__(1024) void k_grad_samples(fem_mesh_t mesh, const double* __restrict__ u, int lists,
-                                                       const double* __restrict__ key, const int32_t* __restrict__ idx,
-                                                       int32_t* __restrict__ pos, int top, int spread,
-                                                       int64_t* __restrict__ out, double* __restrict__ G) {
-  constexpr int N = Cfg::N;
-  __shared__ double s_key[16];
-  __shared__ int s_who[16];
-  __shared__ int64_t s_out[2 * kTop];
-  const int t = threadIdx.x, w = t >> 6;
-  const int64_t n = mesh.num_cells * mesh.num_quads;
-  for (int l = t; l < lists; l += 1024) pos[l] = 0;
-  double best = -4.0;
-  int list = -1;
-  auto scan = [&]() {  // the greatest head of this thread's lists
-    best = -4.0;
-    list = -1;
-    for (int l = t; l < lists; l += 1024) {
-      const int p = pos[l];
-      const double k = p < kTop ? key[l * kTop + p] : -4.0;
-      if (k > best) {
-        best = k;
-        list = l;
-      }
-    }
-  };
-  scan();
-  for (int r = 0; r < top; ++r) {
-    const int lane = wave_argmax(best);
-    if ((t & 63) == lane) {
-      s_key[w] = best;
-      s_who[w] = t;
-    }
-    __syncthreads();
-    int win = 0;
-    for (int k = 1; k < 16; ++k) win = s_key[k] > s_key[win] ? k : win;
-    if (t == s_who[win]) {
-      s_out[r] = idx[list * kTop + pos[list]];
-      pos[list] += 1;
-      scan();
-    }
-    __syncthreads();
+// The kTop largest of kMergeKeys entries of the lists; unused entries have index -1.
+__device__ inline void merge_load(int64_t n, const TopKey* __restrict__ key, const int32_t* __restrict__ idx,
+                                  TopKey (&k)[kMergeKeys / kMergeThreads], int32_t (&id)[kMergeKeys / kMergeThreads],
+                                  bool (&real)[kMergeKeys / kMergeThreads], int* m) {
+  constexpr int PER = kMergeKeys / kMergeThreads;
+  __shared__ int s_m[kMergeThreads / 64];
+  int c = 0;
+#pragma unroll
+  for (int s = 0; s < PER; ++s) {
+    const int64_t i = (int64_t)blockIdx.x * kMergeKeys + threadIdx.x + s * kMergeThreads;
+    id[s] = i < n ? idx[i] : -1;
+    real[s] = id[s] >= 0;
+    k[s] = real[s] ? key[i] : 0;
+    c += real[s] ? 1 : 0;
   }
-  if (t < spread) s_out[top + t] = spread > 1 ? (int64_t)((double)t * (double)(n - 1) / (double)(spread - 1)) : 0;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+  if ((threadIdx.x & 63) == 0) s_m[threadIdx.x >> 6] = c;
   __syncthreads();
-  if (t < top + spread) {
-    const int64_t e = min(max(s_out[t], (int64_t)0), n - 1);
-    const int64_t c = e / mesh.num_quads;
-    const int q = (int)(e - c * mesh.num_quads);
-    double Gl[V][3], Ul[V];
-    point_grad<N, V>(mesh, reinterpret_cast<const double(*)[N][3]>(mesh.shape_grads_ref)[q], c, q, u, Gl, Ul);
-    out[t] = e;
-#pragma unroll
-    for (int i = 0; i < V; ++i)
-#pragma unroll
-      for (int j = 0; j < 3; ++j) G[(t * V + i) * 3 + j] = Gl[i][j];
+  *m = 0;
+  for (int w = 0; w < kMergeThreads / 64; ++w) *m += s_m[w];
+}
+
+__global__ __launch_bounds__(kMergeThreads) void k_merge_top(int64_t n, const TopKey* __restrict__ key,
+                                                             const int32_t* __restrict__ idx,
+                                                             TopKey* __restrict__ key_out,
+                                                             int32_t* __restrict__ idx_out) {
+  constexpr int PER = kMergeKeys / kMergeThreads;
+  TopKey k[PER];
+  int32_t id[PER];
+  bool real[PER];
+  int m;
+  merge_load(n, key, idx, k, id, real, &m);
+  const int64_t o = (int64_t)blockIdx.x * kTop;
+  select_top<kMergeThreads, PER>(k, real, m, [&](int slot, int s) {
+    key_out[o + slot] = k[s];
+    idx_out[o + slot] = id[s];
+  });
+  if ((int)threadIdx.x >= m && threadIdx.x < kTop) idx_out[o + threadIdx.x] = -1;
+}
+
+// The last selection, in descending order, and the spread points.
+__global__ __launch_bounds__(kMergeThreads) void k_order_top(int64_t n, const TopKey* __restrict__ key,
+                                                             const int32_t* __restrict__ idx, int64_t points, int top,
+                                                             int spread, int64_t* __restrict__ out) {
+  constexpr int PER = kMergeKeys / kMergeThreads;
+  __shared__ TopKey s_key[kTop];
+  __shared__ int32_t s_idx[kTop];
+  TopKey k[PER];
+  int32_t id[PER];
+  bool real[PER];
+  int m;
+  merge_load(n, key, idx, k, id, real, &m);
+  select_top<kMergeThreads, PER>(k, real, m, [&](int slot, int s) {
+    s_key[slot] = k[s];
+    s_idx[slot] = id[s];
+  });
+  __syncthreads();
+  const int t = threadIdx.x, have = min(m, kTop);
+  if (t < have) {
+    int rank = 0;
+    for (int i = 0; i < have; ++i)
+      rank += s_key[i] > s_key[t] || (s_key[i] == s_key[t] && s_idx[i] < s_idx[t]) ? 1 : 0;
+    if (rank < top) out[rank] = s_idx[t];
   }
+  if (t < spread)
+    out[top + t] = spread > 1 ? min((int64_t)((double)t * (double)(points - 1) / (double)(spread - 1)), points - 1) : 0;
+}
+
+// Gradients of chosen points, one workgroup of a wave each (the node data is loaded side by side).
+template <class Cfg, int V>
+__global__ __launch_bounds__(64) void k_grad_at(fem_mesh_t mesh, const double* __restrict__ u,
+                                                const int64_t* __restrict__ pts, double* __restrict__ G) {
+  constexpr int N = Cfg::N;
+  __shared__ double x[N][3], f[N][V], dN[N][3];
+  const int64_t e = pts[blockIdx.x], c = e / mesh.num_quads;
+  const int q = (int)(e - c * mesh.num_quads);
+  if (threadIdx.x < N) {
+    const int a = threadIdx.x;
+    const int64_t node = mesh.cells[c * N + a];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      x[a][j] = mesh.points[node * 3 + j];
+      dN[a][j] = mesh.shape_grads_ref[((size_t)q * N + a) * 3 + j];
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) f[a][i] = u[node * V + i];
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  double Gl[V][3], Ul[V];
+  point_grad<N, V>(x, f, dN, nullptr, Gl, Ul);
+#pragma unroll
+  for (int i = 0; i < V; ++i)
+#pragma unroll
+    for (int j = 0; j < 3; ++j) G[((size_t)blockIdx.x * V + i) * 3 + j] = Gl[i][j];
 }
 
 // -------------------------------------------------- u-dependent mass term
@@ -1143,7 +1281,7 @@ int fem_quad_grad(const fem_mesh_t* mesh, const double* u, double* G, double* U,
   if (mesh->num_cells == 0) return FEM_OK;
   return with_cfg(*mesh, [&](auto cfg) -> int {
     using Cfg = decltype(cfg);
-    const dim3 grid((unsigned)ceil_div(mesh->num_cells * mesh->num_quads, 256));
+    const dim3 grid((unsigned)ceil_div(mesh->num_cells * mesh->num_quads, PointCells<Cfg, 1>::round(*mesh)));
     if (mesh->vec == 1)
       hipLaunchKernelGGL((k_quad_grad<Cfg, 1>), grid, dim3(256), 0, as_stream(stream), *mesh, u, G, U);
     else
@@ -1153,35 +1291,60 @@ int fem_quad_grad(const fem_mesh_t* mesh, const double* u, double* G, double* U,
   });
 }
 
-static int64_t sample_lists(const fem_mesh_t* m) { return ceil_div(m->num_cells * m->num_quads, kPerWave); }
+// lists of the first pass (the rounds do not depend on vec)
+static int64_t sample_lists(const fem_mesh_t* m) {
+  int per = 256;
+  (void)with_cfg(*m, [&](auto cfg) -> int {
+    per = PointCells<decltype(cfg), 1>::round(*m);
+    return FEM_OK;
+  });
+  return ceil_div(m->num_cells * m->num_quads, (int64_t)kListRounds * std::max(per, 1));
+}
 
 int64_t fem_grad_samples_ws_bytes(const fem_mesh_t* mesh) {
   if (!mesh || mesh->num_cells <= 0) return 0;
-  const int64_t lists = sample_lists(mesh);
-  return lists * kTop * 12 + lists * 4 + 512;
+  // the lists and, beside them, those of the first merge
+  const int64_t n = sample_lists(mesh) * kTop;
+  return (n + ceil_div(n, kMergeKeys) * kTop) * 12 + 512;
 }
 
 int fem_grad_samples(const fem_mesh_t* mesh, const double* u, int32_t top, int32_t spread, int64_t* idx, double* G,
                      void* ws, void* stream) {
   if (int rc = check_mesh(mesh)) return rc;
-  const int64_t n = mesh->num_cells * mesh->num_quads;
+  const int64_t points = mesh->num_cells * mesh->num_quads;
   FEM_CHECK_ARG(u && idx && G && ws, "fem_grad_samples: NULL argument");
   FEM_CHECK_ARG(mesh->vec == 1 || mesh->vec == 3, "fem_grad_samples: vec must be 1 or 3 (got %d)", mesh->vec);
-  FEM_CHECK_ARG(top >= 1 && top <= kTop && spread >= 0 && spread <= kTop && top <= n,
+  FEM_CHECK_ARG(top >= 1 && top <= kTop && spread >= 0 && spread <= kTop && top <= points,
                 "fem_grad_samples: 1 to %d points, at most the mesh's", kTop);
-  FEM_CHECK_ARG(n < (int64_t)INT32_MAX, "fem_grad_samples: %lld points exceed 32-bit indices", (long long)n);
+  FEM_CHECK_ARG(points < (int64_t)INT32_MAX, "fem_grad_samples: %lld points exceed 32-bit indices",
+                (long long)points);
   const int64_t lists = sample_lists(mesh);
-  double* key = static_cast<double*>(ws);
-  int32_t* li = reinterpret_cast<int32_t*>(key + lists * kTop);
-  int32_t* pos = li + lists * kTop;
+  int64_t n = lists * kTop;
+  // two sets of lists: keys, then indices
+  TopKey* key[2];
+  int32_t* li[2];
+  key[0] = static_cast<TopKey*>(ws);
+  key[1] = key[0] + n;
+  li[0] = reinterpret_cast<int32_t*>(key[1] + ceil_div(n, kMergeKeys) * kTop);
+  li[1] = li[0] + n;
   hipStream_t s = as_stream(stream);
   return with_cfg(*mesh, [&](auto cfg) -> int {
     using Cfg = decltype(cfg);
     auto go = [&](auto vc) {
       constexpr int V = decltype(vc)::value;
-      hipLaunchKernelGGL((k_grad_top<Cfg, V>), dim3((unsigned)ceil_div(lists, 4)), dim3(256), 0, s, *mesh, u, key, li);
-      hipLaunchKernelGGL((k_grad_samples<Cfg, V>), dim3(1), dim3(1024), 0, s, *mesh, u, (int)lists,
-                         (const double*)key, (const int32_t*)li, pos, top, spread, idx, G);
+      hipLaunchKernelGGL((k_grad_top<Cfg, V>), dim3((unsigned)lists), dim3(256), 0, s, *mesh, u, key[0], li[0]);
+      int at = 0;
+      while (n > kMergeKeys) {
+        const int64_t groups = ceil_div(n, kMergeKeys);
+        hipLaunchKernelGGL(k_merge_top, dim3((unsigned)groups), dim3(kMergeThreads), 0, s, n, key[at], li[at],
+                           key[1 - at], li[1 - at]);
+        n = groups * kTop;
+        at = 1 - at;
+      }
+      hipLaunchKernelGGL(k_order_top, dim3(1), dim3(kMergeThreads), 0, s, n, (const TopKey*)key[at],
+                         (const int32_t*)li[at], points, top, spread, idx);
+      hipLaunchKernelGGL((k_grad_at<Cfg, V>), dim3((unsigned)(top + spread)), dim3(64), 0, s, *mesh, u,
+                         (const int64_t*)idx, G);
     };
     if (mesh->vec == 1)
       go(std::integral_constant<int, 1>{});
