@@ -53,14 +53,6 @@ __device__ inline LdsD* lds_base(double* p) {
   return q;
 }
 
-// Orders LDS accesses of one wave: the hardware executes them in order, so only the compiler
-// has to keep the order.
-__device__ inline void wave_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // ------------------------------------------------------------------ plan
 // Cell lists of each slice: kGroups end offsets, then the groups' unique incident
 // cells, ascending.  FILL = false writes the slice's entry and pair counts;

@@ -54,6 +54,14 @@ constexpr int kDppXor2 = 0x4E;        // quad_perm [2, 3, 0, 1]
 constexpr int kDppHalfMirror = 0x141; // lane i of 8 <- 7 - i
 constexpr int kDppMirror = 0x140;     // lane i of 16 <- 15 - i
 
+// Orders LDS accesses of one wave: the hardware executes them in order, so only the compiler
+// has to keep the order.
+__device__ inline void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <typename T>
 __device__ inline T wave_sum(T v) {
 #pragma unroll
