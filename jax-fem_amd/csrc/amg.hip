@@ -1476,9 +1476,7 @@ __global__ __launch_bounds__(256, 6) void k_bcsr_apply_blk(int64_t rows, const i
   double t = 0.0;
 #pragma unroll
   for (int i = 0; i < BR; ++i) {
-    double si = acc[i];
-#pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1) si += __shfl_xor(si, off, 64);
+    const double si = group_sum<G>(acc[i]);
     t = sub == i ? si : t;
   }
   if (fin) epilogue_store<MODE>(a, idx, t, e);
@@ -1652,11 +1650,49 @@ __global__ __launch_bounds__(AmgSliceCfg<T>::NT) void k_sell_apply(fem_pattern_t
   }
 }
 
-// first Chebyshev step from a zero iterate: d = c2 D^-1 rhs, x = d
-template <typename TX>
-__global__ void k_cheb_first(int64_t n, const double* __restrict__ rhs, const double* __restrict__ dinv, double c2,
-                             TX* __restrict__ d, TX* __restrict__ x, const int32_t* __restrict__ done) {
+__device__ inline double sum_parts(const double* part, int np, double* red) {
+  // four independent sums keep four loads in flight per thread (a fixed order)
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  int i = threadIdx.x;
+  for (; i + 768 < np; i += 1024) {
+    s0 += part[i];
+    s1 += part[i + 256];
+    s2 += part[i + 512];
+    s3 += part[i + 768];
+  }
+  for (; i < np; i += 256) s0 += part[i];
+  return block_sum_256((s0 + s1) + (s2 + s3), red);
+}
+
+// The end of CG iteration `it` (counted from 1) where the kernel that follows does it: |r|^2 from
+// the update's partials and the stop test.  Every block finds the same; block 0 writes it.
+struct CgEnd {
+  AmgScalars* sc;
+  const double* part;
+  int parts, it, maxiter;
+};
+__device__ inline bool cg_end(const CgEnd& e, double rr) {  // true: done
+  const bool bad = !isfinite(rr), done = bad || rr <= e.sc->stop2 || e.it >= e.maxiter;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    e.sc->rr = rr;
+    e.sc->iter = e.it;
+    if (bad) e.sc->nan = 1;
+    if (done) e.sc->done = 1;
+  }
+  return done;
+}
+
+// First Chebyshev step from a zero iterate: d = c2 D^-1 rhs, x = d.  END: ends a CG iteration first
+// (a sum of 1024 partials by every block, about 1 us, for a launch of 2 us and its gap).
+template <typename TX, bool END>
+__global__ __launch_bounds__(256) void k_cheb_first(int64_t n, const double* __restrict__ rhs,
+                                                    const double* __restrict__ dinv, double c2, TX* __restrict__ d,
+                                                    TX* __restrict__ x, const int32_t* __restrict__ done, CgEnd end) {
   if (done && *done) return;
+  if constexpr (END) {
+    __shared__ double red[4];
+    if (cg_end(end, sum_parts(end.part, end.parts, red))) return;
+  }
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const TX v = TX(c2 * dinv[i] * rhs[i]);
     d[i] = v;
@@ -1699,11 +1735,6 @@ __global__ __launch_bounds__(256) void k_norm2_part_f32(int64_t n, const float* 
 }
 
 // ---------------------------------------------------------------- CG
-struct AmgScalars {
-  double rz, alpha, beta, rr, stop2, bb;
-  int32_t done, iter, nan, first, maxiter, pad;
-};
-
 __global__ __launch_bounds__(256) void k_dot_part(int64_t n, const double* __restrict__ x,
                                                   const double* __restrict__ y, double* __restrict__ part,
                                                   const int32_t* __restrict__ done) {
@@ -1714,20 +1745,6 @@ __global__ __launch_bounds__(256) void k_dot_part(int64_t n, const double* __res
     s = fma(x[i], y[i], s);
   s = block_sum_256(s, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;
-}
-
-__device__ inline double sum_parts(const double* part, int np, double* red) {
-  // four independent sums keep four loads in flight per thread (a fixed order)
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-  int i = threadIdx.x;
-  for (; i + 768 < np; i += 1024) {
-    s0 += part[i];
-    s1 += part[i + 256];
-    s2 += part[i + 512];
-    s3 += part[i + 768];
-  }
-  for (; i < np; i += 256) s0 += part[i];
-  return block_sum_256((s0 + s1) + (s2 + s3), red);
 }
 
 __global__ __launch_bounds__(256) void k_finish(const double* __restrict__ part, int np, double* __restrict__ out) {
@@ -1741,26 +1758,14 @@ __global__ void k_cg_start(AmgScalars* sc, double rtol, double atol, int maxiter
   const double stop = fmax(rtol * sqrt(sc->bb), atol);
   sc->stop2 = stop * stop;
   sc->iter = 0;
-  sc->first = 1;
-  sc->maxiter = maxiter;
   sc->nan = !isfinite(sc->rr);
   sc->done = sc->nan || sc->rr <= sc->stop2 || maxiter <= 0;
 }
 
-__global__ __launch_bounds__(256) void k_cg_beta(const double* __restrict__ part, int np, AmgScalars* sc) {
+__global__ __launch_bounds__(256) void k_cg_beta(CgHead h) {
   __shared__ double red[4];
-  if (sc->done) return;
-  const double rz = sum_parts(part, np, red);
-  if (threadIdx.x == 0) {
-    if (!isfinite(rz)) {
-      sc->nan = 1;
-      sc->done = 1;
-      return;
-    }
-    sc->beta = sc->first ? 0.0 : rz / sc->rz;
-    sc->rz = rz;
-    sc->first = 0;
-  }
+  bool done;
+  (void)cg_head<256>(h, red, &done);
 }
 
 __global__ void k_cg_p(int64_t n, const double* __restrict__ z, double* __restrict__ p, const AmgScalars* sc) {
@@ -1770,7 +1775,8 @@ __global__ void k_cg_p(int64_t n, const double* __restrict__ z, double* __restri
     p[i] = beta == 0.0 ? z[i] : fma(beta, p[i], z[i]);
 }
 
-__global__ __launch_bounds__(256) void k_cg_alpha(const double* __restrict__ part, int np, AmgScalars* sc) {
+// alpha of an iteration with more <p, q> partials than every block of k_cg_xr should sum
+__global__ __launch_bounds__(256) void k_cg_alpha(const double* __restrict__ part, int np, int it, AmgScalars* sc) {
   __shared__ double red[4];
   if (sc->done) return;
   const double pq = sum_parts(part, np, red);
@@ -1781,16 +1787,31 @@ __global__ __launch_bounds__(256) void k_cg_alpha(const double* __restrict__ par
       sc->alpha = 0.0;
       return;
     }
-    sc->alpha = sc->rz / pq;
+    sc->alpha = sc->rz[it & 1] / pq;
   }
 }
 
+// x += alpha p, r -= alpha q and the partials of <r, r>; np > 0: alpha from the np <p, q> partials.
 __global__ __launch_bounds__(256) void k_cg_xr(int64_t n, const double* __restrict__ p, const double* __restrict__ q,
                                                double* __restrict__ x, double* __restrict__ r,
-                                               double* __restrict__ part, const AmgScalars* sc) {
+                                               const double* __restrict__ pq_part, int np, int it,
+                                               double* __restrict__ part, AmgScalars* sc) {
   __shared__ double red[4];
   if (sc->done) return;
-  const double alpha = sc->alpha;
+  double alpha;
+  if (np > 0) {
+    const double rz = sc->rz[it & 1], pq = sum_parts(pq_part, np, red);
+    if (!isfinite(pq) || pq == 0.0) {  // x and r stay as they are
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sc->nan = !isfinite(pq);
+        sc->done = 1;
+      }
+      return;
+    }
+    alpha = rz / pq;
+  } else {
+    alpha = sc->alpha;
+  }
   double s = 0.0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     x[i] = fma(alpha, p[i], x[i]);
@@ -1803,25 +1824,15 @@ __global__ __launch_bounds__(256) void k_cg_xr(int64_t n, const double* __restri
 }
 
 // after an FP64 residual replacement (sc->rr = |b - A x|^2): the stop test
-__global__ void k_cg_replaced(AmgScalars* sc) {
+__global__ void k_cg_replaced(AmgScalars* sc, int maxiter) {
   sc->nan = sc->nan || !isfinite(sc->rr);
-  sc->done = sc->nan || sc->rr <= sc->stop2 || sc->iter >= sc->maxiter;
+  sc->done = sc->nan || sc->rr <= sc->stop2 || sc->iter >= maxiter;
 }
 
-__global__ __launch_bounds__(256) void k_cg_rr(const double* __restrict__ part, int np, AmgScalars* sc) {
+__global__ __launch_bounds__(256) void k_cg_rr(CgEnd e) {
   __shared__ double red[4];
-  if (sc->done) return;
-  const double rr = sum_parts(part, np, red);
-  if (threadIdx.x == 0) {
-    sc->rr = rr;
-    sc->iter += 1;
-    if (!isfinite(rr)) {
-      sc->nan = 1;
-      sc->done = 1;
-    } else if (rr <= sc->stop2 || sc->iter >= sc->maxiter) {
-      sc->done = 1;
-    }
-  }
+  if (e.sc->done) return;
+  (void)cg_end(e, sum_parts(e.part, e.parts, red));
 }
 
 // ------------------------------------------------------------ dispatch
@@ -1970,14 +1981,23 @@ int level_apply(const fem_amg_t& amg, int l, int mode, const ApplyArgsT<TX, TY>&
 // Pre-smoothing (Chebyshev from a zero iterate), residual and restriction on
 // level l, vectors stored as TX.  On return *xo is the smoothed iterate and
 // *oo the other iterate buffer.  ev: see vcycle_impl.
+// The first step of a level below another is done by the restriction to it (AP_FIRST, into x_next
+// and dd_next).  end (level 0, may be NULL): the CG iteration to end first.
 template <typename T, typename TX>
 int level_down(const fem_amg_t& amg, int l, int64_t n, const double* rhs, double* rhs_next, TX* x, TX* other,
-               TX* dd, TX* res, TX** xo, TX** oo, hipStream_t s, hipEvent_t* ev, const int32_t* done) {
+               TX* dd, TX* res, TX* x_next, TX* dd_next, TX** xo, TX** oo, hipStream_t s, hipEvent_t* ev,
+               const int32_t* done, const CgEnd* end) {
   const fem_amg_level_t& L = amg.levels[l];
   const Cheb cb(L.lmax);
-  hipLaunchKernelGGL(k_cheb_first<TX>, dim3(grid_for(n, 256)), dim3(256), 0, s, n, rhs, L.dinv, 1.0 / cb.theta, dd,
-                     x, done);
-  FEM_LAUNCHED();
+  if (l == 0) {
+    const dim3 grid(grid_for(n, 256)), nt(256);
+    if (end)
+      hipLaunchKernelGGL((k_cheb_first<TX, true>), grid, nt, 0, s, n, rhs, L.dinv, 1.0 / cb.theta, dd, x, done, *end);
+    else
+      hipLaunchKernelGGL((k_cheb_first<TX, false>), grid, nt, 0, s, n, rhs, L.dinv, 1.0 / cb.theta, dd, x, done,
+                         CgEnd{});
+    FEM_LAUNCHED();
+  }
   double rho = 1.0 / cb.sigma;
   const int deg = level_degree(amg, l);
   for (int k = 1; k < deg; ++k) {
@@ -1993,18 +2013,26 @@ int level_down(const fem_amg_t& amg, int l, int64_t n, const double* rhs, double
   ApplyArgsT<TX, TX> ar{x, res, rhs, nullptr, nullptr, 0.0, 0.0, nullptr, done};
   if (int rc = level_apply<T>(amg, l, AP_RESID, ar, s)) return rc;
   ApplyArgsT<TX, double> arr{res, rhs_next, nullptr, nullptr, nullptr, 0.0, 0.0, nullptr, done};
-  if (int rc = bcsr_apply<AP_STORE, T>(L.R, arr, s)) return rc;
+  if (l + 1 < amg.num_levels) {
+    arr.dinv = amg.levels[l + 1].dinv;
+    arr.d = dd_next;
+    arr.c2 = 1.0 / Cheb(amg.levels[l + 1].lmax).theta;
+    arr.first = x_next;
+    if (int rc = bcsr_apply<AP_FIRST, T>(L.R, arr, s)) return rc;
+  } else if (int rc = bcsr_apply<AP_STORE, T>(L.R, arr, s)) {
+    return rc;
+  }
   *xo = x;
   *oo = other;
   return FEM_OK;
 }
 
 // Prolongation of the coarse correction xc into x and post-smoothing on level
-// l.  z (level 0 only, FP64): the output of the last Chebyshev step.  ev: see
-// vcycle_impl.
+// l.  z (level 0 only, FP64): the output of the last Chebyshev step; rz (may be NULL): its *parts
+// partials of <rhs, z>, where level 0 is matrix-free.  ev: see vcycle_impl.
 template <typename T, typename TX>
 int level_up(const fem_amg_t& amg, int l, const double* rhs, const double* xc, TX* x, TX* other, TX* dd, double* z,
-             TX** xo, hipStream_t s, hipEvent_t* ev, const int32_t* done) {
+             TX** xo, hipStream_t s, hipEvent_t* ev, const int32_t* done, double* rz, int* parts) {
   const fem_amg_level_t& L = amg.levels[l];
   const Cheb cb(L.lmax);
   ApplyArgsT<double, TX> ap{xc, x, nullptr, nullptr, nullptr, 0.0, 0.0, nullptr, done};
@@ -2024,8 +2052,10 @@ int level_up(const fem_amg_t& amg, int l, const double* rhs, const double* xc, T
     if (timed) FEM_HIP(hipEventRecord(ev[0], s));
     if (timed_last) FEM_HIP(hipEventRecord(ev[6], s));
     if (z && k == deg - 1) {
-      ApplyArgsT<TX, double> a{x, z, rhs, L.dinv, dd, c1, c2, nullptr, done};
-      if (int rc = level_apply<T>(amg, l, AP_CHEB, a, s)) return rc;
+      ApplyArgsT<TX, double> a{x, z, rhs, L.dinv, dd, c1, c2, rz, done};
+      if (int rc = rz ? patch_apply<AP_CHEBZ, TX, double>(*level0_operator(amg), a, s, parts)
+                      : level_apply<T>(amg, l, AP_CHEB, a, s))
+        return rc;
     } else {
       ApplyArgsT<TX, TX> a{x, other, rhs, L.dinv, dd, c1, c2, nullptr, done};
       if (int rc = level_apply<T>(amg, l, AP_CHEB, a, s)) return rc;
@@ -2049,9 +2079,12 @@ int level_up(const fem_amg_t& amg, int l, const double* rhs, const double* xc, T
 // multiplies, and on the high-contrast SIMP cantilever (160x80x40, E ratio
 // 10^3) the adjoint solve then took 84 instead of 76 iterations (106 with the
 // power iteration on FP32 iterates as well).
+// end (may be NULL): a CG iteration that the first kernel ends; rz (may be NULL, a matrix-free level
+// 0 only): receives the *parts partials of <r, z>.
 template <typename T>
 int vcycle_impl(const fem_amg_t& amg, const double* r, double* z, char* ws, hipStream_t s,
-                hipEvent_t* ev = nullptr, const int32_t* done = nullptr) {
+                hipEvent_t* ev = nullptr, const int32_t* done = nullptr, const CgEnd* end = nullptr,
+                double* rz = nullptr, int* parts = nullptr) {
   if (ev) FEM_HIP(hipEventRecord(ev[2], s));
   const int NL = amg.num_levels;
   std::vector<double*> rhs(NL + 1), xa(NL), xb(NL), dd(NL), res(NL), cur(NL + 1);
@@ -2076,8 +2109,10 @@ int vcycle_impl(const fem_amg_t& amg, const double* r, double* z, char* ws, hipS
   for (int l = 0; l < NL; ++l) {
     const int64_t n = level_n(amg, l);
     double *x = nullptr, *o = nullptr;
-    if (int rc = level_down<T, double>(amg, l, n, rhs[l], rhs[l + 1], xa[l], xb[l], dd[l], res[l], &x, &o, s,
-                                       ev, done))
+    const bool below = l + 1 < NL;
+    if (int rc = level_down<T, double>(amg, l, n, rhs[l], rhs[l + 1], xa[l], xb[l], dd[l], res[l],
+                                       below ? xa[l + 1] : nullptr, below ? dd[l + 1] : nullptr, &x, &o, s, ev, done,
+                                       end))
       return rc;
     cur[l] = x;
     xb[l] = o;
@@ -2092,7 +2127,7 @@ int vcycle_impl(const fem_amg_t& amg, const double* r, double* z, char* ws, hipS
   for (int l = NL - 1; l >= 0; --l) {
     double* x = nullptr;
     if (int rc = level_up<T, double>(amg, l, rhs[l], cur[l + 1], cur[l], xb[l], dd[l], l == 0 ? z : nullptr, &x, s,
-                                     ev, done))
+                                     ev, done, l == 0 ? rz : nullptr, parts))
       return rc;
     cur[l] = x;
   }
@@ -2804,7 +2839,8 @@ int64_t fem_amg_solve_ws_bytes(const fem_pattern_t* pat, const fem_amg_t* amg) {
   if (!pat) return 0;
   const int64_t n = std::max<int64_t>(pat->num_rows * pat->vec, 1);
   const int64_t np = std::max<int64_t>(pat->num_slices, kDotBlocks);
-  return fem_amg_ws_bytes(amg) + (int64_t)(4 * align256(n * 8) + align256(np * 8) + align256(sizeof(AmgScalars)));
+  return fem_amg_ws_bytes(amg) + (int64_t)(4 * align256(n * 8) + align256(np * 8) + align256(kDotBlocks * 8) +
+                                         align256(sizeof(AmgScalars)));
 }
 
 int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float* vals32, const fem_amg_t* amg,
@@ -2837,6 +2873,8 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
   w += align256(std::max<int64_t>(n, 1) * 8);
   double* part = reinterpret_cast<double*>(w);
   w += align256(std::max<int64_t>(pat->num_slices, kDotBlocks) * 8);
+  double* rr_part = reinterpret_cast<double*>(w);  // written while the <p, q> partials are read
+  w += align256(kDotBlocks * 8);
   AmgScalars* sc = reinterpret_cast<AmgScalars*>(w);
   const int32_t* done = &sc->done;
   const unsigned g = grid_for(n, 256);
@@ -2857,6 +2895,7 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
   FEM_LAUNCHED();
   if (int rc = true_residual()) return rc;
   hipLaunchKernelGGL(k_cg_start, dim3(1), dim3(1), 0, s, sc, opt->rtol, opt->atol, opt->maxiter);
+  if (pop) hipLaunchKernelGGL(k_dense_zero, dim3(g), dim3(256), 0, s, n, p);  // the first product reads 0 p + z
   FEM_LAUNCHED();
   AmgScalars h{};
   if (int rc = read_dev(sc, sizeof(AmgScalars), host_status, s, &h)) return rc;
@@ -2876,6 +2915,7 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
   double cheb_ms = 0.0, cycle_ms = 0.0;
   int samples = 0;
   int it = 0;
+  bool ended = true;  // the stop test of iteration `it` is done (or there is none yet)
   // FP32 outer operator: the recursive residual is replaced by the FP64 true
   // residual when it has fallen by reliable_delta since the last replacement,
   // and when it meets the tolerance (convergence is decided on the true one)
@@ -2884,25 +2924,40 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
   int replacements = 0;
   while (!h.done) {
     hipEvent_t* e = opt->timing ? ev : nullptr;
-    if (int rc = (amg->precision == FEM_F32 ? vcycle_impl<float>(*amg, r, z, cyc, s, e, done)
-                                            : vcycle_impl<double>(*amg, r, z, cyc, s, e, done)))
+    // Matrix-free: <r, z> comes with the cycle's last step, beta and p = z + beta p with the product.
+    // The end of an iteration that the host does not look at is left to the next cycle's first kernel.
+    const CgEnd end{sc, rr_part, kDotBlocks, it, opt->maxiter};
+    const CgEnd* pending = ended ? nullptr : &end;
+    int parts = kDotBlocks, np = (int)pat->num_slices;
+    if (int rc = (amg->precision == FEM_F32
+                      ? vcycle_impl<float>(*amg, r, z, cyc, s, e, done, pending, pop ? part : nullptr, &parts)
+                      : vcycle_impl<double>(*amg, r, z, cyc, s, e, done, pending, pop ? part : nullptr, &parts)))
       return rc;
-    hipLaunchKernelGGL(k_dot_part, dim3(kDotBlocks), dim3(256), 0, s, n, r, z, part, done);
-    hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(256), 0, s, part, kDotBlocks, sc);
-    hipLaunchKernelGGL(k_cg_p, dim3(g), dim3(256), 0, s, n, z, p, sc);
-    FEM_LAUNCHED();
-    ApplyArgs apq{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, part, done};
-    int np = (int)pat->num_slices;
-    if (int rc = pop       ? patch_apply<AP_PQ, double, double>(*pop, apq, s, &np)
-                 : outer32 ? sell_apply<AP_PQ, float, true>(*pat, vals32, apq, done, s)
+    const CgHead head{sc, part, parts, it};
+    if (pop) {
+      if (int rc = patch_pcg_product(*pop, head, (const double*)z, (const double*)p, p, q, part, s, &np)) return rc;
+    } else {
+      hipLaunchKernelGGL(k_dot_part, dim3(kDotBlocks), dim3(256), 0, s, n, r, z, part, done);
+      hipLaunchKernelGGL(k_cg_beta, dim3(1), dim3(256), 0, s, head);
+      hipLaunchKernelGGL(k_cg_p, dim3(g), dim3(256), 0, s, n, z, p, sc);
+      FEM_LAUNCHED();
+      ApplyArgs apq{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, part, done};
+      if (int rc = outer32 ? sell_apply<AP_PQ, float, true>(*pat, vals32, apq, done, s)
                            : sell_apply<AP_PQ, double>(*pat, vals, apq, done, s))
-      return rc;
-    hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, s, part, np, sc);
-    hipLaunchKernelGGL(k_cg_xr, dim3(kDotBlocks), dim3(256), 0, s, n, p, q, x, r, part, sc);
-    hipLaunchKernelGGL(k_cg_rr, dim3(1), dim3(256), 0, s, part, kDotBlocks, sc);
+        return rc;
+    }
+    const bool own = np > kSumParts;
+    if (own) hipLaunchKernelGGL(k_cg_alpha, dim3(1), dim3(256), 0, s, part, np, it, sc);
+    hipLaunchKernelGGL(k_cg_xr, dim3(kDotBlocks), dim3(256), 0, s, n, p, q, x, r, part, own ? 0 : np, it, rr_part, sc);
     FEM_LAUNCHED();
     ++it;
-    if (it % opt->check_every == 0 || it >= opt->maxiter) {
+    const bool look = it % opt->check_every == 0 || it >= opt->maxiter;
+    ended = look || amg->num_levels == 0;
+    if (ended) {
+      hipLaunchKernelGGL(k_cg_rr, dim3(1), dim3(256), 0, s, CgEnd{sc, rr_part, kDotBlocks, it, opt->maxiter});
+      FEM_LAUNCHED();
+    }
+    if (look) {
       if (int rc = read_dev(sc, sizeof(AmgScalars), host_status, s, &h)) return rc;
       // (a cycle queued after convergence exits at once: h.iter < it, no sample)
       if (opt->timing && h.iter >= it) {
@@ -2921,7 +2976,7 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
       }
       if (outer32 && !h.nan && (h.done ? h.iter < opt->maxiter : h.rr < delta2 * rr_repl)) {
         if (int rc = true_residual()) return rc;
-        hipLaunchKernelGGL(k_cg_replaced, dim3(1), dim3(1), 0, s, sc);
+        hipLaunchKernelGGL(k_cg_replaced, dim3(1), dim3(1), 0, s, sc, opt->maxiter);
         FEM_LAUNCHED();
         if (int rc = read_dev(sc, sizeof(AmgScalars), host_status, s, &h)) return rc;
         rr_repl = h.rr;
@@ -2941,14 +2996,14 @@ int fem_amg_pcg_solve(const fem_pattern_t* pat, const double* vals, const float*
                    : sell_apply<AP_RESID, double>(*pat, vals, af, nullptr, s))
     return rc;
   hipLaunchKernelGGL(k_dot_part, dim3(kDotBlocks), dim3(256), 0, s, n, q, q, part, (const int32_t*)nullptr);
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(256), 0, s, part, kDotBlocks, &sc->rz);
+  hipLaunchKernelGGL(k_finish, dim3(1), dim3(256), 0, s, part, kDotBlocks, &sc->rz[0]);
   FEM_LAUNCHED();
   AmgScalars fin{};
   if (int rc = read_dev(sc, sizeof(AmgScalars), host_status, s, &fin)) return rc;
   result->iterations = fin.iter;
   result->replacements = replacements;
   result->b_norm = sqrt(fin.bb);
-  result->res_norm = sqrt(fin.rz);
+  result->res_norm = sqrt(fin.rz[0]);
   result->status = fin.nan ? FEM_ERR_NAN : (fin.rr > fin.stop2 ? FEM_ERR_NOT_CONVERGED : FEM_OK);
   return FEM_OK;
 }

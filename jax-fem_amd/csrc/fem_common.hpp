@@ -82,6 +82,18 @@ __device__ inline double wave_sum<double>(double v) {
   return v;
 }
 
+// Sum over the aligned group of G lanes (a power of two), in every lane of it; steps as above.
+template <int G>
+__device__ inline double group_sum(double v) {
+  if (G >= 2) v += dpp_move<kDppXor1>(v);
+  if (G >= 4) v += dpp_move<kDppXor2>(v);
+  if (G >= 8) v += dpp_move<kDppHalfMirror>(v);
+  if (G >= 16) v += dpp_move<kDppMirror>(v);
+  if (G >= 32) v += __shfl_xor(v, 16, 64);
+  if (G >= 64) v += __shfl_xor(v, 32, 64);
+  return v;
+}
+
 // Block-wide sum for blockDim.x == 256 (4 waves); result valid in all threads.
 template <typename T>
 __device__ inline T block_sum_256(T v, T* smem /* >= 4 */) {

@@ -335,38 +335,54 @@ __device__ inline void neo_hookean_tangent(const fem_material_t& m, int64_t cq, 
 
 // The field a cells' pass gathers: x, or z + beta x (the direction of a CG iteration that the
 // pass begins, in the vectors' precision as the gather kernel stores it).
-template <typename TX>
+struct NoHead {
+  const int32_t* done;
+};
+template <typename TX, typename HEAD>
 struct PatchField {
   const TX* x;
   const TX* z;
-  PcgHead head;
-  const int32_t* done;
+  HEAD head;
 };
 
-template <bool CG, typename TX, int NT>
-__device__ inline TX patch_begin(const PatchField<TX>& f, bool* done) {
-  if constexpr (CG) {
+template <int NT>
+__device__ inline double begin(const NoHead& h, double*, bool* done) {
+  *done = h.done && *h.done;
+  return 0.0;
+}
+template <int NT>
+__device__ inline double begin(const PcgHead& h, double* smem, bool* done) {
+  return pcg_head<NT>(h, smem, done);
+}
+template <int NT>
+__device__ inline double begin(const CgHead& h, double* smem, bool* done) {
+  return cg_head<NT>(h, smem, done);
+}
+template <typename TX, typename HEAD, int NT>
+__device__ inline TX patch_begin(const PatchField<TX, HEAD>& f, bool* done) {
+  if constexpr (std::is_same<HEAD, NoHead>::value) {
+    return TX(begin<NT>(f.head, nullptr, done));
+  } else {
     __shared__ double smem[2 * (NT / 64)];
-    return TX(pcg_head<NT>(f.head, smem, done));
+    return TX(begin<NT>(f.head, smem, done));
   }
-  *done = f.done && *f.done;
-  return TX(0);
 }
 
 // MODE 0: internal force at x (u unused); MODE 1: tangent at u times x.
-template <class MAT, int MODE, typename TX, bool CG>
+template <class MAT, int MODE, typename TX, typename HEAD>
 __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh, fem_material_t mat,
                                                                 fem_patch_plan_t plan, const double* __restrict__ u,
-                                                                PatchField<TX> field, double* __restrict__ part) {
+                                                                PatchField<TX, HEAD> field, double* __restrict__ part) {
   constexpr int N = 8, V = MAT::V, NT = 2 * kPatchCells, STRIDE = N * V + 1;  // odd: no bank conflicts between cells
   constexpr bool kNeo = MODE == 1 && MAT::kNeedsU;     // the tangent of the hyperelastic law
   constexpr bool kLinear = !MAT::kNeedsU;
   static_assert(!MAT::kNeedsU || std::is_same<MAT, MatNeoHookean>::value, "one nonlinear law");
+  constexpr bool CG = !std::is_same<HEAD, NoHead>::value;
   using Sums = PatchSums<N, V, STRIDE, kPatchCells, NT>;
   __shared__ double s_r[kPatchCells * STRIDE];
   __shared__ typename Sums::Lds s_plan;
   bool done;
-  const TX beta = patch_begin<CG, TX, NT>(field, &done);
+  const TX beta = patch_begin<TX, HEAD, NT>(field, &done);
   if (done) return;
   const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
   Sums sums;
@@ -515,17 +531,18 @@ __device__ const int8_t kVtk27[27] = {0, 16, 4, 11, 20, 15, 3,  19, 7,  8, 22, 1
 // holding a line of three values, contract one axis at a time with the 1-D tables and hand
 // the results on through LDS (seven cells per wave, so no barrier is needed).  MODE as in
 // k_patch_hex8; the tangent covers the laws that are linear in grad u.
-template <class MAT, int MODE, typename TX, bool CG>
+template <class MAT, int MODE, typename TX, typename HEAD>
 __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_material_t mat, fem_patch_plan_t plan,
-                                                     PatchField<TX> field, double* __restrict__ part) {
+                                                     PatchField<TX, HEAD> field, double* __restrict__ part) {
   constexpr int N = 27, V = MAT::V, NT = 256, STRIDE = 243;  // doubles of LDS per cell: 3 fields, 3 kinds, 27 points
   constexpr bool kLinear = !MAT::kNeedsU;
   static_assert(MODE == 0 || kLinear, "the hyperelastic tangent runs on HEX8 patches only");
+  constexpr bool CG = !std::is_same<HEAD, NoHead>::value;
   using Sums = PatchSums<N, V, STRIDE, kPatchCells27, NT>;
   __shared__ double s_r[kPatchCells27 * STRIDE];
   __shared__ typename Sums::Lds s_plan;
   bool done;
-  const TX beta = patch_begin<CG, TX, NT>(field, &done);
+  const TX beta = patch_begin<TX, HEAD, NT>(field, &done);
   if (done) return;
   const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
   const int lane = min((int)(threadIdx.x & 63), 62);  // lane 63 repeats lane 62
@@ -710,7 +727,7 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
 
 // ------------------------------------------------------------------ gather
 // AP_STORE adds a.rhs where it is given (the residual's constant loads).
-// AP_PQ runs at most kPatchDotBlocks blocks (one partial each) of kDotThreads threads, which
+// AP_PQ and AP_CHEBZ run at most kPatchDotBlocks blocks (one partial each) of kDotThreads threads, which
 // still fill the chip; the others one thread per dof.
 constexpr int kDotThreads = 512;
 
@@ -734,12 +751,14 @@ __device__ inline void patch_range(int64_t n, int64_t* begin, int64_t* end) {
   *end = min(n, *begin + per);
 }
 
-template <int V, int MODE, typename TX, typename TY>
-__global__ __launch_bounds__(MODE == AP_PQ ? kDotThreads : 256) void k_patch_gather(int64_t n, const int32_t* __restrict__ inc_ptr,
+constexpr bool has_dot(int mode) { return mode == AP_PQ || mode == AP_CHEBZ; }
+
+template <int V, int MODE0, typename TX, typename TY>
+__global__ __launch_bounds__(has_dot(MODE0) ? kDotThreads : 256) void k_patch_gather(int64_t n, const int32_t* __restrict__ inc_ptr,
                                                       const int32_t* __restrict__ inc_idx,
                                                       const double* __restrict__ part,
                                                       const uint8_t* __restrict__ mask, ApplyArgsT<TX, TY> a) {
-  constexpr int NT = MODE == AP_PQ ? kDotThreads : 256;
+  constexpr int MODE = MODE0 == AP_CHEBZ ? AP_CHEB : MODE0, NT = has_dot(MODE0) ? kDotThreads : 256;
   __shared__ double red[NT / 64];
   if (a.done && *a.done) return;
   double pq = 0.0;
@@ -753,21 +772,22 @@ __global__ __launch_bounds__(MODE == AP_PQ ? kDotThreads : 256) void k_patch_gat
     double t = patch_sum<V>(idx, inc_ptr, inc_idx, part);
     if (fixed) t = double(a.x[idx]);
     if (MODE == AP_STORE) t += e.rhs;
-    epilogue_store<MODE>(a, idx, t, e);
-    if (MODE == AP_PQ) pq = fma(e.x, double(TY(t)), pq);
+    const double y = epilogue_store<MODE>(a, idx, t, e);
+    if (has_dot(MODE0)) pq = fma(MODE == AP_PQ ? e.x : e.rhs, y, pq);
   }
-  if (MODE == AP_PQ) {
+  if (has_dot(MODE0)) {
     pq = block_sum<NT>(pq, red);
     if (threadIdx.x == 0) a.part[blockIdx.x] = pq;
   }
 }
 
 // The gather of a CG product: p_new = z + beta p_old (as the cells' pass formed it), q, <p, q>.
-template <int V, typename T>
+// (p_old and p_new may be one vector: an entry is read and written by one thread)
+template <int V, typename T, typename SC>
 __global__ __launch_bounds__(kDotThreads) void k_patch_gather_cg(
     int64_t n, const int32_t* __restrict__ inc_ptr, const int32_t* __restrict__ inc_idx,
-    const double* __restrict__ part, const uint8_t* __restrict__ mask, const PcgScalars* __restrict__ sc,
-    const T* __restrict__ z, const T* __restrict__ p_old, T* __restrict__ p_new, T* __restrict__ q,
+    const double* __restrict__ part, const uint8_t* __restrict__ mask, const SC* __restrict__ sc,
+    const T* __restrict__ z, const T* p_old, T* p_new, T* __restrict__ q,
     double* __restrict__ pq_part) {
   __shared__ double red[kDotThreads / 64];
   if (sc->done) return;
@@ -838,21 +858,21 @@ bool patch_operator_ok(const fem_patch_operator_t* op, bool residual) {
 }
 
 // the cells' pass: partials of the internal force (MODE 0) or of the tangent product (MODE 1)
-template <int MODE, bool CG, typename TX>
-static int patch_cells(const fem_patch_operator_t& op, const PatchField<TX>& field, hipStream_t s) {
+template <int MODE, typename TX, typename HEAD>
+static int patch_cells(const fem_patch_operator_t& op, const PatchField<TX, HEAD>& field, hipStream_t s) {
   fem_material_t mat;
   const fem_mesh_t& m = *op.mesh;
   return with_patch_law(op, &mat, [&](auto tag) -> int {
     using MAT = decltype(tag);
     if (m.nodes_per_cell == 27) {
       if constexpr (MODE == 0 || !MAT::kNeedsU) {
-        hipLaunchKernelGGL((k_patch_hex27<MAT, MODE, TX, CG>), dim3((unsigned)op.plan->num_patches), dim3(256), 0, s,
+        hipLaunchKernelGGL((k_patch_hex27<MAT, MODE, TX, HEAD>), dim3((unsigned)op.plan->num_patches), dim3(256), 0, s,
                            m, mat, *op.plan, field, op.partials);
         FEM_LAUNCHED();
       }
       return FEM_OK;
     }
-    hipLaunchKernelGGL((k_patch_hex8<MAT, MODE, TX, CG>), dim3((unsigned)op.plan->num_patches), dim3(2 * kPatchCells),
+    hipLaunchKernelGGL((k_patch_hex8<MAT, MODE, TX, HEAD>), dim3((unsigned)op.plan->num_patches), dim3(2 * kPatchCells),
                        0, s, m, mat, *op.plan, op.u, field, op.partials);
     FEM_LAUNCHED();
     return FEM_OK;
@@ -863,9 +883,9 @@ template <int MODE, typename TX, typename TY>
 static int patch_gather(const fem_patch_operator_t& op, const uint8_t* mask, const ApplyArgsT<TX, TY>& a, hipStream_t s,
                         int* parts) {
   const int64_t n = op.mesh->num_nodes * op.mesh->vec;
-  constexpr int NT = MODE == AP_PQ ? kDotThreads : 256;
+  constexpr int NT = has_dot(MODE) ? kDotThreads : 256;
   const int64_t want = ceil_div(n, NT);
-  const unsigned grid = (unsigned)(MODE == AP_PQ ? std::min<int64_t>(want, kPatchDotBlocks) : want);
+  const unsigned grid = (unsigned)(has_dot(MODE) ? std::min<int64_t>(want, kPatchDotBlocks) : want);
   if (parts) *parts = (int)grid;
   if (op.mesh->vec == 3)
     hipLaunchKernelGGL((k_patch_gather<3, MODE, TX, TY>), dim3(grid), dim3(NT), 0, s, n, op.plan->inc_ptr,
@@ -879,20 +899,24 @@ static int patch_gather(const fem_patch_operator_t& op, const uint8_t* mask, con
 
 template <int MODE, typename TX, typename TY>
 int patch_apply(const fem_patch_operator_t& op, const ApplyArgsT<TX, TY>& a, hipStream_t s, int* parts) {
-  if (int rc = patch_cells<1, false, TX>(op, PatchField<TX>{a.x, nullptr, PcgHead{}, a.done}, s)) return rc;
+  if (int rc = patch_cells<1>(op, PatchField<TX, NoHead>{a.x, nullptr, NoHead{a.done}}, s)) return rc;
   return patch_gather<MODE, TX, TY>(op, op.bc_mask, a, s, parts);
 }
 
-template <typename T>
-int patch_pcg_product(const fem_patch_operator_t& op, const PcgHead& head, const T* z, const T* p_old, T* p_new, T* q,
+inline const PcgScalars* head_scalars(const PcgHead& h) { return h.next; }
+inline const AmgScalars* head_scalars(const CgHead& h) { return h.sc; }
+
+template <typename HEAD, typename T>
+int patch_pcg_product(const fem_patch_operator_t& op, const HEAD& head, const T* z, const T* p_old, T* p_new, T* q,
                       double* part, hipStream_t s, int* parts) {
-  if (int rc = patch_cells<1, true, T>(op, PatchField<T>{p_old, z, head, nullptr}, s)) return rc;
+  if (int rc = patch_cells<1>(op, PatchField<T, HEAD>{p_old, z, head}, s)) return rc;
   const int64_t n = op.mesh->num_nodes * op.mesh->vec;
   *parts = (int)std::min<int64_t>(ceil_div(n, kDotThreads), kPatchDotBlocks);
   auto go = [&](auto vc) {
     constexpr int V = decltype(vc)::value;
-    hipLaunchKernelGGL((k_patch_gather_cg<V, T>), dim3((unsigned)*parts), dim3(kDotThreads), 0, s, n,
-                       op.plan->inc_ptr, op.plan->inc_idx, op.partials, op.bc_mask, (const PcgScalars*)head.next, z,
+    using S = typename std::remove_pointer<decltype(head_scalars(head))>::type;
+    hipLaunchKernelGGL((k_patch_gather_cg<V, T, S>), dim3((unsigned)*parts), dim3(kDotThreads), 0, s, n,
+                       op.plan->inc_ptr, op.plan->inc_idx, op.partials, op.bc_mask, head_scalars(head), z,
                        p_old, p_new, q, part);
   };
   if (op.mesh->vec == 3)
@@ -903,10 +927,12 @@ int patch_pcg_product(const fem_patch_operator_t& op, const PcgHead& head, const
   return FEM_OK;
 }
 
-template int patch_pcg_product<double>(const fem_patch_operator_t&, const PcgHead&, const double*, const double*,
-                                       double*, double*, double*, hipStream_t, int*);
-template int patch_pcg_product<float>(const fem_patch_operator_t&, const PcgHead&, const float*, const float*, float*,
-                                      float*, double*, hipStream_t, int*);
+template int patch_pcg_product(const fem_patch_operator_t&, const PcgHead&, const double*, const double*, double*,
+                               double*, double*, hipStream_t, int*);
+template int patch_pcg_product(const fem_patch_operator_t&, const PcgHead&, const float*, const float*, float*, float*,
+                               double*, hipStream_t, int*);
+template int patch_pcg_product(const fem_patch_operator_t&, const CgHead&, const double*, const double*, double*,
+                               double*, double*, hipStream_t, int*);
 
 template int patch_apply<AP_STORE, double, double>(const fem_patch_operator_t&, const ApplyArgsT<double, double>&,
                                                    hipStream_t, int*);
@@ -914,6 +940,8 @@ template int patch_apply<AP_RESID, double, double>(const fem_patch_operator_t&, 
                                                    hipStream_t, int*);
 template int patch_apply<AP_CHEB, double, double>(const fem_patch_operator_t&, const ApplyArgsT<double, double>&,
                                                   hipStream_t, int*);
+template int patch_apply<AP_CHEBZ, double, double>(const fem_patch_operator_t&, const ApplyArgsT<double, double>&,
+                                                   hipStream_t, int*);
 template int patch_apply<AP_DSTORE, double, double>(const fem_patch_operator_t&, const ApplyArgsT<double, double>&,
                                                     hipStream_t, int*);
 template int patch_apply<AP_PQ, double, double>(const fem_patch_operator_t&, const ApplyArgsT<double, double>&,
@@ -993,7 +1021,7 @@ int fem_patch_residual(const fem_patch_operator_t* op, const double* u, const do
   o.u = u;
   FEM_CHECK_ARG(patch_operator_ok(&o, true), "fem_patch_residual: the operator is incomplete or not covered");
   hipStream_t s = as_stream(stream);
-  if (int rc = patch_cells<0, false, double>(o, PatchField<double>{u, nullptr, PcgHead{}, nullptr}, s)) return rc;
+  if (int rc = patch_cells<0>(o, PatchField<double, NoHead>{u, nullptr, NoHead{nullptr}}, s)) return rc;
   ApplyArgs a{u, res, base, nullptr, nullptr, 0.0, 0.0, nullptr, nullptr};
   return patch_gather<AP_STORE, double, double>(o, nullptr, a, s, nullptr);
 }

@@ -280,7 +280,6 @@ __global__ __launch_bounds__(256) void k_spmv_x(fem_pattern_t pat, const T* __re
 }
 
 constexpr int kVecGrid = 1024;  // blocks of the vector kernels (partials per reduction)
-constexpr int kSumParts = 2048;  // most <p, q> partials that every block of the update kernel sums itself
 // Largest matrix whose product forms its direction itself (us per iteration, with and without):
 // FP64 3 MB 13 / 18, 28 MB 15.9 / 19.5, 38 MB 21.9 / 22.1; FP32 39 MB 17.3 / 18.9, 59 MB 35 / 32.5.
 constexpr double kFuseBytes = 48e6;
@@ -448,7 +447,7 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
       if (!fused) hipLaunchKernelGGL(k_pcg_p<T>, dim3(gV), dim3(256), 0, s, n, (const T*)z, p, head);
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 1], s));
       if (pop && fused) {
-        if (int rc = patch_pcg_product<T>(*pop, head, z, pc, pn, q, w.partA, s, &gA)) return rc;
+        if (int rc = patch_pcg_product<PcgHead, T>(*pop, head, z, pc, pn, q, w.partA, s, &gA)) return rc;
       } else if (pop) {
         ApplyArgsT<T, T> a{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, w.partA, &sc->done};
         if (int rc = patch_apply<AP_PQ, T, T>(*pop, a, s, &gA)) return rc;

@@ -1,5 +1,5 @@
-// Scalars of the Jacobi-PCG iteration and the reductions that a consuming kernel does
-// itself (pcg.hip, patch.hip).
+// Scalars of the CG iterations (Jacobi-PCG and AMG-CG) and the reductions that a consuming
+// kernel does itself (pcg.hip, amg.hip, patch.hip).
 #pragma once
 #include "fem_common.hpp"
 
@@ -82,6 +82,48 @@ __device__ inline double pcg_head(const PcgHead& h, double* smem, bool* done) {
   if (blockIdx.x == 0 && threadIdx.x == 0) pcg_store(h.next, s, 0);
   *done = s.done != 0;
   return s.beta;
+}
+
+constexpr int kSumParts = 2048;  // most partials that every block of a consuming kernel sums itself
+
+// AMG-CG.  rz: <r, z> of the last two iterations (slot = iteration & 1), so that the kernel that
+// forms a new one reads what none of its blocks writes.
+struct AmgScalars {
+  double rz[2], alpha, beta, rr, stop2, bb;
+  int32_t done, iter, nan, pad;
+};
+static_assert(sizeof(AmgScalars) <= 128, "host status buffer");
+
+// beta of iteration `it` (0: the first), summed by every block of the product that needs it from
+// the <r, z> partials of the V-cycle's last kernel.
+struct CgHead {
+  AmgScalars* sc;
+  const double* part;
+  int parts, it;
+};
+
+template <int NT>
+__device__ inline double cg_head(const CgHead& h, double* smem, bool* done) {
+  double a = 0.0;
+  for (int i = threadIdx.x; i < h.parts; i += NT) a += h.part[i];
+  const double old = h.sc->rz[(h.it + 1) & 1];
+  if (h.sc->done) {
+    *done = true;
+    return 0.0;
+  }
+  a = block_sum<NT>(a, smem);
+  *done = !isfinite(a);
+  const double beta = h.it == 0 ? 0.0 : a / old;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (*done) {
+      h.sc->nan = 1;
+      h.sc->done = 1;
+    } else {
+      h.sc->rz[h.it & 1] = a;
+      h.sc->beta = beta;
+    }
+  }
+  return beta;
 }
 
 }  // namespace fem
