@@ -1444,7 +1444,7 @@ __global__ __launch_bounds__(256, 6) void k_bcsr_apply_blk(int64_t rows, const i
                                                            const int32_t* __restrict__ ci, const T* __restrict__ v,
                                                            ApplyArgsT<TX, TY> a) {
   static_assert(G >= BR && G <= 64 && (G & (G - 1)) == 0, "G: a power of two, at least the block rows");
-  if (a.done && *a.done) return;
+  const int32_t done = a.done ? *a.done : 0;  // looked at once the first loads are on their way
   const int sub = threadIdx.x & (G - 1);
   const int64_t row = ((int64_t)blockIdx.x * 256 + threadIdx.x) / G;
   const bool live = row < rows;  // a group is live or dead as a whole: its shuffles stay inside it
@@ -1455,10 +1455,11 @@ __global__ __launch_bounds__(256, 6) void k_bcsr_apply_blk(int64_t rows, const i
   double acc[BR];
 #pragma unroll
   for (int i = 0; i < BR; ++i) acc[i] = 0.0;
-  if (live) {
-    const int k1 = rp[row + 1];
+  const int k0 = live ? rp[row] : 0, k1 = live ? rp[row + 1] : 0;
+  if (done) return;
+  {
 #pragma unroll 1
-    for (int k = rp[row] + sub; k < k1; k += G) {
+    for (int k = k0 + sub; k < k1; k += G) {
       // the block stays in its storage type until each product (FP32 blocks: half the
       // registers of an FP64 copy, so more waves stay resident)
       T blk[BR * BC];
@@ -1489,7 +1490,7 @@ __global__ __launch_bounds__(256) void k_bcsr_apply_row(int64_t rows, const int3
                                                         const int32_t* __restrict__ ci, const T* __restrict__ v,
                                                         ApplyArgsT<TX, TY> a) {
   __shared__ double smem[4][BR];
-  if (a.done && *a.done) return;
+  const int32_t done = a.done ? *a.done : 0;  // looked at once the first loads are on their way
   const int64_t row = blockIdx.x;
   const int w = threadIdx.x >> 6;
   EpiOperands e{0.0, 0.0, 0.0, 0.0, 0.0};
@@ -1499,6 +1500,7 @@ __global__ __launch_bounds__(256) void k_bcsr_apply_row(int64_t rows, const int3
   for (int i = 0; i < BR; ++i) acc[i] = 0.0;
   const int b = rp[row];
   const int nf = (rp[row + 1] - b) * BC;
+  if (done) return;
   // unrolled so that several pairs' loads are in flight (the sums keep their order)
 #pragma unroll 4
   for (int f = threadIdx.x; f < nf; f += 256) {
@@ -1688,15 +1690,32 @@ template <typename TX, bool END>
 __global__ __launch_bounds__(256) void k_cheb_first(int64_t n, const double* __restrict__ rhs,
                                                     const double* __restrict__ dinv, double c2, TX* __restrict__ d,
                                                     TX* __restrict__ x, const int32_t* __restrict__ done, CgEnd end) {
+  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  double bi = 0.0, di = 0.0;
+  auto load = [&]() {
+    if (i < n) {
+      bi = rhs[i];
+      di = dinv[i];
+    }
+  };
+  double part[4] = {0.0, 0.0, 0.0, 0.0};
+  if constexpr (END)
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if ((int)threadIdx.x + 256 * k < end.parts) part[k] = end.part[threadIdx.x + 256 * k];
+  load();
   if (done && *done) return;
   if constexpr (END) {
     __shared__ double red[4];
-    if (cg_end(end, sum_parts(end.part, end.parts, red))) return;
+    static_assert(kDotBlocks <= 1024, "the partials a thread holds");
+    if (cg_end(end, block_sum_256((part[0] + part[1]) + (part[2] + part[3]), red))) return;
   }
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    const TX v = TX(c2 * dinv[i] * rhs[i]);
+  while (i < n) {
+    const TX v = TX(c2 * di * bi);
     d[i] = v;
     x[i] = v;
+    i += (int64_t)gridDim.x * blockDim.x;
+    load();
   }
 }
 
@@ -1765,7 +1784,7 @@ __global__ void k_cg_start(AmgScalars* sc, double rtol, double atol, int maxiter
 __global__ __launch_bounds__(256) void k_cg_beta(CgHead h) {
   __shared__ double red[4];
   bool done;
-  (void)cg_head<256>(h, red, &done);
+  (void)cg_head<256>(h, cg_raw<256>(h), red, &done);
 }
 
 __global__ void k_cg_p(int64_t n, const double* __restrict__ z, double* __restrict__ p, const AmgScalars* sc) {
@@ -1797,10 +1816,28 @@ __global__ __launch_bounds__(256) void k_cg_xr(int64_t n, const double* __restri
                                                const double* __restrict__ pq_part, int np, int it,
                                                double* __restrict__ part, AmgScalars* sc) {
   __shared__ double red[4];
+  // the first entry's loads and the partials' are in flight together
+  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  double xi = 0.0, pi = 0.0, ri = 0.0, qi = 0.0;
+  auto load = [&]() {
+    if (i < n) {
+      xi = x[i];
+      pi = p[i];
+      ri = r[i];
+      qi = q[i];
+    }
+  };
+  double pa[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if ((int)threadIdx.x + 256 * k < np) pa[k] = pq_part[threadIdx.x + 256 * k];
+  load();
   if (sc->done) return;
   double alpha;
   if (np > 0) {
-    const double rz = sc->rz[it & 1], pq = sum_parts(pq_part, np, red);
+    double sum = (pa[0] + pa[1]) + (pa[2] + pa[3]);
+    for (int k = threadIdx.x + 1024; k < np; k += 256) sum += pq_part[k];
+    const double rz = sc->rz[it & 1], pq = block_sum_256(sum, red);
     if (!isfinite(pq) || pq == 0.0) {  // x and r stay as they are
       if (blockIdx.x == 0 && threadIdx.x == 0) {
         sc->nan = !isfinite(pq);
@@ -1813,11 +1850,13 @@ __global__ __launch_bounds__(256) void k_cg_xr(int64_t n, const double* __restri
     alpha = sc->alpha;
   }
   double s = 0.0;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    x[i] = fma(alpha, p[i], x[i]);
-    const double ri = fma(-alpha, q[i], r[i]);
-    r[i] = ri;
-    s = fma(ri, ri, s);
+  while (i < n) {
+    x[i] = fma(alpha, pi, xi);
+    const double rn = fma(-alpha, qi, ri);
+    r[i] = rn;
+    s = fma(rn, rn, s);
+    i += (int64_t)gridDim.x * blockDim.x;
+    load();
   }
   s = block_sum_256(s, red);
   if (threadIdx.x == 0) part[blockIdx.x] = s;

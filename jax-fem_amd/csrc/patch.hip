@@ -345,26 +345,42 @@ struct PatchField {
   HEAD head;
 };
 
+// A cells' pass takes raw() first, loads its cells' data and then finishes the head (begin()).
+struct NoRaw {
+  int32_t done;
+};
 template <int NT>
-__device__ inline double begin(const NoHead& h, double*, bool* done) {
-  *done = h.done && *h.done;
+__device__ inline NoRaw raw(const NoHead& h) {
+  return NoRaw{h.done ? *h.done : 0};
+}
+template <int NT>
+__device__ inline PcgRaw<NT> raw(const PcgHead& h) {
+  return pcg_raw<NT>(h);
+}
+template <int NT>
+__device__ inline CgRaw<NT> raw(const CgHead& h) {
+  return cg_raw<NT>(h);
+}
+template <int NT>
+__device__ inline double begin(const NoHead&, const NoRaw& r, double*, bool* done) {
+  *done = r.done != 0;
   return 0.0;
 }
 template <int NT>
-__device__ inline double begin(const PcgHead& h, double* smem, bool* done) {
-  return pcg_head<NT>(h, smem, done);
+__device__ inline double begin(const PcgHead& h, const PcgRaw<NT>& r, double* smem, bool* done) {
+  return pcg_head<NT>(h, r, smem, done);
 }
 template <int NT>
-__device__ inline double begin(const CgHead& h, double* smem, bool* done) {
-  return cg_head<NT>(h, smem, done);
+__device__ inline double begin(const CgHead& h, const CgRaw<NT>& r, double* smem, bool* done) {
+  return cg_head<NT>(h, r, smem, done);
 }
-template <typename TX, typename HEAD, int NT>
-__device__ inline TX patch_begin(const PatchField<TX, HEAD>& f, bool* done) {
+template <int NT, typename TX, typename HEAD, typename RAW>
+__device__ inline TX patch_begin(const PatchField<TX, HEAD>& f, const RAW& r, bool* done) {
   if constexpr (std::is_same<HEAD, NoHead>::value) {
-    return TX(begin<NT>(f.head, nullptr, done));
+    return TX(begin<NT>(f.head, r, nullptr, done));
   } else {
     __shared__ double smem[2 * (NT / 64)];
-    return TX(begin<NT>(f.head, smem, done));
+    return TX(begin<NT>(f.head, r, smem, done));
   }
 }
 
@@ -381,9 +397,7 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
   using Sums = PatchSums<N, V, STRIDE, kPatchCells, NT>;
   __shared__ double s_r[kPatchCells * STRIDE];
   __shared__ typename Sums::Lds s_plan;
-  bool done;
-  const TX beta = patch_begin<TX, HEAD, NT>(field, &done);
-  if (done) return;
+  const auto head = raw<NT>(field.head);
   const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
   Sums sums;
   const int h = threadIdx.x & 1, cl = threadIdx.x >> 1;
@@ -397,6 +411,7 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
     const int4 node = *reinterpret_cast<const int4*>(mesh.cells + c * N + 4 * h);
     const int id[4] = {node.x, node.y, node.z, node.w};
     double nx[4][3], nf[4][V];
+    TX fx[4][V], fz[CG ? 4 : 1][V];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
 #pragma unroll
@@ -404,10 +419,18 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         const int64_t at = (int64_t)id[k] * V + v;
-        nf[k][v] = double(CG ? fma(beta, field.x[at], field.z[at]) : field.x[at]);
+        fx[k][v] = field.x[at];
+        if (CG) fz[k][v] = field.z[at];
       }
     }
     sums.load(plan, patch, mesh.num_cells);
+    bool done;
+    const TX beta = patch_begin<NT>(field, head, &done);
+    if (done) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int v = 0; v < V; ++v) nf[k][v] = double(CG ? fma(beta, fx[k][v], fz[k][v]) : fx[k][v]);
     // coordinates from the cell's first node, so that their differences round like the cell's size
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -541,9 +564,7 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
   using Sums = PatchSums<N, V, STRIDE, kPatchCells27, NT>;
   __shared__ double s_r[kPatchCells27 * STRIDE];
   __shared__ typename Sums::Lds s_plan;
-  bool done;
-  const TX beta = patch_begin<TX, HEAD, NT>(field, &done);
-  if (done) return;
+  const auto head = raw<NT>(field.head);
   const int64_t patch = xcd_logical_block(blockIdx.x, gridDim.x);
   const int lane = min((int)(threadIdx.x & 63), 62);  // lane 63 repeats lane 62
   const int cl = (threadIdx.x >> 6) * 7 + lane / 9, t = lane % 9, ta = t / 3, tb = t % 3;
@@ -595,6 +616,7 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
   int vtk[3];
   {
     double nx[3][3], nf[3][V];
+    TX fx[3][V], fz[CG ? 3 : 1][V];
     const int32_t* cn = mesh.cells + c * N;
     const double* p0 = mesh.points + (int64_t)cn[0] * 3;
 #pragma unroll
@@ -606,10 +628,18 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
 #pragma unroll
       for (int v = 0; v < V; ++v) {
         const int64_t at = id * V + v;
-        nf[i][v] = double(CG ? fma(beta, field.x[at], field.z[at]) : field.x[at]);
+        fx[i][v] = field.x[at];
+        if (CG) fz[i][v] = field.z[at];
       }
     }
     sums.load(plan, patch, mesh.num_cells);
+    bool done;
+    const TX beta = patch_begin<NT>(field, head, &done);
+    if (done) return;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int v = 0; v < V; ++v) nf[i][v] = double(CG ? fma(beta, fx[i][v], fz[i][v]) : fx[i][v]);
     contract(nx, hx);
     contract(nf, hf);
   }
@@ -733,14 +763,16 @@ constexpr int kDotThreads = 512;
 
 // sum of the partials of dof idx
 template <int V>
-__device__ inline double patch_sum(int64_t idx, const int32_t* __restrict__ inc_ptr,
-                                   const int32_t* __restrict__ inc_idx, const double* __restrict__ part) {
-  const int64_t node = idx / V;
-  const int v = (int)(idx - node * V);
-  const int k1 = inc_ptr[node + 1];
+__device__ inline double patch_sum(int64_t idx, int2 inc, const int32_t* __restrict__ inc_idx,
+                                   const double* __restrict__ part) {
+  const int v = (int)(idx % V);
   double t = 0.0;
-  for (int k = inc_ptr[node]; k < k1; ++k) t += part[(int64_t)inc_idx[k] * V + v];
+  for (int k = inc.x; k < inc.y; ++k) t += part[(int64_t)inc_idx[k] * V + v];
   return t;
+}
+template <int V>
+__device__ inline int2 patch_inc(int64_t idx, const int32_t* __restrict__ inc_ptr) {
+  return make_int2(inc_ptr[idx / V], inc_ptr[idx / V + 1]);
 }
 
 // the dofs of a block: one contiguous range, in the order of the patches
@@ -760,7 +792,7 @@ __global__ __launch_bounds__(has_dot(MODE0) ? kDotThreads : 256) void k_patch_ga
                                                       const uint8_t* __restrict__ mask, ApplyArgsT<TX, TY> a) {
   constexpr int MODE = MODE0 == AP_CHEBZ ? AP_CHEB : MODE0, NT = has_dot(MODE0) ? kDotThreads : 256;
   __shared__ double red[NT / 64];
-  if (a.done && *a.done) return;
+  const int32_t done = a.done ? *a.done : 0;  // looked at once the first loads are on their way
   double pq = 0.0;
   int64_t begin, end;
   patch_range(n, &begin, &end);
@@ -769,13 +801,15 @@ __global__ __launch_bounds__(has_dot(MODE0) ? kDotThreads : 256) void k_patch_ga
     if (MODE == AP_PQ) e.x = double(a.x[idx]);
     if (MODE == AP_STORE && a.rhs) e.rhs = a.rhs[idx];
     const bool fixed = mask && mask[idx];
-    double t = patch_sum<V>(idx, inc_ptr, inc_idx, part);
+    const int2 inc = patch_inc<V>(idx, inc_ptr);
+    if (done) break;
+    double t = patch_sum<V>(idx, inc, inc_idx, part);
     if (fixed) t = double(a.x[idx]);
     if (MODE == AP_STORE) t += e.rhs;
     const double y = epilogue_store<MODE>(a, idx, t, e);
     if (has_dot(MODE0)) pq = fma(MODE == AP_PQ ? e.x : e.rhs, y, pq);
   }
-  if (has_dot(MODE0)) {
+  if (has_dot(MODE0) && !done) {
     pq = block_sum<NT>(pq, red);
     if (threadIdx.x == 0) a.part[blockIdx.x] = pq;
   }
@@ -790,20 +824,24 @@ __global__ __launch_bounds__(kDotThreads) void k_patch_gather_cg(
     const T* __restrict__ z, const T* p_old, T* p_new, T* __restrict__ q,
     double* __restrict__ pq_part) {
   __shared__ double red[kDotThreads / 64];
-  if (sc->done) return;
+  const int32_t done = sc->done;  // (as above)
   const T beta = T(sc->beta);
   double pq = 0.0;
   int64_t begin, end;
   patch_range(n, &begin, &end);
   for (int64_t idx = begin + threadIdx.x; idx < end; idx += kDotThreads) {
-    const T p = fma(beta, p_old[idx], z[idx]);
+    const T po = p_old[idx], zi = z[idx];
     const bool fixed = mask && mask[idx];
-    const double t = patch_sum<V>(idx, inc_ptr, inc_idx, part);
+    const int2 inc = patch_inc<V>(idx, inc_ptr);
+    if (done) return;
+    const T p = fma(beta, po, zi);
+    const double t = patch_sum<V>(idx, inc, inc_idx, part);
     const T qi = fixed ? p : T(t);
     p_new[idx] = p;
     q[idx] = qi;
     pq = fma(double(p), double(qi), pq);
   }
+  if (done) return;
   pq = block_sum<kDotThreads>(pq, red);
   if (threadIdx.x == 0) pq_part[blockIdx.x] = pq;
 }

@@ -49,7 +49,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void k_pcg_p(int64_t n, const T* __restrict__ z, T* __restrict__ p, PcgHead head) {
   __shared__ double smem[8];
   bool done;
-  const T beta = T(pcg_head<256>(head, smem, &done));
+  const T beta = T(pcg_head<256>(head, pcg_raw<256>(head), smem, &done));
   if (done) return;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     p[i] = fma(beta, p[i], z[i]);
@@ -67,30 +67,97 @@ __global__ __launch_bounds__(64 * W) void k_pcg_a(fem_pattern_t pat, const T* __
                                                            const PcgScalars* sc, PcgHead head,
                                                            double* __restrict__ partA, int remap) {
   constexpr int U = SliceCfg<T>::U, NT = 64 * W;
+  // small matrices (W >= 8): a wave's first slots (all of them for rows of up to 32 blocks at W = 16
+  // or scalar blocks) are loaded, and their vector entries gathered, before the head's reduction is
+  // waited for; as many as leave two workgroups on a CU
+  constexpr int NS = FUSED && W >= 8 && V <= 3 ? (W == 8 && V == 1 ? 4 : 2) : 0, VV = V * V;
   __shared__ double smem[2 * (NT / 64)];
   __shared__ double red[W][kSlice][V];
-  T beta = T(0);
-  if (FUSED) {
-    bool done;
-    beta = T(pcg_head<NT>(head, smem, &done));
-    if (done) return;
-  } else if (sc->done) {
+  PcgRaw<NT> raw;
+  if constexpr (FUSED)
+    raw = pcg_raw<NT>(head);
+  else if (sc->done)
     return;
-  }
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t s = remap ? xcd_logical_block(blockIdx.x, gridDim.x) : blockIdx.x;
   const int64_t row = pat.sell_row[s * kSlice + lane];
   const bool real = row >= 0;
+  const int base = NS ? pat.slice_ptr[s] : 0, L = NS ? (pat.slice_ptr[s + 1] - base) >> 6 : 0;
+  int32_t sc_[NS ? NS : 1];
+  T sv[NS ? NS : 1][VV], sp[NS ? NS : 1][V], sz[NS ? NS : 1][V], rp[V], rz[V];
+  if constexpr (NS > 0) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int k = w + W * i;
+      sc_[i] = k < L ? pat.sell_col[base + lane + k * kSlice] : 0;
+#pragma unroll
+      for (int v = 0; v < VV; ++v)
+        sv[i][v] = k < L ? vals[((size_t)base + (size_t)k * kSlice) * VV + (size_t)v * kSlice + lane] : T(0);
+    }
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+#pragma unroll
+      for (int j = 0; j < V; ++j) {
+        sp[i][j] = p[(int64_t)sc_[i] * V + j];
+        sz[i][j] = z[(int64_t)sc_[i] * V + j];
+      }
+#pragma unroll
+    for (int j = 0; j < V; ++j) {
+      rp[j] = p[(real ? row : 0) * V + j];
+      rz[j] = z[(real ? row : 0) * V + j];
+    }
+  }
+  T beta = T(0);
+  if constexpr (FUSED) {
+    bool done;
+    beta = T(pcg_head<NT>(head, raw, smem, &done));
+    if (done) return;
+  }
   auto xat = [&](int64_t c, T (&xc)[V]) {
 #pragma unroll
     for (int j = 0; j < V; ++j) xc[j] = FUSED ? fma(beta, p[c * V + j], z[c * V + j]) : p[c * V + j];
   };
   T pr[V];
-  xat(real ? row : 0, pr);
+  if constexpr (NS > 0) {
+#pragma unroll
+    for (int j = 0; j < V; ++j) pr[j] = fma(beta, rp[j], rz[j]);
+  } else {
+    xat(real ? row : 0, pr);
+  }
   double xr[V], acc[V];
 #pragma unroll
   for (int j = 0; j < V; ++j) xr[j] = double(pr[j]);
-  sell_slice_partial<V, DIFF, W, U, T>(pat, vals, s, w, lane, row, xat, xr, acc);
+  if constexpr (NS > 0) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] = 0.0;
+    auto add = [&](int64_t c, const T (&xt)[V], const T (&a)[VV]) {
+      double xc[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) xc[j] = (DIFF && c != row) ? double(xt[j]) - xr[j] : double(xt[j]);
+#pragma unroll
+      for (int i = 0; i < V; ++i)
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[i] = fma(double(a[i * V + j]), xc[j], acc[i]);
+    };
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      if (w + W * i >= L) continue;
+      T xt[V];
+#pragma unroll
+      for (int j = 0; j < V; ++j) xt[j] = fma(beta, sp[i][j], sz[i][j]);
+      add(sc_[i], xt, sv[i]);
+    }
+    for (int k = w + W * NS; k < L; k += W) {
+      const int64_t c = pat.sell_col[base + lane + k * kSlice];
+      T xt[V], a[VV];
+      xat(c, xt);
+#pragma unroll
+      for (int v = 0; v < VV; ++v) a[v] = vals[((size_t)base + (size_t)k * kSlice) * VV + (size_t)v * kSlice + lane];
+      add(c, xt, a);
+    }
+  } else {
+    sell_slice_partial<V, DIFF, W, U, T>(pat, vals, s, w, lane, row, xat, xr, acc);
+  }
   if (FUSED && w == 0 && real) {
 #pragma unroll
     for (int j = 0; j < V; ++j) pn[row * V + j] = pr[j];
@@ -139,7 +206,7 @@ __global__ __launch_bounds__(1024) void k_pcg_ra(const double* __restrict__ part
 // RB: rz, rr and beta of the iteration that ended, its stop test (head.next may be head.cur).
 __global__ __launch_bounds__(1024) void k_pcg_rb(PcgHead head) {
   __shared__ double smem[32];
-  const PcgState s = pcg_state<1024>(head, smem);
+  const PcgState s = pcg_state<1024>(head, pcg_raw<1024>(head), smem);
   __syncthreads();
   if (threadIdx.x == 0) pcg_store(head.next, s, 1);
 }
@@ -151,19 +218,44 @@ __global__ __launch_bounds__(256) void k_pcg_b(int64_t n, TX* __restrict__ x, T*
                                                const PcgScalars* sc, const double* __restrict__ partA, int nA,
                                                double* __restrict__ partB) {
   __shared__ double smem[8];
+  // the first entry's loads and the partials' are in flight together, and with the state's
+  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  TX xi = TX(0);
+  T pi = T(0), ri = T(0), qi = T(0), di = T(0);
+  auto load = [&]() {
+    if (i < n) {
+      xi = x[i];
+      pi = p[i];
+      ri = r[i];
+      qi = q[i];
+      di = dinv[i];
+    }
+  };
+  double pa[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    if ((int)threadIdx.x + 256 * k < nA) pa[k] = partA[threadIdx.x + 256 * k];
+  load();
   if (sc->done) return;
   // nA > 0: every block sums the <p, q> partials itself
-  const double alpha_d = nA > 0 ? sc->rz / block_reduce_partials(partA, nA, smem) : sc->alpha;
+  double alpha_d = sc->alpha;
+  if (nA > 0) {
+    double s = (pa[0] + pa[1]) + (pa[2] + pa[3]);
+    for (int k = threadIdx.x + 1024; k < nA; k += 256) s += partA[k];
+    alpha_d = sc->rz / block_sum_256(s, smem);
+  }
   const T alpha = T(alpha_d);
   T rz = T(0), rr = T(0);
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    x[i] += TX(alpha_d) * TX(p[i]);
-    const T ri = r[i] - alpha * q[i];
-    const T zi = dinv[i] * ri;
-    r[i] = ri;
+  while (i < n) {
+    x[i] = xi + TX(alpha_d) * TX(pi);
+    const T rn = ri - alpha * qi;
+    const T zi = di * rn;
+    r[i] = rn;
     z[i] = zi;
-    rz += ri * zi;
-    rr += ri * ri;
+    rz += rn * zi;
+    rr += rn * rn;
+    i += (int64_t)gridDim.x * blockDim.x;
+    load();
   }
   const double s1 = block_sum_256(double(rz), smem);
   const double s2 = block_sum_256(double(rr), smem + 4);
