@@ -466,8 +466,18 @@ __device__ inline void select_top(const TopKey (&key)[PER], const bool (&real)[P
     for (int i = t; i < 256; i += NT) s_hist[i] = 0;
     __syncthreads();
 #pragma unroll
-    for (int s = 0; s < PER; ++s)
-      if (real[s] && (key[s] & mask) == prefix) atomicAdd(&s_hist[(int)((key[s] >> shift) & 255u)], 1);
+    for (int s = 0; s < PER; ++s) {
+      const bool in = real[s] && (key[s] & mask) == prefix;
+      const int digit = (int)((key[s] >> shift) & 255u);
+      // a wave of one digit (equal gradients) counts once: 64 adds to one address take their turns
+      const unsigned long long who = __ballot(in);
+      const int lead = who ? __ffsll(who) - 1 : 0;
+      if (__ballot(in && digit == __shfl(digit, lead, 64)) == who) {
+        if (who && lane == lead) atomicAdd(&s_hist[digit], (int)__popcll(who));
+      } else if (in) {
+        atomicAdd(&s_hist[digit], 1);
+      }
+    }
     __syncthreads();
     if (w == 0) {
       // lane l holds the digits 255 - 4 l .. 252 - 4 l; the digit where the count from the top
