@@ -21,7 +21,7 @@
 //          accumulation (about 16 significant bits per product); Ke in FP32.
 // One workgroup of 4 waves per cell, persistent over cells.  46 KB of LDS, so three of them share
 // a CU and one's Jacobians run beside another's products and stores; with all of Z in LDS (91 KB)
-// there was one, which waited for each phase in turn: 24^3 cells 940 -> 420 us (726 MB written).
+// there was one, which waited for each phase in turn: 24^3 cells 940 -> 350 us (726 MB written, 115 us).
 #include "element.hpp"
 #include "tangent_mfma.hpp"
 
@@ -34,6 +34,9 @@ namespace {
 
 constexpr int kN = 27, kQ = 27, kM = 81;
 constexpr int kTN = 5, kTiles = 6;  // nodes per tile; 27 nodes padded to 6 tiles
+constexpr int kZS = 3 * kTN + 2;    // row stride of a staged tile (its entries number below 256)
+constexpr int kEntries = (kTN * kTN * 9 + 63) / 64;
+constexpr uint32_t kDiag = 1u << 24;
 constexpr int kGrid = 768;          // persistent workgroups: three per CU
 
 typedef double double4_t __attribute__((ext_vector_type(4)));
@@ -63,12 +66,30 @@ __global__ __launch_bounds__(256) void k_tangent_hex27_mfma(fem_mesh_t mesh, fem
                                                             TO* __restrict__ Ke) {
   using TZ = typename std::conditional<kBf16, float, double>::type;
   __shared__ Hex27Lds S;
-  __shared__ TZ s_z[4][3 * kTN][3 * kTN + 2];
+  __shared__ TZ s_z[4][3 * kTN][kZS];
   const int t = threadIdx.x;
   const int wave = t >> 6, lane = t & 63;
   load_tables(mesh, S.dN, S.w);
   const double c0 = mat.c[0], c1 = mat.c[1];
-  TZ(*z)[3 * kTN + 2] = s_z[wave];
+  TZ(*z)[kZS] = s_z[wave];
+  // The lane's values of a tile, the same in every tile: where Z[(a,i),(b,k)], Z[(a,k),(b,i)] and the
+  // block's trace stand, whether i = k, and (a, b) against the last tile's edge; off: the value's
+  // place in Ke.  ent of the tile's blocks, entT of their transposes (45 values of a block row are
+  // consecutive in either).  Taken apart again in every tile, the indices cost more than the MFMA.
+  uint32_t ent[kEntries], entT[kEntries];
+  int off[kEntries];
+#pragma unroll
+  for (int t = 0; t < kEntries; ++t) {
+    const int e = lane + 64 * t, hi = e / (9 * kTN), lo = (e / 9) % kTN, i = (e % 9) / 3, k = e % 3;
+    auto pack = [&](int a, int b, int i, int k) {
+      return (uint32_t)((3 * a + i) * kZS + 3 * b + k) | (uint32_t)((3 * a + k) * kZS + 3 * b + i) << 8 |
+             (uint32_t)(3 * a * kZS + 3 * b) << 16 | (i == k ? kDiag : 0u) | (uint32_t)a << 25 | (uint32_t)b << 28;
+    };
+    const bool in = e < kTN * kTN * 9;
+    ent[t] = in ? pack(hi, lo, i, k) : 7u << 25;    // a = 7: outside every tile
+    entT[t] = in ? pack(lo, hi, k, i) : 7u << 25;
+    off[t] = (hi * kN + lo) * 9 + e % 9;
+  }
   const int l = lane & 15;  // row of A, column of B and of the result; 15 is padding
   for (int64_t c = blockIdx.x; c < mesh.num_cells; c += gridDim.x) {
     __syncthreads();  // the previous cell's gradients are no longer read
@@ -134,21 +155,24 @@ __global__ __launch_bounds__(256) void k_tangent_hex27_mfma(fem_mesh_t mesh, fem
       __builtin_amdgcn_wave_barrier();
       const int a0 = tm * kTN, b0 = tn * kTN;
       const int na = min(kTN, kN - a0), nb = min(kTN, kN - b0);
-      // value (i, k) of block (a, b) of the tile
-      auto value = [&](int a, int b, int i, int k) {
-        double v = c0 * double(z[3 * a + i][3 * b + k]) + c1 * double(z[3 * a + k][3 * b + i]);
-        if (i == k)
-          v += c1 * (double(z[3 * a][3 * b]) + double(z[3 * a + 1][3 * b + 1]) + double(z[3 * a + 2][3 * b + 2]));
-        return TO(v);
+      const TZ* zf = &z[0][0];
+      auto emit = [&](uint32_t e, TO* o) {
+        double v = c0 * double(zf[e & 255u]) + c1 * double(zf[(e >> 8) & 255u]);
+        const TZ* d = zf + ((e >> 16) & 255u);
+        const double tr = double(d[0]) + double(d[kZS + 1]) + double(d[2 * kZS + 2]);
+        if (e & kDiag) v += c1 * tr;
+        *o = TO(v);
       };
-      for (int e = lane; e < kTN * kTN * 9; e += 64) {
-        const int a = e / (9 * kTN), b = (e / 9) % kTN, ik = e % 9;
-        if (a < na && b < nb) out[((a0 + a) * kN + b0 + b) * 9 + ik] = value(a, b, ik / 3, ik % 3);
+#pragma unroll
+      for (int t = 0; t < kEntries; ++t) {
+        const int a = (ent[t] >> 25) & 7, b = (int)(ent[t] >> 28) & 7;
+        if (a < na && b < nb) emit(ent[t], out + (a0 * kN + b0) * 9 + off[t]);
       }
       if (tm != tn)
-        for (int e = lane; e < kTN * kTN * 9; e += 64) {
-          const int b = e / (9 * kTN), a = (e / 9) % kTN, ki = e % 9;
-          if (a < na && b < nb) out[((b0 + b) * kN + a0 + a) * 9 + ki] = value(a, b, ki % 3, ki / 3);
+#pragma unroll
+        for (int t = 0; t < kEntries; ++t) {
+          const int a = (entT[t] >> 25) & 7, b = (int)(entT[t] >> 28) & 7;
+          if (a < na && b < nb) emit(entT[t], out + (b0 * kN + a0) * 9 + off[t]);
         }
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
       __builtin_amdgcn_wave_barrier();
