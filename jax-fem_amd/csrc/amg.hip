@@ -801,73 +801,60 @@ __global__ __launch_bounds__(NT) void k_spgemm_row_big(BView X, BView Y, int32_t
   }
 }
 
-// n consecutive entries in their storage type, with 16-byte loads where n and
-// the entry size allow (p is then 16-byte aligned: blocks of 36 FP32 entries)
+// n consecutive entries in their storage type, 16 bytes at a time: a lane's block begins at any
+// multiple of the entry size, which global accesses of four dwords allow.  Lanes read blocks of
+// their own, so the number of accesses is what such a kernel costs (a 3x3 FP32 block: 3 for 9,
+// a 3x6 one 5 for 9: level-0 prolongator smoothing of the 1.6M-dof cantilever 800 -> 630 us; the
+// products A P and R (A P), bound by the blocks' bytes, stay at 1.3 ms each).
+template <typename T, int k>
+struct Wide {
+  typedef T type __attribute__((ext_vector_type(k), aligned(alignof(T))));
+};
 template <int n, typename T>
 __device__ inline void load_raw(const T* __restrict__ p, T (&a)[n]) {
-  if constexpr (sizeof(T) == 4 && n % 4 == 0) {
-    const float4* p4 = reinterpret_cast<const float4*>(p);
+  constexpr int W = 16 / (int)sizeof(T);
+  using V = typename Wide<T, W>::type;
 #pragma unroll
-    for (int k = 0; k < n / 4; ++k) {
-      const float4 v = p4[k];
-      a[4 * k] = v.x;
-      a[4 * k + 1] = v.y;
-      a[4 * k + 2] = v.z;
-      a[4 * k + 3] = v.w;
-    }
-  } else if constexpr (sizeof(T) == 8 && n % 2 == 0) {
-    const double2* p2 = reinterpret_cast<const double2*>(p);
+  for (int k = 0; k + W <= n; k += W) {
+    const V v = *reinterpret_cast<const V*>(p + k);
 #pragma unroll
-    for (int k = 0; k < n / 2; ++k) {
-      const double2 v = p2[k];
-      a[2 * k] = v.x;
-      a[2 * k + 1] = v.y;
-    }
-  } else {
-#pragma unroll
-    for (int k = 0; k < n; ++k) a[k] = p[k];
+    for (int j = 0; j < W; ++j) a[k + j] = v[j];
+  }
+  constexpr int r = n / W * W;
+  if constexpr (W == 4 && n - r >= 2) {
+    using H = typename Wide<T, 2>::type;
+    const H v = *reinterpret_cast<const H*>(p + r);
+    a[r] = v[0];
+    a[r + 1] = v[1];
+    if constexpr (n - r == 3) a[r + 2] = p[r + 2];
+  } else if constexpr (n - r == 1) {
+    a[r] = p[r];
   }
 }
+template <int n, typename T>
+__device__ inline void store_raw(const T (&a)[n], T* __restrict__ p) {
+  constexpr int W = 16 / (int)sizeof(T);
+  using V = typename Wide<T, W>::type;
+#pragma unroll
+  for (int k = 0; k + W <= n; k += W) {
+    V v;
+#pragma unroll
+    for (int j = 0; j < W; ++j) v[j] = a[k + j];
+    *reinterpret_cast<V*>(p + k) = v;
+  }
+#pragma unroll
+  for (int k = n / W * W; k < n; ++k) p[k] = a[k];
+}
 
-// Load an R x C block (FP64 or FP32 storage) into FP64 registers.  Blocks whose
-// size is a multiple of 16 bytes (given 256-byte aligned bases: FP64 blocks but
-// 3x3 and 1x1, FP32 6x6 blocks) use 16-byte loads; FP32 blocks of an even
-// count (3x6, 6x3) 8-byte loads.
+// Load an R x C block (FP64 or FP32 storage) into FP64 registers.
 template <int R, int C, typename T = double>
 __device__ inline void load_block(const T* __restrict__ p, double (&a)[R][C]) {
-  constexpr int n = R * C;
-  if constexpr (sizeof(T) == 8 && n % 2 == 0 && n > 9) {
-    const double2* p2 = reinterpret_cast<const double2*>(p);
+  T raw[R * C];
+  load_raw<R * C, T>(p, raw);
 #pragma unroll
-    for (int k = 0; k < n / 2; ++k) {
-      const double2 v = p2[k];
-      a[(2 * k) / C][(2 * k) % C] = v.x;
-      a[(2 * k + 1) / C][(2 * k + 1) % C] = v.y;
-    }
-  } else if constexpr (sizeof(T) == 4 && n % 4 == 0 && (n * 4) % 16 == 0 && n > 9) {
-    const float4* p4 = reinterpret_cast<const float4*>(p);
+  for (int i = 0; i < R; ++i)
 #pragma unroll
-    for (int k = 0; k < n / 4; ++k) {
-      const float4 v = p4[k];
-      a[(4 * k) / C][(4 * k) % C] = v.x;
-      a[(4 * k + 1) / C][(4 * k + 1) % C] = v.y;
-      a[(4 * k + 2) / C][(4 * k + 2) % C] = v.z;
-      a[(4 * k + 3) / C][(4 * k + 3) % C] = v.w;
-    }
-  } else if constexpr (sizeof(T) == 4 && n % 2 == 0 && n > 9) {
-    const float2* p2 = reinterpret_cast<const float2*>(p);
-#pragma unroll
-    for (int k = 0; k < n / 2; ++k) {
-      const float2 v = p2[k];
-      a[(2 * k) / C][(2 * k) % C] = v.x;
-      a[(2 * k + 1) / C][(2 * k + 1) % C] = v.y;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < R; ++i)
-#pragma unroll
-      for (int j = 0; j < C; ++j) a[i][j] = double(p[i * C + j]);
-  }
+    for (int j = 0; j < C; ++j) a[i][j] = double(raw[i * C + j]);
 }
 
 // C = X Y by its plan: one thread per output block, products in plan order.
@@ -932,11 +919,12 @@ __global__ __launch_bounds__(256) void k_spgemm_numeric(int64_t nb, const int32_
             for (int m = 0; m < XC; ++m) acc[i][j] = fma(xa[i][m], ya[m][j], acc[i][j]);
       }
     }
-    T* c = cv + (size_t)b * XR * YC;
+    T c[XR * YC];
 #pragma unroll
     for (int i = 0; i < XR; ++i)
 #pragma unroll
       for (int j = 0; j < YC; ++j) c[i * YC + j] = T(acc[i][j]);
+    store_raw<XR * YC, T>(c, cv + (size_t)b * XR * YC);
   }
 }
 
@@ -1076,7 +1064,7 @@ __global__ __launch_bounds__(256) void k_smooth_numeric(int64_t nb, int64_t rows
       }
     }
     const bool own = cci[b] == agg[i];
-    T* out = pv + (size_t)b * BS * NS;
+    T out[BS * NS];
 #pragma unroll
     for (int r = 0; r < BS; ++r) {
       const double sc = -omega * dinv[i * BS + r];
@@ -1087,6 +1075,7 @@ __global__ __launch_bounds__(256) void k_smooth_numeric(int64_t nb, int64_t rows
         out[r * NS + j] = T(v);
       }
     }
+    store_raw<BS * NS, T>(out, pv + (size_t)b * BS * NS);
   }
 }
 
@@ -2020,17 +2009,24 @@ int level_apply(const fem_amg_t& amg, int l, int mode, const ApplyArgsT<TX, TY>&
 // Pre-smoothing (Chebyshev from a zero iterate), residual and restriction on
 // level l, vectors stored as TX.  On return *xo is the smoothed iterate and
 // *oo the other iterate buffer.  ev: see vcycle_impl.
-// The first step of a level below another is done by the restriction to it (AP_FIRST, into x_next
-// and dd_next).  end (level 0, may be NULL): the CG iteration to end first.
+// The restriction to a level of few block rows does that level's first step as well (a launch of
+// 3.7 us less on the HEX27 and Neo-Hookean cubes).  To a large one it does not: D^-1, by then out of
+// the caches, is waited for by every wave before its row (1.6M-dof cantilever: 46.2 us and 4.7 for a
+// first step of its own, 56.8 in one).
+bool restriction_first(const fem_amg_t& amg, int l) {
+  return l + 1 < amg.num_levels && amg.levels[l].R.rows < kRowKernelRows;
+}
+
+// x_next, dd_next: of the next level, for restriction_first.  end (level 0, may be NULL): the CG iteration to end first.
 template <typename T, typename TX>
 int level_down(const fem_amg_t& amg, int l, int64_t n, const double* rhs, double* rhs_next, TX* x, TX* other,
                TX* dd, TX* res, TX* x_next, TX* dd_next, TX** xo, TX** oo, hipStream_t s, hipEvent_t* ev,
                const int32_t* done, const CgEnd* end) {
   const fem_amg_level_t& L = amg.levels[l];
   const Cheb cb(L.lmax);
-  if (l == 0) {
+  if (l == 0 || !restriction_first(amg, l - 1)) {
     const dim3 grid(grid_for(n, 256)), nt(256);
-    if (end)
+    if (l == 0 && end)
       hipLaunchKernelGGL((k_cheb_first<TX, true>), grid, nt, 0, s, n, rhs, L.dinv, 1.0 / cb.theta, dd, x, done, *end);
     else
       hipLaunchKernelGGL((k_cheb_first<TX, false>), grid, nt, 0, s, n, rhs, L.dinv, 1.0 / cb.theta, dd, x, done,
@@ -2052,7 +2048,7 @@ int level_down(const fem_amg_t& amg, int l, int64_t n, const double* rhs, double
   ApplyArgsT<TX, TX> ar{x, res, rhs, nullptr, nullptr, 0.0, 0.0, nullptr, done};
   if (int rc = level_apply<T>(amg, l, AP_RESID, ar, s)) return rc;
   ApplyArgsT<TX, double> arr{res, rhs_next, nullptr, nullptr, nullptr, 0.0, 0.0, nullptr, done};
-  if (l + 1 < amg.num_levels) {
+  if (restriction_first(amg, l)) {
     arr.dinv = amg.levels[l + 1].dinv;
     arr.d = dd_next;
     arr.c2 = 1.0 / Cheb(amg.levels[l + 1].lmax).theta;
