@@ -359,9 +359,10 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
   __syncthreads();
   AsmWave<MAT, RES>& L = s_wave[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63, hi8 = lane >> 3, j = lane & 7;
-  const int64_t gid = blockIdx.x * (int64_t)(kAsmThreads / 64) + (threadIdx.x >> 6);
-  const int64_t s = gid / kGroups;
-  const int gr = (int)(gid % kGroups), rl = gr * kGroupRows + hi8;  // the lane's row in the slice
+  // (uniform in the wave, and known to be: what follows from it stays in scalar registers)
+  const int gid = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kAsmThreads / 64) + (threadIdx.x >> 6)));
+  const int s = gid / kGroups;
+  const int gr = gid % kGroups, rl = gr * kGroupRows + hi8;  // the lane's row in the slice
 
   const int sbase = pat.slice_ptr[s], nslots = (pat.slice_ptr[s + 1] - sbase) >> 6;
   const int row = pat.sell_row[s * kSlice + rl];
