@@ -112,13 +112,31 @@ def cheb_bytes(dev, elem_bytes, vec=3):
     return dev.nnzb * (vec * vec * elem_bytes + 4) + dev.n * 8 * (5 + 6 + 6) / 3
 
 
+# FP64 operations of a matrix-free HEX8 elastic product per cell, from the instruction counters of
+# k_patch_hex8<MatModulus> (two lanes of 372 multiply-adds, 222 additions and 136 products)
+PATCH_FLOP_PER_CELL = 2 * (2 * 372 + 222 + 136)
+PEAK_FP64_TFLOPS = 78.6
+
+
+def matrix_free(dev, storage):
+    """True where the solver runs the products of this problem on the elements, not on the matrix."""
+    return bool(dev.patch_law) and dev.dm.C >= dev.patch_min_cells(storage)
+
+
+def patch_bytes(dev, vector_bytes, reads, writes):
+    """Algorithmic bytes of one matrix-free product: connectivity, coordinates, the per-quad modulus
+    field and the Dirichlet mask read once, and `reads` + `writes` vectors (the cells' partial sums,
+    which pass from the first kernel to the second, are not counted)."""
+    dm = dev.dm
+    return dm.C * dm.N * 4 + dm.Nn * 24 + dm.C * dm.Q * 8 + dev.n + dev.n * vector_bytes * (reads + writes)
+
+
 def assembly_bytes(dev):
     """Algorithmic bytes of one FP64 single-pass tangent assembly: the SELL values (padding not
     counted) and the inverse diagonal written once; connectivity, coordinates, the per-quad
-    modulus field and the plan's index data (slice-local contribution ids, slot bounds) read once."""
+    modulus field and the plan's words (eight per cell and node) read once."""
     dm = dev.dm
-    return (dev.nnzb * 72 + dev.n * 8 + dm.C * dm.N * 4 + dm.Nn * 24 + dm.C * dm.Q * 8 + dm.C * dm.N * dm.N * 4
-            + (dev.nnzb + 1) * 4)
+    return dev.nnzb * 72 + dev.n * 8 + dm.C * dm.N * 4 + dm.Nn * 24 + dm.C * dm.Q * 8 + dm.C * dm.N * dm.N * 4
 
 
 def sell_bytes(dev, elem_bytes, vec=3):
@@ -259,12 +277,43 @@ def run(args):
     head = res['amg_mixed']
     amg_traffic = measured_traffic(args.cells, AMG_TRAFFIC_PROFILE)
     traffic = measured_traffic(args.cells)
-    cb = cheb_bytes(dev, 4)
-    achieved = cb / (head['spmv_ms'] * 1e-3) / 1e9 if head['spmv_ms'] else None
-    spmv_bytes = sell_bytes(dev, 4)
-    pcg_achieved = spmv_bytes / (res['mixed']['spmv_ms'] * 1e-3) / 1e9 if res['mixed']['spmv_ms'] else None
-    fp64_bytes = sell_bytes(dev, 8)
-    fp64_achieved = fp64_bytes / (res['fp64']['spmv_ms'] * 1e-3) / 1e9 if res['fp64']['spmv_ms'] else None
+    rate = lambda nbytes, ms: nbytes / (ms * 1e-3) / 1e9 if ms else None
+    if matrix_free(dev, _lib.FEM_F64):
+        cb = patch_bytes(dev, 8, (4 + 5 + 5) / 3, 2)   # x, rhs, D^-1, (d); d and the new x
+        flop = PATCH_FLOP_PER_CELL * dev.dm.C
+        tflops = flop / (head['spmv_ms'] * 1e-3) / 1e12 if head['spmv_ms'] else None
+        roofline = {"bound": "fp64 vector arithmetic (cells' kernel), hbm (gather)",
+                    "kernel": "k_patch_hex8<MatModulus> + k_patch_gather<CHEB> (level-0 Chebyshev steps of the "
+                              "V-cycle, the mean of three per cycle: matrix-free HEX8 product, node sums with the "
+                              "fused D^-1 residual and update)",
+                    "achieved": tflops, "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
+                    "frac": tflops / PEAK_FP64_TFLOPS if tflops else None, "traffic": None, "traffic_source": None,
+                    "algorithmic_flop": flop, "algorithmic_bytes": cb, "achieved_GBs": rate(cb, head['spmv_ms']),
+                    "avg_launch_ms": head['spmv_ms']}
+    else:
+        cb = cheb_bytes(dev, 4)
+        achieved = rate(cb, head['spmv_ms'])
+        roofline = {"bound": "hbm",
+                    "kernel": "k_sell_apply<3,CHEB,float,true> (level-0 Chebyshev steps of the V-cycle, the "
+                              "mean of its three launches per cycle: SELL-64 3x3-block product on FP32 "
+                              "difference-form storage with FP64 vectors and arithmetic, fused D^-1 "
+                              "residual and update)",
+                    "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
+                    "frac": achieved / PEAK_HBM_GBS if achieved else None,
+                    "traffic": amg_traffic.get('k_sell_apply_cheb_f32'),
+                    "traffic_source": os.path.relpath(AMG_TRAFFIC_PROFILE, ROOT) if amg_traffic else None,
+                    "algorithmic_bytes": cb, "avg_launch_ms": head['spmv_ms']}
+
+    def product(path, storage, kernel, key):
+        """The Jacobi path's product q = A p: matrix-free (z, p read; p, q written) or the SELL SpMV."""
+        es = 4 if storage == _lib.FEM_F32 else 8
+        mf = matrix_free(dev, storage)
+        nbytes = patch_bytes(dev, es, 2, 2) if mf else sell_bytes(dev, es)
+        got = rate(nbytes, res[path]['spmv_ms'])
+        return {"kernel": "k_patch_hex8<MatModulus> + k_patch_gather_cg (matrix-free q = A p, p = z + beta p)" if mf
+                else kernel, "achieved_GBs": got, "frac": got / PEAK_HBM_GBS if got else None,
+                "avg_launch_ms": res[path]['spmv_ms'], "algorithmic_bytes": nbytes,
+                "traffic": None if mf else traffic.get(key)}
     out = {
         "metric": METRIC, "value": head['s_per_newton_step'], "unit": "s", "n_gpus": 1,
         "steps": args.steps, "warmup": args.warmup, "ms_per_step": head['s_per_newton_step'] * 1e3,
@@ -288,22 +337,12 @@ def run(args):
         "assembly": dict(asm, kernel="k_assemble_hex8<MatElastic<true>, double> (single-pass HEX8 tangent into the "
                                      "FP64 SELL values, Jacobi diagonal) + k_bc_rows, timed together with HIP events",
                          bytes_formula="nnzb*72 (values) + n*8 (D^-1) + C*32 (cells) + Nn*24 (points) + C*Q*8 "
-                                       "(modulus field) + C*64*4 (slice-local contribution ids) + (nnzb+1)*4 "
-                                       "(slot bounds)"),
+                                       "(modulus field) + C*64*4 (pair words)"),
         "rel_err_vs_fp64_ref": {k: v['rel_err'] for k, v in res.items()},
         "adjoint_grad_rel_diff_vs_fp64": gerr,
         "s_per_adjoint_gradient": {"mixed": head['s_per_adjoint_gradient'],
                                    "fp64": res['fp64']['s_per_adjoint_gradient']},
-        "roofline": {"bound": "hbm",
-                     "kernel": "k_sell_apply<3,CHEB,float,true> (level-0 Chebyshev steps of the V-cycle, the "
-                               "mean of its three launches per cycle: SELL-64 3x3-block product on FP32 "
-                               "difference-form storage with FP64 vectors and arithmetic, fused D^-1 "
-                               "residual and update)",
-                     "achieved": achieved, "peak": PEAK_HBM_GBS, "unit": "GB/s",
-                     "frac": achieved / PEAK_HBM_GBS if achieved else None,
-                     "traffic": amg_traffic.get('k_sell_apply_cheb_f32'),
-                     "traffic_source": os.path.relpath(AMG_TRAFFIC_PROFILE, ROOT) if amg_traffic else None,
-                     "algorithmic_bytes": cb, "avg_launch_ms": head['spmv_ms']},
+        "roofline": roofline,
         "level0_fp16": {"kernel": "k_sell_apply<3,CHEB,_Float16,true> (level-0 Chebyshev step on FP16 D^-1 A)",
                         "s_per_newton_step": res['amg_mixed_l0fp16']['s_per_newton_step'],
                         "iterations": res['amg_mixed_l0fp16']['iterations'],
@@ -312,14 +351,9 @@ def run(args):
                         "traffic": measured_traffic(args.cells, F16_TRAFFIC_PROFILE).get('k_sell_apply_cheb_f16'),
                         "achieved_GBs": (cheb_bytes(dev, 2) / (res['amg_mixed_l0fp16']['spmv_ms'] * 1e-3) / 1e9
                                          if res['amg_mixed_l0fp16']['spmv_ms'] else None)},
-        "pcg_spmv": {"kernel": "k_pcg_a<3,true,float> (Jacobi-PCG SpMV q = Ap, FP32 storage)",
-                     "achieved_GBs": pcg_achieved, "frac": pcg_achieved / PEAK_HBM_GBS if pcg_achieved else None,
-                     "avg_launch_ms": res['mixed']['spmv_ms'], "algorithmic_bytes": spmv_bytes,
-                     "traffic": traffic.get('k_pcg_a_f32')},
-        "fp64_spmv": {"kernel": "k_pcg_a<3,false,double>", "achieved_GBs": fp64_achieved,
-                      "frac": fp64_achieved / PEAK_HBM_GBS if fp64_achieved else None,
-                      "avg_launch_ms": res['fp64']['spmv_ms'], "algorithmic_bytes": fp64_bytes,
-                      "traffic": traffic.get('k_pcg_a_f64')},
+        "pcg_spmv": product('mixed', _lib.FEM_F32, "k_pcg_a<3,true,float> (Jacobi-PCG SpMV q = Ap, FP32 storage)",
+                            'k_pcg_a_f32'),
+        "fp64_spmv": product('fp64', _lib.FEM_F64, "k_pcg_a<3,false,double>", 'k_pcg_a_f64'),
         "detail": res,
     }
     if args.cpu_baseline:
@@ -760,7 +794,9 @@ def workload_hex27(args):
     res['mixed']['grad_rel_diff_vs_fp64'] = _rel(grads['mixed'], grads['fp64'])
     # compliance self-adjointness: dC/dE_e = -u_e^T K_e(1) u_e = -(energy of cell e) / E_e * 2 ... checked by sign
     assert bool((grads['fp64'] < 0).all()), "compliance gradient w.r.t. E must be negative"
-    spmv_b = {nm: sell_bytes(dev, es) for nm, es in (('mixed', 4), ('fp64', 8))}
+    from jax_fem_amd import _lib
+    spmv_b = {nm: sell_bytes(dev, es) for nm, es, st in (('mixed', 4, _lib.FEM_F32), ('fp64', 8, _lib.FEM_F64))
+              if not matrix_free(dev, st)}
     cpu = None
     if args.cpu_baseline:
         from oracle import fem as OF
