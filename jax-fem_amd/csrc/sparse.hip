@@ -77,7 +77,7 @@ template <int V, bool DIFF, typename TS, typename T>
 __global__ __launch_bounds__(64 * kGatherWaves) void k_gather_matrix(fem_pattern_t pat, const TS* __restrict__ Ke,
                                                                      T* __restrict__ vals, T* __restrict__ dinv) {
   constexpr int VV = V * V;
-  __shared__ TS s_sum[DIFF ? kGatherWaves : 1][DIFF ? VV : 1][DIFF ? kSlice : 1];
+  __shared__ double s_sum[DIFF ? kGatherWaves : 1][DIFF ? VV : 1][DIFF ? kSlice : 1];
   const int64_t s = blockIdx.x;
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int base = pat.slice_ptr[s];
@@ -88,9 +88,10 @@ __global__ __launch_bounds__(64 * kGatherWaves) void k_gather_matrix(fem_pattern
   const int len = real ? pat.row_ptr[row + 1] - rb : 0;
   const int ds = real ? pat.diag_slot[row] : -1;
   T* vp = vals + (size_t)base * VV + lane;
-  TS rsum[VV];
+  // (FP64 whatever the tangents' type: rounded row sums let CG stagnate, 64x32x32 cantilever)
+  double rsum[VV];
 #pragma unroll
-  for (int v = 0; v < VV; ++v) rsum[v] = TS(0);
+  for (int v = 0; v < VV; ++v) rsum[v] = 0.;
   ListWindow<4> cptr(pat.contrib_ptr, pat.nnzb + 1);
   ListWindow<8> cidx(pat.contrib_idx, (int64_t)pat.num_cells * pat.nodes_per_cell * pat.nodes_per_cell);
   const int K = (L + kGatherWaves - 1) / kGatherWaves, k0 = w * K, k1 = min(L, k0 + K);
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(64 * kGatherWaves) void k_gather_matrix(fem_pattern
     __syncthreads();
     if (ds >= 0)
       for (int v = w; v < VV; v += kGatherWaves) {
-        TS t = s_sum[0][v][lane];
+        double t = s_sum[0][v][lane];
 #pragma unroll
         for (int o = 1; o < kGatherWaves; ++o) t += s_sum[o][v][lane];
         vp[((size_t)ds * VV + v) * kSlice] = T(t);
@@ -144,14 +145,19 @@ __global__ __launch_bounds__(64 * kGatherWaves) void k_gather_matrix(fem_pattern
 // workgroup's eight rows are stored together (64-byte segments).  Sums run over the cells in
 // ascending order, as above.  Rows of more than kRowSlots slots are done in windows and rows of
 // more than kRowPairs pairs slot by slot, into the same LDS.
-// 24^3 cells: 610 -> 365 us (1.29 GB, 250 us at the copy rate); with two rows to a wave 525: what is
-// left is the chain row -> lists -> runs, which 16 waves on a CU (the LDS's limit) do not cover.
+// The adds are LDS atomics in FP64 (one instruction; loads, adds and stores 416 us instead of 405 in
+// the same run) and plain ones in FP32, whose atomics are the slower ones (777 us; plain 400), unless
+// a cell names a node twice.
+// 24^3 cells: 610 -> 365 us (1.29 GB, 250 us at the copy rate), from FP32 tangents 553 -> 400; with two
+// rows to a wave 525: what is left is the chain row -> lists -> runs, which 16 waves on a CU (the LDS's
+// limit) do not cover.
 constexpr int kRowSlots = 128, kRowPairs = 16, kRowWaves = 8, kRowsPerGroup = 8;
 
 template <int V, int N, bool DIFF, typename TS, typename T>
 __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pat, const TS* __restrict__ Ke,
                                                                 T* __restrict__ vals, T* __restrict__ dinv) {
   constexpr int VV = V * V, RUN = N * VV, PER = (RUN + 63) / 64, STRIDE = kRowSlots * VV + 1;
+  constexpr bool kPlainAdds = sizeof(TS) == 4;
   __shared__ TS s_acc[kRowsPerGroup][STRIDE];
   __shared__ uint8_t s_slot[kRowWaves][kRowPairs][N + 1];
   __shared__ uint8_t s_first[kRowWaves][kRowPairs * N + 64];
@@ -161,11 +167,11 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
   const int base = pat.slice_ptr[s], L = (pat.slice_ptr[s + 1] - base) >> 6;
   T* vp = vals + (size_t)base * VV + l0;
   constexpr int RPW = kRowsPerGroup / kRowWaves;
-  TS rsum[RPW][VV];
+  double rsum[RPW][VV];
 #pragma unroll
   for (int r = 0; r < RPW; ++r)
 #pragma unroll
-    for (int v = 0; v < VV; ++v) rsum[r][v] = TS(0);
+    for (int v = 0; v < VV; ++v) rsum[r][v] = 0.;
   for (int k0 = 0; k0 < L; k0 += kRowSlots) {
     const int kn = min(kRowSlots, L - k0);
 #pragma unroll
@@ -191,6 +197,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
         wave_fence();
         for (int k = lane; k < len; k += 64) s_first[w][pat.contrib_ptr[rb + k] - t0] = 1;
         wave_fence();
+        bool twice = false;
         int slots = 0;  // slots that begin before the 64 contributions at hand
         for (int i = lane; i - lane < n * N; i += 64) {
           const bool in = i < n * N;
@@ -202,8 +209,12 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
             const int b = e - __shfl(first, p, 64);
             if (in && b >= 0 && b < N) s_slot[w][p][b] = (uint8_t)slot;
           }
+          // (a slot's contributions are in ascending order: a pair's two blocks of it are neighbours)
+          if (kPlainAdds)
+            twice |= i + 1 < n * N && !s_first[w][i + 1] && pat.contrib_idx[t0 + i + 1] / N == e / N;
         }
         wave_fence();
+        const bool unique = kPlainAdds && !__any(twice);
         for (int p = 0; p < n; p += 4) {
           TS x[4][PER];
 #pragma unroll
@@ -215,6 +226,21 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             if (p + j >= n) break;
+            if (unique) {
+              int at[PER];
+              TS y[PER];
+#pragma unroll
+              for (int i = 0; i < PER; ++i) {
+                const int o = min(lane + 64 * i, RUN - 1);
+                at[i] = s_slot[w][p + j][o / VV] * VV + o % VV;
+                y[i] = acc[at[i]];
+              }
+#pragma unroll
+              for (int i = 0; i < PER; ++i)
+                if (lane + 64 * i < RUN) acc[at[i]] = y[i] + x[j][i];
+              wave_fence();
+              continue;
+            }
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
               const int o = lane + 64 * i;
@@ -264,7 +290,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
       const int ds = row >= 0 ? pat.diag_slot[row] : -1;
 #pragma unroll
       for (int v = 0; v < VV; ++v) {
-        const TS t = wave_sum(rsum[r][v]);
+        const double t = wave_sum(rsum[r][v]);
         if (ds >= 0 && lane == 0) vp[((size_t)ds * VV + v) * kSlice + rl] = T(t);
       }
     }
