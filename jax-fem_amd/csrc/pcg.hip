@@ -501,9 +501,20 @@ __global__ __launch_bounds__(256) void k_spmv_x(fem_pattern_t pat, const T* __re
 }
 
 constexpr int kVecGrid = 1024;  // blocks of the vector kernels (partials per reduction)
-// Largest matrix whose product forms its direction itself (us per iteration, with and without):
-// FP64 3 MB 13 / 18, 28 MB 15.9 / 19.5, 38 MB 21.9 / 22.1; FP32 39 MB 17.3 / 18.9, 59 MB 35 / 32.5.
-constexpr double kFuseBytes = 48e6;
+// Mean slots of a row from which eight waves share a slice whatever the size of the matrix (HEX27: 64;
+// HEX8: 27).  us per iteration with eight and with the usual waves: 32^3 HEX27 Poisson FP64 60 / 78, FP32
+// 58 / 59; 18^3 and 20^3 HEX27 J2 FP64 71 / 80 and 83 / 111, 20^3 FP32 53 / 61.
+constexpr int kLongRow = 40;
+
+// Largest matrix whose product forms its direction itself (us per iteration, with and without).
+// Scalar rows: FP64 37 MB 19.7 / 19.9, 59 MB 28 / 25.6; FP32 39 MB 25.0 / 26.1, 58 MB 33.0 / 32.7.  Blocks in
+// FP64: 72 MB 22.5 / 24.2, 139 MB 33.8 / 37.2, 237 MB 52.7 / 55.2 (HEX27 52 / 71), 325 MB 96 / 83; in FP32:
+// 45 MB 17.0 / 19.2, 73 MB 23.2 / 24.9, 125 MB 34.4 / 34.2, of long rows 125 MB 39 / 46, 171 MB 50 / 53.
+template <int V, typename T>
+inline double fuse_bytes(bool long_rows) {
+  if (V == 1 || V > 3) return 45e6;
+  return sizeof(T) == 8 ? 240e6 : long_rows ? 180e6 : 100e6;
+}
 
 struct EventPool {
   std::vector<hipEvent_t> e;
@@ -641,13 +652,17 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
   const int check = std::max(1, opt->check_every);
   // Small matrices leave most of the chip idle at one workgroup of W waves per slice: up to 256
   // slices (one per CU) 16 waves share a slice's slots, up to 768 eight (FP64 Poisson of 13,824
-  // cells 15.3 -> 12.0 us per iteration, of 32,768 cells 16.0 -> 14.9).
+  // cells 15.3 -> 12.0 us per iteration, of 32,768 cells 16.0 -> 14.9).  FP32 blocks leave room for two
+  // workgroups of eight waves on a CU: eight waves only up to 512 slices (562 slices: 25 us, with four
+  // 16.3).  FP64 blocks keep eight at any size (139 MB: 33.8 us, with two 37.7).
   // The direction update runs inside the product (which then gathers z and the old direction) where
   // the matrix stays in the caches or is not read; the new direction goes to a second buffer.  That is
   // y's, free between the true residuals: so a batch of status-free iterations has to be even.
   T* p2 = (T*)w.y;
   const double sell_bytes = double(pat->sell_blocks) * (V * V * sizeof(T) + 4);
-  const bool fused = check % 2 == 0 && (pop ? true : sell_bytes <= kFuseBytes);
+  const bool long_rows = pat->sell_blocks >= pat->num_slices * kSlice * kLongRow;
+  const bool fused = check % 2 == 0 && (pop ? true : sell_bytes <= fuse_bytes<V, T>(long_rows));
+  const bool eight = long_rows || (fused && (V == 1 ? gA <= 768 : gA <= 512 || (V <= 3 && sizeof(T) == 8)));
   // one workgroup for the whole batch: few scalar rows of, on average, at most kOneSlots slots
   const bool one = V == 1 && !pop && !opt->timing && pat->num_slices <= kOneSlices &&
                    pat->sell_blocks <= pat->num_slices * kSlice * kOneSlots;
@@ -681,21 +696,25 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
       } else if (pop) {
         ApplyArgsT<T, T> a{p, q, nullptr, nullptr, nullptr, 0.0, 0.0, w.partA, &sc->done};
         if (int rc = patch_apply<AP_PQ, T, T>(*pop, a, s, &gA)) return rc;
-      } else if (fused) {
-        auto product = [&](auto waves) {
-          constexpr int W = decltype(waves)::value;
-          hipLaunchKernelGGL((k_pcg_a<V, kDiff, T, true, W>), dim3(gA), dim3(64 * W), 0, s, *pat, vals, (const T*)pc,
-                             (const T*)z, pn, q, (const PcgScalars*)sc, head, w.partA, opt->xcd_remap);
-        };
-        if (gA <= 256)
-          product(std::integral_constant<int, 16>{});
-        else if (gA <= 768)
-          product(std::integral_constant<int, 8>{});
-        else
-          product(std::integral_constant<int, SliceCfg<T>::W>{});
       } else {
-        hipLaunchKernelGGL((k_pcg_a<V, kDiff, T, false>), dim3(gA), dim3(SliceCfg<T>::NT), 0, s, *pat, vals,
-                           (const T*)p, (const T*)z, p, q, (const PcgScalars*)sc, head, w.partA, opt->xcd_remap);
+        auto product = [&](auto fuse, auto waves) {
+          constexpr int W = decltype(waves)::value;
+          hipLaunchKernelGGL((k_pcg_a<V, kDiff, T, decltype(fuse)::value, W>), dim3(gA), dim3(64 * W), 0, s, *pat, vals,
+                             (const T*)pc, (const T*)z, pn, q, (const PcgScalars*)sc, head, w.partA, opt->xcd_remap);
+        };
+        using Few = std::integral_constant<int, 16>;
+        using Some = std::integral_constant<int, 8>;
+        using Many = std::integral_constant<int, SliceCfg<T>::W>;
+        if (fused && gA <= 256)
+          product(std::true_type{}, Few{});
+        else if (fused && eight)
+          product(std::true_type{}, Some{});
+        else if (fused)
+          product(std::true_type{}, Many{});
+        else if (eight)
+          product(std::false_type{}, Some{});
+        else
+          product(std::false_type{}, Many{});
       }
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 2], s));
       const int sumA = gA <= kSumParts ? gA : 0;
