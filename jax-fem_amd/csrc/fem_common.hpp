@@ -193,6 +193,12 @@ struct SliceCfg {
   static constexpr int NT = 64 * W;
 };
 
+// Mean slots of a row from which eight waves share a slice whatever the size of the matrix (HEX27: 64;
+// HEX8: 27).  us per CG iteration with eight and with SliceCfg's waves: 32^3 HEX27 Poisson FP64 60 / 78,
+// FP32 58 / 59; 18^3 and 20^3 HEX27 J2 FP64 71 / 80 and 83 / 111, 20^3 FP32 53 / 61.
+constexpr int kLongRow = 40;
+inline bool long_rows(const fem_pattern_t& pat) { return pat.sell_blocks >= pat.num_slices * kSlice * kLongRow; }
+
 // XCD-contiguous block order: hardware dispatches block b to XCD b % 8; this
 // maps the blocks of one XCD onto a contiguous range of logical block ids so
 // neighbouring rows (which share gathered vector entries) stay in one L2.

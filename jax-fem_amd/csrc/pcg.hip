@@ -472,48 +472,15 @@ __global__ void k_pcg_copy(int64_t n, const T* __restrict__ a, T* __restrict__ b
     b[i] = a[i];
 }
 
-// y = A x for FP64 x, y (standard form values of precision T).
-template <int V, typename T>
-__global__ __launch_bounds__(256) void k_spmv_x(fem_pattern_t pat, const T* __restrict__ vals,
-                                                const double* __restrict__ x, double* __restrict__ y) {
-  constexpr int VV = V * V;
-  const int64_t row = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (row >= pat.num_rows) return;
-  const int64_t pos = pat.sell_pos[row];
-  const int64_t s = pos >> 6;
-  const int lane = (int)(pos & 63);
-  const int base = pat.slice_ptr[s];
-  const int L = (pat.slice_ptr[s + 1] - base) >> 6;
-  const int32_t* cp = pat.sell_col + base + lane;
-  const T* vp = vals + (size_t)base * VV + lane;
-  double acc[V];
-#pragma unroll
-  for (int i = 0; i < V; ++i) acc[i] = 0.0;
-  for (int k = 0; k < L; ++k) {
-    const int64_t c = cp[(size_t)k * kSlice];
-#pragma unroll
-    for (int i = 0; i < V; ++i)
-#pragma unroll
-      for (int j = 0; j < V; ++j) acc[i] += double(vp[((size_t)k * VV + i * V + j) * kSlice]) * x[c * V + j];
-  }
-#pragma unroll
-  for (int i = 0; i < V; ++i) y[row * V + i] = acc[i];
-}
-
 constexpr int kVecGrid = 1024;  // blocks of the vector kernels (partials per reduction)
-// Mean slots of a row from which eight waves share a slice whatever the size of the matrix (HEX27: 64;
-// HEX8: 27).  us per iteration with eight and with the usual waves: 32^3 HEX27 Poisson FP64 60 / 78, FP32
-// 58 / 59; 18^3 and 20^3 HEX27 J2 FP64 71 / 80 and 83 / 111, 20^3 FP32 53 / 61.
-constexpr int kLongRow = 40;
-
 // Largest matrix whose product forms its direction itself (us per iteration, with and without).
 // Scalar rows: FP64 37 MB 19.7 / 19.9, 59 MB 28 / 25.6; FP32 39 MB 25.0 / 26.1, 58 MB 33.0 / 32.7.  Blocks in
 // FP64: 72 MB 22.5 / 24.2, 139 MB 33.8 / 37.2, 237 MB 52.7 / 55.2 (HEX27 52 / 71), 325 MB 96 / 83; in FP32:
 // 45 MB 17.0 / 19.2, 73 MB 23.2 / 24.9, 125 MB 34.4 / 34.2, of long rows 125 MB 39 / 46, 171 MB 50 / 53.
 template <int V, typename T>
-inline double fuse_bytes(bool long_rows) {
+inline double fuse_bytes(bool longs) {
   if (V == 1 || V > 3) return 45e6;
-  return sizeof(T) == 8 ? 240e6 : long_rows ? 180e6 : 100e6;
+  return sizeof(T) == 8 ? 240e6 : longs ? 180e6 : 100e6;
 }
 
 struct EventPool {
@@ -617,9 +584,7 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
     } else if (kMixed) {
       if (int rc = fem_operator_apply_impl(op, x, w.y, s)) return rc;
     } else {
-      hipLaunchKernelGGL((k_spmv_x<V, T>), dim3((unsigned)ceil_div(pat->num_rows, 256)), dim3(256), 0, s, *pat, vals,
-                         (const double*)x, w.y);
-      FEM_LAUNCHED();
+      if (int rc = fem_spmv(pat, FEM_F64, FEM_FORM_STANDARD, vals, x, w.y, s)) return rc;
     }
     return residual_from(w.y);
   };
@@ -654,15 +619,15 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
   // slices (one per CU) 16 waves share a slice's slots, up to 768 eight (FP64 Poisson of 13,824
   // cells 15.3 -> 12.0 us per iteration, of 32,768 cells 16.0 -> 14.9).  FP32 blocks leave room for two
   // workgroups of eight waves on a CU: eight waves only up to 512 slices (562 slices: 25 us, with four
-  // 16.3).  FP64 blocks keep eight at any size (139 MB: 33.8 us, with two 37.7).
+  // 16.3) unless the direction has its own kernel.  FP64 blocks keep eight at any size (139 MB: 33.8 us,
+  // with two 37.7).
   // The direction update runs inside the product (which then gathers z and the old direction) where
   // the matrix stays in the caches or is not read; the new direction goes to a second buffer.  That is
   // y's, free between the true residuals: so a batch of status-free iterations has to be even.
   T* p2 = (T*)w.y;
   const double sell_bytes = double(pat->sell_blocks) * (V * V * sizeof(T) + 4);
-  const bool long_rows = pat->sell_blocks >= pat->num_slices * kSlice * kLongRow;
-  const bool fused = check % 2 == 0 && (pop ? true : sell_bytes <= fuse_bytes<V, T>(long_rows));
-  const bool eight = long_rows || (fused && (V == 1 ? gA <= 768 : gA <= 512 || (V <= 3 && sizeof(T) == 8)));
+  const bool fused = check % 2 == 0 && (pop ? true : sell_bytes <= fuse_bytes<V, T>(long_rows(*pat)));
+  const bool eight = long_rows(*pat) || (V == 1 ? fused && gA <= 768 : !fused || gA <= 512 || sizeof(T) == 8);
   // one workgroup for the whole batch: few scalar rows of, on average, at most kOneSlots slots
   const bool one = V == 1 && !pop && !opt->timing && pat->num_slices <= kOneSlices &&
                    pat->sell_blocks <= pat->num_slices * kSlice * kOneSlots;

@@ -351,10 +351,10 @@ __global__ void k_residual_bc(int64_t n_bc, const int32_t* __restrict__ dofs, co
 
 // ------------------------------------------------------------ SpMV
 // One block per slice; the W waves split the slots and wave 0 combines them.
-template <int V, bool DIFF, typename T>
-__global__ __launch_bounds__(SliceCfg<T>::NT) void k_spmv(fem_pattern_t pat, const T* __restrict__ vals,
-                                                          const T* __restrict__ x, T* __restrict__ y) {
-  constexpr int W = SliceCfg<T>::W, U = SliceCfg<T>::U;
+template <int V, bool DIFF, typename T, int W>
+__global__ __launch_bounds__(64 * W) void k_spmv(fem_pattern_t pat, const T* __restrict__ vals,
+                                                 const T* __restrict__ x, T* __restrict__ y) {
+  constexpr int U = SliceCfg<T>::U;
   __shared__ double red[W][kSlice][V];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int64_t s = blockIdx.x;
@@ -620,13 +620,23 @@ int fem_spmv(const fem_pattern_t* pat, int32_t precision, int32_t form, const vo
   return with_vt(pat->vec, precision, [&](auto vc, auto tv) -> int {
     constexpr int V = decltype(vc)::value;
     using T = decltype(tv);
-    const dim3 grid((unsigned)pat->num_slices), block(SliceCfg<T>::NT);
+    const dim3 grid((unsigned)pat->num_slices);
+    auto product = [&](auto diff, auto waves) {
+      constexpr int W = decltype(waves)::value;
+      hipLaunchKernelGGL((k_spmv<V, decltype(diff)::value, T, W>), grid, dim3(64 * W), 0, as_stream(stream), *pat,
+                         (const T*)vals, (const T*)x, (T*)y);
+    };
+    // Eight waves per slice for blocks and long rows, SliceCfg's for short scalar rows.  us with SliceCfg's
+    // and with eight: HEX8 elastic 64^3 FP64 97 / 92, FP32 49.6 / 48.2, HEX27 12^3 32 / 20 and 17 / 11.5, 32^3
+    // 343 / 319 and 165 / 161, HEX27 scalar 32^3 72 / 57 and 45 / 45; HEX8 scalar 64^3 19.6 / 18.5 and 16 / 18.2,
+    // 100^3 66 / 68 and 54 / 64.
+    using Some = std::integral_constant<int, 8>;
+    using Many = std::integral_constant<int, SliceCfg<T>::W>;
+    const bool some = V > 1 || long_rows(*pat);
     if (form == FEM_FORM_DIFFERENCE)
-      hipLaunchKernelGGL((k_spmv<V, true, T>), grid, block, 0, as_stream(stream), *pat, (const T*)vals, (const T*)x,
-                         (T*)y);
+      some ? product(std::true_type{}, Some{}) : product(std::true_type{}, Many{});
     else
-      hipLaunchKernelGGL((k_spmv<V, false, T>), grid, block, 0, as_stream(stream), *pat, (const T*)vals, (const T*)x,
-                         (T*)y);
+      some ? product(std::false_type{}, Some{}) : product(std::false_type{}, Many{});
     FEM_LAUNCHED();
     return FEM_OK;
   });
