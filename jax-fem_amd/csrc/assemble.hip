@@ -21,9 +21,9 @@
 // What bounds it: LDS (60 to 70 % of its cycles: gradients read per block, blocks
 // handed over) and the latencies that two waves per SIMD leave open; the matrix
 // itself is written at 6 TB/s, past the caches.  64^3 Neo-Hookean cells with FP64
-// values 2630 -> 930 us, 128 x 64 x 64 elastic cells 2000 -> 870 us (the stores alone
+// values 2630 -> 940 us, 128 x 64 x 64 elastic cells 2000 -> 855 us (the stores alone
 // take 220 us of these, a wave's first loads 130 us), 80 x 31 x 31 SIMP cells 342 ->
-// 170 us, against one workgroup per slice that met at four barriers per chunk (80 to
+// 160 us, against one workgroup per slice that met at four barriers per chunk (80 to
 // 110 KB of LDS, one or two workgroups per CU, most threads idle in most phases).
 #include "element.hpp"
 

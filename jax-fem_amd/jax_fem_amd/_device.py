@@ -118,7 +118,7 @@ class DeviceMesh:
 
     def patch_plan(self):
         """Plan of the matrix-free patch products (csrc/patch.hip), built once per mesh; None where
-        they do not apply (HEX8 cells with the 2x2x2 Gauss rule only)."""
+        they do not apply (HEX8 cells with the 2x2x2, HEX27 with the 3x3x3 Gauss rule)."""
         if self._patch is None:
             self._patch = False
             cpp = int(self.L.fem_patch_cells(self.ref)) if self.C > 0 else 0
