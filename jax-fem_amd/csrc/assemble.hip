@@ -21,7 +21,7 @@
 // What bounds it: LDS (60 to 70 % of its cycles: gradients read per block, blocks
 // handed over) and the latencies that two waves per SIMD leave open; the matrix
 // itself is written at 6 TB/s, past the caches.  64^3 Neo-Hookean cells with FP64
-// values 2630 -> 940 us, 128 x 64 x 64 elastic cells 2000 -> 855 us (the stores alone
+// values 2630 -> 925 us, 128 x 64 x 64 elastic cells 2000 -> 850 us (the stores alone
 // take 220 us of these, a wave's first loads 130 us), 80 x 31 x 31 SIMP cells 342 ->
 // 160 us, against one workgroup per slice that met at four barriers per chunk (80 to
 // 110 KB of LDS, one or two workgroups per CU, most threads idle in most phases).
@@ -354,9 +354,6 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
   constexpr bool kParam = !std::is_same<MAT, MatJ2>::value;
   __shared__ double s_dN[8 * kGQ], s_w[8];
   __shared__ AsmWave<MAT, RES> s_wave[kAsmThreads / 64];
-  for (int i = threadIdx.x; i < 8 * 24; i += kAsmThreads) s_dN[(i / 24) * kGQ + i % 24] = mesh.shape_grads_ref[i];
-  if (threadIdx.x < 8) s_w[threadIdx.x] = mesh.quad_weights[threadIdx.x];
-  __syncthreads();
   AsmWave<MAT, RES>& L = s_wave[threadIdx.x >> 6];
   const int lane = threadIdx.x & 63, hi8 = lane >> 3, j = lane & 7;
   // (uniform in the wave, and known to be: what follows from it stays in scalar registers)
@@ -364,16 +361,45 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
   const int s = gid / kGroups;
   const int gr = gid % kGroups, rl = gr * kGroupRows + hi8;  // the lane's row in the slice
 
+  // The wave's two chains of lists, row -> pairs and group -> cells -> nodes -> coordinates, are
+  // begun side by side and before the tables' barrier (one after the other: 128 x 64 x 64 elastic
+  // cells 867 us instead of 849, 64^3 Neo-Hookean with the residual 1070 instead of 1045).
   const int sbase = pat.slice_ptr[s], nslots = (pat.slice_ptr[s + 1] - sbase) >> 6;
   const int row = pat.sell_row[s * kSlice + rl];
-  int ds = -1, np = 0;  // pairs of the row
-  const uint32_t* pw = loc + j;
-  if (row >= 0) {
-    const int rb = pat.row_ptr[row], t0 = pat.contrib_ptr[rb];
-    np = (pat.contrib_ptr[pat.row_ptr[row + 1]] - t0) >> 3;
-    pw += np > 0 ? t0 : 0;
-    ds = pat.diag_slot[row];
-  }
+  const int32_t* cl = sc + sc_ptr[s];
+  const int first = gr ? cl[gr - 1] : 0, nc = cl[gr] - first;
+  cl += kGroups + first;
+  auto cell_at = [&](int k) { return cl[min(k * 8 + hi8, nc - 1)]; };
+  // loaded ahead: cell, node, coordinates and parameter of the coming chunk (1), cell and node of
+  // the one after it (2), cells of the third
+  int32_t c1 = 0, n1 = 0, c2 = 0, n2 = 0, c3 = 0;
+  if (nc > 0) c1 = cell_at(0), c2 = cell_at(1), c3 = cell_at(2);
+  for (int i = threadIdx.x; i < 8 * 24; i += kAsmThreads) s_dN[(i / 24) * kGQ + i % 24] = mesh.shape_grads_ref[i];
+  if (threadIdx.x < 8) s_w[threadIdx.x] = mesh.quad_weights[threadIdx.x];
+  const int rr = max(row, 0), rb = pat.row_ptr[rr], re = pat.row_ptr[rr + 1];
+  int ds = pat.diag_slot[rr];
+  if (nc > 0) n1 = mesh.cells[(int64_t)c1 * 8 + j], n2 = mesh.cells[(int64_t)c2 * 8 + j];
+  const int t0 = pat.contrib_ptr[rb];
+  int np = (pat.contrib_ptr[re] - t0) >> 3;  // pairs of the row
+  __syncthreads();
+  double xr[3] = {0, 0, 0}, ur[V], par = 1.0;
+#pragma unroll
+  for (int i = 0; i < V; ++i) ur[i] = 0.0;
+  // without parameters the load reads a weight and is not used (a branch would split the geometry)
+  const bool has_par = kParam && mat.has_param;
+  const double* par_base = has_par ? mat.param : mesh.quad_weights;
+  auto load_chunk = [&]() {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) xr[i] = mesh.points[(int64_t)n1 * 3 + i];
+    if constexpr (kU)
+#pragma unroll
+      for (int i = 0; i < V; ++i) ur[i] = u[(int64_t)n1 * V + i];
+    if constexpr (kParam) par = par_base[has_par ? (int64_t)c1 * 8 + j : 0];
+  };
+  if (nc > 0) load_chunk();
+  np = row >= 0 ? np : 0;
+  ds = row >= 0 ? ds : -1;
+  const uint32_t* pw = loc + (np > 0 ? t0 : 0) + j;
   // word: the row's next pair; ahead: what was loaded for pair ip, the one after it (beyond the
   // row's last pair the load repeats that one and is not used)
   int ip = 1;
@@ -382,11 +408,6 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
   constexpr int NX = AsmWave<MAT, RES>::NX;
   LdsD *const lg = lds_base(L.g), *const lr = lds_base(&L.rec[0][0]), *const lx = lds_base(L.ex);
   if (lane < NX) lx[64 * NX + lane] = 0.0;
-
-  const int32_t* cl = sc + sc_ptr[s];
-  const int first = gr ? cl[gr - 1] : 0, nc = cl[gr] - first;
-  cl += kGroups + first;
-  auto cell_at = [&](int k) { return cl[min(k * 8 + hi8, nc - 1)]; };
 
   // the point's reference gradients: kept where the registers suffice, else read from LDS each time
   constexpr bool kKeep = TP::kIso && !RES;
@@ -402,32 +423,6 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
   double rs[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) rs[i] = 0.0;
-
-  // loaded ahead: cell, node, coordinates and parameter of the coming chunk (1), cell and node of
-  // the one after it (2), cells of the third
-  double xr[3] = {0, 0, 0}, ur[V], par = 1.0;
-#pragma unroll
-  for (int i = 0; i < V; ++i) ur[i] = 0.0;
-  int32_t c1 = 0, n1 = 0, c2 = 0, n2 = 0, c3 = 0;
-  // without parameters the load reads a weight and is not used (a branch would split the geometry)
-  const bool has_par = kParam && mat.has_param;
-  const double* par_base = has_par ? mat.param : mesh.quad_weights;
-  auto load_chunk = [&]() {
-#pragma unroll
-    for (int i = 0; i < 3; ++i) xr[i] = mesh.points[(int64_t)n1 * 3 + i];
-    if constexpr (kU)
-#pragma unroll
-      for (int i = 0; i < V; ++i) ur[i] = u[(int64_t)n1 * V + i];
-    if constexpr (kParam) par = par_base[has_par ? (int64_t)c1 * 8 + j : 0];
-  };
-  if (nc > 0) {
-    c1 = cell_at(0);
-    n1 = mesh.cells[(int64_t)c1 * 8 + j];
-    c2 = cell_at(1);
-    n2 = mesh.cells[(int64_t)c2 * 8 + j];
-    c3 = cell_at(2);
-    load_chunk();
-  }
 
   for (int k = 0; k * 8 < nc; ++k) {
     // ---- 1: the chunk's coordinates to LDS; fetch the next chunk's
