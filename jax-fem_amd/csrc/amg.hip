@@ -1515,24 +1515,28 @@ __global__ __launch_bounds__(256) void k_bcsr_apply_row(int64_t rows, const int3
 // Slice split of the V-cycle's SELL kernels: FP32 storage with FP64 vectors 3 waves
 // per slice (one thread per (row, component) in the epilogue; on the 1.6M-dof HEX8
 // cantilever 3, 4, 6, 8 waves: Chebyshev step 122.5, 123.2, 130.3, 125.6 us, residual
-// 111.9, 113.6, 125.9, 121.7 us), otherwise the split of the Jacobi path's kernels.
-template <typename T>
+// 111.9, 113.6, 125.9, 121.7 us), FP16 and short scalar FP64 rows the split of the Jacobi
+// path's kernels; EIGHT: eight waves, for FP64 blocks and for long rows.  Chebyshev step, us:
+// J2 HEX8 64^3 FP64 113 -> 109, 16^3 11.4 -> 9.0; HEX27 24^3 FP64 155 -> 120, FP32 82 -> 71,
+// 8^3 33 -> 21 and 23 -> 15, 16^3 59 -> 60 and 38 -> 30.
+template <typename T, bool EIGHT>
 struct AmgSliceCfg {
-  static constexpr int W = sizeof(T) == 4 ? 3 : SliceCfg<T>::W;
+  static constexpr int W = EIGHT ? 8 : sizeof(T) == 4 ? 3 : SliceCfg<T>::W;
   static constexpr int NT = 64 * W;
 };
 
 // Standard-form SELL-64 operator (level 0), FP64 vectors, one block per slice.
 // DIFF: the matrix is in difference form (the diagonal slot holds the row
 // sum); the own-row entries of the input then enter every product.
-template <int V, int MODE, typename T, bool DIFF = false, typename TX = double, typename TY = double>
-__global__ __launch_bounds__(AmgSliceCfg<T>::NT) void k_sell_apply(fem_pattern_t pat, const T* __restrict__ vals,
-                                                                ApplyArgsT<TX, TY> a,
-                                                                const int32_t* __restrict__ done) {
+template <int V, int MODE, typename T, bool DIFF, typename TX, typename TY, bool EIGHT>
+__global__ __launch_bounds__((AmgSliceCfg<T, EIGHT>::NT)) void k_sell_apply(fem_pattern_t pat,
+                                                                       const T* __restrict__ vals,
+                                                                       ApplyArgsT<TX, TY> a,
+                                                                       const int32_t* __restrict__ done) {
   // FP32 products unroll the slots by 4 (the residual: 124 -> 112 us on the 1.6M-dof
   // cantilever), the Chebyshev step, with its larger epilogue, by 2 (119.5 against 124.6 us);
   // FP16 storage keeps 2 (its residual: 74 us unrolled by 2, 78 us by 4)
-  constexpr int W = AmgSliceCfg<T>::W;
+  constexpr int W = AmgSliceCfg<T, EIGHT>::W;
   constexpr int U = sizeof(T) == 4 ? (MODE == AP_CHEB ? 2 : 4) : SliceCfg<T>::U;
   __shared__ double red[W][kSlice][V];
   if ((done && *done) || (a.done && *a.done)) return;
@@ -1553,11 +1557,11 @@ __global__ __launch_bounds__(AmgSliceCfg<T>::NT) void k_sell_apply(fem_pattern_t
   // FP16 values hold D^-1 A (rows scaled by dinv): the epilogues undo or skip the scaling
   constexpr bool kScaled = sizeof(T) == 2;
   // The epilogue's own-row operands are loaded before the matrix stream, so their
-  // latency overlaps it.  With a thread per (row, component) pair (kDist: 4 waves),
+  // latency overlaps it.  With a thread per (row, component) pair (kDist: a thread for each),
   // thread p finishes component p % V of lane p / V after the partial sums meet in
   // LDS, holding 4 operands; otherwise wave 0 finishes its lanes' rows (the outer
   // product's <p, q> partial is then one wave sum).
-  constexpr bool kDist = MODE != AP_PQ && AmgSliceCfg<T>::NT >= kSlice * V;
+  constexpr bool kDist = MODE != AP_PQ && AmgSliceCfg<T, EIGHT>::NT >= kSlice * V;
   const int pl = threadIdx.x / V, pi = threadIdx.x % V;
   int64_t prow = -1;
   double p_rhs = 0.0, p_dinv = 0.0, p_d = 0.0, p_x = 0.0;
@@ -1931,12 +1935,18 @@ int sell_apply(const fem_pattern_t& pat, const void* vals, const ApplyArgsT<TX, 
   if (pat.num_slices == 0) return FEM_OK;
   const unsigned grid = (unsigned)pat.num_slices;
   const T* v = static_cast<const T*>(vals);
+  auto product = [&](auto vec, auto eight) {
+    constexpr int V = decltype(vec)::value;
+    constexpr bool EIGHT = decltype(eight)::value;
+    hipLaunchKernelGGL((k_sell_apply<V, MODE, T, DIFF, TX, TY, EIGHT>), dim3(grid), dim3(AmgSliceCfg<T, EIGHT>::NT), 0, s,
+                       pat, v, a, done);
+  };
+  using Vec3 = std::integral_constant<int, 3>;
+  using Vec1 = std::integral_constant<int, 1>;
   if (pat.vec == 3)
-    hipLaunchKernelGGL((k_sell_apply<3, MODE, T, DIFF, TX, TY>), dim3(grid), dim3(AmgSliceCfg<T>::NT), 0, s, pat, v, a,
-                       done);
+    sizeof(T) == 8 || long_rows(pat) ? product(Vec3{}, std::true_type{}) : product(Vec3{}, std::false_type{});
   else if (pat.vec == 1)
-    hipLaunchKernelGGL((k_sell_apply<1, MODE, T, DIFF, TX, TY>), dim3(grid), dim3(AmgSliceCfg<T>::NT), 0, s, pat, v, a,
-                       done);
+    long_rows(pat) ? product(Vec1{}, std::true_type{}) : product(Vec1{}, std::false_type{});
   else
     FEM_CHECK_ARG(false, "AMG: vec must be 1 or 3");
   FEM_LAUNCHED();

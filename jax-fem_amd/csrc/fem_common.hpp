@@ -185,7 +185,8 @@ __device__ inline void sell_slice_partial(const fem_pattern_t& pat, const T* __r
 
 // Slice split chosen by a sweep of (W, U) on the 1.6M-dof HEX8 elasticity
 // matrix: FP32 4 waves x unroll 2, FP64 2 waves x unroll 2 (FP16 storage
-// takes the FP32 split).
+// takes the FP32 split).  Products of blocks and of long rows take eight where
+// that measured faster (fem_spmv, k_pcg_a's and k_sell_apply's launches).
 template <typename T>
 struct SliceCfg {
   static constexpr int W = sizeof(T) <= 4 ? 4 : 2;
