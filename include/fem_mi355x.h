@@ -618,9 +618,9 @@ int fem_amg_dinv(const fem_bcsr_t* A, int32_t fix_zero, double* dinv, void* stre
 /* Largest-eigenvalue estimate of D^-1 A by `steps` power steps from a fixed
  * start vector.  A is the SELL matrix (pat, sell_vals) if pat != NULL --
  * sell_f32 = 0: FP64 standard form, 1: FP32 difference form, 2: FP16 scaled
- * difference form (FEM_FORM_SCALED_DIFF16) -- else the FP64 block CSR matrix
- * A.  sell_f32 = 3: sell_vals is a host fem_patch_operator_t (pat is not read
- * beyond its sizes).  ws >= fem_amg_lmax_ws_bytes(unknowns).  Synchronises the
+ * difference form (FEM_FORM_SCALED_DIFF16), 3: sell_vals is a host
+ * fem_patch_operator_t and pat gives the sizes -- else the block CSR matrix A
+ * (sell_vals and sell_f32 are not read).  ws >= fem_amg_lmax_ws_bytes(unknowns).  Synchronises the
  * stream. */
 int64_t fem_amg_lmax_ws_bytes(int64_t n);
 int fem_amg_lmax(const fem_bcsr_t* A, const fem_pattern_t* pat, const void* sell_vals, int32_t sell_f32,

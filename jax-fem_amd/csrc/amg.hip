@@ -2521,11 +2521,11 @@ int fem_amg_lmax_async(const fem_bcsr_t* A, const fem_pattern_t* pat, const void
   FEM_CHECK_ARG(dinv && lmax_dev && ws && steps >= 1, "fem_amg_lmax: bad arguments");
   FEM_CHECK_ARG(pat ? (sell_vals != nullptr && pat->num_rows > 0) : (A && A->br == A->bc && A->rows > 0),
                 "fem_amg_lmax: give a SELL matrix (pat, sell_vals) or a square block CSR matrix");
-  if (pat && sell_f32 == 3) {
-    const fem_patch_operator_t* op = static_cast<const fem_patch_operator_t*>(sell_vals);
+  // (without a pattern the matrix is A, whatever sell_f32 is)
+  const fem_patch_operator_t* op = pat && sell_f32 == 3 ? static_cast<const fem_patch_operator_t*>(sell_vals) : nullptr;
+  if (op)
     FEM_CHECK_ARG(patch_operator_ok(op) && op->mesh->num_nodes == pat->num_rows && op->mesh->vec == pat->vec,
                   "fem_amg_lmax: the matrix-free operator is incomplete, not covered or of another size");
-  }
   hipStream_t s = as_stream(stream);
   const int64_t n = pat ? pat->num_rows * pat->vec : A->rows * A->br;
   char* w = static_cast<char*>(ws);
@@ -2565,8 +2565,7 @@ int fem_amg_lmax_async(const fem_bcsr_t* A, const fem_pattern_t* pat, const void
       if constexpr (sizeof(TV) == 4) {
         rc = sell_apply<AP_DSTORE, float, true>(*pat, static_cast<const float*>(sell_vals), a, nullptr, s);
       } else {
-        rc = sell_f32 == 3 ? patch_apply<AP_DSTORE, double, double>(
-                                 *static_cast<const fem_patch_operator_t*>(sell_vals), a, s)
+        rc = op ? patch_apply<AP_DSTORE, double, double>(*op, a, s)
              : !pat ? (A->f32 ? bcsr_apply<AP_DSTORE, float>(*A, a, s) : bcsr_apply<AP_DSTORE, double>(*A, a, s))
              : sell_f32 == 2 ? sell_apply<AP_DSTORE, _Float16, true>(*pat, sell_vals, a, nullptr, s)
                              : sell_apply<AP_DSTORE, double>(*pat, static_cast<const double*>(sell_vals), a, nullptr, s);
