@@ -143,11 +143,11 @@ __global__ __launch_bounds__(64 * kGatherWaves) void k_gather_matrix(fem_pattern
 // A wave takes a row: it lists the row's pairs (the diagonal slot's contributions) and the slot of
 // each of their blocks, then adds run after run, lane-contiguous, to the row's slots in LDS; the
 // workgroup's eight rows are stored together (64-byte segments).  Sums run over the cells in
-// ascending order, as above.  Rows of more than kRowSlots slots are done in windows and rows of
-// more than kRowPairs pairs slot by slot, into the same LDS.
+// ascending order, as above.  Rows of more than kRowSlots slots are done in windows; rows of more
+// than kRowPairs pairs, and rows of a cell that names a node twice (two lanes of one run on one
+// slot: their order would be the hardware's), slot by slot, into the same LDS.
 // The adds are LDS atomics in FP64 (one instruction; loads, adds and stores 416 us instead of 405 in
-// the same run) and plain ones in FP32, whose atomics are the slower ones (777 us; plain 400), unless
-// a cell names a node twice.
+// the same run) and plain ones in FP32, whose atomics are the slower ones (777 us; plain 400).
 // 24^3 cells: 610 -> 365 us (1.29 GB, 250 us at the copy rate), from FP32 tangents 553 -> 400; with two
 // rows to a wave 525: what is left is the chain row -> lists -> runs, which 16 waves on a CU (the LDS's
 // limit) do not cover.
@@ -186,9 +186,10 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
       const int d0 = ds >= 0 ? pat.contrib_ptr[rb + ds] : 0;
       const int n = ds >= 0 ? pat.contrib_ptr[rb + ds + 1] - d0 : 0;
       const int t0 = pat.contrib_ptr[rb], t1 = pat.contrib_ptr[rb + len];
-      if (len <= kRowSlots && n <= kRowPairs && t1 - t0 == n * N) {
+      bool listed = len <= kRowSlots && n <= kRowPairs && t1 - t0 == n * N;
+      int first = 0;
+      if (listed) {
         // first block of each pair (the diagonal's contribution is its block a)
-        int first = 0;
         if (lane < n) {
           const int32_t e = pat.contrib_idx[d0 + lane];
           first = e - e % N;
@@ -199,22 +200,30 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
         wave_fence();
         bool twice = false;
         int slots = 0;  // slots that begin before the 64 contributions at hand
+        int last = -1;  // pair of the contribution before them
         for (int i = lane; i - lane < n * N; i += 64) {
           const bool in = i < n * N;
           const unsigned long long begins = __ballot(in && s_first[w][i]);
           const int slot = slots + __popcll(begins & (~0ull >> (63 - lane))) - 1;
           slots += __popcll(begins);
           const int e = in ? pat.contrib_idx[t0 + i] : -1;
+          int pair = -1;
           for (int p = 0; p < n; ++p) {
             const int b = e - __shfl(first, p, 64);
-            if (in && b >= 0 && b < N) s_slot[w][p][b] = (uint8_t)slot;
+            if (in && b >= 0 && b < N) {
+              s_slot[w][p][b] = (uint8_t)slot;
+              pair = p;
+            }
           }
           // (a slot's contributions are in ascending order: a pair's two blocks of it are neighbours)
-          if (kPlainAdds)
-            twice |= i + 1 < n * N && !s_first[w][i + 1] && pat.contrib_idx[t0 + i + 1] / N == e / N;
+          const int up = __shfl_up(pair, 1, 64);
+          twice |= in && !(begins >> lane & 1) && pair == (lane ? up : last);
+          last = __shfl(pair, 63, 64);
         }
         wave_fence();
-        const bool unique = kPlainAdds && !__any(twice);
+        listed = !__any(twice);
+      }
+      if (listed) {
         for (int p = 0; p < n; p += 4) {
           TS x[4][PER];
 #pragma unroll
@@ -226,7 +235,7 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             if (p + j >= n) break;
-            if (unique) {
+            if constexpr (kPlainAdds) {
               int at[PER];
               TS y[PER];
 #pragma unroll
@@ -239,13 +248,12 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_gather_rows(fem_pattern_t pa
               for (int i = 0; i < PER; ++i)
                 if (lane + 64 * i < RUN) acc[at[i]] = y[i] + x[j][i];
               wave_fence();
-              continue;
-            }
+            } else {
 #pragma unroll
-            for (int i = 0; i < PER; ++i) {
-              const int o = lane + 64 * i;
-              // (an LDS atomic only for a cell that names a node twice: two lanes on one slot)
-              if (o < RUN) atomicAdd(&acc[s_slot[w][p + j][o / VV] * VV + o % VV], x[j][i]);
+              for (int i = 0; i < PER; ++i) {
+                const int o = lane + 64 * i;
+                if (o < RUN) atomicAdd(&acc[s_slot[w][p + j][o / VV] * VV + o % VV], x[j][i]);
+              }
             }
           }
         }
