@@ -484,7 +484,9 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
       inv3(J, det, iJ);
       [[maybe_unused]] double P[6];
       if constexpr (TP::kSpatial) {
-        // F = j J^-1 with j = J + grad_ref u; h = j^-T dN
+        // F = I + grad_ref u J^-1; h = j^-T dN with j = J + grad_ref u.  (F, and its determinant, from
+        // the displacement's gradient: from j they carry j's rounding, which the stress of a small
+        // strain, a difference of terms of order 1, shows undiminished.)
         double jc[9], F[9];
 #pragma unroll
         for (int i = 0; i < 9; ++i) jc[i] = J[i] + U[i / 3][i % 3];
@@ -492,18 +494,17 @@ __global__ __launch_bounds__(kAsmThreads, 2) void k_assemble_hex8(
         for (int i = 0; i < 3; ++i)
 #pragma unroll
           for (int l = 0; l < 3; ++l)
-            F[i * 3 + l] = jc[i * 3] * iJ[l] + jc[i * 3 + 1] * iJ[3 + l] + jc[i * 3 + 2] * iJ[6 + l];
+            F[i * 3 + l] = (U[i][0] * iJ[l] + U[i][1] * iJ[3 + l] + U[i][2] * iJ[6 + l]) + (i == l ? 1.0 : 0.0);
         const double b[6] = {F[0] * F[0] + F[1] * F[1] + F[2] * F[2], F[3] * F[3] + F[4] * F[4] + F[5] * F[5],
                              F[6] * F[6] + F[7] * F[7] + F[8] * F[8], F[0] * F[3] + F[1] * F[4] + F[2] * F[5],
                              F[0] * F[6] + F[1] * F[7] + F[2] * F[8], F[3] * F[6] + F[4] * F[7] + F[5] * F[8]};
-        const double detc = det3(jc), Jd = detc / det;
-        inv3(jc, detc, iJ);
-        // Jd^-2/3; NaN for an inverted point, like pow(Jd, -2/3)
-        const double rc = rcbrt(Jd), wp = w * p0, I1 = b[0] + b[1] + b[2];
-        const double ma = mat.c[0] * wp * (Jd < 0.0 ? __builtin_nan("") : rc * rc), kp = mat.c[1] * wp;
+        const double Jd = det3(F);
+        inv3(jc, det3(jc), iJ);
+        const double wp = w * p0, I1 = b[0] + b[1] + b[2];
+        const double ma = mat.c[0] * wp * pow_m23(Jd), kp = mat.c[1] * wp;
 #pragma unroll
         for (int i = 0; i < 6; ++i) r[i] = (-2.0 / 3.0) * ma * b[i];
-        const double kj = kp * (Jd * Jd - Jd), mi = ma * I1 * (1.0 / 3.0);
+        const double kj = kp * Jd * (Jd - 1.0), mi = ma * I1 * (1.0 / 3.0);
         r[6] = (2.0 / 3.0) * mi + kj + kp * (Jd * Jd);
         r[7] = mi - kj;
         if constexpr (RES)

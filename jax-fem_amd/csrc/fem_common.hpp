@@ -54,6 +54,18 @@ constexpr int kDppXor2 = 0x4E;        // quad_perm [2, 3, 0, 1]
 constexpr int kDppHalfMirror = 0x141; // lane i of 8 <- 7 - i
 constexpr int kDppMirror = 0x140;     // lane i of 16 <- 15 - i
 
+// x^-2/3 to half an ulp for x > 0, NaN for x < 0 (like pow): rcbrt squared, with the rounding of the
+// square and the error of rcbrt put back.  With c = rcbrt(x) and r = 1 - x c^3 (exact to 1e-32),
+// x^-2/3 = c^2 (1 - r)^-2/3.  The square alone is off by up to 2.3 ulp (pow: 0.5 to 18 over
+// e^-50 .. e^50, at several times the instructions).
+__device__ inline double pow_m23(double x) {
+#pragma clang fp contract(off)  // (a product folded into the next sum would lose its rounding error)
+  const double c = rcbrt(x), p = c * c, pe = fma(c, c, -p);
+  const double q = p * c, qe = fma(p, c, -q) + pe * c;
+  const double r = fma(-x, q, 1.0) - x * qe;
+  return x < 0.0 ? __builtin_nan("") : p + fma(p * (2.0 / 3.0), r, pe);
+}
+
 // Orders LDS accesses of one wave: the hardware executes them in order, so only the compiler
 // has to keep the order.
 __device__ inline void wave_fence() {

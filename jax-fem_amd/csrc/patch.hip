@@ -308,10 +308,8 @@ __device__ inline void neo_hookean_tangent(const fem_material_t& m, int64_t cq, 
   for (int i = 0; i < 3; ++i)
 #pragma unroll
     for (int l = 0; l < 3; ++l) L[i][l] = Lr[i][0] * A[l] + Lr[i][1] * A[3 + l] + Lr[i][2] * A[6 + l];
-  // J^-2/3; NaN for an inverted point, like pow(J, -2/3)
-  const double rc = rcbrt(J), a = J < 0.0 ? __builtin_nan("") : rc * rc;
   const double s = W * id * id * param_at(m, cq);
-  const double ma = m.c[0] * s * a, k = m.c[1] * s, I1 = b[0] + b[1] + b[2];
+  const double ma = m.c[0] * s * pow_m23(J), k = m.c[1] * s, I1 = b[0] + b[1] + b[2];
   const double tr = L[0][0] + L[1][1] + L[2][2];
   const double bL = b[0] * L[0][0] + b[1] * L[1][1] + b[2] * L[2][2] + b[3] * (L[0][1] + L[1][0]) +
                     b[4] * (L[0][2] + L[2][0]) + b[5] * (L[1][2] + L[2][1]);
