@@ -429,13 +429,19 @@ __global__ __launch_bounds__(2 * kPatchCells) void k_patch_hex8(fem_mesh_t mesh,
     for (int k = 0; k < 4; ++k)
 #pragma unroll
       for (int v = 0; v < V; ++v) nf[k][v] = double(CG ? fma(beta, fx[k][v], fz[k][v]) : fx[k][v]);
-    // coordinates from the cell's first node, so that their differences round like the cell's size
+    // coordinates, and the residual's field, from the cell's first node, so that their differences
+    // round like the cell's size and the field's change over it
+    auto from_first = [&](auto& n) {
+      constexpr int NC = sizeof(n[0]) / sizeof(double);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const double o = swap_lane1(nx[0][j]), x0 = h ? o : nx[0][j];
+      for (int j = 0; j < NC; ++j) {
+        const double o = swap_lane1(n[0][j]), n0 = h ? o : n[0][j];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) nx[k][j] -= x0;
-    }
+        for (int k = 0; k < 4; ++k) n[k][j] -= n0;
+      }
+    };
+    from_first(nx);
+    if constexpr (MODE == 0) from_first(nf);
     layer_grad<3>(nx, g, X);
     layer_grad<V>(nf, g, F);
     if constexpr (kNeo) {
@@ -638,6 +644,13 @@ __global__ __launch_bounds__(256) void k_patch_hex27(fem_mesh_t mesh, fem_materi
     for (int i = 0; i < 3; ++i)
 #pragma unroll
       for (int v = 0; v < V; ++v) nf[i][v] = double(CG ? fma(beta, fx[i][v], fz[i][v]) : fx[i][v]);
+    if constexpr (MODE == 0)  // from the cell's first node (held by its first lane), as the coordinates
+#pragma unroll
+      for (int v = 0; v < V; ++v) {
+        const double f0 = __shfl(nf[0][v], lane - t, 64);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) nf[i][v] -= f0;
+      }
     contract(nx, hx);
     contract(nf, hf);
   }

@@ -55,6 +55,7 @@ def _exact(p, u, stress):
     pts, cells = np.asarray(fe.points, dtype=LD), np.asarray(fe.cells)
     dN, w = np.asarray(fe.shape_grads_ref).astype(LD), np.asarray(fe.quad_weights).astype(LD)
     x, ul = pts[cells], u.astype(LD)[cells]
+    ul = ul - ul[:, :1]     # (exact; the sums below are good to 19 digits of what they add)
     d, iJ = _det_inv((x[:, None, :, :, None] * dN[None, :, :, None, :]).sum(2))
     g = (dN[None, :, :, :, None] * iJ[:, :, None, :, :]).sum(3)
     G = (ul[:, None, :, :, None] * g[:, :, :, None, :]).sum(2)
@@ -91,3 +92,32 @@ def test_hyperelastic_single_pass_residual(gpu, amp):
             e = dev.last_residual.cpu().numpy().reshape(-1, 3) - want
             err[k] += float((e * e).sum() / (want * want).sum())
     assert err[0] ** .5 <= 1.1 * err[1] ** .5, err ** .5
+
+
+@pytest.mark.parametrize('second', [False, True], ids=['hex8', 'hex27'])
+@pytest.mark.parametrize('kind', ['poisson', 'elastic', 'simp'])
+def test_residual_of_a_translated_body(gpu, kind, second):
+    """A strain field of 1e-3 on a translation by a thousand: differences from a cell's first node are
+    exact, so the residual keeps its digits, some 50 roundings of its largest entry (1e-14), where
+    interpolating the field itself loses six (1e3 / 1e-3)."""
+    law = {'poisson': materials.Poisson(k=2.), 'elastic': materials.LinearElastic(E=1., nu=0.3),
+           'simp': materials.SIMPElastic(E0=1., Emin=1e-3, nu=0.3, penal=3.)}[kind]
+    p = _problem(law, (4, 3, 3) if second else (6, 5, 4), second, 1 if kind == 'poisson' else 3)
+    rng = np.random.default_rng(4)
+    u = _field(p, rng, 1e-3) + 1e3
+    E = np.ones((p.num_cells, p.fes[0].num_quads), LD)
+    if kind == 'simp':
+        theta = rng.uniform(0.4, 0.6, E.shape)
+        p.internal_vars = [torch.as_tensor(theta, device='cuda')]
+        E = LD(1e-3) + (1 - LD(1e-3)) * theta.astype(LD) ** 3
+    dev, ut = _dev(p, u)
+    c = [LD(dev.mat_desc.c[i]) for i in range(2)]
+
+    def stress(G):
+        if kind == 'poisson':
+            return c[0] * G
+        tr = np.trace(G, axis1=-2, axis2=-1)[..., None, None]
+        return E[..., None, None] * (c[0] * tr * np.eye(3, dtype=LD) + c[1] * (G + np.swapaxes(G, -1, -2)))
+    want = _exact(p, u, stress)
+    got = dev.residual_unconstrained(ut).cpu().numpy().reshape(want.shape)
+    assert np.abs(got - want).max() <= 1e-14 * np.abs(want).max()
