@@ -270,7 +270,6 @@ class DeviceProblem:
         self.cperm_inv = onp.argsort(self.cperm)
         self.inc_ptr, self.inc_idx = dm.incidence(dm.cells)
         self._build_pattern()
-        self.patch_plan = dm.patch_plan()
         self.surfaces = []
         for bi in problem.boundary_inds_list:
             faces = dm.faces_tensor(bi)
@@ -282,8 +281,8 @@ class DeviceProblem:
         self._bc_sources = None
         self._mat_cache = {}
         self.buffers = {}
-        if self.patch_plan is not None:
-            self.buffers['patch_part'] = dm.empty(self.patch_plan.entries * self.V)
+        if self._names_patch_law():
+            self.patch_plan
         self.material = None
         self.param = None
         self.load = None
@@ -841,9 +840,29 @@ class DeviceProblem:
     _PATCH_KINDS = (_lib.FEM_MAT_POISSON, _lib.FEM_MAT_LINEAR_ELASTIC, _lib.FEM_MAT_SIMP, _lib.FEM_MAT_NEO_HOOKEAN)
 
     @property
+    def patch_plan(self):
+        """The mesh's patch plan (None: not covered); with it, the products' partials.  Built on first
+        use, which for a law that no patch kernel runs (J2, tabulated, weak forms) never comes: 120 us
+        and some 8 V bytes per node and patch it appears in."""
+        plan = self.dm.patch_plan()
+        if plan is not None and 'patch_part' not in self.buffers:
+            self.buffers['patch_part'] = self.dm.empty(plan.entries * self.V)
+        return plan
+
+    def _names_patch_law(self):
+        """True when the problem names a law of the patch kernels outright (a user's callable is only
+        recognised once its parameters are there): the plan is then built with the pattern."""
+        from .materials import Material
+        try:
+            law = self.problem.get_tensor_map()
+        except Exception:
+            return False    # no laplace term, or a law that the program sets later
+        return isinstance(law, Material) and law.kind in self._PATCH_KINDS
+
+    @property
     def patch_law(self):
         """True when the cells' integrals are a closed-form law the patch kernels run."""
-        return self.patch_plan is not None and not self.cell_terms and self.material.kind in self._PATCH_KINDS
+        return not self.cell_terms and self.material.kind in self._PATCH_KINDS and self.patch_plan is not None
 
     def patch_operator(self, mat_desc, u=None, modulus=None):
         """Descriptor of the matrix-free tangent at u (fem_patch_operator_t); u is needed by the
