@@ -398,8 +398,12 @@ typedef struct {
   const int32_t* slice_cells;    /* per slice: the end offsets of its 8 groups'
                                     lists, then the lists: the group's unique
                                     incident cells, ascending                 */
-  const int32_t* slice_pair_ptr; /* not read (may be NULL)                     */
-  const int32_t* slice_pairs;    /* not read (may be NULL)                     */
+  const int32_t* slice_pair_ptr; /* (num_slices + 1), or NULL: fem_assemble
+                                    reads neither this nor slice_pairs        */
+  const int32_t* slice_pairs;    /* NULL, or the slice's (cell, local node a,
+                                    row lane) pairs, sorted keys (rank * 8 + a)
+                                    * 64 + lane, rank = position in the slice's
+                                    lists (behind the end offsets)            */
   const int32_t* contrib_loc;    /* (num_cells*N*N), rows where contrib_idx has
                                     them: 8 words per (cell, local node a) pair,
                                     by ascending cell.  Word j, of the slots
@@ -419,8 +423,8 @@ int fem_assembly_plan_counts(const fem_pattern_t* pat, const int32_t* inc_ptr, c
                              int32_t* slice_cell_counts, int32_t* slice_pair_counts, int32_t* err_flag,
                              void* stream);
 /* Plan, pass 2: slice_cells and contrib_loc (err_flag as above, or 1 when the
- * pattern and the incidences do not belong together).  slice_pair_ptr and
- * slice_pairs are not used (may be NULL). */
+ * pattern and the incidences do not belong together).  slice_pairs (with
+ * slice_pair_ptr, the scan of the pair counts) may be NULL. */
 int fem_assembly_plan_fill(const fem_pattern_t* pat, const int32_t* inc_ptr, const int32_t* inc_idx,
                            const int32_t* slice_cell_ptr, const int32_t* slice_pair_ptr, int32_t* slice_cells,
                            int32_t* slice_pairs, int32_t* contrib_loc, int32_t* err_flag, void* stream);

@@ -214,6 +214,63 @@ __global__ __launch_bounds__(kSlice* kGroupRows) void k_pair_words(fem_pattern_t
   }
 }
 
+// The pairs of each slice for callers that ask for them (the assembly reads their words above):
+// keys (rank * 8 + a) * 64 + lane, rank = place of the cell among the slice's lists, ascending.
+__global__ __launch_bounds__(256) void k_slice_pairs(fem_pattern_t pat, const int32_t* __restrict__ inc_ptr,
+                                                     const int32_t* __restrict__ inc_idx,
+                                                     const int32_t* __restrict__ sc_ptr,
+                                                     const int32_t* __restrict__ sc,
+                                                     const int32_t* __restrict__ pair_ptr,
+                                                     int32_t* __restrict__ pairs, const int32_t* __restrict__ err) {
+  __shared__ int32_t s_key[kSliceIncCap];
+  __shared__ int32_t s_off[kSlice + 1];
+  if (*err) return;  // the plan is refused
+  const int64_t s = blockIdx.x;
+  const int t = threadIdx.x;
+  const int row = t < kSlice ? pat.sell_row[s * kSlice + t] : -1;
+  const int b = row >= 0 ? inc_ptr[row] : 0, e = row >= 0 ? inc_ptr[row + 1] : 0;
+  if (t < kSlice) s_off[t + 1] = e - b;
+  if (t == 0) s_off[0] = 0;
+  __syncthreads();
+  if (t == 0)
+    for (int i = 1; i <= kSlice; ++i) s_off[i] += s_off[i - 1];
+  __syncthreads();
+  const int n = s_off[kSlice];
+  if (n > kSliceIncCap || pair_ptr[s + 1] - pair_ptr[s] != n) return;
+  if (t < kSlice) {
+    const int32_t* hd = sc + sc_ptr[s];
+    const int g = t / kGroupRows, first = g ? hd[g - 1] : 0, end = hd[g];
+    const int32_t* list = hd + kGroups;
+    for (int j = b; j < e; ++j) {
+      int lo = first, hi = end;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (list[mid] < inc_idx[j] >> 3) lo = mid + 1; else hi = mid;
+      }
+      s_key[s_off[t] + j - b] = (lo * 8 + (inc_idx[j] & 7)) * kSlice + t;
+    }
+  }
+  int P = 1;
+  while (P < n) P <<= 1;
+  for (int i = n + t; i < P; i += 256) s_key[i] = INT32_MAX;
+  __syncthreads();
+  for (int k = 2; k <= P; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int i = t; i < P; i += 256) {
+        const int l = i ^ j;
+        if (l > i) {
+          const int32_t x = s_key[i], y = s_key[l];
+          if ((x > y) == ((i & k) == 0)) {
+            s_key[i] = y;
+            s_key[l] = x;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  for (int i = t; i < n; i += 256) pairs[pair_ptr[s] + i] = s_key[i];
+}
+
 // ------------------------------------------------------- point records
 // What a block K_ab needs of a quadrature point besides the gradients h_a, h_b of its
 // shape functions: NR doubles, weighted with JxW (point()), and the block itself (add(),
@@ -766,10 +823,9 @@ int fem_assembly_plan_counts(const fem_pattern_t* pat, const int32_t* inc_ptr, c
 int fem_assembly_plan_fill(const fem_pattern_t* pat, const int32_t* inc_ptr, const int32_t* inc_idx,
                            const int32_t* slice_cell_ptr, const int32_t* slice_pair_ptr, int32_t* slice_cells,
                            int32_t* slice_pairs, int32_t* contrib_loc, int32_t* err_flag, void* stream) {
-  (void)slice_pair_ptr;
-  (void)slice_pairs;
   FEM_CHECK_ARG(pat && inc_ptr && inc_idx && slice_cell_ptr && slice_cells && contrib_loc && err_flag,
                 "fem_assembly_plan_fill: NULL argument");
+  FEM_CHECK_ARG(!slice_pairs || slice_pair_ptr, "fem_assembly_plan_fill: slice_pairs without slice_pair_ptr");
   FEM_CHECK_ARG(pat->nodes_per_cell == 8, "fem_assembly_plan_fill: HEX8 patterns only");
   if (pat->num_slices == 0) return FEM_OK;
   hipStream_t st = as_stream(stream);
@@ -780,6 +836,11 @@ int fem_assembly_plan_fill(const fem_pattern_t* pat, const int32_t* inc_ptr, con
   hipLaunchKernelGGL(k_pair_words, dim3((unsigned)pat->num_slices), dim3(kSlice * kGroupRows), 0, st, *pat, inc_ptr,
                      inc_idx, slice_cell_ptr, slice_cells, (uint32_t*)contrib_loc, err_flag);
   FEM_LAUNCHED();
+  if (slice_pairs) {
+    hipLaunchKernelGGL(k_slice_pairs, dim3((unsigned)pat->num_slices), dim3(256), 0, st, *pat, inc_ptr, inc_idx,
+                       slice_cell_ptr, slice_cells, slice_pair_ptr, slice_pairs, err_flag);
+    FEM_LAUNCHED();
+  }
   return FEM_OK;
 }
 
