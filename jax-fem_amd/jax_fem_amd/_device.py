@@ -1008,9 +1008,13 @@ class DeviceProblem:
             check(self.L.fem_patch_modulus(self.dm.ref, self.mref, ptr(mod), stream_ptr()), 'fem_patch_modulus')
         else:
             mod = None
-        lin = u.clone() if self.material.kind == _lib.FEM_MAT_NEO_HOOKEAN else None
-        op = self.patch_operator(self.mat_desc, lin, mod)
-        return op, (self.mat_desc, self.param, lin, mod, self.bc_mask)
+        neo = self.material.kind == _lib.FEM_MAT_NEO_HOOKEAN
+        lin = u.clone() if neo else None
+        # (a program's own tensor may be edited between the tangent and a solve with it)
+        param = self.param.clone() if neo and self.param is not None else self.param
+        mat = self.material.to_struct(param.data_ptr() if param is not None else None)
+        op = self.patch_operator(mat, lin, mod)
+        return op, (mat, param, lin, mod, self.bc_mask)
 
     def operator(self, u):
         op = _lib.FemOperator()
