@@ -73,6 +73,6 @@ def test_reused_hierarchy_follows_the_tangent(gpu, kind, monkeypatch):
         v = (1. + step) * u
         dev.tangent(v, cfg['precision_code'])
         assert dev.fine_for(_lib.FEM_F64) is not None
-            err = _solved(dev, cfg, v, b)
+        err = _solved(dev, cfg, v, b)
         assert err <= 1.1 * RTOL * float(torch.linalg.norm(b)), (step, err)
         assert dev._amg_uses == (0, 1, 2, 0)[step]
