@@ -180,7 +180,11 @@ typedef struct {
                                     recursive |r| fell by this factor         */
   int32_t xcd_remap;             /* 1: XCD-contiguous block order in SpMV     */
   int32_t timing;                /* 1: time the iteration phases with HIP
-                                    events (adds a record per launch)         */
+                                    events (adds a record per launch).  Scalar
+                                    systems of up to 1408 rows, otherwise whole
+                                    batches of iterations in one workgroup, then
+                                    run by launches like larger ones: the means
+                                    below are those launches'                 */
 } fem_pcg_options_t;
 
 typedef struct {

@@ -1515,10 +1515,11 @@ __global__ __launch_bounds__(256) void k_bcsr_apply_row(int64_t rows, const int3
 // Slice split of the V-cycle's SELL kernels: FP32 storage with FP64 vectors 3 waves
 // per slice (one thread per (row, component) in the epilogue; on the 1.6M-dof HEX8
 // cantilever 3, 4, 6, 8 waves: Chebyshev step 122.5, 123.2, 130.3, 125.6 us, residual
-// 111.9, 113.6, 125.9, 121.7 us), FP16 and short scalar FP64 rows the split of the Jacobi
-// path's kernels; EIGHT: eight waves, for FP64 blocks and for long rows.  Chebyshev step, us:
-// J2 HEX8 64^3 FP64 113 -> 109, 16^3 11.4 -> 9.0; HEX27 24^3 FP64 155 -> 120, FP32 82 -> 71,
-// 8^3 33 -> 21 and 23 -> 15, 16^3 59 -> 60 and 38 -> 30.
+// 111.9, 113.6, 125.9, 121.7 us), short FP16 and short scalar FP64 rows the split of the Jacobi
+// path's kernels; EIGHT: eight waves, for FP64 blocks and for long rows of any type.  Chebyshev
+// step, us: J2 HEX8 64^3 FP64 113 -> 109, 16^3 11.4 -> 9.0; HEX27 24^3 FP64 155 -> 120, FP32
+// 82 -> 71, 8^3 33 -> 21 and 23 -> 15, 16^3 59 -> 60 and 38 -> 30.  AMG-CG iteration with FP16 at
+// level 0: HEX27 8^3 185 -> 156, 16^3 368 -> 342, 24^3 672 -> 610.
 template <typename T, bool EIGHT>
 struct AmgSliceCfg {
   static constexpr int W = EIGHT ? 8 : sizeof(T) == 4 ? 3 : SliceCfg<T>::W;
@@ -1943,9 +1944,12 @@ int sell_apply(const fem_pattern_t& pat, const void* vals, const ApplyArgsT<TX, 
   };
   using Vec3 = std::integral_constant<int, 3>;
   using Vec1 = std::integral_constant<int, 1>;
-  if (pat.vec == 3)
-    sizeof(T) == 8 || long_rows(pat) ? product(Vec3{}, std::true_type{}) : product(Vec3{}, std::false_type{});
-  else if (pat.vec == 1)
+  if (pat.vec == 3) {
+    if constexpr (sizeof(T) == 8)
+      product(Vec3{}, std::true_type{});
+    else
+      long_rows(pat) ? product(Vec3{}, std::true_type{}) : product(Vec3{}, std::false_type{});
+  } else if (pat.vec == 1)
     long_rows(pat) ? product(Vec1{}, std::true_type{}) : product(Vec1{}, std::false_type{});
   else
     FEM_CHECK_ARG(false, "AMG: vec must be 1 or 3");

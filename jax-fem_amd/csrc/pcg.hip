@@ -477,6 +477,9 @@ constexpr int kVecGrid = 1024;  // blocks of the vector kernels (partials per re
 // Scalar rows: FP64 37 MB 19.7 / 19.9, 59 MB 28 / 25.6; FP32 39 MB 25.0 / 26.1, 58 MB 33.0 / 32.7.  Blocks in
 // FP64: 72 MB 22.5 / 24.2, 139 MB 33.8 / 37.2, 237 MB 52.7 / 55.2 (HEX27 52 / 71), 325 MB 96 / 83; in FP32:
 // 45 MB 17.0 / 19.2, 73 MB 23.2 / 24.9, 125 MB 34.4 / 34.2, of long rows 125 MB 39 / 46, 171 MB 50 / 53.
+// (3 x 3 blocks.)  2 x 2 blocks, to the largest measured: FP64 28 MB 13.2 / 17.0, 87 MB 24.9 / 27.3, FP32
+// 16 MB 12.7 / 16.1, 48 MB 20.2 / 22.6.  4 x 4 blocks: FP64 52 MB 18.8 / 19.2, 104 MB 27.5 / 27.8, 177 MB
+// 45.6 / 43.7; FP32 27 MB 14.6 / 14.8, 53 MB 19.0 / 20.8, 90 MB 28.5 / 30.3.
 template <int V, typename T>
 inline double fuse_bytes(bool longs) {
   if (V == 1 || V > 3) return 45e6;
@@ -628,7 +631,8 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
   const double sell_bytes = double(pat->sell_blocks) * (V * V * sizeof(T) + 4);
   const bool fused = check % 2 == 0 && (pop ? true : sell_bytes <= fuse_bytes<V, T>(long_rows(*pat)));
   const bool eight = long_rows(*pat) || (V == 1 ? fused && gA <= 768 : !fused || gA <= 512 || sizeof(T) == 8);
-  // one workgroup for the whole batch: few scalar rows of, on average, at most kOneSlots slots
+  // one workgroup for the whole batch: few scalar rows of, on average, at most kOneSlots slots (a timed
+  // solve takes the launches that its events can stand between)
   const bool one = V == 1 && !pop && !opt->timing && pat->num_slices <= kOneSlices &&
                    pat->sell_blocks <= pat->num_slices * kSlice * kOneSlots;
   const double delta2 = kMixed ? opt->reliable_delta * opt->reliable_delta : 0.0;
@@ -670,16 +674,19 @@ static int pcg_run(const fem_pattern_t* pat, const T* vals, const T* dinv_in, co
         using Few = std::integral_constant<int, 16>;
         using Some = std::integral_constant<int, 8>;
         using Many = std::integral_constant<int, SliceCfg<T>::W>;
+        // (blocks always take eight waves in FP64 and where the direction has its own kernel)
+        constexpr bool kManyFused = V == 1 || sizeof(T) == 4, kMany = V == 1;
         if (fused && gA <= 256)
           product(std::true_type{}, Few{});
-        else if (fused && eight)
+        else if (fused && (eight || !kManyFused))
           product(std::true_type{}, Some{});
-        else if (fused)
-          product(std::true_type{}, Many{});
-        else if (eight)
+        else if (!fused && (eight || !kMany))
           product(std::false_type{}, Some{});
-        else
-          product(std::false_type{}, Many{});
+        else if (fused) {
+          if constexpr (kManyFused) product(std::true_type{}, Many{});
+        } else {
+          if constexpr (kMany) product(std::false_type{}, Many{});
+        }
       }
       if (opt->timing) FEM_HIP(hipEventRecord(ev.e[4 * m + 2], s));
       const int sumA = gA <= kSumParts ? gA : 0;

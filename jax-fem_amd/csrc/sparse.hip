@@ -640,11 +640,16 @@ int fem_spmv(const fem_pattern_t* pat, int32_t precision, int32_t form, const vo
     // 100^3 66 / 68 and 54 / 64.
     using Some = std::integral_constant<int, 8>;
     using Many = std::integral_constant<int, SliceCfg<T>::W>;
-    const bool some = V > 1 || long_rows(*pat);
+    auto go = [&](auto diff) {
+      if constexpr (V == 1) {
+        if (!long_rows(*pat)) return product(diff, Many{});
+      }
+      product(diff, Some{});
+    };
     if (form == FEM_FORM_DIFFERENCE)
-      some ? product(std::true_type{}, Some{}) : product(std::true_type{}, Many{});
+      go(std::true_type{});
     else
-      some ? product(std::false_type{}, Some{}) : product(std::false_type{}, Many{});
+      go(std::false_type{});
     FEM_LAUNCHED();
     return FEM_OK;
   });

@@ -972,13 +972,20 @@ class DeviceProblem:
         self.fine = self._fine_operator(u) if ke_precision == _lib.FEM_F64 else None
         return self._law_finish(pending)
 
-    # Cells from which a solve's products run matrix-free, by the storage of the matrix they replace.
-    # One product at 28^3, 32^3, 40^3, 64^3 cells in us: elastic law, patches 9.9, 9.8, 12.5, 31;
-    # FP64 matrix 10.9, 13.8, 24, 97; FP32 matrix 6.6, 7.8, 12.9, 49.  Neo-Hookean patches 12.0, 12.2,
-    # 19, 65: faster than the FP64 matrix, slower than the FP32 one at every size.  The scalar Poisson
-    # matrix is read as fast as its cells are integrated (64^3: 19.2 against 19.6).
-    # HEX27, elastic law, 6^3, 8^3, 10^3, 24^3 cells: patches 13, 13, 13, 21; FP64 matrix 15, 23, 30,
-    # 150; FP32 matrix 8.7, 12, 15, 72.
+    # Cells from which a solve's products run matrix-free, by the storage of the matrix they replace:
+    # one line for both solvers.  us per iteration with patches / with the matrix (Jacobi-PCG, then
+    # AMG-CG), SIMP law:
+    #   HEX8 FP64    21,952 cells 17.0 / 17.2, 136 / 149;  24,389  17.0 / 17.6, 136 / 151;  32,768
+    #                17.6 / 22.9, 159 / 184;  64,000  22.7 / 34.7, 191 / 257
+    #   HEX8 FP32    32,768  18.6 / 16.7, 151 / 163;  50,653  21.3 / 20.3, 168 / 186;  64,000
+    #                20.8 / 23.4, 172 / 206
+    #   HEX27 FP64   125  20.5 / 22.7, 100 / 122;  343  21.8 / 22.7, 104 / 126;  1,000  21.5 / 25.5, 104 / 138
+    #   HEX27 FP32   1,000  20.2 / 16.1, 102 / 129;  1,728  21.1 / 20.5, 162 / 191;  2,744  21.1 / 27.0,
+    #                166 / 257
+    # In FP32 AMG-CG gains below the line and Jacobi-PCG only some way above it.  Neo-Hookean HEX8
+    # in FP64: 24,389  20.4 / 18.0, 164 / 162;  32,768  21.1 / 22.9, 170 / 183;  its cells take longer than
+    # the FP32 matrix at every size (64^3 product 65 us against 49).  The scalar Poisson matrix is read
+    # as fast as its cells are integrated (64^3 product: 19.2 us against 19.6).
     PATCH_MIN_CELLS = {(8, _lib.FEM_F64): 24000, (8, _lib.FEM_F32): 48000,
                        (27, _lib.FEM_F64): 250, (27, _lib.FEM_F32): 1000}
 
